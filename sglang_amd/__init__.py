@@ -7,5 +7,6 @@ Modules:
   fused_moe   - block-FP8 fused-experts pipeline
 """
 from . import _lib  # noqa: F401  (fails loudly when the HIP library is not built)
+from . import _host  # noqa: F401  (likewise for the native side of the layer-level calls)
 
 __all__ = ["sgl_kernel", "fp8_kernel", "fp8_utils", "fused_moe"]

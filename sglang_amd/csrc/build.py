@@ -1,4 +1,5 @@
-"""Build libfp8k.so (hand-written HIP kernels for gfx950 + the C ABI) in-tree with hipcc.
+"""Build libfp8k.so (hand-written HIP kernels for gfx950 + the C ABI) in-tree with hipcc, and _host.so (the native side of
+the layer-level calls, a CPython extension over it) with the host compiler.
 
 Usage: python sglang_amd/csrc/build.py [--force] [--jobs N]
 Each .hip file is compiled to an object next to it and linked into sglang_amd/csrc/libfp8k.so.
@@ -14,6 +15,8 @@ from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB = os.path.join(HERE, "libfp8k.so")
+HOST_SRC = "host.cpp"
+HOST = os.path.join(os.path.dirname(HERE), "_host.so")  # the extension module sglang_amd._host, linked against LIB
 SOURCES = ["api.hip", "quant.hip", "gemm.hip", "moe.hip", "tune.hip"]
 HEADERS = ["fp8k_common.h", "quant_math.h", "gemm_kernels.h", "gemm_direct.h", "gemm_moe256.h", "gemm_tile128.h", os.path.join("..", "..", "include", "fp8k.h"),
            os.path.join("..", "..", "include", "fp8k_tune.h")]
@@ -54,6 +57,22 @@ def _run(cmd: list[str]) -> None:
         sys.stderr.write(err + "\n")
 
 
+def _host_command() -> list[str]:
+    """Host code only: the native side of the layer-level calls, against torch's C++ API."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+           sysconfig.get_paths()["include"]]
+    return [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-Wno-deprecated-declarations"] + [
+        "-isystem" + d for d in inc] + [HOST_SRC, "-o", HOST, "-L" + HERE, "-lfp8k", "-L" + os.path.join(root, "lib"),
+                                        "-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lc10",
+                                        "-Wl,-rpath,$ORIGIN/csrc"]
+
+
 def build(force: bool = False, jobs: int = 4, verbose: bool = True) -> str:
     cc = hipcc()
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(HERE, s))]
@@ -73,6 +92,10 @@ def build(force: bool = False, jobs: int = 4, verbose: bool = True) -> str:
         _run([cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
         if verbose:
             print("[fp8k] linked", LIB, flush=True)
+    if force or _stale(HOST, [os.path.join(HERE, HOST_SRC), os.path.abspath(__file__), hdrs[-2]]):
+        _run(_host_command())
+        if verbose:
+            print("[fp8k] linked", HOST, flush=True)
     return LIB
 
 

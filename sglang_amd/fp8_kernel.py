@@ -9,6 +9,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
+from . import _host
 from . import custom_ops as _ops
 from . import sgl_kernel as _k
 
@@ -58,6 +59,10 @@ def sglang_per_token_group_quant_fp8(
     enable_v2: Optional[bool] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """Reference: fp8_kernel.py:481-531."""
+    if masked_m is None and not torch.compiler.is_compiling():
+        done = _host.group_quant(x, group_size, eps, column_major_scales, scale_tma_aligned, scale_ue8m0, fuse_silu_and_mul)
+        if done is not None:
+            return done
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
     out_shape = (*x.shape[:-1], x.shape[-1] // (2 if fuse_silu_and_mul else 1))
@@ -202,6 +207,10 @@ def per_tensor_quant_mla_fp8(x: torch.Tensor, x_s_out: torch.Tensor, eps: float 
     must be zero on entry (the maximum is accumulated atomically) and receives max(absmax, eps) / 448."""
     assert x.dim() == 3, "`x` is not a 3d-tensor"
     assert x_s_out.shape == (1,) and x_s_out.dtype == torch.float32 and x_s_out.device == x.device
+    if not torch.compiler.is_compiling():
+        x_q = _host.mla_quant(x, x_s_out, eps)
+        if x_q is not None:
+            return x_q, x_s_out
     x_q = x.new_empty(x.size(), dtype=fp8_dtype)
     if x.numel() > 0:
         _ops.tensor_quant_mla(x, x_q, x_s_out, eps)
@@ -258,6 +267,10 @@ def w8a8_block_fp8_matmul(
     exponents itself.  Packed activation scales next to ordinary float32 weight scales are expanded to floats and
     take the float-scale kernels: a float scale is never read as a bare exponent.
     """
+    if not torch.compiler.is_compiling():
+        out = _host.block_matmul(A, B, As, Bs, block_size, output_dtype, As.dtype == torch.int32 and _k.is_ue8m0(Bs))
+        if out is not None:
+            return out
     assert len(block_size) == 2
     block_n, block_k = block_size
     if block_n != 128 or block_k != 128:

@@ -8,6 +8,7 @@ from typing import Callable, List, Optional, Tuple
 
 import torch
 
+from . import _host
 from . import custom_ops as _ops
 from .sgl_kernel import mark_ue8m0, unpack_ue8m0_weight_scales  # noqa: F401  (re-exported for weight loading)
 from .fp8_kernel import (
@@ -40,6 +41,10 @@ def w8a8_block_fp8_linear(
     With input_scale the input is e4m3fn already (quantised upstream in groups of block_size[1], scales float32
     [tokens, K/128] in any strides); the result is bf16, as in the reference.
     """
+    if input_scale is None and not torch.compiler.is_compiling():
+        output = _host.block_linear(input, weight, block_size, weight_scale, bias)
+        if output is not None:
+            return output
     input_2d = input.view(-1, input.shape[-1])
     output_shape = [*input.shape[:-1], weight.shape[0]]
     if input_scale is not None:
@@ -79,6 +84,10 @@ def apply_fp8_linear(
     (numel 1) or per channel (numel N).  Static per-tensor activation scale when input_scale is
     given, else dynamic per-token (or per-tensor) quantisation.
     """
+    if input_scale is None and not torch.compiler.is_compiling():
+        output = _host.token_linear(input, weight, weight_scale, bias, use_per_token_if_dynamic)
+        if output is not None:
+            return output
     input_2d = input.view(-1, input.shape[-1])
     N = weight.shape[1]
     output_shape = [*input.shape[:-1], N]

@@ -19,6 +19,7 @@ from typing import Any, Dict, List, Optional, Tuple
 
 import torch
 
+from . import _host
 from . import custom_ops as _ops
 from .fp8_kernel import sglang_per_token_group_quant_fp8
 
@@ -199,6 +200,16 @@ def fused_experts_impl(
     num_tokens, _ = hidden_states.shape
     E, N, _ = w1.shape
     topk = topk_ids.shape[1]
+    if 0 < num_tokens <= CHUNK_SIZE and activation == "silu" and is_gated and not no_combine and not torch.compiler.is_compiling() \
+            and list(block_shape) == [128, 128]:
+        config = get_default_config(num_tokens, E, topk)
+        out = _host.fused_experts(
+            hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, topk_ids, config["BLOCK_SIZE_M"],
+            blocks_want_balancing(config, num_tokens * topk, E),
+            gemm1_fuses_activation(config, N) and not apply_router_weight_on_input, apply_router_weight_on_input,
+            1.0 if routed_scaling_factor is None else float(routed_scaling_factor), inplace)
+        if out is not None:
+            return out
     M = min(num_tokens, CHUNK_SIZE)
     dev, dt = hidden_states.device, hidden_states.dtype
     if topk_weights.dtype != torch.float32:
@@ -300,6 +311,7 @@ def biased_grouped_topk(
     groups, renormalised weights); where the reference falls back to tensor ops for other shapes, this path has no
     second implementation and raises."""
     experts = gating_output.shape[1]
+    scaling = float(routed_scaling_factor) if routed_scaling_factor is not None else 0.0
     fits = (
         renormalize and num_expert_group and topk_group and experts & (experts - 1) == 0
         and experts % num_expert_group == 0 and experts // num_expert_group <= 32 and num_expert_group <= 64
@@ -309,8 +321,12 @@ def biased_grouped_topk(
             "biased_grouped_topk: built for renormalised weights, a power-of-two expert count, at most 32 experts per "
             "group and at most 64 groups (got %d experts, %s groups, renormalize=%s)" % (experts, num_expert_group, renormalize))
     assert hidden_states.shape[0] == gating_output.shape[0], "Number of tokens mismatch"
+    if not torch.compiler.is_compiling():
+        routed = _host.fused_gate(gating_output, correction_bias, num_expert_group, topk_group, topk, num_fused_shared_experts,
+                                  scaling, apply_routed_scaling_factor_on_output)
+        if routed is not None:
+            return routed
     return _ops.moe_fused_gate(
         gating_output.contiguous(), correction_bias.to(gating_output.dtype).contiguous(), num_expert_group, topk_group,
-        topk, num_fused_shared_experts, routed_scaling_factor if routed_scaling_factor is not None else 0.0,
-        apply_routed_scaling_factor_on_output,
+        topk, num_fused_shared_experts, scaling, apply_routed_scaling_factor_on_output,
     )

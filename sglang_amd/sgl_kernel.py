@@ -13,7 +13,7 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _host, _lib
 from ._lib import check, dtype_code, lib, require_cuda, stream_ptr
 
 FP8_DTYPE = torch.float8_e4m3fn
@@ -44,6 +44,9 @@ def _workspace(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
         buf = torch.empty(size, dtype=torch.uint8, device=device)
         _workspaces[key] = buf
     return buf
+
+
+_host.set_workspace(_workspaces, _workspace)  # native calls look their stream's buffer up in the same registry
 
 
 def reserve_workspace(device: torch.device, nbytes: int) -> None:
@@ -347,6 +350,10 @@ def bmm_fp8(A: torch.Tensor, B: torch.Tensor, A_scale: torch.Tensor, B_scale: to
     contiguous, B e4m3fn [b, k, n] column-major per entry (k contiguous: a [b, n, k] weight transposed), one float32
     scale per operand; returns / fills out [b, m, n] = (A @ B) * A_scale * B_scale in `dtype`.  No host synchronisation:
     the scalar scales are broadcast to vectors on the device."""
+    if out is None and not torch.compiler.is_compiling():
+        out = _host.bmm(A, B, A_scale, B_scale, dtype)
+        if out is not None:
+            return out
     require_cuda(A, B, A_scale, B_scale, out)
     if A.dim() != 3 or B.dim() != 3 or A.shape[0] != B.shape[0] or A.shape[2] != B.shape[1]:
         raise RuntimeError("bmm_fp8: A [b, m, k] and B [b, k, n] expected")

@@ -1,0 +1,128 @@
+"""The native calls behind the layer-level entry points (sglang_amd._host).
+
+They must decline - return None before launching anything - whatever they do not take as it is, so that the dispatcher path
+decides; and where they do take a call, its result is that of the dispatcher path, bit for bit.
+"""
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+from sglang_amd import _host, fp8_kernel, fp8_utils, fused_moe, sgl_kernel
+
+BLOCK = [128, 128]
+
+
+def test_declines_what_it_does_not_take():
+    x, w, s = torch.zeros((4, 256), dtype=torch.bfloat16), torch.zeros((128, 256), dtype=torch.float8_e4m3fn), torch.ones((1, 2))
+    assert _host.block_linear(x, w, BLOCK, s, None) is None  # host memory
+    assert _host.group_quant(x, 128, 1e-10, False, False, False, False) is None
+    assert _host.token_linear(x, w.t(), torch.ones(128), None, True) is None
+    assert _host.block_linear(None, w, BLOCK, s, None) is None
+    with FakeTensorMode():
+        f = torch.empty((4, 256), dtype=torch.bfloat16, device="cuda")
+        fw = torch.empty((128, 256), dtype=torch.float8_e4m3fn, device="cuda")
+        assert _host.block_linear(f, fw, BLOCK, torch.empty((1, 2), device="cuda"), None) is None
+        assert _host.group_quant(f, 128, 1e-10, False, False, False, False) is None
+
+
+@pytest.fixture
+def dispatcher(monkeypatch):
+    """Calls fn() with every native call declining."""
+
+    def call(fn):
+        with monkeypatch.context() as m:
+            for name in ("group_quant", "block_linear", "block_matmul", "token_linear", "mla_quant", "bmm", "fused_gate", "fused_experts"):
+                assert hasattr(_host, name)
+                m.setattr(_host, name, lambda *a: None)
+            return fn()
+
+    return call
+
+
+def _same(a, b):
+    if isinstance(a, tuple):
+        return len(a) == len(b) and all(_same(x, y) for x, y in zip(a, b))
+    if a.dtype == torch.float8_e4m3fn:
+        a, b = a.view(torch.uint8), b.view(torch.uint8)
+    return a.shape == b.shape and a.stride() == b.stride() and a.dtype == b.dtype and torch.equal(a, b)
+
+
+def _randn(shape, dtype=torch.bfloat16, seed=0):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+
+
+def _weight(n, k, seed=1):
+    return fp8_utils.per_block_cast_to_fp8(_randn((n, k), torch.float32, seed) * 0.02)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 128, 128), (3, 264, 512), (33, 640, 1536), (300, 72, 256), (700, 1000, 384)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linears_are_the_dispatcher_path(dev, dispatcher, m, n, k, dtype):
+    x, (w, s), bias = _randn((m, k), dtype), _weight(n, k), _randn((n,), dtype, 2)
+    for b in (None, bias):
+        def block():
+            return fp8_utils.w8a8_block_fp8_linear(x, w, BLOCK, s, bias=b)
+
+        assert _host.block_linear(x, w, BLOCK, s, b) is not None
+        assert _same(block(), dispatcher(block))
+        for scale in (torch.rand((n, 1), device=dev) * 1e-2, torch.full((1,), 3e-3, device=dev)):
+            def token():
+                return fp8_utils.apply_fp8_linear(x, w.t(), scale, bias=b, use_per_token_if_dynamic=True)
+
+            assert _host.token_linear(x, w.t(), scale, b, True) is not None
+            assert _same(token(), dispatcher(token))
+    q, xs = fp8_kernel.sglang_per_token_group_quant_fp8(x, 128)
+    matmul = lambda: fp8_kernel.w8a8_block_fp8_matmul(q, w, xs, s, BLOCK, dtype)  # noqa: E731
+    assert _same(matmul(), dispatcher(matmul))
+    qp, xp = fp8_kernel.sglang_per_token_group_quant_fp8(x, 128, column_major_scales=True, scale_tma_aligned=True, scale_ue8m0=True)
+    sgl_kernel.mark_ue8m0(s)
+    packed = lambda: fp8_kernel.w8a8_block_fp8_matmul(qp, w, xp, s, BLOCK, dtype)  # noqa: E731
+    assert (_host.block_matmul(qp, w, xp, s, BLOCK, dtype, True) is not None) == (m > 128)
+    assert _same(packed(), dispatcher(packed))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k", [(1, 128), (5, 640), (130, 7168)])
+def test_group_quant_layouts_are_the_dispatcher_path(dev, dispatcher, m, k):
+    x = _randn((m, k))
+    for kw in ({}, dict(column_major_scales=True), dict(column_major_scales=True, scale_tma_aligned=True),
+               dict(column_major_scales=True, scale_tma_aligned=True, scale_ue8m0=True), dict(fuse_silu_and_mul=True)):
+        if k % 256 and "fuse_silu_and_mul" in kw:
+            continue
+        quant = lambda: fp8_kernel.sglang_per_token_group_quant_fp8(x, 128, **kw)  # noqa: E731
+        assert _same(quant(), dispatcher(quant))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,m,k,n", [(4, 1, 128, 512), (16, 37, 512, 128), (3, 130, 128, 264)])
+def test_mla_products_are_the_dispatcher_path(dev, dispatcher, heads, m, k, n):
+    x = _randn((m, heads, k)).transpose(0, 1)
+    w, ws = fp8_utils.input_to_float8(_randn((heads, n, k), seed=3))
+
+    def product():
+        q, s = fp8_kernel.per_tensor_quant_mla_fp8(x, torch.zeros((1,), device=dev))
+        return q, s, sgl_kernel.bmm_fp8(q, w.transpose(1, 2), s, ws, torch.bfloat16)
+
+    assert _same(product(), dispatcher(product))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [1, 20, 100, 700])
+def test_experts_are_the_dispatcher_path(dev, dispatcher, tokens):
+    E, H, inter, topk = 16, 512, 256, 4
+    x = _randn((tokens, H))
+    parts = [[_weight(n, k, 10 * e + n) for e in range(E)] for n, k in ((2 * inter, H), (H, inter))]
+    (w13, s13), (w2, s2) = [(torch.stack([q for q, _ in p]), torch.stack([s for _, s in p])) for p in parts]
+    logits, bias = _randn((tokens, E), torch.float32, 7), _randn((E,), torch.float32, 8)
+
+    def layer(inplace, on_input=False):
+        tw, ids = fused_moe.biased_grouped_topk(x, logits, bias, topk, True, 4, 2)
+        h = x.clone() if inplace else x
+        out = fused_moe.fused_experts_impl(h, w13, w2, tw, ids, inplace=inplace, use_fp8_w8a8=True, w1_scale=s13, w2_scale=s2,
+                                           block_shape=BLOCK, routed_scaling_factor=2.5, apply_router_weight_on_input=on_input)
+        assert (out.data_ptr() == h.data_ptr()) == inplace
+        return tw, ids, out
+
+    for args in ((False,), (True,), (False, True)):
+        assert _same(layer(*args), dispatcher(lambda: layer(*args)))
