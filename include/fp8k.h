@@ -124,6 +124,16 @@ int fp8k_block_gemm(const void* A, const void* B, const float* As, const float* 
                     int64_t workspace_bytes, void* stream);
 
 /*
+ * fp8k_block_gemm followed by `+ bias` (the two statements of the reference's linear, fp8_utils.py:220-226), in the
+ * kernel's write-out: the product is rounded to out_dtype, then bias[n] (out_dtype, [N], may be NULL) is added in float32
+ * and the sum rounded again, so the result is the elementwise addition's bit for bit.
+ */
+int fp8k_block_gemm_bias(const void* A, const void* B, const float* As, const float* Bs, const void* bias, void* C,
+                         int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t as_stride_m,
+                         int64_t as_stride_k, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, int out_dtype,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * The same product with power-of-two scales that the matrix core applies itself (no float promote per K block):
  * As_packed int32 words of four UE8M0 exponent bytes, as fp8k_group_quant writes them with FP8K_SCALE_UE8M0_PACKED
  * (row m, K blocks 4j..4j+3 in the word at As_packed[m*as_stride_m + j*as_stride_w]); Bs float32, every value a power of
@@ -165,6 +175,14 @@ int fp8k_block_gemm_noalloc(const void* A, const void* B, const float* As, const
 int fp8k_scaled_mm(const void* A, const void* B, const float* sa, const float* sb, const void* bias, void* C,
                    int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int out_dtype,
                    int bias_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+/*
+ * fp8k_scaled_mm with strides for the two scale vectors: 1 as above, 0 for one scale that holds for every row / column
+ * (a per-tensor scale needs no broadcast copy).  Same workspace.
+ */
+int fp8k_scaled_mm_strided(const void* A, const void* B, const float* sa, int64_t sa_stride, const float* sb,
+                           int64_t sb_stride, const void* bias, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
+                           int64_t ldb, int64_t ldc, int out_dtype, int bias_dtype, void* workspace,
+                           int64_t workspace_bytes, void* stream);
 int64_t fp8k_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
@@ -187,6 +205,10 @@ int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H, int64_t S
  * K % 128 == 0, N % 8 == 0, batch <= 65535.  No workspace.
  */
 int fp8k_bmm_fp8(const void* A, const void* B, const float* sa, const float* sb, void* C, int64_t batch, int64_t M,
+                 int64_t N, int64_t K, int64_t a_stride_b, int64_t lda, int64_t b_stride_b, int64_t ldb,
+                 int64_t c_stride_b, int64_t ldc, int out_dtype, void* stream);
+/* The same with sa and sb pointing at one float each (the op's own per-tensor scales, no broadcast). */
+int fp8k_bmm_fp8_tensor_scales(const void* A, const void* B, const float* sa, const float* sb, void* C, int64_t batch, int64_t M,
                  int64_t N, int64_t K, int64_t a_stride_b, int64_t lda, int64_t b_stride_b, int64_t ldb,
                  int64_t c_stride_b, int64_t ldc, int out_dtype, void* stream);
 

@@ -46,6 +46,7 @@ SIGNATURES = {
     "fp8k_tensor_quant": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_ptr]),
     "fp8k_tensor_quant_mla": (_c_int, [_c_ptr, _c_ptr, _c_ptr] + [_c_i64] * 5 + [_c_f32, _c_int, _c_ptr]),
     "fp8k_bmm_fp8": (_c_int, [_c_ptr] * 5 + [_c_i64] * 10 + [_c_int, _c_ptr]),
+    "fp8k_bmm_fp8_tensor_scales": (_c_int, [_c_ptr] * 5 + [_c_i64] * 10 + [_c_int, _c_ptr]),
     "fp8k_moe_prepare_input": (_c_int, [_c_ptr] + [_c_i64] * 5 + [_c_ptr] * 7),
     "fp8k_shuffle_rows": (_c_int, [_c_ptr] * 3 + [_c_i64] * 3 + [_c_ptr]),
     "fp8k_apply_shuffle_mul_sum": (_c_int, [_c_ptr] * 4 + [_c_i64] * 4 + [_c_int, _c_ptr]),
@@ -56,6 +57,10 @@ SIGNATURES = {
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr] + [_c_i64] * 10 + [_c_int, _c_ptr, _c_i64, _c_ptr],
     ),
+    "fp8k_block_gemm_bias": (
+        _c_int,
+        [_c_ptr] * 6 + [_c_i64] * 10 + [_c_int, _c_ptr, _c_i64, _c_ptr],
+    ),
     "fp8k_block_gemm_ue8m0": (
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr] + [_c_i64] * 10 + [_c_int, _c_ptr, _c_i64, _c_ptr],
@@ -65,6 +70,10 @@ SIGNATURES = {
     "fp8k_scaled_mm": (
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr] + [_c_i64] * 6 + [_c_int, _c_int, _c_ptr, _c_i64, _c_ptr],
+    ),
+    "fp8k_scaled_mm_strided": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr] + [_c_i64] * 6 + [_c_int, _c_int, _c_ptr, _c_i64, _c_ptr],
     ),
     "fp8k_scaled_mm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "fp8k_tune_force_gemm_plan": (None, [_c_int, _c_int]),

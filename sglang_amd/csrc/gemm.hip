@@ -380,7 +380,7 @@ extern "C" void fp8k_tune_force_gemm_plan(int kind, int splits) {
 extern "C" int64_t fp8k_block_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) { return block_gemm_workspace_bytes(M, N, K); }
 extern "C" int64_t fp8k_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) { return workspace_bytes(M, N, K); }
 
-static int block_gemm_impl(const void* A, const void* B, const float* As, const float* Bs, void* C, int64_t M, int64_t N,
+static int block_gemm_impl(const void* A, const void* B, const float* As, const float* Bs, const void* bias, void* C, int64_t M, int64_t N,
                            int64_t K, int64_t lda, int64_t ldb, int64_t as_stride_m, int64_t as_stride_k,
                            int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, int out_dtype, void* workspace,
                            int64_t workspace_bytes_given, void* stream) {
@@ -400,7 +400,7 @@ static int block_gemm_impl(const void* A, const void* B, const float* As, const 
     return fail(FP8K_ERR_WORKSPACE, "fp8_blockwise_scaled_mm: workspace of %lld bytes required, %lld given",
                 (long long)need, (long long)(workspace ? workspace_bytes_given : 0));
   GemmArgs a{};
-  a.X = (const uint8_t*)A; a.W = (const uint8_t*)B; a.sx = As; a.sw = Bs; a.bias = nullptr; a.C = C;
+  a.X = (const uint8_t*)A; a.W = (const uint8_t*)B; a.sx = As; a.sw = Bs; a.bias = bias; a.C = C;
   a.partial = (float*)workspace;
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = lda; a.ldw = ldb; a.ldc = ldc;
   a.sx_m = as_stride_m; a.sx_k = as_stride_k; a.sw_n = bs_stride_n; a.sw_k = bs_stride_k;
@@ -413,8 +413,8 @@ static int block_gemm_impl(const void* A, const void* B, const float* As, const 
     if (rc) return rc;
     a.sx = cm; a.sx_m = 1; a.sx_k = M;
   }
-  return out_dtype == FP8K_BF16 ? launch<kModeBlock, FP8K_BF16, FP8K_F32>(a, pl, st)
-                                : launch<kModeBlock, FP8K_F16, FP8K_F32>(a, pl, st);
+  return out_dtype == FP8K_BF16 ? launch<kModeBlock, FP8K_BF16, FP8K_BF16>(a, pl, st)
+                                : launch<kModeBlock, FP8K_F16, FP8K_F16>(a, pl, st);
 }
 
 extern "C" int fp8k_block_gemm(const void* A, const void* B, const float* As, const float* Bs, void* C, int64_t M,
@@ -422,7 +422,16 @@ extern "C" int fp8k_block_gemm(const void* A, const void* B, const float* As, co
                                int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, int out_dtype, void* workspace,
                                int64_t workspace_bytes_given, void* stream) {
   clear_error();
-  return block_gemm_impl(A, B, As, Bs, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
+  return block_gemm_impl(A, B, As, Bs, nullptr, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
+                         out_dtype, workspace, workspace_bytes_given, stream);
+}
+
+extern "C" int fp8k_block_gemm_bias(const void* A, const void* B, const float* As, const float* Bs, const void* bias, void* C,
+                                    int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t as_stride_m,
+                                    int64_t as_stride_k, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, int out_dtype,
+                                    void* workspace, int64_t workspace_bytes_given, void* stream) {
+  clear_error();
+  return block_gemm_impl(A, B, As, Bs, bias, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
                          out_dtype, workspace, workspace_bytes_given, stream);
 }
 
@@ -483,7 +492,7 @@ extern "C" int fp8k_block_gemm_noalloc(const void* A, const void* B, const float
   }
   // nothing in the buffer has to start at zero: every float partial and every copied scale that a launch reads was
   // written by the same call
-  return block_gemm_impl(A, B, As, Bs, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
+  return block_gemm_impl(A, B, As, Bs, nullptr, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
                          out_dtype, ws, need > 0 ? kStaticScratchBytes : 0, stream);
 }
 
@@ -522,13 +531,22 @@ extern "C" int fp8k_block_gemm_ue8m0(const void* A, const void* B, const int32_t
 extern "C" int fp8k_scaled_mm(const void* A, const void* B, const float* sa, const float* sb, const void* bias, void* C,
                               int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int out_dtype,
                               int bias_dtype, void* workspace, int64_t workspace_bytes_given, void* stream) {
+  return fp8k_scaled_mm_strided(A, B, sa, 1, sb, 1, bias, C, M, N, K, lda, ldb, ldc, out_dtype, bias_dtype, workspace,
+                                workspace_bytes_given, stream);
+}
+
+extern "C" int fp8k_scaled_mm_strided(const void* A, const void* B, const float* sa, int64_t sa_stride, const float* sb,
+                                      int64_t sb_stride, const void* bias, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
+                                      int64_t ldb, int64_t ldc, int out_dtype, int bias_dtype, void* workspace,
+                                      int64_t workspace_bytes_given, void* stream) {
   clear_error();
   int rc = common_checks("fp8_scaled_mm", A, B, C, M, N, K, lda, ldb, ldc, out_dtype);
   if (rc) return rc;
   if (M == 0 || N == 0) return FP8K_OK;
   FP8K_REQUIRE(K > 0, "fp8_scaled_mm: K must be positive");
   FP8K_REQUIRE(sa && sb, "fp8_scaled_mm: null scale pointer");
-  FP8K_REQUIRE(aligned(sb, 16), "fp8_scaled_mm: scales_b must be 16-byte aligned");
+  FP8K_REQUIRE((sa_stride == 0 || sa_stride == 1) && (sb_stride == 0 || sb_stride == 1), "fp8_scaled_mm: scale strides must be 0 or 1");
+  FP8K_REQUIRE(sb_stride == 0 || aligned(sb, 16), "fp8_scaled_mm: scales_b must be 16-byte aligned");
   if (bias)
     FP8K_REQUIRE(bias_dtype == FP8K_F32 || bias_dtype == FP8K_F16 || bias_dtype == FP8K_BF16,
                  "fp8_scaled_mm: bias dtype must be float32, float16 or bfloat16");
@@ -541,6 +559,7 @@ extern "C" int fp8k_scaled_mm(const void* A, const void* B, const float* sa, con
   a.X = (const uint8_t*)A; a.W = (const uint8_t*)B; a.sx = sa; a.sw = sb; a.bias = bias; a.C = C;
   a.partial = (float*)workspace;
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = lda; a.ldw = ldb; a.ldc = ldc;
+  a.sx_m = sa_stride; a.sw_n = sb_stride;
   hipStream_t st = (hipStream_t)stream;
   const int bd = bias ? bias_dtype : FP8K_F32;
 #define FP8K_SMM(O, B) launch<kModeRow, O, B>(a, pl, st)
@@ -557,9 +576,9 @@ extern "C" int fp8k_scaled_mm(const void* A, const void* B, const float* sa, con
 
 // ---- batched per-tensor-scaled FP8 GEMM (the MLA absorbed products): every batch entry is a row-mode GEMM on the
 // 128x128 tile kernel (grid y = entry), whose per-row / per-column scale vectors are shared by all entries.
-extern "C" int fp8k_bmm_fp8(const void* A, const void* B, const float* sa, const float* sb, void* C, int64_t batch, int64_t M,
-                            int64_t N, int64_t K, int64_t a_stride_b, int64_t lda, int64_t b_stride_b, int64_t ldb,
-                            int64_t c_stride_b, int64_t ldc, int out_dtype, void* stream) {
+static int bmm_impl(const void* A, const void* B, const float* sa, const float* sb, int64_t scale_stride, void* C, int64_t batch,
+                    int64_t M, int64_t N, int64_t K, int64_t a_stride_b, int64_t lda, int64_t b_stride_b, int64_t ldb,
+                    int64_t c_stride_b, int64_t ldc, int out_dtype, void* stream) {
   clear_error();
   const char* op = "bmm_fp8";
   int rc = common_checks(op, A, B, C, M, N, K, lda, ldb, ldc, out_dtype);
@@ -569,12 +588,13 @@ extern "C" int fp8k_bmm_fp8(const void* A, const void* B, const float* sa, const
   FP8K_REQUIRE(K > 0 && K % kTileK == 0, "%s: K must be a positive multiple of 128 (got %lld)", op, (long long)K);
   FP8K_REQUIRE(N % 8 == 0, "%s: N must be a multiple of 8 (got %lld)", op, (long long)N);
   FP8K_REQUIRE(sa && sb, "%s: null scale pointer", op);
-  FP8K_REQUIRE(aligned(sb, 16), "%s: the column scale vector must be 16-byte aligned", op);
+  FP8K_REQUIRE(scale_stride == 0 || aligned(sb, 16), "%s: the column scale vector must be 16-byte aligned", op);
   FP8K_REQUIRE(a_stride_b % 16 == 0 && b_stride_b % 16 == 0 && (c_stride_b * 2) % 16 == 0 && a_stride_b >= 0 && b_stride_b >= 0 &&
                c_stride_b >= 0, "%s: batch strides must be non-negative multiples of 16 bytes", op);
   GemmArgs a{};
   a.X = (const uint8_t*)A; a.W = (const uint8_t*)B; a.sx = sa; a.sw = sb; a.bias = nullptr; a.C = C; a.partial = nullptr;
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = lda; a.ldw = ldb; a.ldc = ldc;
+  a.sx_m = a.sw_n = scale_stride;
   a.batch_x = a_stride_b; a.batch_w = b_stride_b; a.batch_c = c_stride_b;
   a.tiles_m = (int)((M + kT128 - 1) / kT128);
   a.tiles_n = (int)((N + kT128 - 1) / kT128);
@@ -587,4 +607,16 @@ extern "C" int fp8k_bmm_fp8(const void* A, const void* B, const float* sa, const
   else
     hipLaunchKernelGGL((gemm_tile128_kernel<kModeRow, FP8K_F16, FP8K_F32, false>), dim3(nwg, (unsigned)batch), dim3(512), 0, st, a);
   return check_launch(op);
+}
+
+extern "C" int fp8k_bmm_fp8(const void* A, const void* B, const float* sa, const float* sb, void* C, int64_t batch, int64_t M,
+                            int64_t N, int64_t K, int64_t a_stride_b, int64_t lda, int64_t b_stride_b, int64_t ldb,
+                            int64_t c_stride_b, int64_t ldc, int out_dtype, void* stream) {
+  return bmm_impl(A, B, sa, sb, 1, C, batch, M, N, K, a_stride_b, lda, b_stride_b, ldb, c_stride_b, ldc, out_dtype, stream);
+}
+
+extern "C" int fp8k_bmm_fp8_tensor_scales(const void* A, const void* B, const float* sa, const float* sb, void* C, int64_t batch,
+                                          int64_t M, int64_t N, int64_t K, int64_t a_stride_b, int64_t lda, int64_t b_stride_b,
+                                          int64_t ldb, int64_t c_stride_b, int64_t ldc, int out_dtype, void* stream) {
+  return bmm_impl(A, B, sa, sb, 0, C, batch, M, N, K, a_stride_b, lda, b_stride_b, ldb, c_stride_b, ldc, out_dtype, stream);
 }

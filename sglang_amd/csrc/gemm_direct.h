@@ -250,15 +250,9 @@ __global__ __launch_bounds__(512, 2) void gemm_direct_kernel(const GemmArgs p) {
       *reinterpret_cast<float4*>(p.partial + ((int64_t)split * p.M + orow) * p.N + n) = make_float4(v[0], v[1], v[2], v[3]);
       continue;
     }
-    if (MODE == kModeRow) {
-      const float sa = p.sx[orow];
-      const float4 sb = *reinterpret_cast<const float4*>(p.sw + n);
-      v[0] = v[0] * sb.x * sa; v[1] = v[1] * sb.y * sa; v[2] = v[2] * sb.z * sa; v[3] = v[3] * sb.w * sa;
-      if (p.bias) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] += load_scalar<BIAS_DT>(p.bias, n + i);
-      }
-    } else if (MOE && p.topk_w) {
+    if (!MOE) {
+      finish4<MODE, OUT_DT, BIAS_DT>(p, n, MODE == kModeRow ? row_scale(p, orow) : 1.f, v);
+    } else if (p.topk_w) {
       const float tw = p.topk_w[orow];
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] *= tw;
@@ -397,15 +391,7 @@ __global__ __launch_bounds__(512, 2) void gemm_wavek_kernel(const GemmArgs p) {
       s[0] += o[0]; s[1] += o[1]; s[2] += o[2]; s[3] += o[3];
     }
     float v[4] = {s[0], s[1], s[2], s[3]};
-    if (MODE == kModeRow) {
-      const float sa = p.sx[m];
-      const float4 sb = *reinterpret_cast<const float4*>(p.sw + n);
-      v[0] = v[0] * sb.x * sa; v[1] = v[1] * sb.y * sa; v[2] = v[2] * sb.z * sa; v[3] = v[3] * sb.w * sa;
-      if (p.bias) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] += load_scalar<BIAS_DT>(p.bias, n + i);
-      }
-    }
+    finish4<MODE, OUT_DT, BIAS_DT>(p, n, MODE == kModeRow ? row_scale(p, m) : 1.f, v);
     store4<OUT_DT>(p.C, (int64_t)m * p.ldc + n, v[0], v[1], v[2], v[3]);
   }
 }

@@ -16,9 +16,9 @@ namespace fp8k {
 struct GemmArgs {
   const uint8_t* X;   // [M,K]
   const uint8_t* W;   // [N,K]
-  const float* sx;    // block mode: as[m*sx_m + kb*sx_k]; row mode: sa[m]
-  const float* sw;    // block mode: bs[nb*sw_n + kb*sw_k]; row mode: sb[n]
-  const void* bias;   // row mode only, may be null
+  const float* sx;    // block mode: as[m*sx_m + kb*sx_k]; row mode: sa[m*sx_m] (sx_m 0: one scale for all rows)
+  const float* sw;    // block mode: bs[nb*sw_n + kb*sw_k]; row mode: sb[n*sw_n] (sw_n 0: one scale for all columns)
+  const void* bias;   // row and block mode, may be null
   void* C;            // [M,N]
   float* partial;     // split-K workspace [splits][M][N] float, or null
   int M, N, K;
@@ -91,6 +91,106 @@ __device__ __forceinline__ float load_scalar(const void* p, int64_t i) {
   if (DT == FP8K_F32) return ((const float*)p)[i];
   if (DT == FP8K_BF16) return __uint_as_float((uint32_t)((const u16*)p)[i] << 16);
   return f16_bits_to_f32(((const u16*)p)[i]);
+}
+
+// Four values of output row m (columns n .. n+3, n < p.N) on their way out: row mode multiplies by the column scales and the
+// row's scale `sa` and adds the bias in float32; block mode, whose bias is the elementwise addition that follows the product,
+// rounds to the output type first, so that the result is the two-step one bit for bit.  (As a separate pass over the output
+// the addition took 18.8 us of a 71 us linear at M = 1000, N = 24576.)
+template <int DT>
+__device__ __forceinline__ void load_bias4(const void* bias, int64_t n, float (&b)[4]) {
+  if (DT == FP8K_F32 && (reinterpret_cast<uintptr_t>(bias) & 15) == 0) {
+    const float4 t = *reinterpret_cast<const float4*>((const float*)bias + n);
+    b[0] = t.x; b[1] = t.y; b[2] = t.z; b[3] = t.w;
+  } else if (DT != FP8K_F32 && (reinterpret_cast<uintptr_t>(bias) & 7) == 0) {
+    const uint2 t = *reinterpret_cast<const uint2*>((const u16*)bias + n);
+    b[0] = DT == FP8K_BF16 ? bf16_lo(t.x) : f16_bits_to_f32(t.x & 0xffff);
+    b[1] = DT == FP8K_BF16 ? bf16_hi(t.x) : f16_bits_to_f32(t.x >> 16);
+    b[2] = DT == FP8K_BF16 ? bf16_lo(t.y) : f16_bits_to_f32(t.y & 0xffff);
+    b[3] = DT == FP8K_BF16 ? bf16_hi(t.y) : f16_bits_to_f32(t.y >> 16);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = load_scalar<DT>(bias, n + i);
+  }
+}
+__device__ __forceinline__ float row_scale(const GemmArgs& p, int64_t m) { return p.sx[m * p.sx_m]; }
+template <int MODE, int OUT_DT, int BIAS_DT>
+__device__ __forceinline__ void finish4(const GemmArgs& p, int n, float sa, float (&v)[4]) {
+  if (MODE == kModeRow) {
+    float4 sb;
+    if (p.sw_n) sb = *reinterpret_cast<const float4*>(p.sw + n);
+    else sb.x = sb.y = sb.z = sb.w = p.sw[0];
+    v[0] = v[0] * sb.x * sa; v[1] = v[1] * sb.y * sa; v[2] = v[2] * sb.z * sa; v[3] = v[3] * sb.w * sa;
+  }
+  if (MODE != kModeScaled && p.bias) {
+    float b[4];
+    load_bias4<BIAS_DT>(p.bias, n, b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (MODE == kModeBlock ? round_to<OUT_DT>(v[i]) : v[i]) + b[i];
+  }
+}
+
+// The same for the quads of a whole tile, whose accumulators stay where they are: every column scale of a lane is requested
+// before the first is used (Q quads of columns, each for R rows).  One load per value just ahead of its use cost a 256x256
+// tile 32 memory round trips in its write-out: 231 -> 214 us at M = 2048, N = 28672, K = 4096 with a bias.
+// col(j): first column of quad j; apply(j, r, q, f): f on the accumulator of column q of quad j in row r; sa[r]: that row's scale.
+template <int Q, int R, int BIAS_DT, class COL, class APPLY>
+__device__ __forceinline__ void finish_rows(const GemmArgs& p, const float (&sa)[R], COL col, APPLY apply) {
+  if (p.sw_n) {
+    float4 sb[Q];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) sb[j] = *reinterpret_cast<const float4*>(p.sw + min(col(j), p.N - 4));
+#pragma unroll
+    for (int j = 0; j < Q; ++j)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        apply(j, r, 0, [&](float v) { return v * sb[j].x * sa[r]; });
+        apply(j, r, 1, [&](float v) { return v * sb[j].y * sa[r]; });
+        apply(j, r, 2, [&](float v) { return v * sb[j].z * sa[r]; });
+        apply(j, r, 3, [&](float v) { return v * sb[j].w * sa[r]; });
+      }
+  } else {
+    const float sb = p.sw[0];
+#pragma unroll
+    for (int j = 0; j < Q; ++j)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) apply(j, r, q, [&](float v) { return v * sb * sa[r]; });
+  }
+  if (p.bias) {
+    float b[Q][4];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) load_bias4<BIAS_DT>(p.bias, min(col(j), p.N - 4), b[j]);
+#pragma unroll
+    for (int j = 0; j < Q; ++j)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) apply(j, r, q, [&](float v) { return v + b[j][q]; });
+  }
+}
+// Block mode's bias on eight 16-bit results that are about to be stored: `b` holds the lane's columns, loaded once per tile.
+template <int DT>
+__device__ __forceinline__ uint4 add_bias8(uint4 o, const float (&b)[8]) {
+  uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (DT == FP8K_BF16) {
+      w[i] = pack_bf16x2(bf16_lo(w[i]) + b[2 * i], bf16_hi(w[i]) + b[2 * i + 1]);
+    } else {
+      w[i] = f32_to_f16_bits(f16_bits_to_f32(w[i] & 0xffff) + b[2 * i]) | (f32_to_f16_bits(f16_bits_to_f32(w[i] >> 16) + b[2 * i + 1]) << 16);
+    }
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+template <int BIAS_DT>
+__device__ __forceinline__ void load_bias8(const void* bias, int64_t n, float (&b)[8]) {
+  float lo[4], hi[4];
+  load_bias4<BIAS_DT>(bias, n, lo);
+  load_bias4<BIAS_DT>(bias, n + 4, hi);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) { b[i] = lo[i]; b[4 + i] = hi[i]; }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -580,21 +680,22 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
       SB();
     }
 
-    // value (ns, rg) of row slot ms of this lane, scaled / biased (row mode) and packed to two 16-bit pairs
-    auto out_pair = [&](int ns, int ms, int rg, float sa) -> uint2 {
-      const int n = n0 + wn * 128 + ns * 32 + rg * 8 + h * 4;
+    const auto col_of = [&](int ns, int rg) { return n0 + wn * 128 + ns * 32 + rg * 8 + h * 4; };
+    if (MODE == kModeRow && !is_split) {
+      float sa[2];
+#pragma unroll
+      for (int ms = 0; ms < 2; ++ms) {
+        const int m = slot_at(wm * 64 + ms * 32 + lr);
+        sa[ms] = m < nrows ? row_scale(p, m) : 1.f;
+      }
+      finish_rows<16, 2, BIAS_DT>(p, sa, [&](int j) { return col_of(j >> 2, j & 3); },
+                                  [&](int j, int ms, int q, auto f) { acc[j >> 2][ms][(j & 3) * 4 + q] = f(acc[j >> 2][ms][(j & 3) * 4 + q]); });
+    }
+    // value (ns, rg) of row slot ms of this lane, packed to two 16-bit pairs
+    auto out_pair = [&](int ns, int ms, int rg) -> uint2 {
       float v[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] = acc[ns][ms][rg * 4 + q];
-      if (MODE == kModeRow) {
-        float4 sb = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (n < p.N) sb = *reinterpret_cast<const float4*>(p.sw + n);
-        v[0] = v[0] * sb.x * sa; v[1] = v[1] * sb.y * sa; v[2] = v[2] * sb.z * sa; v[3] = v[3] * sb.w * sa;
-        if (p.bias && n < p.N) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] += load_scalar<BIAS_DT>(p.bias, n + q);
-        }
-      }
       uint2 o;
       if (OUT_DT == FP8K_BF16) {
         o.x = pack_bf16x2(v[0], v[1]);
@@ -607,23 +708,23 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
     };
 
     if (wide) {
+      float bias8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (MODE == kModeBlock && p.bias) load_bias8<BIAS_DT>(p.bias, min(n0 + wn * 128 + ((ln & 15) << 3), p.N - 8), bias8);
       uint8_t* ep = smem + (w < 4 ? ews * kWStage + w * 8192 : kXBase + exs * kXStage + (w - 4) * 8192);  // 32 rows x 256 B per pass
 #pragma unroll
       for (int ms = 0; ms < 2; ++ms) {
-        const int mrow = slot_at(wm * 64 + ms * 32 + lr);
-        float sa = 1.f;
-        if (MODE == kModeRow && mrow < nrows) sa = p.sx[mrow];
 #pragma unroll
         for (int ns = 0; ns < 4; ++ns)
 #pragma unroll
           for (int rg = 0; rg < 4; ++rg)
-            *reinterpret_cast<uint2*>(ep + lr * 256 + (((ns * 4 + rg) ^ (lr & 15)) << 4) + h * 8) = out_pair(ns, ms, rg, sa);
+            *reinterpret_cast<uint2*>(ep + lr * 256 + (((ns * 4 + rg) ^ (lr & 15)) << 4) + h * 8) = out_pair(ns, ms, rg);
         __builtin_amdgcn_wave_barrier();  // one wave's LDS accesses complete in order: no wait needed
         const int rr = ln >> 4, pc = ln & 15;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int r = i * 4 + rr;
-          const uint4 o = *reinterpret_cast<const uint4*>(ep + r * 256 + ((pc ^ (r & 15)) << 4));
+          uint4 o = *reinterpret_cast<const uint4*>(ep + r * 256 + ((pc ^ (r & 15)) << 4));
+          if (MODE == kModeBlock && p.bias) o = add_bias8<OUT_DT>(o, bias8);
           const int m = slot_at(wm * 64 + ms * 32 + r);
           const int n = n0 + wn * 128 + (pc << 3);  // consecutive lanes store consecutive 16-byte chunks
           if (m < nrows && n < p.N) *reinterpret_cast<uint4*>((u16*)p.C + (int64_t)m * p.ldc + n) = o;
@@ -636,7 +737,6 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
         const int ml = wm * 64 + ms * 32 + lr;  // row inside the tile
         const int m = slot_at(ml);               // output row
         if (m >= nrows) continue;
-        const float sa = (MODE == kModeRow && !is_split) ? p.sx[m] : 1.f;
 #pragma unroll
         for (int ns = 0; ns < 4; ++ns) {
 #pragma unroll
@@ -648,7 +748,15 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
               *reinterpret_cast<float4*>(tile_part + ml * kTileN + (n - n0)) =
                   make_float4(acc[ns][ms][rg * 4], acc[ns][ms][rg * 4 + 1], acc[ns][ms][rg * 4 + 2], acc[ns][ms][rg * 4 + 3]);
             } else {
-              *reinterpret_cast<uint2*>((u16*)p.C + (int64_t)m * p.ldc + n) = out_pair(ns, ms, rg, sa);
+              if (MODE == kModeBlock && p.bias) {
+                float v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = acc[ns][ms][rg * 4 + q];
+                finish4<MODE, OUT_DT, BIAS_DT>(p, n, 1.f, v);
+                store4<OUT_DT>(p.C, (int64_t)m * p.ldc + n, v[0], v[1], v[2], v[3]);
+              } else {
+                *reinterpret_cast<uint2*>((u16*)p.C + (int64_t)m * p.ldc + n) = out_pair(ns, ms, rg);
+              }
             }
           }
         }
@@ -999,7 +1107,7 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const GemmArgs 
     for (int ms = 0; ms < MS; ++ms) {
       const int row = mrow0 + ms * 32 + lr;
       float rs = 1.f;
-      if (MODE == kModeRow && out_ok[ms]) rs = p.sx[out_slot[ms]];
+      if (MODE == kModeRow && out_ok[ms]) rs = row_scale(p, out_slot[ms]);
       if (MOE) rs = rsw[ms];
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg) {
@@ -1007,17 +1115,11 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const GemmArgs 
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = acc[ms][rg * 4 + r];
-        if (MODE == kModeRow) {
-          float4 sb = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (n < p.N) sb = *reinterpret_cast<const float4*>(p.sw + n);
-          v[0] = v[0] * sb.x * rs; v[1] = v[1] * sb.y * rs; v[2] = v[2] * sb.z * rs; v[3] = v[3] * sb.w * rs;
-          if (p.bias && n < p.N) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] += load_scalar<BIAS_DT>(p.bias, n + r);
-          }
-        } else if (MOE) {
+        if (MOE) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] *= rs;
+        } else if (n < p.N) {
+          finish4<MODE, OUT_DT, BIAS_DT>(p, n, rs, v);
         }
         uint2 o;
         if (OUT_DT == FP8K_BF16) {
@@ -1047,7 +1149,7 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const GemmArgs 
     if (!out_ok[ms]) continue;
     const int64_t orow = out_slot[ms];
     float rs = 1.f;
-    if (MODE == kModeRow && !SPLIT) rs = p.sx[orow];
+    if (MODE == kModeRow && !SPLIT) rs = row_scale(p, orow);
     if (MOE) rs = rsw[ms];
 #pragma unroll
     for (int rg = 0; rg < 4; ++rg) {
@@ -1059,16 +1161,11 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const GemmArgs 
       if (SPLIT) {
         *reinterpret_cast<float4*>(p.partial + ((int64_t)split * p.M + orow) * p.N + n) = make_float4(v[0], v[1], v[2], v[3]);
       } else {
-        if (MODE == kModeRow) {
-          const float4 sb = *reinterpret_cast<const float4*>(p.sw + n);
-          v[0] = v[0] * sb.x * rs; v[1] = v[1] * sb.y * rs; v[2] = v[2] * sb.z * rs; v[3] = v[3] * sb.w * rs;
-          if (p.bias) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] += load_scalar<BIAS_DT>(p.bias, n + r);
-          }
-        } else if (MOE) {
+        if (MOE) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] *= rs;
+        } else {
+          finish4<MODE, OUT_DT, BIAS_DT>(p, n, rs, v);
         }
         store4<OUT_DT>(p.C, orow * p.ldc + n, v[0], v[1], v[2], v[3]);
       }
@@ -1077,7 +1174,7 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_stream_kernel(const GemmArgs 
 }
 
 // ------------------------------------------------------------------------------------------------
-// split-K reduction: C = cast( sum_s partial[s] (* sa*sb + bias in row mode) )
+// split-K reduction: C = cast( sum_s partial[s] (* sa*sb in row mode, + bias) )
 // ------------------------------------------------------------------------------------------------
 template <int MODE, int OUT_DT, int BIAS_DT>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p) {
@@ -1086,21 +1183,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p) {
   if (i >= quads) return;
   const int m = (int)(i / (p.N / 4));
   const int n = (int)(i % (p.N / 4)) * 4;
-  float4 s = make_float4(0, 0, 0, 0);
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
   for (int k = 0; k < p.splits; ++k) {
     const float4 v = *reinterpret_cast<const float4*>(p.partial + ((int64_t)k * p.M + m) * p.N + n);
-    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+    s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
   }
-  if (MODE == kModeRow) {
-    const float sa = p.sx[m];
-    const float4 sb = *reinterpret_cast<const float4*>(p.sw + n);
-    s.x = s.x * sb.x * sa; s.y = s.y * sb.y * sa; s.z = s.z * sb.z * sa; s.w = s.w * sb.w * sa;
-    if (p.bias) {
-      s.x += load_scalar<BIAS_DT>(p.bias, n); s.y += load_scalar<BIAS_DT>(p.bias, n + 1);
-      s.z += load_scalar<BIAS_DT>(p.bias, n + 2); s.w += load_scalar<BIAS_DT>(p.bias, n + 3);
-    }
-  }
-  store4<OUT_DT>(p.C, (int64_t)m * p.ldc + n, s.x, s.y, s.z, s.w);
+  finish4<MODE, OUT_DT, BIAS_DT>(p, n, MODE == kModeRow ? row_scale(p, m) : 1.f, s);
+  store4<OUT_DT>(p.C, (int64_t)m * p.ldc + n, s[0], s[1], s[2], s[3]);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1116,21 +1205,13 @@ __global__ __launch_bounds__(256) void tile_reduce_kernel(const GemmArgs p) {
   const int m = tile_m * kTileM + ml, n = tile_n * kTileN + nl;
   if (m >= p.M || n >= p.N) return;
   const float* src = p.partial + (int64_t)tl * p.splits * (kTileM * kTileN) + ml * kTileN + nl;
-  float4 s = make_float4(0, 0, 0, 0);
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
   for (int k = 0; k < p.splits; ++k) {
     const float4 v = *reinterpret_cast<const float4*>(src + (int64_t)k * (kTileM * kTileN));
-    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+    s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
   }
-  if (MODE == kModeRow) {
-    const float sa = p.sx[m];
-    const float4 sb = *reinterpret_cast<const float4*>(p.sw + n);
-    s.x = s.x * sb.x * sa; s.y = s.y * sb.y * sa; s.z = s.z * sb.z * sa; s.w = s.w * sb.w * sa;
-    if (p.bias) {
-      s.x += load_scalar<BIAS_DT>(p.bias, n); s.y += load_scalar<BIAS_DT>(p.bias, n + 1);
-      s.z += load_scalar<BIAS_DT>(p.bias, n + 2); s.w += load_scalar<BIAS_DT>(p.bias, n + 3);
-    }
-  }
-  store4<OUT_DT>(p.C, (int64_t)m * p.ldc + n, s.x, s.y, s.z, s.w);
+  finish4<MODE, OUT_DT, BIAS_DT>(p, n, MODE == kModeRow ? row_scale(p, m) : 1.f, s);
+  store4<OUT_DT>(p.C, (int64_t)m * p.ldc + n, s[0], s[1], s[2], s[3]);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1172,8 +1253,10 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p) {
     }
   }
   if (MODE == kModeRow) {
-    acc = acc * p.sw[n] * p.sx[m];
+    acc = acc * p.sw[(int64_t)n * p.sw_n] * row_scale(p, m);
     if (p.bias) acc += load_scalar<BIAS_DT>(p.bias, n);
+  } else if (p.bias) {
+    acc = round_to<OUT_DT>(acc) + load_scalar<BIAS_DT>(p.bias, n);
   }
   if (OUT_DT == FP8K_BF16)
     ((u16*)p.C)[(int64_t)m * p.ldc + n] = (u16)f32_to_bf16_bits(acc);

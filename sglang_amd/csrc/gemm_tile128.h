@@ -274,20 +274,17 @@ __global__ __launch_bounds__(512, 1) void gemm_tile128_kernel(const GemmArgs p) 
     return;
   }
 
-  // scaling of row mode + conversion of one run of 4 n
-  auto finish4 = [&](int ns, int rg, int n, float sa) -> uint2 {
+  const int m_own = m0 + wm * 32 + lr;
+  if (MODE == kModeRow) {
+    const float sa[1] = {m_own < nrows ? row_scale(p, m_own) : 1.f};
+    finish_rows<8, 1, BIAS_DT>(p, sa, [&](int j) { return n0 + wn * 64 + (j >> 2) * 32 + (j & 3) * 8 + h * 4; },
+                               [&](int j, int, int q, auto f) { acc[j >> 2][(j & 3) * 4 + q] = f(acc[j >> 2][(j & 3) * 4 + q]); });
+  }
+  // conversion of one run of 4 n
+  auto out_quad = [&](int ns, int rg) -> uint2 {
     float v[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = acc[ns][rg * 4 + q];
-    if (MODE == kModeRow) {
-      float4 sb = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (n < p.N) sb = *reinterpret_cast<const float4*>(p.sw + n);
-      v[0] = v[0] * sb.x * sa; v[1] = v[1] * sb.y * sa; v[2] = v[2] * sb.z * sa; v[3] = v[3] * sb.w * sa;
-      if (p.bias && n < p.N) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] += load_scalar<BIAS_DT>(p.bias, n + q);
-      }
-    }
     uint2 o;
     if (OUT_DT == FP8K_BF16) {
       o.x = pack_bf16x2(v[0], v[1]);
@@ -301,21 +298,19 @@ __global__ __launch_bounds__(512, 1) void gemm_tile128_kernel(const GemmArgs p) 
 
   // Finished tiles leave through LDS so that a store instruction writes whole 128-byte row segments: each wave
   // re-lays its 32(m) x 64(n) block out in a private 4 KB slot, 16-byte chunks XOR-swizzled by the row.
-  const int m_own = m0 + wm * 32 + lr;
-  float sa = 1.f;
-  if (MODE == kModeRow && m_own < nrows) sa = p.sx[m_own];
   const bool wide = (p.ldc & 7) == 0 && (reinterpret_cast<uintptr_t>(Cb) & 15) == 0;
   if (wide) {
     wait_vm0_lgkm0();                // own stray loads have landed ...
     __builtin_amdgcn_s_barrier();    // ... and so have everyone's; every wave has taken its last operands
     asm volatile("" ::: "memory");
+    float bias8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (MODE == kModeBlock && p.bias) load_bias8<BIAS_DT>(p.bias, min(n0 + wn * 64 + ((lane & 7) << 3), p.N - 8), bias8);
     uint8_t* ep = smem + w * 4096;
 #pragma unroll
     for (int ns = 0; ns < 2; ++ns)
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg) {
-        const int n = n0 + wn * 64 + ns * 32 + rg * 8 + h * 4;
-        const uint2 o = finish4(ns, rg, n, sa);
+        const uint2 o = out_quad(ns, rg);
         const int chunk = (ns * 4 + rg) ^ (lr & 7);
         *reinterpret_cast<uint2*>(ep + lr * 128 + chunk * 16 + h * 8) = o;
       }
@@ -324,7 +319,8 @@ __global__ __launch_bounds__(512, 1) void gemm_tile128_kernel(const GemmArgs p) 
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = i * 8 + rr;
-      const uint4 o = *reinterpret_cast<const uint4*>(ep + r * 128 + ((pc ^ (r & 7)) << 4));
+      uint4 o = *reinterpret_cast<const uint4*>(ep + r * 128 + ((pc ^ (r & 7)) << 4));
+      if (MODE == kModeBlock && p.bias) o = add_bias8<OUT_DT>(o, bias8);
       const int m = m0 + wm * 32 + r;
       const int n = n0 + wn * 64 + (pc << 3);
       if (m < nrows && n < p.N) *reinterpret_cast<uint4*>(Cb + (int64_t)m * p.ldc + n) = o;
@@ -340,7 +336,15 @@ __global__ __launch_bounds__(512, 1) void gemm_tile128_kernel(const GemmArgs p) 
     for (int rg = 0; rg < 4; ++rg) {
       const int n = n0 + wn * 64 + ns * 32 + rg * 8 + h * 4;
       if (n >= p.N) continue;
-      const uint2 o = finish4(ns, rg, n, sa);
+      if (MODE == kModeBlock && p.bias) {
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = acc[ns][rg * 4 + q];
+        finish4<MODE, OUT_DT, BIAS_DT>(p, n, 1.f, v);
+        store4<OUT_DT>(Cb, (int64_t)m_own * p.ldc + n, v[0], v[1], v[2], v[3]);
+        continue;
+      }
+      const uint2 o = out_quad(ns, rg);
       *reinterpret_cast<uint2*>(Cb + (int64_t)m_own * p.ldc + n) = o;
     }
 }

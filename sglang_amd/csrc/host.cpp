@@ -248,7 +248,7 @@ PyObject* block_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (K % 128 != 0 || !block_weight(w, ws, K, dev)) DECLINE;
   const int64_t N = w.size(0);
   if (a[4] != Py_None) {
-    if (!tensor_arg(a[4], bias) || !plain(bias, dev) || bias.dim() != 1 || bias.size(0) != N || bias.scalar_type() != dt) DECLINE;
+    if (!tensor_arg(a[4], bias) || !plain(bias, dev) || bias.dim() != 1 || bias.size(0) != N || bias.scalar_type() != dt || !bias.is_contiguous()) DECLINE;
   }
 
   Call c(x);
@@ -261,9 +261,8 @@ PyObject* block_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   float* s = mem.take<float>(M * kb * 4);
   void* work = mem.take(wsb);
   check(fp8k_group_quant(x.data_ptr(), q, s, M, K, 128, kEps, -448.f, 448.f, code(dt), 1, M, FP8K_SCALE_F32, c.stream));
-  check(fp8k_block_gemm(q, w.data_ptr(), s, ws.data_ptr<float>(), out.data_ptr(), M, N, K, K, K, 1, M, ws.stride(0), ws.stride(1),
-                        N, code(dt), wsb ? work : nullptr, wsb, c.stream));
-  if (bias.defined()) out = out + bias;
+  check(fp8k_block_gemm_bias(q, w.data_ptr(), s, ws.data_ptr<float>(), bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(), M, N, K,
+                             K, K, 1, M, ws.stride(0), ws.stride(1), N, code(dt), wsb ? work : nullptr, wsb, c.stream));
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -329,7 +328,6 @@ PyObject* token_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
 
   Call c(x);
-  if (ws.numel() == 1) ws = ws.reshape({1}).expand({N}).contiguous();
   c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = N;
   Tensor out = empty(shape, dt, x.device());
@@ -339,8 +337,8 @@ PyObject* token_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   float* s = mem.take<float>(M * 4);
   void* work = mem.take(wsb);
   check(fp8k_token_quant(x.data_ptr(), q, s, M, K, code(dt), c.stream));
-  check(fp8k_scaled_mm(q, w.data_ptr(), s, ws.data_ptr<float>(), bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(), M, N, K,
-                       K, N > 1 ? w.stride(1) : K, N, code(dt), bias.defined() ? code(bias.scalar_type()) : FP8K_F32,
+  check(fp8k_scaled_mm_strided(q, w.data_ptr(), s, 1, ws.data_ptr<float>(), ws.numel() == 1 ? 0 : 1,
+                       bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(), M, N, K, K, N > 1 ? w.stride(1) : K, N, code(dt), bias.defined() ? code(bias.scalar_type()) : FP8K_F32,
                        wsb ? work : nullptr, wsb, c.stream));
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -379,9 +377,8 @@ PyObject* bmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (A.stride(2) != 1 || B.stride(1) != 1 || k % 128 != 0 || nn % 8 != 0) DECLINE;
   if (as.numel() != 1 || bs.numel() != 1 || as.scalar_type() != ScalarType::Float || bs.scalar_type() != ScalarType::Float) DECLINE;
   Call c(A);
-  const Tensor sa = as.reshape({1}).expand({m}).contiguous(), sb = bs.reshape({1}).expand({nn}).contiguous();
   Tensor out = empty({b, m, nn}, dt, A.device());
-  check(fp8k_bmm_fp8(A.data_ptr(), B.data_ptr(), sa.data_ptr<float>(), sb.data_ptr<float>(), out.data_ptr(), b, m, nn, k,
+  check(fp8k_bmm_fp8_tensor_scales(A.data_ptr(), B.data_ptr(), as.data_ptr<float>(), bs.data_ptr<float>(), out.data_ptr(), b, m, nn, k,
                      b > 1 ? A.stride(0) : m * k, m > 1 ? A.stride(1) : k, b > 1 ? B.stride(0) : nn * k, nn > 1 ? B.stride(2) : k,
                      m * nn, nn, code(dt), c.stream));
   return THPVariable_Wrap(std::move(out));

@@ -56,7 +56,8 @@ def _weight(n, k, seed=1):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [(1, 128, 128), (3, 264, 512), (33, 640, 1536), (300, 72, 256), (700, 1000, 384)])
+@pytest.mark.parametrize("m,n,k", [(1, 128, 128), (3, 264, 512), (33, 640, 1536), (300, 72, 256), (700, 1000, 384), (100, 1024, 4096),
+                                   (1100, 4096, 256), (1300, 9224, 1024)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_linears_are_the_dispatcher_path(dev, dispatcher, m, n, k, dtype):
     x, (w, s), bias = _randn((m, k), dtype), _weight(n, k), _randn((n,), dtype, 2)
