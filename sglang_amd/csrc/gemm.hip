@@ -4,6 +4,7 @@
 #include <atomic>
 #include <mutex>
 
+#include "gemm_bmm.h"
 #include "gemm_direct.h"
 #include "gemm_tile128.h"
 
@@ -574,8 +575,12 @@ extern "C" int fp8k_scaled_mm_strided(const void* A, const void* B, const float*
 #undef FP8K_SMM
 }
 
-// ---- batched per-tensor-scaled FP8 GEMM (the MLA absorbed products): every batch entry is a row-mode GEMM on the
-// 128x128 tile kernel (grid y = entry), whose per-row / per-column scale vectors are shared by all entries.
+// ---- batched per-tensor-scaled FP8 GEMM (the MLA absorbed products): every batch entry is a row-mode GEMM on the short-K
+// kernel or, for long K, on the 128x128 tile kernel (grid y = entry), whose per-row / per-column scale vectors are shared by all entries.
+// Up to eight K blocks the short-K kernel is ahead at every row count (1 .. 4096 rows, 16 and 128 entries: level to 3.6 times;
+// 128 entries of 64 x 512 x 128: 14.6 -> 5.7 us); at 16 and more blocks the tile kernel's ring and larger tile win from about
+// 1000 rows on and below it the two are within 15 % on a part-filled chip.
+constexpr int64_t kBmmShortK = 1024;
 static int bmm_impl(const void* A, const void* B, const float* sa, const float* sb, int64_t scale_stride, void* C, int64_t batch,
                     int64_t M, int64_t N, int64_t K, int64_t a_stride_b, int64_t lda, int64_t b_stride_b, int64_t ldb,
                     int64_t c_stride_b, int64_t ldc, int out_dtype, void* stream) {
@@ -596,12 +601,22 @@ static int bmm_impl(const void* A, const void* B, const float* sa, const float* 
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = lda; a.ldw = ldb; a.ldc = ldc;
   a.sx_m = a.sw_n = scale_stride;
   a.batch_x = a_stride_b; a.batch_w = b_stride_b; a.batch_c = c_stride_b;
+  hipStream_t st = (hipStream_t)stream;
+  a.batch = (int)batch;
+  if ((g_force_kind == 6 || (g_force_kind < 0 && K <= kBmmShortK)) && M * lda < (1LL << 31) && N * ldb < (1LL << 31)) {
+    a.tiles_m = (int)((M + kBmmTileM - 1) / kBmmTileM);
+    a.tiles_n = (int)((N + kBmmTileN - 1) / kBmmTileN);
+    const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n * ((batch + 7) / 8 * 8);
+    FP8K_REQUIRE(blocks <= 0x7fffffffLL, "%s: too many tiles for one launch", op);
+    if (out_dtype == FP8K_BF16) hipLaunchKernelGGL(gemm_bmm_short_kernel<FP8K_BF16>, dim3((unsigned)blocks), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(gemm_bmm_short_kernel<FP8K_F16>, dim3((unsigned)blocks), dim3(256), 0, st, a);
+    return check_launch(op);
+  }
   a.tiles_m = (int)((M + kT128 - 1) / kT128);
   a.tiles_n = (int)((N + kT128 - 1) / kT128);
   a.splits = 1;
   a.kb_per_split = (int)(K / kTileK);
   const unsigned nwg = (unsigned)(((int64_t)a.tiles_m * a.tiles_n + 7) / 8 * 8);
-  hipStream_t st = (hipStream_t)stream;
   if (out_dtype == FP8K_BF16)
     hipLaunchKernelGGL((gemm_tile128_kernel<kModeRow, FP8K_BF16, FP8K_F32, false>), dim3(nwg, (unsigned)batch), dim3(512), 0, st, a);
   else

@@ -51,7 +51,8 @@ struct GemmArgs {
   int64_t qs_ld;                // floats between the scale rows of two activation column blocks (>= capacity)
   float q_eps;                  // lower clamp of the group maximum (already rounded to the element type)
   int64_t sw_expert_stride;     // floats between experts in sw
-  // batched form of the 128x128 tile kernel (grid y = batch entry); zero for a single GEMM
+  // batched form of the 128x128 tile kernel (grid y = batch entry), and gemm_bmm_short_kernel; zero for a single GEMM
+  int batch;                    // entries (gemm_bmm_short_kernel)
   int64_t batch_x, batch_w;     // bytes between batch entries of X and W
   int64_t batch_c;              // elements between batch entries of C
 };

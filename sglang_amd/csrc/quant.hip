@@ -2,6 +2,8 @@
 //
 // All three are HBM-bound streaming kernels: 16-byte loads, 8/16-byte stores, one pass over the
 // input held in registers, amax by DPP lane exchange inside the wavefront.
+#include <algorithm>
+
 #include "fp8k_common.h"
 #include "quant_math.h"
 
@@ -400,37 +402,51 @@ __global__ __launch_bounds__(256) void tensor_quant_kernel(const void* __restric
 }
 
 // ------------------------------------------------------------------------------------------------
-// per-tensor quant of a strided [H, S, D] tensor into a contiguous one (the MLA absorbed products): a workgroup takes
-// whole rows (h, s) in grid-stride, a lane 8 elements at a time
+// per-tensor quant of a strided [H, S, D] tensor into a contiguous one (the MLA absorbed products): 8 elements (a chunk) a
+// lane, four chunks in flight, in grid-stride.  Bound by latency at decode sizes: with 2048 workgroups the maxima queued up
+// at the one atomic (8.0 us for 64 tokens x 128 heads x 128, 2 MB), so the maximum pass takes at most 512 workgroups and four
+// chunks per lane before it takes a second workgroup's atomic; IDX is 32-bit wherever the chunks can be counted so, because
+// the two divisions per chunk (row, then head) are the arithmetic of this kernel.
 // ------------------------------------------------------------------------------------------------
-template <int DT, bool QUANT>
+template <int DT, bool QUANT, typename IDX>
 __global__ __launch_bounds__(256) void rows_tensor_quant_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
                                                                 float* __restrict__ s, int64_t rows, int S, int D,
                                                                 int64_t stride_h, int64_t stride_s, float eps) {
   __shared__ float red[4];
-  const int chunks = D / 8;                 // per row; the host checks D % 8 == 0 and the alignment of every row
-  const int64_t total = rows * chunks;
-  const int64_t step = (int64_t)gridDim.x * 256;
+  const IDX chunks = (IDX)(D / 8);          // per row; the host checks D % 8 == 0 and the alignment of every row
+  const IDX total = (IDX)rows * chunks;
+  const IDX step = (IDX)gridDim.x * 256;
   const float inv = QUANT ? 1.0f / s[0] : 0.f;
   float m = 0.f;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += step) {
-    const int64_t row = i / chunks;
-    const int c = (int)(i - row * chunks);
-    const int64_t hh = row / S, ss = row - hh * S;
-    Raw8<DT> t;
-    t.load(x, hh * stride_h + ss * stride_s + c * 8);
-    float a[8];
-    t.unpack(a);
-    if (QUANT) {
-      float y[8];
+  constexpr int U = 4;
+  for (IDX i0 = (IDX)blockIdx.x * 256 + threadIdx.x; i0 < total; i0 += U * step) {
+    Raw8<DT> t[U];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) y[j] = fmaxf(fminf(a[j] * inv, kFp8Max), -kFp8Max);
-      uint2 o;
-      o.x = cvt4_fp8(y[0], y[1], y[2], y[3]);
-      o.y = cvt4_fp8(y[4], y[5], y[6], y[7]);
-      *reinterpret_cast<uint2*>(q + row * D + c * 8) = o;
-    } else {
-      m = fmaxf(m, absmax8(a));
+    for (int u = 0; u < U; ++u) {
+      const IDX i = i0 + u * step;
+      if (i < total) {
+        const IDX row = i / chunks, c = i - row * chunks;
+        const IDX hh = row / (IDX)S, ss = row - hh * (IDX)S;
+        t[u].load(x, (int64_t)hh * stride_h + (int64_t)ss * stride_s + (int64_t)c * 8);
+      } else {
+        t[u].zero();
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float a[8];
+      t[u].unpack(a);
+      if (!QUANT) {
+        m = fmaxf(m, absmax8(a));
+      } else if (const IDX i = i0 + u * step; i < total) {
+        float y[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[j] = fmaxf(fminf(a[j] * inv, kFp8Max), -kFp8Max);
+        uint2 o;
+        o.x = cvt4_fp8(y[0], y[1], y[2], y[3]);
+        o.y = cvt4_fp8(y[4], y[5], y[6], y[7]);
+        *reinterpret_cast<uint2*>(q + (int64_t)i * 8) = o;  // the output is contiguous
+      }
     }
   }
   if (!QUANT) {
@@ -438,6 +454,55 @@ __global__ __launch_bounds__(256) void rows_tensor_quant_kernel(const void* __re
     // non-negative floats order like their bit patterns
     if (threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned int*>(s), __float_as_uint(m / kFp8Max));
   }
+}
+
+// The same for a tensor that one workgroup can hold in its registers (kMlaSmallChunks x 8 elements): one launch instead of
+// two, no atomic.  4.9 us of two launches -> 3.1 us at 1 KB, 3.7 at 16 KB, 5.1 at 64 KB, where the line lies: with more, the
+// one CU's load path (64 bytes a clock) takes longer than the second launch (7.2 us at 128 KB).
+constexpr int kMlaHold = 4, kMlaSmallChunks = 1024 * kMlaHold;
+template <int DT>
+__global__ __launch_bounds__(1024) void rows_tensor_quant_small_kernel(const void* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ s,
+                                                                       uint32_t total, uint32_t chunks, uint32_t S, int64_t stride_h,
+                                                                       int64_t stride_s, float eps) {
+  __shared__ float red[16];
+  Raw8<DT> t[kMlaHold];
+#pragma unroll
+  for (int u = 0; u < kMlaHold; ++u) {
+    const uint32_t i = u * 1024 + threadIdx.x;
+    if (i < total) {
+      const uint32_t row = i / chunks, c = i - row * chunks, hh = row / S, ss = row - hh * S;
+      t[u].load(x, (int64_t)hh * stride_h + (int64_t)ss * stride_s + (int64_t)c * 8);
+    } else {
+      t[u].zero();
+    }
+  }
+  float m = eps;
+#pragma unroll
+  for (int u = 0; u < kMlaHold; ++u) {
+    float a[8];
+    t[u].unpack(a);
+    m = fmaxf(m, absmax8(a));
+  }
+  m = group_max<64>(m);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) m = fmaxf(m, red[i]);
+  const float sc = fmaxf(m / kFp8Max, s[0]);  // accumulates onto what the scale holds, as the atomic form does
+  const float inv = 1.0f / sc;
+#pragma unroll
+  for (int u = 0; u < kMlaHold; ++u) {
+    const uint32_t i = u * 1024 + threadIdx.x;
+    if (i < total) {
+      float a[8], y[8];
+      t[u].unpack(a);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] = fmaxf(fminf(a[j] * inv, kFp8Max), -kFp8Max);
+      *reinterpret_cast<uint2*>(q + (int64_t)i * 8) = make_uint2(cvt4_fp8(y[0], y[1], y[2], y[3]), cvt4_fp8(y[4], y[5], y[6], y[7]));
+    }
+  }
+  __syncthreads();  // every wave has read the old scale
+  if (threadIdx.x == 0) s[0] = sc;
 }
 
 }  // namespace fp8k
@@ -637,15 +702,24 @@ extern "C" int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H
   FP8K_REQUIRE(x_stride_h >= 0 && x_stride_s >= 0 && (x_stride_h * esz) % 16 == 0 && (x_stride_s * esz) % 16 == 0 && aligned(x, 16) &&
                aligned(q, 8), "%s: rows of x must be 16-byte aligned, q 8-byte aligned", op);
   hipStream_t st = (hipStream_t)stream;
-  const int64_t rows = H * S;
-  const int64_t want = (rows * (D / 8) + 255) / 256;
-  dim3 grid((unsigned)(want < 1 ? 1 : (want > 2048 ? 2048 : want))), block(256);
-#define FP8K_MLAQ(DT)                                                                                                    \
-  do {                                                                                                                   \
-    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, false>), grid, block, 0, st, x, (uint8_t*)q, s, rows, (int)S, (int)D, \
-                       x_stride_h, x_stride_s, eps);                                                                     \
-    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, true>), grid, block, 0, st, x, (uint8_t*)q, s, rows, (int)S, (int)D,  \
-                       x_stride_h, x_stride_s, eps);                                                                     \
+  const int64_t rows = H * S, chunks = rows * (D / 8);
+  const bool narrow = chunks < (1LL << 31);  // room for the four steps past the end
+  const dim3 block(256);
+  const dim3 grid_max((unsigned)std::min<int64_t>(512, (chunks + 1023) / 1024)), grid_q((unsigned)std::min<int64_t>(2048, (chunks + 255) / 256));
+#define FP8K_MLAQ2(DT, IDX)                                                                                                 \
+  do {                                                                                                                      \
+    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, false, IDX>), grid_max, block, 0, st, x, (uint8_t*)q, s, rows, (int)S, \
+                       (int)D, x_stride_h, x_stride_s, eps);                                                                \
+    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, true, IDX>), grid_q, block, 0, st, x, (uint8_t*)q, s, rows, (int)S,    \
+                       (int)D, x_stride_h, x_stride_s, eps);                                                                \
+  } while (0)
+#define FP8K_MLAQ(DT)                                                                                                          \
+  do {                                                                                                                         \
+    if (chunks <= kMlaSmallChunks)                                                                                             \
+      hipLaunchKernelGGL(rows_tensor_quant_small_kernel<DT>, dim3(1), dim3(1024), 0, st, x, (uint8_t*)q, s, (uint32_t)chunks,  \
+                         (uint32_t)(D / 8), (uint32_t)S, x_stride_h, x_stride_s, eps);                                         \
+    else if (narrow) FP8K_MLAQ2(DT, uint32_t);                                                                                 \
+    else FP8K_MLAQ2(DT, int64_t);             \
   } while (0)
   switch (in_dtype) {
     case FP8K_BF16: FP8K_MLAQ(FP8K_BF16); break;
@@ -653,5 +727,6 @@ extern "C" int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H
     default: FP8K_MLAQ(FP8K_F32); break;
   }
 #undef FP8K_MLAQ
+#undef FP8K_MLAQ2
   return check_launch(op);
 }

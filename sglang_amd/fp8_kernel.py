@@ -205,12 +205,12 @@ def per_tensor_quant_mla_fp8(x: torch.Tensor, x_s_out: torch.Tensor, eps: float 
     """Reference: fp8_kernel.py:1221-1266 - tensor-wise quantisation specialised for the MLA absorbed products: x is a
     (possibly transposed) [num_head, num_seq, head_size] view, the result is contiguous.  x_s_out: one float32 that
     must be zero on entry (the maximum is accumulated atomically) and receives max(absmax, eps) / 448."""
-    assert x.dim() == 3, "`x` is not a 3d-tensor"
-    assert x_s_out.shape == (1,) and x_s_out.dtype == torch.float32 and x_s_out.device == x.device
     if not torch.compiler.is_compiling():
         x_q = _host.mla_quant(x, x_s_out, eps)
         if x_q is not None:
             return x_q, x_s_out
+    assert x.dim() == 3, "`x` is not a 3d-tensor"
+    assert x_s_out.shape == (1,) and x_s_out.dtype == torch.float32 and x_s_out.device == x.device
     x_q = x.new_empty(x.size(), dtype=fp8_dtype)
     if x.numel() > 0:
         _ops.tensor_quant_mla(x, x_q, x_s_out, eps)

@@ -127,3 +127,20 @@ def test_experts_are_the_dispatcher_path(dev, dispatcher, tokens):
 
     for args in ((False,), (True,), (False, True)):
         assert _same(layer(*args), dispatcher(lambda: layer(*args)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,m,n,k", [(1, 1, 8, 128), (9, 64, 128, 256), (8, 65, 136, 384), (17, 127, 120, 1024), (3, 70, 200, 1152)])
+def test_bmm_tile_edges(dev, b, m, n, k):
+    """Row, column and batch remainders of the short-K kernel's 64 x 128 tiles, one to nine K blocks, strided operands and
+    output; exact on integer data."""
+    g = torch.Generator().manual_seed(m)
+    A = torch.randint(-4, 5, (b, m + 3, k), generator=g).float()
+    B = torch.randint(-4, 5, (b, n, k), generator=g).float()
+    out = torch.zeros((b, m + 1, n + 8), dtype=torch.float16, device=dev)
+    fa, fb = A.to(dev).to(torch.float8_e4m3fn), B.to(dev).to(torch.float8_e4m3fn)
+    one = torch.ones((1,), device=dev)
+    sgl_kernel.bmm_fp8(fa[:, :m], fb.transpose(1, 2), one * 0.5, one * 0.25, torch.float16, out[:, :m, :n])
+    ref = (A[:, :m] @ B.transpose(1, 2)) * 0.125
+    assert torch.equal(out[:, :m, :n].float().cpu(), ref.half().float())
+    assert not out[:, m:].any() and not out[:, :, n:].any()
