@@ -6,6 +6,7 @@
 
 #include "gemm_bmm.h"
 #include "gemm_direct.h"
+#include "gemm_direct_quant.h"
 #include "gemm_tile128.h"
 
 #include "../../include/fp8k_tune.h"
@@ -573,6 +574,71 @@ extern "C" int fp8k_scaled_mm_strided(const void* A, const void* B, const float*
   if (bd == FP8K_BF16) return FP8K_SMM(FP8K_F16, FP8K_BF16);
   return FP8K_SMM(FP8K_F16, FP8K_F16);
 #undef FP8K_SMM
+}
+
+// ---- decode linears of a few rows, quantisation included (gemm_wavek_quant_kernel)
+// Up to 16 rows of at most kQuantFuseMax elements together, where the wave-cut kernel would take the GEMM: every workgroup
+// repeats the quantisation, whose share grows with M * K while the launch it saves does not (the gain falls from 1.5 .. 1.85
+// times at 4096 elements to 1.2 .. 1.3 at 32768; twice as many would take another 32 registers per lane and with them the
+// second workgroup of a CU).
+static bool fuses_quant(int64_t M, int64_t N, int64_t K) {
+  if (M < 1 || M > 16 || N < 1 || N % 8 != 0 || K < kTileK || K % kTileK != 0 || M * K > kQuantFuseMax) return false;
+  return g_force_kind < 0 && prefers_wavek(M, N, K);
+}
+
+template <int MODE, int OUT_DT, int BIAS_DT>
+static int launch_quant_linear(const GemmArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)((a.N + 16 * a.wk_nw - 1) / (16 * a.wk_nw))), block(512);
+  const unsigned lds = (unsigned)(a.M * wq_row_bytes(a.K));
+  const int64_t pieces = (int64_t)a.M * a.K / 8;
+  if (pieces <= 2 * 512) hipLaunchKernelGGL((gemm_wavek_quant_kernel<2, 8, MODE, OUT_DT, BIAS_DT>), grid, block, lds, st, a);
+  else if (pieces <= 4 * 512) hipLaunchKernelGGL((gemm_wavek_quant_kernel<4, 8, MODE, OUT_DT, BIAS_DT>), grid, block, lds, st, a);
+  else hipLaunchKernelGGL((gemm_wavek_quant_kernel<8, 4, MODE, OUT_DT, BIAS_DT>), grid, block, lds, st, a);
+  return check_launch("gemm_wavek_quant");
+}
+
+static int quant_linear(const char* op, bool block_mode, const void* x, const void* B, const float* Bs, int64_t bs_n, int64_t bs_k,
+                        const void* bias, int bias_dtype, void* C, int64_t M, int64_t N, int64_t K, int64_t ldb, int64_t ldc, float eps,
+                        int dtype, void* stream) {
+  clear_error();
+  int rc = common_checks(op, x, B, C, M, N, K, K, ldb, ldc, dtype);
+  if (rc) return rc;
+  FP8K_REQUIRE(fuses_quant(M, N, K), "%s: M=%lld N=%lld K=%lld is not a size of the one-launch form (fp8k_linear_fuses_quant)", op,
+               (long long)M, (long long)N, (long long)K);
+  FP8K_REQUIRE(Bs, "%s: null scale pointer", op);
+  FP8K_REQUIRE(bs_n >= 0 && bs_k >= 0, "%s: negative scale stride", op);
+  FP8K_REQUIRE(block_mode || ((bs_n == 0 || bs_n == 1) && (bs_n == 0 || aligned(Bs, 16))),
+               "%s: channel scales must be contiguous and 16-byte aligned", op);
+  FP8K_REQUIRE(!bias || bias_dtype == FP8K_F32 || bias_dtype == FP8K_F16 || bias_dtype == FP8K_BF16,
+               "%s: bias dtype must be float32, float16 or bfloat16", op);
+  const Plan pl = plan_wavek(M, N, K);
+  GemmArgs a{};
+  a.X = (const uint8_t*)x; a.W = (const uint8_t*)B; a.sw = Bs; a.bias = bias; a.C = C;
+  a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldw = ldb; a.ldc = ldc;
+  a.sw_n = bs_n; a.sw_k = bs_k; a.q_eps = quant_eps(eps, dtype);
+  a.wk_nw = pl.halves; a.kb_per_split = pl.kb_per_split;
+  hipStream_t st = (hipStream_t)stream;
+  if (block_mode)
+    return dtype == FP8K_BF16 ? launch_quant_linear<kModeBlock, FP8K_BF16, FP8K_BF16>(a, st)
+                              : launch_quant_linear<kModeBlock, FP8K_F16, FP8K_F16>(a, st);
+  const int bd = bias ? bias_dtype : FP8K_F32;
+#define FP8K_QL(O) (bd == FP8K_F32    ? launch_quant_linear<kModeRow, O, FP8K_F32>(a, st) \
+                    : bd == FP8K_BF16 ? launch_quant_linear<kModeRow, O, FP8K_BF16>(a, st) \
+                                      : launch_quant_linear<kModeRow, O, FP8K_F16>(a, st))
+  return dtype == FP8K_BF16 ? FP8K_QL(FP8K_BF16) : FP8K_QL(FP8K_F16);
+#undef FP8K_QL
+}
+
+extern "C" int fp8k_linear_fuses_quant(int64_t M, int64_t N, int64_t K) { return fuses_quant(M, N, K) ? 1 : 0; }
+
+extern "C" int fp8k_block_linear(const void* x, const void* B, const float* Bs, const void* bias, void* C, int64_t M, int64_t N, int64_t K,
+                                 int64_t ldb, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, float eps, int dtype, void* stream) {
+  return quant_linear("block_linear", true, x, B, Bs, bs_stride_n, bs_stride_k, bias, dtype, C, M, N, K, ldb, ldc, eps, dtype, stream);
+}
+
+extern "C" int fp8k_token_linear(const void* x, const void* B, const float* sb, int64_t sb_stride, const void* bias, int bias_dtype,
+                                 void* C, int64_t M, int64_t N, int64_t K, int64_t ldb, int64_t ldc, int dtype, void* stream) {
+  return quant_linear("token_linear", false, x, B, sb, sb_stride, 0, bias, bias_dtype, C, M, N, K, ldb, ldc, 0.f, dtype, stream);
 }
 
 // ---- batched per-tensor-scaled FP8 GEMM (the MLA absorbed products): every batch entry is a row-mode GEMM on the short-K

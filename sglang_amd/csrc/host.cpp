@@ -255,6 +255,11 @@ PyObject* block_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = N;
   Tensor out = empty(shape, dt, x.device());
+  if (fp8k_linear_fuses_quant(M, N, K)) {
+    check(fp8k_block_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(),
+                            M, N, K, K, ws.stride(0), ws.stride(1), N, kEps, code(dt), c.stream));
+    return THPVariable_Wrap(std::move(out));
+  }
   const int64_t kb = K / 128, wsb = fp8k_block_gemm_workspace_bytes(M, N, K);
   Scratch mem(Scratch::room(M * K) + Scratch::room(M * kb * 4) + Scratch::room(wsb), c.stream);
   void* q = mem.take(M * K);
@@ -331,6 +336,12 @@ PyObject* token_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = N;
   Tensor out = empty(shape, dt, x.device());
+  if (fp8k_linear_fuses_quant(M, N, K)) {
+    check(fp8k_token_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), ws.numel() == 1 ? 0 : 1, bias.defined() ? bias.data_ptr() : nullptr,
+                            bias.defined() ? code(bias.scalar_type()) : FP8K_F32, out.data_ptr(), M, N, K, N > 1 ? w.stride(1) : K, N, code(dt),
+                            c.stream));
+    return THPVariable_Wrap(std::move(out));
+  }
   const int64_t wsb = fp8k_scaled_mm_workspace_bytes(M, N, K);
   Scratch mem(Scratch::room(M * K) + Scratch::room(M * 4) + Scratch::room(wsb), c.stream);
   void* q = mem.take(M * K);

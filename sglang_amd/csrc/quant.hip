@@ -10,55 +10,6 @@
 namespace fp8k {
 
 // ------------------------------------------------------------------------------------------------
-// loading 8 consecutive elements as float
-// ------------------------------------------------------------------------------------------------
-template <int DT>
-struct Raw8;
-template <>
-struct Raw8<FP8K_BF16> {
-  uint4 v;
-  __device__ __forceinline__ void load(const void* base, int64_t elem) { v = *reinterpret_cast<const uint4*>((const u16*)base + elem); }
-  __device__ __forceinline__ void zero() { v = make_uint4(0, 0, 0, 0); }
-  __device__ __forceinline__ void unpack(float (&a)[8]) const {
-    a[0] = bf16_lo(v.x); a[1] = bf16_hi(v.x); a[2] = bf16_lo(v.y); a[3] = bf16_hi(v.y);
-    a[4] = bf16_lo(v.z); a[5] = bf16_hi(v.z); a[6] = bf16_lo(v.w); a[7] = bf16_hi(v.w);
-  }
-};
-template <>
-struct Raw8<FP8K_F16> {
-  uint4 v;
-  __device__ __forceinline__ void load(const void* base, int64_t elem) { v = *reinterpret_cast<const uint4*>((const u16*)base + elem); }
-  __device__ __forceinline__ void zero() { v = make_uint4(0, 0, 0, 0); }
-  __device__ __forceinline__ void unpack(float (&a)[8]) const {
-    a[0] = f16_bits_to_f32(v.x & 0xffff); a[1] = f16_bits_to_f32(v.x >> 16);
-    a[2] = f16_bits_to_f32(v.y & 0xffff); a[3] = f16_bits_to_f32(v.y >> 16);
-    a[4] = f16_bits_to_f32(v.z & 0xffff); a[5] = f16_bits_to_f32(v.z >> 16);
-    a[6] = f16_bits_to_f32(v.w & 0xffff); a[7] = f16_bits_to_f32(v.w >> 16);
-  }
-};
-template <>
-struct Raw8<FP8K_F32> {
-  float4 lo, hi;
-  __device__ __forceinline__ void load(const void* base, int64_t elem) {
-    const float4* p = reinterpret_cast<const float4*>((const float*)base + elem);
-    lo = p[0];
-    hi = p[1];
-  }
-  __device__ __forceinline__ void zero() { lo = make_float4(0, 0, 0, 0); hi = lo; }
-  __device__ __forceinline__ void unpack(float (&a)[8]) const {
-    a[0] = lo.x; a[1] = lo.y; a[2] = lo.z; a[3] = lo.w; a[4] = hi.x; a[5] = hi.y; a[6] = hi.z; a[7] = hi.w;
-  }
-};
-
-__device__ __forceinline__ float absmax8(const float (&a)[8]) {
-  float m = fmaxf(fabsf(a[0]), fabsf(a[1]));
-  m = fmaxf(fmaxf(m, fabsf(a[2])), fabsf(a[3]));
-  m = fmaxf(fmaxf(m, fabsf(a[4])), fabsf(a[5]));
-  m = fmaxf(fmaxf(m, fabsf(a[6])), fabsf(a[7]));
-  return m;
-}
-
-// ------------------------------------------------------------------------------------------------
 // per-token-group quant
 //
 // The unit of work is a 1 KB "segment" (64 lanes x 8 elements = 512 columns of one row, i.e.
@@ -533,14 +484,7 @@ extern "C" int fp8k_group_quant(const void* x, void* q, void* s, int64_t M, int6
   } else {
     FP8K_REQUIRE(s_stride_m > 0 && ((G + 3) / 4 == 1 || s_stride_g > 0), "group_quant: packed scale strides must be positive");
   }
-  // the torch-native formula clamps amax in the input dtype: bf16 sees eps rounded to bf16
-  float eps_eff = eps;
-  if (in_dtype == FP8K_BF16) {
-    uint32_t u;
-    memcpy(&u, &eps, 4);
-    u = ((u + 0x7fffu + ((u >> 16) & 1u)) >> 16) << 16;
-    memcpy(&eps_eff, &u, 4);
-  }
+  const float eps_eff = quant_eps(eps, in_dtype);
   hipStream_t st = (hipStream_t)stream;
 #define FP8K_GQ(DT)                                                                                               \
   (scale_kind == FP8K_SCALE_F32                                                                                   \
@@ -577,13 +521,7 @@ extern "C" int fp8k_silu_mul_group_quant(const void* x, void* q, void* s, int64_
   } else {
     FP8K_REQUIRE(s_stride_m > 0 && ((G + 3) / 4 == 1 || s_stride_g > 0), "%s: packed scale strides must be positive", op);
   }
-  float eps_eff = eps;  // clamped in the input dtype, as in fp8k_group_quant
-  if (in_dtype == FP8K_BF16) {
-    uint32_t u;
-    memcpy(&u, &eps, 4);
-    u = ((u + 0x7fffu + ((u >> 16) & 1u)) >> 16) << 16;
-    memcpy(&eps_eff, &u, 4);
-  }
+  const float eps_eff = quant_eps(eps, in_dtype);
   hipStream_t st = (hipStream_t)stream;
 #define FP8K_SGQ(DT)                                                                                                 \
   (scale_kind == FP8K_SCALE_F32                                                                                     \
@@ -616,13 +554,7 @@ extern "C" int fp8k_group_quant_masked(const void* x, void* q, void* s, int64_t 
   FP8K_REQUIRE(x && q && s && masked_m, "%s: null pointer", op);
   FP8K_REQUIRE(aligned(x, 16) && aligned(q, 8) && aligned(s, 4) && aligned(masked_m, 4), "%s: x must be 16-byte, q 8-byte aligned", op);
   FP8K_REQUIRE(s_stride_e >= 0 && s_stride_m >= 0 && s_stride_g >= 0, "%s: negative scale stride", op);
-  float eps_eff = eps;  // clamped in the input dtype, as in fp8k_group_quant
-  if (in_dtype == FP8K_BF16) {
-    uint32_t u;
-    memcpy(&u, &eps, 4);
-    u = ((u + 0x7fffu + ((u >> 16) & 1u)) >> 16) << 16;
-    memcpy(&eps_eff, &u, 4);
-  }
+  const float eps_eff = quant_eps(eps, in_dtype);
   hipStream_t st = (hipStream_t)stream;
   const int64_t M = E * m_max;
 #define FP8K_MQ3(DT, KIND, FUSE) \

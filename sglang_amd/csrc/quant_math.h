@@ -1,11 +1,70 @@
-// The exact arithmetic of the FP8 group quantisation, shared by the quant kernels and by the GEMM epilogue that
-// quantises its own output: scale = amax / 448 correctly rounded, bytes = RNE_e4m3fn(clamp(x / scale)) bit-identical
-// to an IEEE divide followed by the cast.
+// The exact arithmetic of the FP8 group quantisation, shared by the quant kernels, by the GEMM epilogue that quantises its
+// own output and by the decode GEMM that quantises its own activations: scale = amax / 448 correctly rounded,
+// bytes = RNE_e4m3fn(clamp(x / scale)) bit-identical to an IEEE divide followed by the cast.
 #pragma once
 
 #include "fp8k_common.h"
 
 namespace fp8k {
+
+// ------------------------------------------------------------------------------------------------
+// loading 8 consecutive elements as float
+// ------------------------------------------------------------------------------------------------
+template <int DT>
+struct Raw8;
+template <>
+struct Raw8<FP8K_BF16> {
+  uint4 v;
+  __device__ __forceinline__ void load(const void* base, int64_t elem) { v = *reinterpret_cast<const uint4*>((const u16*)base + elem); }
+  __device__ __forceinline__ void zero() { v = make_uint4(0, 0, 0, 0); }
+  __device__ __forceinline__ void unpack(float (&a)[8]) const {
+    a[0] = bf16_lo(v.x); a[1] = bf16_hi(v.x); a[2] = bf16_lo(v.y); a[3] = bf16_hi(v.y);
+    a[4] = bf16_lo(v.z); a[5] = bf16_hi(v.z); a[6] = bf16_lo(v.w); a[7] = bf16_hi(v.w);
+  }
+};
+template <>
+struct Raw8<FP8K_F16> {
+  uint4 v;
+  __device__ __forceinline__ void load(const void* base, int64_t elem) { v = *reinterpret_cast<const uint4*>((const u16*)base + elem); }
+  __device__ __forceinline__ void zero() { v = make_uint4(0, 0, 0, 0); }
+  __device__ __forceinline__ void unpack(float (&a)[8]) const {
+    a[0] = f16_bits_to_f32(v.x & 0xffff); a[1] = f16_bits_to_f32(v.x >> 16);
+    a[2] = f16_bits_to_f32(v.y & 0xffff); a[3] = f16_bits_to_f32(v.y >> 16);
+    a[4] = f16_bits_to_f32(v.z & 0xffff); a[5] = f16_bits_to_f32(v.z >> 16);
+    a[6] = f16_bits_to_f32(v.w & 0xffff); a[7] = f16_bits_to_f32(v.w >> 16);
+  }
+};
+template <>
+struct Raw8<FP8K_F32> {
+  float4 lo, hi;
+  __device__ __forceinline__ void load(const void* base, int64_t elem) {
+    const float4* p = reinterpret_cast<const float4*>((const float*)base + elem);
+    lo = p[0];
+    hi = p[1];
+  }
+  __device__ __forceinline__ void zero() { lo = make_float4(0, 0, 0, 0); hi = lo; }
+  __device__ __forceinline__ void unpack(float (&a)[8]) const {
+    a[0] = lo.x; a[1] = lo.y; a[2] = lo.z; a[3] = lo.w; a[4] = hi.x; a[5] = hi.y; a[6] = hi.z; a[7] = hi.w;
+  }
+};
+
+// eps as the torch-native formula sees it: amax is clamped in the input dtype, so bf16 sees eps rounded to bf16
+inline float quant_eps(float eps, int in_dtype) {
+  if (in_dtype != FP8K_BF16) return eps;
+  uint32_t u;
+  memcpy(&u, &eps, 4);
+  u = ((u + 0x7fffu + ((u >> 16) & 1u)) >> 16) << 16;
+  memcpy(&eps, &u, 4);
+  return eps;
+}
+
+__device__ __forceinline__ float absmax8(const float (&a)[8]) {
+  float m = fmaxf(fabsf(a[0]), fabsf(a[1]));
+  m = fmaxf(fmaxf(m, fabsf(a[2])), fabsf(a[3]));
+  m = fmaxf(fmaxf(m, fabsf(a[4])), fabsf(a[5]));
+  m = fmaxf(fmaxf(m, fabsf(a[6])), fabsf(a[7]));
+  return m;
+}
 
 // q = RNE_e4m3fn(clamp(RN32(a / sc))) for 8 values - bit-identical to an IEEE float32 divide followed by the
 // cast - without a divide and without a branch.  The quotient is bracketed by two multiplies with reciprocals

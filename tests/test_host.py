@@ -84,6 +84,31 @@ def test_linears_are_the_dispatcher_path(dev, dispatcher, m, n, k, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 8, 128), (16, 136, 2048), (15, 1000, 128), (8, 4104, 4096), (7, 16376, 640), (1, 72, 18432), (2, 520, 8320),
+                                   (1, 264, 32768), (3, 128, 10880)])
+def test_quantising_decode_linear(dev, dispatcher, m, n, k):
+    """One launch with the quantisation in it: smallest and largest activations it takes, rows of one to 256 groups, remainders of
+    lane pieces, wave shares and weight rows, outliers, an all-zero row, a subnormal group scale; bit for bit the two launches."""
+    from sglang_amd._lib import lib
+
+    assert lib.fp8k_linear_fuses_quant(m, n, k) == 1
+    assert lib.fp8k_linear_fuses_quant(32768 // k + 1, n, k) == 0 and lib.fp8k_linear_fuses_quant(17, n, k) == 0
+    w, s = _weight(n, k)
+    for dtype in (torch.bfloat16, torch.float16):
+        x = _randn((m, k), dtype)
+        x[:, ::97] *= 50
+        x[m // 2, :128] *= 1e-7
+        x[m - 1] = 0 if m > 1 else x[m - 1]
+        for bias in (None, _randn((n,), dtype, 2), _randn((n,), torch.float32, 2)):
+            calls = [lambda: fp8_utils.apply_fp8_linear(x, w.t(), torch.rand((n, 1), generator=torch.Generator().manual_seed(4)).to(dev),
+                                                        bias=bias, use_per_token_if_dynamic=True)]
+            if bias is None or bias.dtype == dtype:
+                calls.append(lambda: fp8_utils.w8a8_block_fp8_linear(x, w, BLOCK, s, bias=bias))
+            for call in calls:
+                assert _same(call(), dispatcher(call))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m,k", [(1, 128), (5, 640), (130, 7168)])
 def test_group_quant_layouts_are_the_dispatcher_path(dev, dispatcher, m, k):
     x = _randn((m, k))
