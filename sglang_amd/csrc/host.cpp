@@ -457,6 +457,9 @@ PyObject* fused_experts(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (topk <= 0 || bm <= 0 || (fuse && (bm != 256 || on_input)) || (balanced && bm != 256)) DECLINE;
 
   const int64_t cap = slots + (E + 1) * (bm - 1), blocks = ceil_div(cap, bm);
+  // what of the table can be in use (a block holds at least one slot, and only an expert's last is not full): the launches
+  // are sized by it, 7168 workgroups less for 2 tokens of 128 experts
+  const int64_t cap_used = std::min(cap, bm * std::min(slots, E + 1 + slots / bm));
   const int64_t kb1 = H / 128, kb2 = I / 128;
   const bool sorted = bm >= 64;  // blocks of 64 slots and more read their activation scales in slot order
   Call c(x);
@@ -495,7 +498,7 @@ PyObject* fused_experts(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (sorted) check(fp8k_moe_sort_scales(s1, ss1, sorted_ids, padded, cap, kb1, topk, slots, kb1, 1, st));
   auto gemm = [&](const void* A, const Tensor& W, const Tensor& Ws, const float* As, int64_t as_m, int64_t as_k, void* C, bool weigh,
                   int64_t per_row) {
-    check(fp8k_moe_block_gemm(A, W.data_ptr(), As, Ws.data_ptr<float>(), C, sorted_ids, block_expert, padded, weigh ? twp : nullptr, cap,
+    check(fp8k_moe_block_gemm(A, W.data_ptr(), As, Ws.data_ptr<float>(), C, sorted_ids, block_expert, padded, weigh ? twp : nullptr, cap_used,
                               bm, slots, per_row, E, W.size(1), W.size(2), W.size(2), as_m, as_k, W.stride(0), W.stride(1), Ws.stride(0),
                               Ws.stride(1), Ws.stride(2), W.size(1), dc, (sorted ? 1 : 0) | (balanced ? 2 : 0), st));
   };

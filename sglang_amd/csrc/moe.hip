@@ -2,6 +2,7 @@
 // GEMM (host side; the device code is the grouped form of gemm_direct_kernel for 16/32-slot blocks, of
 // gemm_stream_kernel for 64/128 and moe_stream256_kernel for 256), silu_and_mul and the top-k sum.  No allocation, no synchronisation, no host reads of device data.
 #include "gemm_direct.h"
+#include "gemm_moe_shortk.h"
 #include "gemm_moe256.h"
 
 namespace fp8k {
@@ -444,6 +445,11 @@ static bool moe256_walks(int64_t num_valid_tokens, int64_t num_experts, int64_t 
   return (balanced || num_valid_tokens <= num_experts * 192) && K >= 2 * kTileK;
 }
 
+// blocks that can be in use: every one holds a slot, and only an expert's last (or that of the slots without one) is not full
+static int64_t moe_blocks_in_use(int64_t slots, int64_t num_experts, int64_t block_m, int64_t capacity) {
+  return std::min(capacity, std::min(slots, num_experts + 1 + slots / block_m));
+}
+
 static int moe_block_gemm_impl(const void* A, const void* B, const float* As, const float* Bs, void* C,
                                const int32_t* sorted_token_ids, const int32_t* expert_ids,
                                const int32_t* num_tokens_post_padded, const float* topk_weights,
@@ -498,6 +504,25 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
   hipStream_t st = (hipStream_t)stream;
 #define FP8K_MOE_DIRECT(TM, O) \
   hipLaunchKernelGGL((gemm_direct_kernel<TM, kModeBlock, O, FP8K_F32, false, true>), dim3((unsigned)nwg), dim3(512), 0, st, a)
+  // Short K: a run of tiles per workgroup, where there are more tiles than workgroups (two per CU) to make runs of.  With 16
+  // slots a tile is all weight stream, and from 16 K blocks on a workgroup per tile with eight K blocks in flight is level or
+  // 2 % ahead (128 experts, H = 4096, 8 .. 64 tokens, K = 2048); with 32 slots the run is ahead at every K that fits.
+  const int64_t blocks_max = moe_blocks_in_use(num_valid_tokens, num_experts, block_m, a.m_blocks);
+  const int64_t most = 2 * (int64_t)num_cu() / 8 * 8;
+  if (direct && K <= (block_m == 16 ? kMoeShortKMax / 2 : kMoeShortKMax) && blocks_max * a.tiles_n > most && N * ldb < (1LL << 31)) {
+    const dim3 grid((unsigned)most), block(512);
+    const unsigned lds = (unsigned)(block_m * moe_shortk_row((int)K));
+#define FP8K_SHORTK(TM, O) hipLaunchKernelGGL((moe_shortk_kernel<TM, O>), grid, block, lds, st, a)
+    if (out_dtype == FP8K_BF16) {
+      if (block_m == 16) FP8K_SHORTK(16, FP8K_BF16);
+      else FP8K_SHORTK(32, FP8K_BF16);
+    } else {
+      if (block_m == 16) FP8K_SHORTK(16, FP8K_F16);
+      else FP8K_SHORTK(32, FP8K_F16);
+    }
+#undef FP8K_SHORTK
+    return check_launch(op);
+  }
   if (direct) {
     if (out_dtype == FP8K_BF16) {
       if (block_m == 16) FP8K_MOE_DIRECT(16, FP8K_BF16);

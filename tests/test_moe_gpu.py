@@ -411,6 +411,39 @@ def test_grouped_gemm_256_slot_blocks_every_group_count(dev):
             assert torch.equal(outs[0], C)
 
 
+@pytest.mark.parametrize("T,E,topk,N,K,block", [(64, 40, 2, 2056, 128, 16), (70, 24, 3, 3080, 384, 16), (33, 40, 1, 2048, 1024, 16),
+                                                (90, 64, 4, 1160, 640, 32), (200, 8, 4, 2568, 2048, 32), (130, 96, 6, 1032, 256, 32)])
+def test_grouped_gemm_short_k_runs_exact(dev, T, E, topk, N, K, block):
+    """More tiles than workgroups, so that each takes a run of them: runs that start and end inside a block, blocks of one slot and
+    full ones, one to 16 K blocks, a last tile of 8 weight rows, ids of -1 (stored as zeros); exact on integer data."""
+    from sglang_amd.fused_moe import moe_align_block_size
+    from sglang_amd.sgl_kernel import moe_block_gemm
+
+    g = torch.Generator().manual_seed(K + T)
+    pow2 = lambda *s: 2.0 ** torch.randint(-3, 3, s, generator=g).float()  # noqa: E731
+    x, w = (torch.randint(-4, 5, s, generator=g).float() for s in ((T, K), (E, N, K)))
+    xs, ws = pow2(T, K // 128), pow2(E, (N + 127) // 128, K // 128)
+    ids = torch.rand((T, E), generator=g).argsort(dim=1)[:, :topk].int()
+    ids[:T // 3, 0] = 1  # one expert with full blocks
+    ids[torch.rand(ids.shape, generator=g) < 0.05] = -1
+    tw = pow2(T, topk)
+    sorted_ids, expert_ids, npad = moe_align_block_size(ids.to(dev), block, E)
+    for weigh in (False, True):
+        C = torch.full((T * topk, N), float("nan"), dtype=torch.bfloat16, device=dev)
+        moe_block_gemm(x.to(dev).to(torch.float8_e4m3fn), w.to(dev).to(torch.float8_e4m3fn), C, xs.to(dev), ws.to(dev), tw.to(dev), sorted_ids,
+                       expert_ids, npad, weigh, topk, block, ids.numel())
+        got = C.float().cpu()
+        assert not got[ids.flatten() < 0].any()
+        for e in range(E):
+            slots = (ids.flatten() == e).nonzero().flatten()
+            if len(slots):
+                rows = x[slots // topk] * xs[slots // topk].repeat_interleave(128, 1)
+                ref = rows @ (w[e] * ws[e].repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)).t()
+                if weigh:
+                    ref *= tw.flatten()[slots, None]
+                assert torch.equal(got[slots], ref.bfloat16().float())
+
+
 def test_grouped_gemm_random_routings_exact(dev):
     """Forty seeded random routings (1..600 tokens, 2..40 experts, top-1..6, every block size, skewed and absent
     experts, ids of -1) on integer data with power-of-two scales: exact, with per-token and with sorted scales."""
