@@ -851,6 +851,24 @@ def test_moe_fused_gate_bf16_and_ties(dev, dtype, name):
     assert torch.allclose(w0, torch.full_like(w0, 0.125))
 
 
+@pytest.mark.parametrize("params", [(64, 8, 3, 6), (64, 4, 1, 16), (128, 8, 4, 8), (128, 16, 16, 20), (64, 16, 2, 4)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_moe_fused_gate_forms_agree(dev, params, dtype):
+    """Many rows take the form with a lane per expert group, few rows a wavefront per row: the same picks and weights bit for bit,
+    ties included (16-bit inputs, logits from a small set, biases that leave fewer finite choices than picks)."""
+    from sglang_amd.sgl_kernel import moe_fused_gate
+
+    E, G, tg, topk = params
+    g = torch.Generator().manual_seed(E + G)
+    x, bias = torch.randn((8197, E), generator=g), torch.randn((E,), generator=g) * 0.1
+    x[1::3] = torch.randint(-2, 3, x[1::3].shape, generator=g).float()
+    for b in (bias, torch.zeros(E), torch.where(torch.arange(E) % 8 == 3, bias, torch.tensor(-float("inf")))):
+        for shared, scale_out in ((0, True), (1, False)):
+            many = moe_fused_gate(x.to(dtype).to(dev), b.to(dtype).to(dev), G, tg, topk, shared, 2.5, scale_out)
+            few = moe_fused_gate(x[-77:].to(dtype).to(dev), b.to(dtype).to(dev), G, tg, topk, shared, 2.5, scale_out)
+            assert torch.equal(many[0][-77:], few[0]) and torch.equal(many[1][-77:], few[1])
+
+
 def test_biased_grouped_topk_is_the_gate_kernel_and_matches_the_tensor_op_restatement(dev):
     """The layer-level routing entry point runs the fused gate kernel; on well-separated float32 logits its expert sets
     and weights are those of the tensor-op restatement of topk.py:665-738 kept with the tests.  Shapes the kernel does
