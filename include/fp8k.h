@@ -186,16 +186,19 @@ int fp8k_scaled_mm_strided(const void* A, const void* B, const float* sa, int64_
 int64_t fp8k_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
- * A whole linear of a few rows in one launch: the group quantisation (fp8k_group_quant, group 128, float scales) or the
- * per-token one (fp8k_token_quant) of the 16-bit activations x [M, K] (contiguous), then fp8k_block_gemm_bias resp.
- * fp8k_scaled_mm_strided on them; the results are those of the two calls bit for bit.  Only for the sizes for which
- * fp8k_linear_fuses_quant returns 1 (few activations: every workgroup quantises them for itself).  dtype: of x and C.
+ * A whole linear on 16-bit activations x [M, K] (contiguous): the group quantisation (fp8k_group_quant, group 128, float
+ * scales; K a multiple of 128) or the per-token one (fp8k_token_quant; K a multiple of 16), then fp8k_block_gemm_bias resp.
+ * fp8k_scaled_mm_strided; the results are those of the two calls bit for bit.  A few rows (the sizes for which
+ * fp8k_linear_fuses_quant returns 1) take one launch.  dtype: of x and C.  Workspace: 256-byte aligned, fp8k_linear_workspace_bytes of it (0 possible), nothing in it has to be initialised.
  */
 int fp8k_linear_fuses_quant(int64_t M, int64_t N, int64_t K);
+int64_t fp8k_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int block_mode);
 int fp8k_block_linear(const void* x, const void* B, const float* Bs, const void* bias, void* C, int64_t M, int64_t N, int64_t K,
-                      int64_t ldb, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, float eps, int dtype, void* stream);
+                      int64_t ldb, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, float eps, int dtype, void* workspace,
+                      int64_t workspace_bytes, void* stream);
 int fp8k_token_linear(const void* x, const void* B, const float* sb, int64_t sb_stride, const void* bias, int bias_dtype, void* C,
-                      int64_t M, int64_t N, int64_t K, int64_t ldb, int64_t ldc, int dtype, void* stream);
+                      int64_t M, int64_t N, int64_t K, int64_t ldb, int64_t ldc, int dtype, void* workspace, int64_t workspace_bytes,
+                      void* stream);
 
 /*
  * Per-tensor FP8 quantisation of a strided [H, S, D] tensor into a contiguous [H, S, D] one (the activations of the

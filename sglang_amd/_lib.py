@@ -77,8 +77,9 @@ SIGNATURES = {
     ),
     "fp8k_scaled_mm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "fp8k_linear_fuses_quant": (_c_int, [_c_i64] * 3),
-    "fp8k_block_linear": (_c_int, [_c_ptr] * 5 + [_c_i64] * 7 + [_c_f32, _c_int, _c_ptr]),
-    "fp8k_token_linear": (_c_int, [_c_ptr] * 3 + [_c_i64, _c_ptr, _c_int, _c_ptr] + [_c_i64] * 5 + [_c_int, _c_ptr]),
+    "fp8k_linear_workspace_bytes": (_c_i64, [_c_i64] * 3 + [_c_int]),
+    "fp8k_block_linear": (_c_int, [_c_ptr] * 5 + [_c_i64] * 7 + [_c_f32, _c_int, _c_ptr, _c_i64, _c_ptr]),
+    "fp8k_token_linear": (_c_int, [_c_ptr] * 3 + [_c_i64, _c_ptr, _c_int, _c_ptr] + [_c_i64] * 5 + [_c_int, _c_ptr, _c_i64, _c_ptr]),
     "fp8k_tune_force_gemm_plan": (None, [_c_int, _c_int]),
     "fp8k_tune_stream_read": (_c_int, [_c_ptr, _c_i64, _c_ptr]),
     "fp8k_tune_stream_read_tiles": (_c_int, [_c_ptr, _c_i64, _c_i64, _c_ptr]),

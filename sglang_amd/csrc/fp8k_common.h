@@ -17,6 +17,10 @@ int fail(int code, const char* fmt, ...);
 void clear_error();
 int num_cu();  // compute units of the current device (256 when no device is visible)
 
+// the quantisation of a linear's 16-bit activations (quant.hip; operands checked by the caller): in groups of 128 with
+// column-major scales, or per token
+int quant_for_linear(bool groups, const void* x, void* q, float* s, int64_t M, int64_t K, float eps, int dtype, hipStream_t st);
+
 #define FP8K_REQUIRE(cond, ...)                                   \
   do {                                                            \
     if (!(cond)) return ::fp8k::fail(FP8K_ERR_INVALID, __VA_ARGS__); \

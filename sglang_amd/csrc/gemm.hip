@@ -7,6 +7,7 @@
 #include "gemm_bmm.h"
 #include "gemm_direct.h"
 #include "gemm_direct_quant.h"
+#include "gemm_skinny.h"
 #include "gemm_tile128.h"
 
 #include "../../include/fp8k_tune.h"
@@ -15,12 +16,13 @@ namespace fp8k {
 
 struct Plan {
   int kind;    // 0 = generic, 1 = tile256, 2 = weight-streaming through LDS (33..128 rows), 3 = direct (<= 32 rows),
-               // 4 = tile128, 5 = direct with K cut across the waves of a workgroup (<= 32 rows, N below 16 K)
+               // 4 = tile128, 5 = direct with K cut across the waves of a workgroup (<= 16 rows, N below 16 K), 7 = skinny
+               // strips over all of K (<= 64 rows, N up to 16 K)
   int splits;  // >1: split-K through the float workspace
   int kb_per_split;
   int tm;      // rows per block of the streaming kernels
   int tail_first;   // tile256: first tile that is cut along K or into halves (== number of tiles when none is)
-  int halves;       // tile256: the tiles from tail_first on are computed as two 128-row halves
+  int halves;       // tile256: the tiles from tail_first on are computed as two 128-row halves; kinds 5, 7: waves along n
   int64_t ws_bytes; // float workspace the plan needs
 };
 
@@ -76,7 +78,7 @@ constexpr int64_t kWaveKMaxN = 16384;
 static Plan plan_wavek(int64_t M, int64_t N, int64_t K) {
   Plan pl{5, 1, 0, 0, 0, 0};
   const int kb = (int)(K / kTileK);
-  pl.tm = M <= 16 ? 16 : 32;
+  pl.tm = 16;
   // waves along n: the choice that leaves the busiest CU the fewest weight rows (workgroups go two to a CU at most);
   // among equals the widest workgroup whose waves still get at most 16 K blocks each (measured: wider workgroups
   // re-read less of the activations, longer per-wave K ranges start to serialise)
@@ -95,14 +97,36 @@ static Plan plan_wavek(int64_t M, int64_t N, int64_t K) {
   pl.kb_per_split = (kb + 8 / nw - 1) / (8 / nw);
   return pl;
 }
-// Which of the two decode kernels: every workgroup of the wave-cut kernel reads all of the activations' K range for its
-// 16 * nw weight rows, so its traffic through the CUs' load path grows with the rows of the batch; the workgroup-cut
-// kernel shares the activations among 128 weight rows but pays float partials and a reduction launch.  Measured
-// (M = 1 .. 32 on the DeepSeek-V3 and Llama projection shapes): the wave cut wins for up to 8 rows, and for up to 32
-// rows while the weights are at most about 24 MB.
-static bool prefers_wavek(int64_t M, int64_t N, int64_t K) {
-  if (N >= kWaveKMaxN) return false;  // 128 and more tiles of 128 rows: the workgroup-cut kernel runs uncut
-  return M <= 8 || N * K <= (24LL << 20);
+// Up to 64 rows: the strips of weight rows that one workgroup each runs over all of K are as narrow as leaves every CU one.
+constexpr int64_t kSkinnyMaxN = 16384;
+static Plan plan_skinny(int64_t M, int64_t N, int64_t K) {
+  Plan pl{7, 1, 0, 0, 0, 0};
+  pl.tm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  pl.halves = N <= 16 * num_cu() ? 1 : N <= 32 * num_cu() ? 2 : 4;
+  if (g_force_kind == 7 && (g_force_splits == 1 || g_force_splits == 2 || g_force_splits == 4)) pl.halves = g_force_splits;  // tuning aid
+  return pl;
+}
+// Where it is ahead (M = 4 .. 64 x 16 widths up to 20480 x 9 depths up to 18432, timed against the other decode kernels and the
+// 128-row tiles under every K cut: what the rule takes is within 1 % of the best on average up to 32 rows, 4 % above):
+//  * more than 64 weight rows per CU's strip cost more activation traffic than a K cut costs partials, from 9 rows on;
+//  * that traffic grows with rows x K: above 32 rows a K of more than 8192 is left to the 128-row tiles with a K cut, and with
+//    64-row strips, whose waves have little of the LDS traffic to hide it behind, K of more than 4096 unless they fill the chip;
+//  * 17 .. 32 rows in 64-row strips that leave a quarter of the CUs idle: up to K = 6144.
+static bool prefers_skinny(int64_t M, int64_t N, int64_t K) {
+  if (M > kSkinnyMaxM || N > kSkinnyMaxN) return false;
+  const bool wide = N > 32 * num_cu(), fills = N >= 48 * num_cu();
+  if (M <= 8) return K <= 9216;  // above: the wave-cut kernel, whose waves keep all of their K range in flight
+  if (M <= 16) return true;
+  if (M <= 32) return !wide || fills || K <= 6144;
+  return wide ? K >= 1024 && K <= (fills ? 10240 : 4096) : K <= 8192;
+}
+// Activations few enough for every workgroup to quantise them for itself (gemm_wavek_quant_kernel): up to 16 rows of at most
+// kQuantFuseMax elements together.  The share of the quantisation grows with M * K while the launch it saves does not (the gain
+// falls from 1.5 .. 1.85 times at 4096 elements to 1.2 .. 1.3 at 32768; twice as many would take another 32 registers per lane
+// and with them the second workgroup of a CU).  The GEMM of these sizes is the wave-cut kernel's also where the activations come
+// quantised, so that a linear's result does not depend on the way it took.
+static bool few_activations(int64_t M, int64_t N, int64_t K) {
+  return M <= 16 && M * K <= kQuantFuseMax && N < kWaveKMaxN && (M <= 8 || N * K <= (24LL << 20));
 }
 
 // up to 128 rows: stream the weights once, every CU takes a K slice of one 256-row weight tile
@@ -150,10 +174,13 @@ static Plan plan_tile256(int64_t M, int64_t N, int64_t K) {
 static Plan plan_base(int64_t M, int64_t N, int64_t K) {
   const bool fits32 = M * K < (1LL << 31);
   if (g_force_kind == 3 && M <= 32 && fits32) return plan_direct(M, N, K);
-  if (g_force_kind == 5 && M <= 32 && fits32) return plan_wavek(M, N, K);
+  if (g_force_kind == 5 && M <= 16 && fits32) return plan_wavek(M, N, K);
+  if (g_force_kind == 7 && M <= kSkinnyMaxM && fits32) return plan_skinny(M, N, K);
   if (g_force_kind == 2 && M <= 128 && fits32) return plan_stream(M, N, K);
   if (g_force_kind == 1) return plan_tile256(M, N, K);
-  if (M <= 32 && fits32 && prefers_wavek(M, N, K)) return plan_wavek(M, N, K);
+  if (fits32 && few_activations(M, N, K)) return plan_wavek(M, N, K);
+  if (fits32 && prefers_skinny(M, N, K)) return plan_skinny(M, N, K);
+  if (fits32 && M <= 8 && N < kWaveKMaxN) return plan_wavek(M, N, K);
   if (M <= 32 && fits32) return plan_direct(M, N, K);
   if (M <= 128 && fits32) return plan_stream(M, N, K);
   return plan_tile256(M, N, K);
@@ -226,11 +253,15 @@ static int64_t workspace_bytes(int64_t M, int64_t N, int64_t K) {
 // them into column-major order behind the float partials (a few microseconds for at most M*K/128 floats) and
 // runs on the copy; fp8k_block_gemm_workspace_bytes counts that area for every call that could need it.
 static int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
-static bool wants_scale_copy(const Plan& pl, int64_t M) { return M > 32 && (pl.kind == 1 || pl.kind == 2 || pl.kind == 4); }
+// The skinny kernel's waves fetch 16 scales per load instead of 32: there the copy (2 - 3 us) is level at 16 rows x 128 K blocks
+// and ahead above (without it 32 x 128 takes 34.8 us against 27.4 with column-major scales, 64 x 64 32.4 against 21.1).
+static bool wants_scale_copy(const Plan& pl, int64_t M, int64_t K) {
+  return pl.kind == 7 ? M * (K / kTileK) >= 2048 : M > 32 && (pl.kind == 1 || pl.kind == 2 || pl.kind == 4);
+}
 static int64_t block_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const Plan pl = make_plan(M, N, K);
-  return wants_scale_copy(pl, M) ? align256(pl.ws_bytes) + M * ((K + kTileK - 1) / kTileK) * 4 : pl.ws_bytes;
+  return wants_scale_copy(pl, M, K) ? align256(pl.ws_bytes) + M * ((K + kTileK - 1) / kTileK) * 4 : pl.ws_bytes;
 }
 __global__ __launch_bounds__(256) void scale_to_column_major_kernel(const float* __restrict__ src, float* __restrict__ dst,
                                                                     int M, int kb, int64_t stride_m) {
@@ -324,9 +355,26 @@ static int launch(const GemmArgs& a0, const Plan& pl, hipStream_t st) {
   if (pl.kind == 5) {
     a.wk_nw = pl.halves;
     const unsigned nwg = (unsigned)((a.N + 16 * a.wk_nw - 1) / (16 * a.wk_nw));
-    if (pl.tm == 16) hipLaunchKernelGGL((gemm_wavek_kernel<16, MODE, OUT_DT, BIAS_DT>), dim3(nwg), dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((gemm_wavek_kernel<32, MODE, OUT_DT, BIAS_DT>), dim3(nwg), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((gemm_wavek_kernel<MODE, OUT_DT, BIAS_DT>), dim3(nwg), dim3(512), 0, st, a);
     return check_launch("gemm_wavek");
+  }
+  if (pl.kind == 7) {
+    a.wk_nw = pl.halves;
+    a.tiles_n = (a.N + 16 * a.wk_nw - 1) / (16 * a.wk_nw);
+    const dim3 grid((unsigned)((a.tiles_n + 7) / 8 * 8));
+#define FP8K_SKINNY(TM, NW) hipLaunchKernelGGL((gemm_skinny_kernel<TM, NW, MODE, OUT_DT, BIAS_DT>), grid, dim3(TM <= 32 ? 640 : 768), 0, st, a)
+#define FP8K_SKINNY_NW(TM)                    \
+  do {                                        \
+    if (pl.halves == 1) FP8K_SKINNY(TM, 1);   \
+    else if (pl.halves == 2) FP8K_SKINNY(TM, 2); \
+    else FP8K_SKINNY(TM, 4);                  \
+  } while (0)
+    if (pl.tm == 16) FP8K_SKINNY_NW(16);
+    else if (pl.tm == 32) FP8K_SKINNY_NW(32);
+    else FP8K_SKINNY_NW(64);
+#undef FP8K_SKINNY_NW
+#undef FP8K_SKINNY
+    return check_launch("gemm_skinny");
   }
   if (pl.kind == 2) {
     a.m_blocks = 1;
@@ -397,7 +445,7 @@ static int block_gemm_impl(const void* A, const void* B, const float* As, const 
                "fp8_blockwise_scaled_mm: scales_a spans more than 3.5 GiB");
   const Plan pl = make_plan(M, N, K);
   const int64_t kb = (K + kTileK - 1) / kTileK;
-  const int64_t need = wants_scale_copy(pl, M) ? align256(pl.ws_bytes) + M * kb * 4 : pl.ws_bytes;
+  const int64_t need = wants_scale_copy(pl, M, K) ? align256(pl.ws_bytes) + M * kb * 4 : pl.ws_bytes;
   if (need > 0 && (!workspace || workspace_bytes_given < need))
     return fail(FP8K_ERR_WORKSPACE, "fp8_blockwise_scaled_mm: workspace of %lld bytes required, %lld given",
                 (long long)need, (long long)(workspace ? workspace_bytes_given : 0));
@@ -407,7 +455,7 @@ static int block_gemm_impl(const void* A, const void* B, const float* As, const 
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = lda; a.ldw = ldb; a.ldc = ldc;
   a.sx_m = as_stride_m; a.sx_k = as_stride_k; a.sw_n = bs_stride_n; a.sw_k = bs_stride_k;
   hipStream_t st = (hipStream_t)stream;
-  if (wants_scale_copy(pl, M) && as_stride_k == 1 && as_stride_m > 1 && kb > 1) {
+  if (wants_scale_copy(pl, M, K) && as_stride_k == 1 && as_stride_m > 1 && kb > 1) {
     float* cm = reinterpret_cast<float*>(static_cast<char*>(workspace) + align256(pl.ws_bytes));
     hipLaunchKernelGGL(scale_to_column_major_kernel, dim3((unsigned)((M * kb + 255) / 256)), dim3(256), 0, st, As, cm, (int)M,
                        (int)kb, as_stride_m);
@@ -576,14 +624,10 @@ extern "C" int fp8k_scaled_mm_strided(const void* A, const void* B, const float*
 #undef FP8K_SMM
 }
 
-// ---- decode linears of a few rows, quantisation included (gemm_wavek_quant_kernel)
-// Up to 16 rows of at most kQuantFuseMax elements together, where the wave-cut kernel would take the GEMM: every workgroup
-// repeats the quantisation, whose share grows with M * K while the launch it saves does not (the gain falls from 1.5 .. 1.85
-// times at 4096 elements to 1.2 .. 1.3 at 32768; twice as many would take another 32 registers per lane and with them the
-// second workgroup of a CU).
+// ---- whole linears, quantisation included.  Of a few rows: one launch (gemm_wavek_quant_kernel).
 static bool fuses_quant(int64_t M, int64_t N, int64_t K) {
-  if (M < 1 || M > 16 || N < 1 || N % 8 != 0 || K < kTileK || K % kTileK != 0 || M * K > kQuantFuseMax) return false;
-  return g_force_kind < 0 && prefers_wavek(M, N, K);
+  if (M < 1 || N < 1 || N % 8 != 0 || K < kTileK || K % kTileK != 0) return false;
+  return g_force_kind < 0 && few_activations(M, N, K);
 }
 
 template <int MODE, int OUT_DT, int BIAS_DT>
@@ -597,48 +641,91 @@ static int launch_quant_linear(const GemmArgs& a, hipStream_t st) {
   return check_launch("gemm_wavek_quant");
 }
 
+// Workspace of a linear: the quantised activations, their scales, what the GEMM's plan needs.
+struct LinearLayout {
+  Plan pl{};
+  int64_t s = 0, work = 0, bytes = 0;  // offsets behind the quantised activations at 0
+};
+static LinearLayout linear_layout(int64_t M, int64_t N, int64_t K, bool block_mode) {
+  LinearLayout l;
+  l.pl = make_plan(M, N, K);
+  l.s = align256(M * K);
+  l.work = l.s + align256(M * (block_mode ? K / kTileK : 1) * 4);
+  l.bytes = l.work + l.pl.ws_bytes;
+  return l;
+}
+
 static int quant_linear(const char* op, bool block_mode, const void* x, const void* B, const float* Bs, int64_t bs_n, int64_t bs_k,
                         const void* bias, int bias_dtype, void* C, int64_t M, int64_t N, int64_t K, int64_t ldb, int64_t ldc, float eps,
-                        int dtype, void* stream) {
+                        int dtype, void* workspace, int64_t workspace_bytes_given, void* stream) {
   clear_error();
   int rc = common_checks(op, x, B, C, M, N, K, K, ldb, ldc, dtype);
   if (rc) return rc;
-  FP8K_REQUIRE(fuses_quant(M, N, K), "%s: M=%lld N=%lld K=%lld is not a size of the one-launch form (fp8k_linear_fuses_quant)", op,
-               (long long)M, (long long)N, (long long)K);
+  if (M == 0 || N == 0) return FP8K_OK;
+  FP8K_REQUIRE(K > 0 && (!block_mode || K % kTileK == 0), "%s: K must be a positive multiple of %d (got %lld)", op, block_mode ? kTileK : 16,
+               (long long)K);
   FP8K_REQUIRE(Bs, "%s: null scale pointer", op);
   FP8K_REQUIRE(bs_n >= 0 && bs_k >= 0, "%s: negative scale stride", op);
   FP8K_REQUIRE(block_mode || ((bs_n == 0 || bs_n == 1) && (bs_n == 0 || aligned(Bs, 16))),
                "%s: channel scales must be contiguous and 16-byte aligned", op);
+  FP8K_REQUIRE(!block_mode || M * (K / kTileK) < 0x38000000LL, "%s: activation scales span more than 3.5 GiB", op);
   FP8K_REQUIRE(!bias || bias_dtype == FP8K_F32 || bias_dtype == FP8K_F16 || bias_dtype == FP8K_BF16,
                "%s: bias dtype must be float32, float16 or bfloat16", op);
-  const Plan pl = plan_wavek(M, N, K);
+  const int bd = bias ? bias_dtype : FP8K_F32;
   GemmArgs a{};
   a.X = (const uint8_t*)x; a.W = (const uint8_t*)B; a.sw = Bs; a.bias = bias; a.C = C;
-  a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldw = ldb; a.ldc = ldc;
-  a.sw_n = bs_n; a.sw_k = bs_k; a.q_eps = quant_eps(eps, dtype);
-  a.wk_nw = pl.halves; a.kb_per_split = pl.kb_per_split;
+  a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = K; a.ldw = ldb; a.ldc = ldc;
+  a.sw_n = bs_n; a.sw_k = bs_k;
   hipStream_t st = (hipStream_t)stream;
-  if (block_mode)
-    return dtype == FP8K_BF16 ? launch_quant_linear<kModeBlock, FP8K_BF16, FP8K_BF16>(a, st)
-                              : launch_quant_linear<kModeBlock, FP8K_F16, FP8K_F16>(a, st);
-  const int bd = bias ? bias_dtype : FP8K_F32;
-#define FP8K_QL(O) (bd == FP8K_F32    ? launch_quant_linear<kModeRow, O, FP8K_F32>(a, st) \
-                    : bd == FP8K_BF16 ? launch_quant_linear<kModeRow, O, FP8K_BF16>(a, st) \
-                                      : launch_quant_linear<kModeRow, O, FP8K_F16>(a, st))
-  return dtype == FP8K_BF16 ? FP8K_QL(FP8K_BF16) : FP8K_QL(FP8K_F16);
+#define FP8K_QL(FN, O, ...) (bd == FP8K_F32    ? FN<kModeRow, O, FP8K_F32>(__VA_ARGS__) \
+                             : bd == FP8K_BF16 ? FN<kModeRow, O, FP8K_BF16>(__VA_ARGS__) \
+                                               : FN<kModeRow, O, FP8K_F16>(__VA_ARGS__))
+#define FP8K_LINEAR(FN, ...)                                                                                                      \
+  (block_mode ? (dtype == FP8K_BF16 ? FN<kModeBlock, FP8K_BF16, FP8K_BF16>(__VA_ARGS__) : FN<kModeBlock, FP8K_F16, FP8K_F16>(__VA_ARGS__)) \
+   : dtype == FP8K_BF16 ? FP8K_QL(FN, FP8K_BF16, __VA_ARGS__)                                                                     \
+                        : FP8K_QL(FN, FP8K_F16, __VA_ARGS__))
+  if (fuses_quant(M, N, K)) {
+    const Plan pl = plan_wavek(M, N, K);
+    a.q_eps = quant_eps(eps, dtype);
+    a.wk_nw = pl.halves; a.kb_per_split = pl.kb_per_split;
+    return FP8K_LINEAR(launch_quant_linear, a, st);
+  }
+  const LinearLayout l = linear_layout(M, N, K, block_mode);
+  if (!workspace || workspace_bytes_given < l.bytes)
+    return fail(FP8K_ERR_WORKSPACE, "%s: workspace of %lld bytes required, %lld given", op, (long long)l.bytes,
+                (long long)(workspace ? workspace_bytes_given : 0));
+  FP8K_REQUIRE(aligned(workspace, 256), "%s: the workspace must be 256-byte aligned", op);
+  char* const ws = static_cast<char*>(workspace);
+  float* const s = reinterpret_cast<float*>(ws + l.s);
+  rc = quant_for_linear(block_mode, x, ws, s, M, K, eps, dtype, st);
+  if (rc) return rc;
+  a.X = reinterpret_cast<const uint8_t*>(ws);
+  a.sx = s; a.sx_m = 1; a.sx_k = block_mode ? M : 0;
+  a.partial = reinterpret_cast<float*>(ws + l.work);
+  return FP8K_LINEAR(launch, a, l.pl, st);
+#undef FP8K_LINEAR
 #undef FP8K_QL
 }
 
 extern "C" int fp8k_linear_fuses_quant(int64_t M, int64_t N, int64_t K) { return fuses_quant(M, N, K) ? 1 : 0; }
 
+extern "C" int64_t fp8k_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int block_mode) {
+  if (M <= 0 || N <= 0 || K <= 0 || fuses_quant(M, N, K)) return 0;
+  return linear_layout(M, N, K, block_mode != 0).bytes;
+}
+
 extern "C" int fp8k_block_linear(const void* x, const void* B, const float* Bs, const void* bias, void* C, int64_t M, int64_t N, int64_t K,
-                                 int64_t ldb, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, float eps, int dtype, void* stream) {
-  return quant_linear("block_linear", true, x, B, Bs, bs_stride_n, bs_stride_k, bias, dtype, C, M, N, K, ldb, ldc, eps, dtype, stream);
+                                 int64_t ldb, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, float eps, int dtype, void* workspace,
+                                 int64_t workspace_bytes_given, void* stream) {
+  return quant_linear("block_linear", true, x, B, Bs, bs_stride_n, bs_stride_k, bias, dtype, C, M, N, K, ldb, ldc, eps, dtype, workspace,
+                      workspace_bytes_given, stream);
 }
 
 extern "C" int fp8k_token_linear(const void* x, const void* B, const float* sb, int64_t sb_stride, const void* bias, int bias_dtype,
-                                 void* C, int64_t M, int64_t N, int64_t K, int64_t ldb, int64_t ldc, int dtype, void* stream) {
-  return quant_linear("token_linear", false, x, B, sb, sb_stride, 0, bias, bias_dtype, C, M, N, K, ldb, ldc, 0.f, dtype, stream);
+                                 void* C, int64_t M, int64_t N, int64_t K, int64_t ldb, int64_t ldc, int dtype, void* workspace,
+                                 int64_t workspace_bytes_given, void* stream) {
+  return quant_linear("token_linear", false, x, B, sb, sb_stride, 0, bias, bias_dtype, C, M, N, K, ldb, ldc, 0.f, dtype, workspace,
+                      workspace_bytes_given, stream);
 }
 
 // ---- batched per-tensor-scaled FP8 GEMM (the MLA absorbed products): every batch entry is a row-mode GEMM on the short-K

@@ -272,10 +272,9 @@ __global__ __launch_bounds__(512, 2) void gemm_direct_kernel(const GemmArgs p) {
 // D K blocks of weights, activations and scales in flight.  At the end the 8 accumulator sets are summed through LDS
 // in ascending ks (a fixed order: results do not depend on timing) and the ks = 0 waves write the output.
 // ------------------------------------------------------------------------------------------------
-template <int TM, int MODE, int OUT_DT, int BIAS_DT>
+template <int MODE, int OUT_DT, int BIAS_DT>
 __global__ __launch_bounds__(512, 2) void gemm_wavek_kernel(const GemmArgs p) {
-  static_assert(TM == 16 || TM == 32, "gemm_wavek_kernel: 16 or 32 rows");
-  constexpr int MS = TM / 16;
+  constexpr int MS = 1;  // up to 16 rows
   constexpr int D = 4;  // K blocks in flight per wave
   __shared__ __attribute__((aligned(16))) uint8_t wl[8][16 * kTileK];  // per wave: one K block of its 16 weight rows
   __shared__ __attribute__((aligned(16))) float red[8][MS][64][4];

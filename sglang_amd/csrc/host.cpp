@@ -255,19 +255,10 @@ PyObject* block_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = N;
   Tensor out = empty(shape, dt, x.device());
-  if (fp8k_linear_fuses_quant(M, N, K)) {
-    check(fp8k_block_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(),
-                            M, N, K, K, ws.stride(0), ws.stride(1), N, kEps, code(dt), c.stream));
-    return THPVariable_Wrap(std::move(out));
-  }
-  const int64_t kb = K / 128, wsb = fp8k_block_gemm_workspace_bytes(M, N, K);
-  Scratch mem(Scratch::room(M * K) + Scratch::room(M * kb * 4) + Scratch::room(wsb), c.stream);
-  void* q = mem.take(M * K);
-  float* s = mem.take<float>(M * kb * 4);
-  void* work = mem.take(wsb);
-  check(fp8k_group_quant(x.data_ptr(), q, s, M, K, 128, kEps, -448.f, 448.f, code(dt), 1, M, FP8K_SCALE_F32, c.stream));
-  check(fp8k_block_gemm_bias(q, w.data_ptr(), s, ws.data_ptr<float>(), bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(), M, N, K,
-                             K, K, 1, M, ws.stride(0), ws.stride(1), N, code(dt), wsb ? work : nullptr, wsb, c.stream));
+  const int64_t wsb = fp8k_linear_workspace_bytes(M, N, K, 1);
+  Scratch mem(wsb, c.stream);
+  check(fp8k_block_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(), M,
+                          N, K, K, ws.stride(0), ws.stride(1), N, kEps, code(dt), wsb ? mem.take(wsb) : nullptr, wsb, c.stream));
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -336,21 +327,11 @@ PyObject* token_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = N;
   Tensor out = empty(shape, dt, x.device());
-  if (fp8k_linear_fuses_quant(M, N, K)) {
-    check(fp8k_token_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), ws.numel() == 1 ? 0 : 1, bias.defined() ? bias.data_ptr() : nullptr,
-                            bias.defined() ? code(bias.scalar_type()) : FP8K_F32, out.data_ptr(), M, N, K, N > 1 ? w.stride(1) : K, N, code(dt),
-                            c.stream));
-    return THPVariable_Wrap(std::move(out));
-  }
-  const int64_t wsb = fp8k_scaled_mm_workspace_bytes(M, N, K);
-  Scratch mem(Scratch::room(M * K) + Scratch::room(M * 4) + Scratch::room(wsb), c.stream);
-  void* q = mem.take(M * K);
-  float* s = mem.take<float>(M * 4);
-  void* work = mem.take(wsb);
-  check(fp8k_token_quant(x.data_ptr(), q, s, M, K, code(dt), c.stream));
-  check(fp8k_scaled_mm_strided(q, w.data_ptr(), s, 1, ws.data_ptr<float>(), ws.numel() == 1 ? 0 : 1,
-                       bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(), M, N, K, K, N > 1 ? w.stride(1) : K, N, code(dt), bias.defined() ? code(bias.scalar_type()) : FP8K_F32,
-                       wsb ? work : nullptr, wsb, c.stream));
+  const int64_t wsb = fp8k_linear_workspace_bytes(M, N, K, 0);
+  Scratch mem(wsb, c.stream);
+  check(fp8k_token_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), ws.numel() == 1 ? 0 : 1, bias.defined() ? bias.data_ptr() : nullptr,
+                          bias.defined() ? code(bias.scalar_type()) : FP8K_F32, out.data_ptr(), M, N, K, N > 1 ? w.stride(1) : K, N, code(dt),
+                          wsb ? mem.take(wsb) : nullptr, wsb, c.stream));
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }

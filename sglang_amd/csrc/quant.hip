@@ -456,6 +456,17 @@ __global__ __launch_bounds__(1024) void rows_tensor_quant_small_kernel(const voi
   if (threadIdx.x == 0) s[0] = sc;
 }
 
+int quant_for_linear(bool groups, const void* x, void* q, float* s, int64_t M, int64_t K, float eps, int dtype, hipStream_t st) {
+  const bool bf = dtype == FP8K_BF16;
+  if (groups)
+    return bf ? launch_group_quant<FP8K_BF16, 128, FP8K_SCALE_F32>(x, q, s, M, K, quant_eps(eps, dtype), 1, M, st)
+              : launch_group_quant<FP8K_F16, 128, FP8K_SCALE_F32>(x, q, s, M, K, quant_eps(eps, dtype), 1, M, st);
+  const dim3 grid((unsigned)M), block(256);
+  if (bf) hipLaunchKernelGGL(token_quant_kernel<FP8K_BF16>, grid, block, 0, st, x, (uint8_t*)q, s, K);
+  else hipLaunchKernelGGL(token_quant_kernel<FP8K_F16>, grid, block, 0, st, x, (uint8_t*)q, s, K);
+  return check_launch("token_quant");
+}
+
 }  // namespace fp8k
 
 using namespace fp8k;

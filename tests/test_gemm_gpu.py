@@ -210,6 +210,35 @@ def test_block_gemm_random_shapes_every_plan(dev):
         assert np.array_equal(c, ref), "case %d: M=%d N=%d K=%d" % (case, M, N, K)
 
 
+@pytest.mark.parametrize("nw", [0, 1, 2, 4])
+def test_skinny_gemm_is_exact_on_integers(dev, nw):
+    """The decode-batch kernel with loading and streaming waves, pinned with every wave layout (0 = the plan's own): one to 33 K blocks
+    (one trip, remainders of a trip, more trips than stages), 9 .. 64 rows around the row counts it is built for, strips that end
+    inside their 16, 32 or 64 rows, both scale layouts, both outputs; exact whatever the order of the sums; then row mode."""
+    from sglang_amd._lib import lib
+    from sglang_amd.sgl_kernel import fp8_scaled_mm
+
+    rng = np.random.default_rng(99 + nw)
+    lib.fp8k_tune_force_gemm_plan(7, nw)
+    try:
+        for case, (M, N, K) in enumerate([(9, 16, 128), (16, 264, 1024), (17, 1000, 128 * 9), (32, 4104, 128 * 17), (33, 520, 128 * 33),
+                                          (64, 72, 128 * 24), (63, 8200, 640), (1, 8, 256)]):
+            xq = O.f32_to_e4m3fn(rng.integers(-4, 5, (M, K)).astype(np.float32))
+            wq = O.f32_to_e4m3fn(rng.integers(-4, 5, (N, K)).astype(np.float32))
+            xs = (2.0 ** rng.integers(-3, 3, (M, K // 128))).astype(np.float32)
+            ws = (2.0 ** rng.integers(-3, 3, ((N + 127) // 128, K // 128))).astype(np.float32)
+            dt, name = (torch.bfloat16, "bf16") if case & 1 else (torch.float16, "f16")
+            ref = O.w8a8_block_fp8_matmul(xq, wq, xs, ws, out_dtype=name, acc=np.float64)
+            assert np.array_equal(_run_block(xq, xs, wq, ws, dev, col_major_as=bool(case & 2), out_dtype=dt), ref), "nw=%d M=%d N=%d K=%d" % (nw, M, N, K)
+            sa, sb = ((2.0 ** rng.integers(-3, 3, (n,))).astype(np.float32) for n in (M, N))
+            bias = rng.integers(-8, 9, (N,)).astype(np.float32)
+            got = fp8_scaled_mm(fp8_tensor(xq, dev), fp8_tensor(wq, dev).t(), torch.from_numpy(sa).to(dev), torch.from_numpy(sb).to(dev),
+                                torch.bfloat16, torch.from_numpy(bias).to(dev)).float().cpu().numpy()
+            assert np.array_equal(got, O.fp8_scaled_mm(xq, wq, sa, sb, out_dtype="bf16", bias=bias)), "row mode nw=%d M=%d N=%d K=%d" % (nw, M, N, K)
+    finally:
+        lib.fp8k_tune_force_gemm_plan(-1, 0)
+
+
 @pytest.mark.parametrize("nw", [0, 1, 2, 4, 8])
 def test_decode_gemm_with_k_cut_across_waves_is_exact_on_integers(dev, nw):
     """The decode kernel that cuts K across the waves of a workgroup (partial sums meet in LDS), pinned with every
