@@ -17,7 +17,7 @@ namespace fp8k {
 struct Plan {
   int kind;    // 0 = generic, 1 = tile256, 2 = weight-streaming through LDS (33..128 rows), 3 = direct (<= 32 rows),
                // 4 = tile128, 5 = direct with K cut across the waves of a workgroup (<= 16 rows, N below 16 K), 7 = skinny
-               // strips over all of K (<= 64 rows, N up to 16 K)
+               // strips over all of K (<= 128 rows, N up to 16 K)
   int splits;  // >1: split-K through the float workspace
   int kb_per_split;
   int tm;      // rows per block of the streaming kernels
@@ -97,13 +97,14 @@ static Plan plan_wavek(int64_t M, int64_t N, int64_t K) {
   pl.kb_per_split = (kb + 8 / nw - 1) / (8 / nw);
   return pl;
 }
-// Up to 64 rows: the strips of weight rows that one workgroup each runs over all of K are as narrow as leaves every CU one.
+// Up to 128 rows: the strips of weight rows that one workgroup each runs over all of K are as narrow as leaves every CU one.
 constexpr int64_t kSkinnyMaxN = 16384;
 static Plan plan_skinny(int64_t M, int64_t N, int64_t K) {
   Plan pl{7, 1, 0, 0, 0, 0};
-  pl.tm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  pl.tm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
   pl.halves = N <= 16 * num_cu() ? 1 : N <= 32 * num_cu() ? 2 : 4;
   if (g_force_kind == 7 && (g_force_splits == 1 || g_force_splits == 2 || g_force_splits == 4)) pl.halves = g_force_splits;  // tuning aid
+  if (pl.tm == 128) pl.halves = 2;
   return pl;
 }
 // Where it is ahead (M = 4 .. 64 x 16 widths up to 20480 x 9 depths up to 18432, timed against the other decode kernels and the
@@ -111,13 +112,15 @@ static Plan plan_skinny(int64_t M, int64_t N, int64_t K) {
 //  * more than 64 weight rows per CU's strip cost more activation traffic than a K cut costs partials, from 9 rows on;
 //  * that traffic grows with rows x K: above 32 rows a K of more than 8192 is left to the 128-row tiles with a K cut, and with
 //    64-row strips, whose waves have little of the LDS traffic to hide it behind, K of more than 4096 unless they fill the chip;
-//  * 17 .. 32 rows in 64-row strips that leave a quarter of the CUs idle: up to K = 6144.
+//  * 17 .. 32 rows in 64-row strips that leave a quarter of the CUs idle: up to K = 6144;
+//  * 65 .. 128 rows, in 32-row strips only: a middle range of K, 3 - 37 % ahead inside it.
 static bool prefers_skinny(int64_t M, int64_t N, int64_t K) {
   if (M > kSkinnyMaxM || N > kSkinnyMaxN) return false;
   const bool wide = N > 32 * num_cu(), fills = N >= 48 * num_cu();
   if (M <= 8) return K <= 9216;  // above: the wave-cut kernel, whose waves keep all of their K range in flight
   if (M <= 16) return true;
   if (M <= 32) return !wide || fills || K <= 6144;
+  if (M > 64) return !wide && K >= 1536 && K <= (N >= 16 * num_cu() ? 4608 : 3072);
   return wide ? K >= 1024 && K <= (fills ? 10240 : 4096) : K <= 8192;
 }
 // Activations few enough for every workgroup to quantise them for itself (gemm_wavek_quant_kernel): up to 16 rows of at most
@@ -371,7 +374,8 @@ static int launch(const GemmArgs& a0, const Plan& pl, hipStream_t st) {
   } while (0)
     if (pl.tm == 16) FP8K_SKINNY_NW(16);
     else if (pl.tm == 32) FP8K_SKINNY_NW(32);
-    else FP8K_SKINNY_NW(64);
+    else if (pl.tm == 64) FP8K_SKINNY_NW(64);
+    else FP8K_SKINNY(128, 2);
 #undef FP8K_SKINNY_NW
 #undef FP8K_SKINNY
     return check_launch("gemm_skinny");

@@ -1,4 +1,4 @@
-// FP8 GEMM for decode batches (9 .. 64 activation rows), gfx950: no float partials, no reduction launch.
+// FP8 GEMM for decode batches (9 .. 128 activation rows), gfx950: no float partials, no reduction launch.
 //
 // The weights are a stream from HBM that has to be spread over all CUs.  With narrow strips of weight rows per workgroup (16 or
 // 32: one or two to a CU) every workgroup can run over the whole of K and write finished rows; the price is that each of them
@@ -7,11 +7,11 @@
 // empty the weight stream.  Loads of a wave return in order, so a wave that waits for an activation line also waits for every
 // weight line it asked for before.  Hence two kinds of waves:
 //
-//   * eight streaming waves, NW along n (16 weight rows each) x KS = 8 / NW along k.  A trip covers eight K blocks, NW
-//     consecutive ones per wave; a wave keeps its next D K blocks of weights in flight in registers (whole-line loads, re-laid
+//   * eight streaming waves, NW along n (16 weight rows each) x KS = 8 / NW along k.  A trip covers eight K blocks (four above 64
+//     rows), U consecutive ones per wave; a wave keeps its next D K blocks of weights in flight in registers (whole-line loads, re-laid
 //     out through a private LDS slot as in gemm_direct_kernel) and takes its activations from LDS.  It never waits for a load
 //     of anybody else's.
-//   * NL loading waves, which bring the activations of a trip - [rows][1 KB], a row per instruction straight into LDS - one
+//   * NL loading waves, which bring the activations of a trip - [rows][1 KB], 1 KB per instruction straight into LDS - one
 //     or two trips ahead and wait for them in front of the trip's barrier.
 //
 // One LDS-only barrier per trip.  The 16-byte chunk c of row r lies at chunk c ^ (r & 15) of its row, which spreads the 16 rows of
@@ -19,53 +19,53 @@
 //
 // GEMM alone, bf16, against what ran before (K cut across workgroups with partials, or across the waves of one whose lanes fetched
 // their own activations): 32 x 4096 x 4096 10.7 -> 7.4 us, 24 x 7168 x 16384 30.6 -> 24.6 (117 MB: 4.8 TB/s), 64 x 4096 x 4096
-// 14.4 -> 9.3, 13 x 12224 x 3968 18.9 -> 11.0.
+// 14.4 -> 9.3, 13 x 12224 x 3968 18.9 -> 11.0, 128 x 4096 x 4096 16.4 -> 14.3.
 #pragma once
 
 #include "gemm_direct.h"
 
 namespace fp8k {
 
-constexpr int kSkinnyMaxM = 64;
-constexpr int kSkinnyTripK = 8;  // K blocks of a trip
-constexpr int kSkinnyRow = kSkinnyTripK * kTileK;
-// a trip's activations, and how many trips' worth the LDS holds beside the weight slots
-__host__ __device__ constexpr int skinny_stage(int tm) { return tm * kSkinnyRow; }
-__host__ __device__ constexpr int skinny_stages(int tm) { return 3 * skinny_stage(tm) + 8 * 2048 <= 160 * 1024 ? 3 : 2; }
+constexpr int kSkinnyMaxM = 128;
+constexpr int skinny_trip(int tm) { return tm <= 64 ? 8 : 4; }  // K blocks of a trip
 
 template <int TM, int NW, int MODE, int OUT_DT, int BIAS_DT>
 __global__ __launch_bounds__(TM <= 32 ? 640 : 768) void gemm_skinny_kernel(const GemmArgs p) {
-  static_assert(TM == 16 || TM == 32 || TM == 64, "16, 32 or 64 rows");
-  static_assert(NW == 1 || NW == 2 || NW == 4, "waves along n");
-  constexpr int MS = TM / 16, KS = 8 / NW;
+  static_assert(TM == 16 || TM == 32 || TM == 64 || TM == 128, "16, 32, 64 or 128 rows");
+  constexpr int TRIP = skinny_trip(TM), ROW = TRIP * kTileK;  // K blocks of a trip, bytes of a staged row
+  static_assert((NW == 1 || NW == 2 || NW == 4) && TRIP * NW % 8 == 0, "waves along n");
+  constexpr int MS = TM / 16, KS = 8 / NW, U = TRIP / KS;  // U: K blocks of a trip per wave
   // K blocks of weights in flight per wave (whole trips): more is slower, 24 x 7168 x 16384 25.2 us with 8 against 24.6
   constexpr int D = NW == 1 ? 2 : 4;
-  constexpr int NL = TM <= 32 ? 2 : 4;  // loading waves
-  constexpr int NI = TM / NL;           // rows, instructions, of a trip per loading wave
-  constexpr int NST = skinny_stages(TM), STAGE = skinny_stage(TM);
+  constexpr int NL = TM <= 32 ? 2 : 4;       // loading waves
+  constexpr int NI = TM * ROW / 1024 / NL;   // instructions of a trip per loading wave
+  constexpr int STAGE = TM * ROW;
+  constexpr int NST = 3 * STAGE + 8 * 2048 <= 160 * 1024 ? 3 : 2;  // trips' worth of activations beside the weight slots
   __shared__ __attribute__((aligned(16))) uint8_t xs[NST * STAGE];     // the sums at the end
   __shared__ __attribute__((aligned(16))) uint8_t wl[8][16 * kTileK];  // per streaming wave: one K block of its 16 weight rows
   static_assert(MS * 8 * 1024 <= NST * STAGE, "room for the sums");
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int kb_all = p.K / kTileK, trips = (kb_all + kSkinnyTripK - 1) / kSkinnyTripK;
+  const int kb_all = p.K / kTileK, trips = (kb_all + TRIP - 1) / TRIP;
   // an XCD (workgroup id mod 8) takes a contiguous run of strips: neighbours complete each other's output lines in its L2
   const int per_xcd = (p.tiles_n + 7) >> 3;
   const int strip = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
   if (((int)blockIdx.x >> 3) >= per_xcd || strip >= p.tiles_n) return;
 
   if (w >= 8) {
-    // ---- loading wave: rows [NI (w - 8), NI (w - 7)) of the stage, lane l brings the row's chunk l ^ (row & 15)
-    const int row0 = (w - 8) * NI;
+    // ---- loading wave: instruction i brings rows [i R, (i + 1) R) of the stage, the lane at chunk c of a row its chunk c ^ (row & 15)
+    constexpr int LR = ROW / 16, R = 64 / LR;  // lanes per row, rows per instruction
+    const int i0 = (w - 8) * NI;
+    const int sub = lane / LR, pos = lane % LR;
     const rsrc_t rX = make_rsrc(p.X, (uint32_t)((p.M - 1) * p.ldx + p.K));
     auto load = [&](int c) {
       uint8_t* const st = xs + (c % NST) * STAGE;
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
-        const int row = row0 + j;
-        const uint32_t k = (uint32_t)c * (uint32_t)kSkinnyRow + (uint32_t)(lane ^ (row & 15)) * 16u;
-        buf_load16_to_lds(rX, row < p.M && k < (uint32_t)p.K ? (uint32_t)(row * p.ldx) + k : kOutOfRange, 0, st + row * kSkinnyRow);
+        const int row = (i0 + j) * R + sub;
+        const uint32_t k = (uint32_t)c * (uint32_t)ROW + (uint32_t)(pos ^ (row & 15)) * 16u;
+        buf_load16_to_lds(rX, row < p.M && k < (uint32_t)p.K ? (uint32_t)(row * p.ldx) + k : kOutOfRange, 0, st + (i0 + j) * 1024);
       }
     };
     load(0);
@@ -94,8 +94,8 @@ __global__ __launch_bounds__(TM <= 32 ? 640 : 768) void gemm_skinny_kernel(const
   const uint32_t wst1 = (uint32_t)((wrow + 8) * kTileK + ((wc ^ (((wrow + 8) >> 1) & 7)) << 4));
   const uint32_t wrd0 = (uint32_t)(r * kTileK + ((kq ^ ((r >> 1) & 7)) << 4));
   const uint32_t wrd1 = (uint32_t)(r * kTileK + (((4 + kq) ^ ((r >> 1) & 7)) << 4));
-  // operand fetch of K block u: row ms * 16 + r, chunks (ks * NW + u) * 8 + kq and + 4, at their swizzled places
-  auto xr = [&](int u, int half) { return (uint32_t)(r * kSkinnyRow + ((((ks * NW + u) * 8 + kq + half * 4) ^ r) << 4)); };
+  // operand fetch of K block u: row ms * 16 + r, chunks (ks * U + u) * 8 + kq and + 4, at their swizzled places
+  auto xr = [&](int u, int half) { return (uint32_t)(r * ROW + ((((ks * U + u) * 8 + kq + half * 4) ^ r) << 4)); };
   const float* sxp[MS];
   const float* swp = p.sw;
   if (MODE == kModeBlock) {
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(TM <= 32 ? 640 : 768) void gemm_skinny_kernel(const
   v4i wreg[D][2];
   float sxr[D][MS], swr[D];
   auto issue = [&](int slot, int c, int u) {
-    const int kb = c * kSkinnyTripK + ks * NW + u;
+    const int kb = c * TRIP + ks * U + u;
     const bool ok = kb < kb_all;
     const uint32_t ko = (uint32_t)kb * kTileK;
     wreg[slot][0] = buf_load16_stream(rW, ok ? voW0 + ko : kOutOfRange);
@@ -123,9 +123,9 @@ __global__ __launch_bounds__(TM <= 32 ? 640 : 768) void gemm_skinny_kernel(const
 #pragma unroll
   for (int ms = 0; ms < MS; ++ms) acc[ms] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int d = 0; d < D; ++d) issue(d, d / NW, d % NW);
-  constexpr int UT = D / NW;  // trips per turn of the ring
-  static_assert(D % NW == 0, "whole trips");
+  for (int d = 0; d < D; ++d) issue(d, d / U, d % U);
+  constexpr int UT = D / U;  // trips per turn of the ring
+  static_assert(D % U == 0, "whole trips");
   int st = 0;  // stage of the trip
   for (int c0 = 0; c0 < trips; c0 += UT) {
 #pragma unroll
@@ -135,8 +135,8 @@ __global__ __launch_bounds__(TM <= 32 ? 640 : 768) void gemm_skinny_kernel(const
       const uint8_t* const xp = xs + st * STAGE;
       st = st + 1 == NST ? 0 : st + 1;
 #pragma unroll
-      for (int u = 0; u < NW; ++u) {
-        const int d = ct * NW + u;
+      for (int u = 0; u < U; ++u) {
+        const int d = ct * U + u;
         *reinterpret_cast<v4i*>(wslot + wst0) = wreg[d][0];
         *reinterpret_cast<v4i*>(wslot + wst1) = wreg[d][1];
         const v8i wa = join(*reinterpret_cast<const v4i*>(wslot + wrd0), *reinterpret_cast<const v4i*>(wslot + wrd1));
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(TM <= 32 ? 640 : 768) void gemm_skinny_kernel(const
         issue(d, c0 + ct + UT, u);
 #pragma unroll
         for (int ms = 0; ms < MS; ++ms) {
-          const v8i xa = join(*reinterpret_cast<const v4i*>(xp + ms * 16 * kSkinnyRow + xr(u, 0)), *reinterpret_cast<const v4i*>(xp + ms * 16 * kSkinnyRow + xr(u, 1)));
+          const v8i xa = join(*reinterpret_cast<const v4i*>(xp + ms * 16 * ROW + xr(u, 0)), *reinterpret_cast<const v4i*>(xp + ms * 16 * ROW + xr(u, 1)));
           if (MODE == kModeBlock) {
             const v4f t = mfma_16x16x128(wa, xa, v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll

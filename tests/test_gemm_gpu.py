@@ -213,7 +213,7 @@ def test_block_gemm_random_shapes_every_plan(dev):
 @pytest.mark.parametrize("nw", [0, 1, 2, 4])
 def test_skinny_gemm_is_exact_on_integers(dev, nw):
     """The decode-batch kernel with loading and streaming waves, pinned with every wave layout (0 = the plan's own): one to 33 K blocks
-    (one trip, remainders of a trip, more trips than stages), 9 .. 64 rows around the row counts it is built for, strips that end
+    (one trip, remainders of a trip, more trips than stages), 1 .. 128 rows around the row counts it is built for, strips that end
     inside their 16, 32 or 64 rows, both scale layouts, both outputs; exact whatever the order of the sums; then row mode."""
     from sglang_amd._lib import lib
     from sglang_amd.sgl_kernel import fp8_scaled_mm
@@ -222,7 +222,7 @@ def test_skinny_gemm_is_exact_on_integers(dev, nw):
     lib.fp8k_tune_force_gemm_plan(7, nw)
     try:
         for case, (M, N, K) in enumerate([(9, 16, 128), (16, 264, 1024), (17, 1000, 128 * 9), (32, 4104, 128 * 17), (33, 520, 128 * 33),
-                                          (64, 72, 128 * 24), (63, 8200, 640), (1, 8, 256)]):
+                                          (64, 72, 128 * 24), (63, 8200, 640), (1, 8, 256), (65, 136, 128 * 6), (128, 520, 128 * 13)]):
             xq = O.f32_to_e4m3fn(rng.integers(-4, 5, (M, K)).astype(np.float32))
             wq = O.f32_to_e4m3fn(rng.integers(-4, 5, (N, K)).astype(np.float32))
             xs = (2.0 ** rng.integers(-3, 3, (M, K // 128))).astype(np.float32)
