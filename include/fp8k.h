@@ -211,6 +211,15 @@ int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H, int64_t S
                           int64_t x_stride_s, float eps, int in_dtype, void* stream);
 
 /*
+ * The same in one launch for mid-sized tensors (numel = H S D with fp8k_tensor_quant_mla_takes_sync(numel) = 1).  sync: three
+ * int32 in device memory, zero before the first call with them and left zero by every call; calls that share them have to be on
+ * one stream.
+ */
+int fp8k_tensor_quant_mla_takes_sync(int64_t numel);
+int fp8k_tensor_quant_mla_sync(const void* x, void* q, float* s, int64_t H, int64_t S, int64_t D, int64_t x_stride_h,
+                               int64_t x_stride_s, float eps, int in_dtype, int32_t* sync, void* stream);
+
+/*
  * Batched FP8 GEMM with one scale per operand: C[b] = (A[b] . B[b]^T) * sa[m] * sb[n], float32 accumulation.
  * Replaces torch.ops.sgl_kernel.bmm_fp8 (sgl-kernel/python/sgl_kernel/gemm.py:45-82, sgl-kernel/csrc/gemm/bmm_fp8.cu),
  * whose per-tensor scales the caller broadcasts to the vectors sa [M] and sb [N] (shared by all batch entries).

@@ -24,6 +24,8 @@
 
 #include <algorithm>
 #include <initializer_list>
+#include <map>
+#include <mutex>
 
 #include "../../include/fp8k.h"
 
@@ -337,6 +339,24 @@ PyObject* token_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---------------------------------------------------------------------------------------------- absorbed products
+// Three zeroed int32 per (device, stream) for fp8k_tensor_quant_mla_sync, made on first use and kept: at most kMaxSync of them, other
+// streams (and calls under graph capture, whose replays may run on any stream) get none and take the two launches.
+constexpr size_t kMaxSync = 64;
+int32_t* stream_sync(const Tensor& like, hipStream_t st) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return nullptr;
+  static std::mutex mutex;
+  static auto* const words = new std::map<std::pair<int, hipStream_t>, Tensor>;  // lives as long as the process
+  std::lock_guard<std::mutex> lock(mutex);
+  const auto key = std::make_pair((int)like.get_device(), st);
+  auto it = words->find(key);
+  if (it == words->end()) {
+    if (words->size() >= kMaxSync) return nullptr;
+    it = words->emplace(key, at::zeros({3}, like.options().dtype(ScalarType::Int))).first;  // on the current stream, which is st
+  }
+  return it->second.data_ptr<int32_t>();
+}
+
 // mla_quant(x, x_s, eps) -> x_q or None
 PyObject* mla_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -348,8 +368,9 @@ PyObject* mla_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!(is_half(dt) || dt == ScalarType::Float) || s.scalar_type() != ScalarType::Float || s.dim() != 1 || s.size(0) != 1) DECLINE;
   Call c(x);
   Tensor q = empty(x.sizes(), ScalarType::Float8_e4m3fn, x.device());
-  check(fp8k_tensor_quant_mla(x.data_ptr(), q.data_ptr(), s.data_ptr<float>(), x.size(0), x.size(1), x.size(2), x.stride(0),
-                              x.stride(1), (float)PyFloat_AS_DOUBLE(a[2]), code(dt), c.stream));
+  int32_t* const sync = fp8k_tensor_quant_mla_takes_sync(x.numel()) ? stream_sync(x, c.stream) : nullptr;
+  check(fp8k_tensor_quant_mla_sync(x.data_ptr(), q.data_ptr(), s.data_ptr<float>(), x.size(0), x.size(1), x.size(2), x.stride(0),
+                                   x.stride(1), (float)PyFloat_AS_DOUBLE(a[2]), code(dt), sync, c.stream));
   return THPVariable_Wrap(std::move(q));
   END_HANDLE_TH_ERRORS
 }

@@ -456,6 +456,103 @@ __global__ __launch_bounds__(1024) void rows_tensor_quant_small_kernel(const voi
   if (threadIdx.x == 0) s[0] = sc;
 }
 
+// The same in one launch for tensors that the registers of one round of workgroups hold: every workgroup adds its maximum to
+// sync[1], counts itself in at sync[0], waits until all have, and quantises what it still holds - the tensor is read once, and the
+// host pays for one launch (4.2 us of an absorbed product's 18.7 with its zeroed scale).  The counting costs a queue at one line per
+// workgroup, so they are few and large: 256 of 256 threads took 6 us longer than 64 of 1024 at 2 MB.  The wait is bounded: an idle
+// chip holds all of them at once, but work of other streams may keep CUs, so a workgroup that has waited kMlaSpins polls takes the
+// maximum of the whole tensor for itself and goes on; nobody depends on another one's progress.  The last to leave writes the
+// scale and zeroes the three words for the next launch on them, which must be on the same stream.
+constexpr int kMlaOnceHold = 4, kMlaOnceGroups = 64, kMlaSpins = 4096;
+template <int DT>
+__global__ __launch_bounds__(1024) void rows_tensor_quant_once_kernel(const void* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ s,
+                                                                     uint32_t total, uint32_t chunks, uint32_t S, int64_t stride_h,
+                                                                     int64_t stride_s, float eps, uint32_t* __restrict__ sync) {
+  __shared__ float red[16];
+  __shared__ float found;
+  auto at = [&](uint32_t i) -> int64_t {
+    const uint32_t row = i / chunks, c = i - row * chunks, hh = row / S, ss = row - hh * S;
+    return (int64_t)hh * stride_h + (int64_t)ss * stride_s + (int64_t)c * 8;
+  };
+  auto block_max = [&](float v) -> float {
+    v = group_max<64>(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = red[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) v = fmaxf(v, red[i]);
+    __syncthreads();
+    return v;
+  };
+  Raw8<DT> t[kMlaOnceHold];
+  const uint32_t step = gridDim.x * 1024u, i0 = blockIdx.x * 1024u + threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < kMlaOnceHold; ++u) {
+    if (i0 + u * step < total) t[u].load(x, at(i0 + u * step));
+    else t[u].zero();
+  }
+  const float old = threadIdx.x == 0 ? __uint_as_float(__hip_atomic_load(reinterpret_cast<uint32_t*>(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) : 0.f;
+  float m = eps;
+#pragma unroll
+  for (int u = 0; u < kMlaOnceHold; ++u) {
+    float a[8];
+    t[u].unpack(a);
+    m = fmaxf(m, absmax8(a));
+  }
+  m = block_max(m);
+  if (threadIdx.x == 0) {
+    // non-negative floats order like their bit patterns
+    __hip_atomic_fetch_max(sync + 1, __float_as_uint(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the maximum is there, and the old scale has been read, before the count
+    __hip_atomic_fetch_add(sync, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    float all = -1.f;
+    for (int n = 0; n < kMlaSpins; ++n) {
+      if (__hip_atomic_load(sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x) {
+        asm volatile("" ::: "memory");
+        all = __uint_as_float(__hip_atomic_load(sync + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    found = all;
+  }
+  __syncthreads();
+  m = found;
+  if (m < 0.f) {  // uniform: the others did not turn up in time
+    m = eps;
+    for (uint32_t i = threadIdx.x; i < total; i += 1024) {
+      Raw8<DT> r;
+      r.load(x, at(i));
+      float a[8];
+      r.unpack(a);
+      m = fmaxf(m, absmax8(a));
+    }
+    m = block_max(m);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) found = old;
+  __syncthreads();
+  const float sc = fmaxf(m / kFp8Max, found);  // accumulates onto what the scale holds, as the atomic form does
+  const float inv = 1.0f / sc;
+#pragma unroll
+  for (int u = 0; u < kMlaOnceHold; ++u) {
+    const uint32_t i = i0 + u * step;
+    if (i < total) {
+      float a[8], y[8];
+      t[u].unpack(a);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] = fmaxf(fminf(a[j] * inv, kFp8Max), -kFp8Max);
+      *reinterpret_cast<uint2*>(q + (int64_t)i * 8) = make_uint2(cvt4_fp8(y[0], y[1], y[2], y[3]), cvt4_fp8(y[4], y[5], y[6], y[7]));
+    }
+  }
+  if (threadIdx.x == 0 && __hip_atomic_fetch_add(sync + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+    // every workgroup has read the old scale and is past its wait
+    s[0] = sc;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) __hip_atomic_store(sync + i, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 int quant_for_linear(bool groups, const void* x, void* q, float* s, int64_t M, int64_t K, float eps, int dtype, hipStream_t st) {
   const bool bf = dtype == FP8K_BF16;
   if (groups)
@@ -631,8 +728,12 @@ extern "C" int fp8k_tensor_quant(const void* x, void* q, float* s, int64_t numel
   return check_launch("tensor_quant");
 }
 
-extern "C" int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H, int64_t S, int64_t D, int64_t x_stride_h,
-                                     int64_t x_stride_s, float eps, int in_dtype, void* stream) {
+extern "C" int fp8k_tensor_quant_mla_takes_sync(int64_t numel) {
+  return numel / 8 > kMlaSmallChunks && numel / 8 <= (int64_t)kMlaOnceGroups * 1024 * kMlaOnceHold && num_cu() >= kMlaOnceGroups;
+}
+
+static int tensor_quant_mla(const void* x, void* q, float* s, int64_t H, int64_t S, int64_t D, int64_t x_stride_h, int64_t x_stride_s,
+                            float eps, int in_dtype, int32_t* sync, void* stream) {
   clear_error();
   const char* op = "per_tensor_quant_mla_fp8";
   FP8K_REQUIRE(H >= 0 && S >= 0 && D >= 0, "%s: negative shape", op);
@@ -649,6 +750,9 @@ extern "C" int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H
   const bool narrow = chunks < (1LL << 31);  // room for the four steps past the end
   const dim3 block(256);
   const dim3 grid_max((unsigned)std::min<int64_t>(512, (chunks + 1023) / 1024)), grid_q((unsigned)std::min<int64_t>(2048, (chunks + 255) / 256));
+  // one chunk per lane is enough to work on: the more workgroups share it, the shorter the loads
+  const dim3 grid_once((unsigned)std::min<int64_t>(kMlaOnceGroups, (chunks + 1023) / 1024));
+  FP8K_REQUIRE(!sync || fp8k_tensor_quant_mla_takes_sync(H * S * D), "%s: not a size of the one-launch form", op);
 #define FP8K_MLAQ2(DT, IDX)                                                                                                 \
   do {                                                                                                                      \
     hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, false, IDX>), grid_max, block, 0, st, x, (uint8_t*)q, s, rows, (int)S, \
@@ -661,6 +765,9 @@ extern "C" int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H
     if (chunks <= kMlaSmallChunks)                                                                                             \
       hipLaunchKernelGGL(rows_tensor_quant_small_kernel<DT>, dim3(1), dim3(1024), 0, st, x, (uint8_t*)q, s, (uint32_t)chunks,  \
                          (uint32_t)(D / 8), (uint32_t)S, x_stride_h, x_stride_s, eps);                                         \
+    else if (sync)                                                                                                             \
+      hipLaunchKernelGGL(rows_tensor_quant_once_kernel<DT>, grid_once, dim3(1024), 0, st, x, (uint8_t*)q, s, (uint32_t)chunks,      \
+                         (uint32_t)(D / 8), (uint32_t)S, x_stride_h, x_stride_s, eps, reinterpret_cast<uint32_t*>(sync));      \
     else if (narrow) FP8K_MLAQ2(DT, uint32_t);                                                                                 \
     else FP8K_MLAQ2(DT, int64_t);             \
   } while (0)
@@ -672,4 +779,14 @@ extern "C" int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H
 #undef FP8K_MLAQ
 #undef FP8K_MLAQ2
   return check_launch(op);
+}
+
+extern "C" int fp8k_tensor_quant_mla(const void* x, void* q, float* s, int64_t H, int64_t S, int64_t D, int64_t x_stride_h,
+                                     int64_t x_stride_s, float eps, int in_dtype, void* stream) {
+  return tensor_quant_mla(x, q, s, H, S, D, x_stride_h, x_stride_s, eps, in_dtype, nullptr, stream);
+}
+
+extern "C" int fp8k_tensor_quant_mla_sync(const void* x, void* q, float* s, int64_t H, int64_t S, int64_t D, int64_t x_stride_h,
+                                          int64_t x_stride_s, float eps, int in_dtype, int32_t* sync, void* stream) {
+  return tensor_quant_mla(x, q, s, H, S, D, x_stride_h, x_stride_s, eps, in_dtype, sync, stream);
 }

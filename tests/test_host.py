@@ -134,6 +134,52 @@ def test_mla_products_are_the_dispatcher_path(dev, dispatcher, heads, m, k, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,m,k", [(16, 17, 128), (5, 103, 72), (128, 64, 128), (64, 256, 128), (32, 512, 128), (32, 513, 128)])
+def test_mla_quant_in_one_launch(dev, dispatcher, heads, m, k):
+    """From one chunk of eight more than the one-workgroup form takes to one row more than the registers of the launch hold: the bytes
+    and the scale of the two launches, in every one of a run of launches that share their counters, onto a scale that is not zero, on
+    another stream and from a replayed graph in between."""
+    x = _randn((m, heads, k)).transpose(0, 1)
+    x[heads // 2, m // 3, k // 2] = 77
+
+    def quant(start=0.0):
+        return fp8_kernel.per_tensor_quant_mla_fp8(x, torch.full((1,), start, device=dev))
+
+    for start in (0.0, 10.0):
+        want = dispatcher(lambda: quant(start))
+        assert all(_same(got, want) for got in [quant(start) for _ in range(20)])
+    want = dispatcher(quant)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        outs = [quant() for _ in range(5)]
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            captured = quant()
+        for _ in range(3):
+            graph.replay()
+            outs.append(quant())
+    torch.cuda.synchronize()
+    assert all(_same(got, want) for got in outs + [captured])
+
+
+@pytest.mark.gpu
+def test_mla_quant_in_one_launch_ends_its_wait(dev):
+    """A count that never comes out (set from the host): every workgroup gives up its bounded wait and finds the maximum for itself."""
+    from sglang_amd._lib import BF16, check, lib, stream_ptr
+
+    x = _randn((40, 100, 128))
+    want = fp8_kernel.per_tensor_quant_mla_fp8(x, torch.zeros((1,), device=dev))
+    q, s = torch.empty_like(want[0]), torch.zeros((1,), device=dev)
+    sync = torch.tensor([100000, 0, 0], dtype=torch.int32, device=dev)
+    check(lib.fp8k_tensor_quant_mla_sync(x.data_ptr(), q.data_ptr(), s.data_ptr(), 40, 100, 128, x.stride(0), x.stride(1), 1e-12, BF16,
+                                         sync.data_ptr(), stream_ptr(dev)))
+    torch.cuda.synchronize()
+    assert _same((q, s), want) and not sync.any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("tokens", [1, 20, 100, 700])
 def test_experts_are_the_dispatcher_path(dev, dispatcher, tokens):
     E, H, inter, topk = 16, 512, 256, 4
