@@ -356,6 +356,18 @@ int fp8k_moe_slot_blocks_from_offsets(const int32_t* expert_starts, const int32_
                                       int64_t expert_capacity, int32_t* num_tokens_post_pad, void* stream);
 
 /*
+ * fp8k_silu_mul_group_quant (group 128, float scales) of x [slots, 2 K] (16-bit, ldx in elements) followed by fp8k_moe_block_gemm on
+ * it with top_k = 1, in one launch: the second half of an expert layer, bit for bit.  For what fp8k_moe_act_block_gemm_takes
+ * accepts (blocks of 16 or 32 slots and a short K).
+ */
+int fp8k_moe_act_block_gemm_takes(int64_t block_m, int64_t N, int64_t K, int64_t ldb);
+int fp8k_moe_act_block_gemm(const void* x, const void* B, const float* Bs, void* C, const int32_t* sorted_token_ids,
+                            const int32_t* expert_ids, const int32_t* num_tokens_post_padded, const float* topk_weights,
+                            int64_t sorted_capacity, int64_t block_m, int64_t num_valid_tokens, int64_t num_experts, int64_t N, int64_t K,
+                            int64_t ldx, int64_t b_stride_e, int64_t ldb, int64_t bs_stride_e, int64_t bs_stride_n, int64_t bs_stride_k,
+                            int64_t ldc, float eps, int dtype, void* stream);
+
+/*
  * Grouped GEMM 1 of the fused MoE layer with silu_and_mul and the per-token-group requantisation inside its write-out
  * (256-slot blocks): what fp8k_moe_block_gemm into a 16-bit [slots, 2 I] tensor followed by
  * fp8k_silu_mul_group_quant would produce, bit for bit, without that tensor ever being written.

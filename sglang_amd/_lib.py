@@ -55,6 +55,8 @@ SIGNATURES = {
     "fp8k_moe_blocks_from_offsets": (_c_int, [_c_ptr] * 2 + [_c_i64] * 3 + [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr]),
     "fp8k_moe_slot_blocks_from_offsets": (_c_int, [_c_ptr] * 2 + [_c_i64, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr]),
     "fp8k_moe_block_gemm_silu_quant": (_c_int, [_c_ptr] * 9 + [_c_i64] * 15 + [_c_f32, _c_int, _c_int, _c_ptr]),
+    "fp8k_moe_act_block_gemm_takes": (_c_int, [_c_i64] * 4),
+    "fp8k_moe_act_block_gemm": (_c_int, [_c_ptr] * 8 + [_c_i64] * 13 + [_c_f32, _c_int, _c_ptr]),
     "fp8k_block_gemm": (
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr] + [_c_i64] * 10 + [_c_int, _c_ptr, _c_i64, _c_ptr],

@@ -13,17 +13,22 @@
 // Whole layer, before -> now: 128 experts, H = 4096, top 6, 128 tokens, I = 256 176 -> 113 us, I = 512 224 -> 191; 256 experts,
 // H = 7168, I = 512, 865 tokens 739 -> 578 (its second GEMM, 940 MB of weights, 372 -> 211 us).
 //
+// ACT: the rows come as the 16-bit output [slots, 2 K] of the first GEMM, and a workgroup forms silu_and_mul and the group
+// quantisation of its block's rows when it puts them into LDS - bit for bit the bytes and scales of the kernel that does it
+// between the two GEMMs (4.7 us and a launch).  A block is staged by the few workgroups whose runs it spans, padding rows cost nothing.
+//
 // Operand layouts, the LDS round trip of the weights and the order of the K sums are gemm_direct_kernel's.
 #pragma once
 
 #include "gemm_direct.h"
+#include "quant_math.h"
 
 namespace fp8k {
 
 constexpr int kMoeShortKMax = 2048;
 __host__ __device__ constexpr int moe_shortk_row(int K) { return K + 16; }  // LDS row: rows of an operand fetch fall into different banks
 
-template <int TM, int OUT_DT>
+template <int TM, int OUT_DT, bool ACT>
 __global__ __launch_bounds__(512, 4) void moe_shortk_kernel(const GemmArgs p) {
   static_assert(TM == 16 || TM == 32, "16 or 32 slots per block");
   constexpr int MS = TM / 16, D = 4;
@@ -86,7 +91,7 @@ __global__ __launch_bounds__(512, 4) void moe_shortk_kernel(const GemmArgs p) {
 
   // ---- activations of a block: rows, scales and the routed weights of its slots
   const int64_t xrows = (int64_t)((p.num_valid + p.top_k - 1) / p.top_k);
-  const rsrc_t rX = make_rsrc(p.X, (uint32_t)((xrows - 1) * p.ldx + p.K));
+  const rsrc_t rX = make_rsrc(p.X, (uint32_t)((xrows - 1) * p.ldx + (ACT ? 4 * p.K : p.K)));  // ldx: bytes
   int slot[MS];
   float tw[MS];
   bool local = true;
@@ -94,17 +99,21 @@ __global__ __launch_bounds__(512, 4) void moe_shortk_kernel(const GemmArgs p) {
   // `between` runs behind the requests: what it requests is younger, so the rows are not waited for together with it
   auto stage = [&](int mb, auto&& between) {
     local = p.expert_ids[mb] >= 0;
-    const int per_row = p.K / 16, total = TM * per_row;
-    constexpr int U = 4;
-    const bool scaler = tid < TM * kb;
+    const int per_row = p.K / (ACT ? 8 : 16), total = TM * per_row;  // pieces of 8 elements, of 16 bytes
+    constexpr int U = ACT ? 2 : 4;
+    const bool scaler = !ACT && tid < TM * kb;
     float sc = 0.f;
     for (int c0 = 0; c0 < total; c0 += U * 512) {  // uniform: every lane takes part in the first round
-      v4i x[U];
+      v4i x[U], up[ACT ? U : 1];
+      bool there[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int i = c0 + u * 512 + tid, row = i / per_row;
         const int s = i < total ? slot_of(mb, row) : p.num_valid;
-        x[u] = buf_load16(rX, s < p.num_valid ? (uint32_t)((int64_t)(s / p.top_k) * p.ldx) + (uint32_t)(i - row * per_row) * 16 : kOutOfRange);
+        there[u] = s < p.num_valid;
+        const uint32_t off = there[u] ? (uint32_t)((int64_t)(s / p.top_k) * p.ldx) + (uint32_t)(i - row * per_row) * 16 : kOutOfRange;
+        x[u] = buf_load16(rX, off);
+        if (ACT) up[u] = buf_load16(rX, there[u] ? off + 2u * (uint32_t)p.K : kOutOfRange);
       }
       if (c0 == 0) {
         if (scaler) {
@@ -122,8 +131,29 @@ __global__ __launch_bounds__(512, 4) void moe_shortk_kernel(const GemmArgs p) {
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int i = c0 + u * 512 + tid, row = i / per_row;
-        if (i < total) *reinterpret_cast<v4i*>(xs + row * xrow + (i - row * per_row) * 16) = x[u];
+        const int i = c0 + u * 512 + tid, row = i / per_row, piece = i - row * per_row;
+        if (i >= total) continue;
+        if (!ACT) {
+          *reinterpret_cast<v4i*>(xs + row * xrow + piece * 16) = x[u];
+          continue;
+        }
+        // 16 lanes hold a group of 128; rows are multiples of 16 pieces, so a group is there or padding as a whole
+        uint2 o = make_uint2(0, 0);
+        float scale = 0.f;
+        if (there[u]) {
+          Raw8<OUT_DT> g, h;
+          g.v = __builtin_bit_cast(uint4, x[u]);
+          h.v = __builtin_bit_cast(uint4, up[ACT ? u : 0]);
+          float a[8];
+          silu_mul8<OUT_DT>(g, h, a);
+          const float amax = fmaxf(group_max<16>(absmax8(a)), p.q_eps);
+          scale = div448<true>(amax);
+          bool redo;
+          o = quant8_bracket<true>(a, scale, amax, redo);
+          if (__builtin_expect(redo, 0)) o = quant8_divide(a, scale);
+        }
+        *reinterpret_cast<uint2*>(xs + row * xrow + piece * 8) = o;
+        if ((piece & 15) == 0) scx[piece >> 4][row] = scale;
       }
     }
     if (scaler) scx[tid / TM][tid % TM] = sc;

@@ -463,6 +463,7 @@ PyObject* fused_experts(PyObject*, PyObject* const* a, Py_ssize_t n) {
   // are sized by it, 7168 workgroups less for 2 tokens of 128 experts
   const int64_t cap_used = std::min(cap, bm * std::min(slots, E + 1 + slots / bm));
   const int64_t kb1 = H / 128, kb2 = I / 128;
+  const bool act_gemm2 = !fuse && fp8k_moe_act_block_gemm_takes(bm, H, I, I);  // silu_and_mul and requantisation inside GEMM 2
   const bool sorted = bm >= 64;  // blocks of 64 slots and more read their activation scales in slot order
   Call c(x);
   Tensor out = inplace ? x : empty(x.sizes(), dt, x.device());
@@ -510,11 +511,16 @@ PyObject* fused_experts(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                          s13.stride(2), I, cap, kEps, dc, balanced ? 1 : 0, st));
   } else {
     gemm(q1, w13, s13, sorted ? ss1 : s1, 1, sorted ? cap : T, mid, on_input, topk);
+  }
+  if (act_gemm2) {
+    check(fp8k_moe_act_block_gemm(mid, w2.data_ptr(), s2.data_ptr<float>(), down, sorted_ids, block_expert, padded, on_input ? nullptr : twp,
+                                  cap_used, bm, slots, E, H, I, N, w2.stride(0), I, s2.stride(0), s2.stride(1), s2.stride(2), H, kEps, dc, st));
+  } else if (!fuse) {
     check(fp8k_silu_mul_group_quant(mid, q2, sm2, slots, I, 128, kEps, -448.f, 448.f, dc, sorted ? kb2 : 1, sorted ? 1 : slots,
                                     FP8K_SCALE_F32, st));
     if (sorted) check(fp8k_moe_sort_scales(sm2, ss2, sorted_ids, padded, cap, kb2, 1, slots, kb2, 1, st));
   }
-  gemm(q2, w2, s2, sorted ? ss2 : sm2, 1, sorted ? cap : slots, down, !on_input, 1);
+  if (!act_gemm2) gemm(q2, w2, s2, sorted ? ss2 : sm2, 1, sorted ? cap : slots, down, !on_input, 1);
   check(fp8k_moe_sum_reduce(down, out.data_ptr(), T, topk, H, topk * H, H, H, (float)PyFloat_AS_DOUBLE(a[11]), dc, st));
   if (inplace) {
     Py_INCREF(a[0]);

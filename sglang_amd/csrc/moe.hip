@@ -512,7 +512,7 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
   if (direct && K <= (block_m == 16 ? kMoeShortKMax / 2 : kMoeShortKMax) && blocks_max * a.tiles_n > most && N * ldb < (1LL << 31)) {
     const dim3 grid((unsigned)most), block(512);
     const unsigned lds = (unsigned)(block_m * moe_shortk_row((int)K));
-#define FP8K_SHORTK(TM, O) hipLaunchKernelGGL((moe_shortk_kernel<TM, O>), grid, block, lds, st, a)
+#define FP8K_SHORTK(TM, O) hipLaunchKernelGGL((moe_shortk_kernel<TM, O, false>), grid, block, lds, st, a)
     if (out_dtype == FP8K_BF16) {
       if (block_m == 16) FP8K_SHORTK(16, FP8K_BF16);
       else FP8K_SHORTK(32, FP8K_BF16);
@@ -600,6 +600,54 @@ extern "C" int fp8k_moe_block_gemm_ue8m0(const void* A, const void* B, const flo
                              sorted_capacity, block_m, num_valid_tokens, top_k, num_experts, N, K, lda, as_stride_m,
                              as_stride_k, b_stride_e, ldb, bs_stride_e, bs_stride_n, bs_stride_k, ldc, out_dtype, as_sorted,
                              true, stream);
+}
+
+extern "C" int fp8k_moe_act_block_gemm_takes(int64_t block_m, int64_t N, int64_t K, int64_t ldb) {
+  return (block_m == 16 || block_m == 32) && K > 0 && K % kTileK == 0 && K <= kMoeShortKMax / 2 && N > 0 && N % 8 == 0 && N * ldb < (1LL << 31);
+}
+
+extern "C" int fp8k_moe_act_block_gemm(const void* x, const void* B, const float* Bs, void* C, const int32_t* sorted_token_ids,
+                                       const int32_t* expert_ids, const int32_t* num_tokens_post_padded, const float* topk_weights,
+                                       int64_t sorted_capacity, int64_t block_m, int64_t num_valid_tokens, int64_t num_experts, int64_t N,
+                                       int64_t K, int64_t ldx, int64_t b_stride_e, int64_t ldb, int64_t bs_stride_e, int64_t bs_stride_n,
+                                       int64_t bs_stride_k, int64_t ldc, float eps, int dtype, void* stream) {
+  clear_error();
+  const char* op = "moe_act_block_gemm";
+  FP8K_REQUIRE(fp8k_moe_act_block_gemm_takes(block_m, N, K, ldb), "%s: block_m 16 or 32, K a multiple of 128 up to %d, N of 8 (got %lld, %lld, %lld)",
+               op, kMoeShortKMax / 2, (long long)block_m, (long long)K, (long long)N);
+  FP8K_REQUIRE(dtype == FP8K_F16 || dtype == FP8K_BF16, "%s: the activation type must be Half or BFloat16", op);
+  FP8K_REQUIRE(num_experts > 0 && num_valid_tokens >= 0 && num_valid_tokens < 0x7fffffffLL && sorted_capacity >= 0 && sorted_capacity < 0x7fffffffLL,
+               "%s: bad shape", op);
+  FP8K_REQUIRE(ldx >= 2 * K && ldb >= K && ldc >= N, "%s: leading dimension smaller than the row length", op);
+  FP8K_REQUIRE(ldx % 8 == 0 && ldb % 16 == 0 && (ldc * 2) % 8 == 0 && b_stride_e % 16 == 0, "%s: rows must be 16-byte aligned", op);
+  FP8K_REQUIRE(num_valid_tokens * ldx * 2 < 0xE0000000LL && ldb < (1LL << 23), "%s: activation matrix exceeds 3.5 GiB, or rows 8 MiB", op);
+  FP8K_REQUIRE(bs_stride_n >= 0 && bs_stride_k >= 0 && bs_stride_e >= 0, "%s: negative scale stride", op);
+  if (num_valid_tokens == 0 || sorted_capacity < block_m) return FP8K_OK;
+  FP8K_REQUIRE(x && B && Bs && C && sorted_token_ids && expert_ids && num_tokens_post_padded, "%s: null pointer", op);
+  FP8K_REQUIRE(aligned(x, 16) && aligned(B, 16) && aligned(C, 8), "%s: operands must be 16-byte aligned", op);
+  GemmArgs a{};
+  a.X = (const uint8_t*)x; a.W = (const uint8_t*)B; a.sw = Bs; a.C = C;
+  a.M = (int)num_valid_tokens; a.N = (int)N; a.K = (int)K; a.ldx = ldx * 2; a.ldw = ldb; a.ldc = ldc;
+  a.sw_n = bs_stride_n; a.sw_k = bs_stride_k;
+  a.tiles_n = (int)((N + kDirTileN - 1) / kDirTileN);
+  a.sorted_ids = sorted_token_ids; a.expert_ids = expert_ids; a.num_post_pad = num_tokens_post_padded;
+  a.topk_w = topk_weights; a.top_k = 1; a.num_valid = (int)num_valid_tokens;
+  a.m_blocks = (int)(sorted_capacity / block_m); a.block_m = (int)block_m;
+  a.w_expert_stride = b_stride_e; a.sw_expert_stride = bs_stride_e; a.q_eps = quant_eps(eps, dtype);
+  const int64_t tiles = moe_blocks_in_use(num_valid_tokens, num_experts, block_m, a.m_blocks) * a.tiles_n;
+  const dim3 grid((unsigned)(std::min<int64_t>(2 * (int64_t)num_cu(), tiles + 7) / 8 * 8)), block(512);
+  const unsigned lds = (unsigned)(block_m * moe_shortk_row((int)K));
+  hipStream_t st = (hipStream_t)stream;
+#define FP8K_SHORTK(TM, O) hipLaunchKernelGGL((moe_shortk_kernel<TM, O, true>), grid, block, lds, st, a)
+  if (dtype == FP8K_BF16) {
+    if (block_m == 16) FP8K_SHORTK(16, FP8K_BF16);
+    else FP8K_SHORTK(32, FP8K_BF16);
+  } else {
+    if (block_m == 16) FP8K_SHORTK(16, FP8K_F16);
+    else FP8K_SHORTK(32, FP8K_F16);
+  }
+#undef FP8K_SHORTK
+  return check_launch(op);
 }
 
 extern "C" int fp8k_moe_block_gemm_silu_quant(const void* A, const void* B, const float* As_sorted, const float* Bs, void* q_out,

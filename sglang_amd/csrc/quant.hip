@@ -43,17 +43,6 @@ __device__ __forceinline__ void load_stream(Raw8<DT>& r, const void* base, int64
   }
 }
 
-// FUSE: the value that gets quantised is T( T(silu(gate)) * up ) with gate = x[m, c], up = x[m, K + c] of an
-// input row of 2K elements - what silu_and_mul would have written to memory, bit for bit (same two roundings).
-template <int DT>
-__device__ __forceinline__ void silu_mul8(const Raw8<DT>& gate, const Raw8<DT>& up, float (&a)[8]) {
-  float g[8], u[8];
-  gate.unpack(g);
-  up.unpack(u);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) a[i] = round_to<DT>(round_to<DT>(silu_f32(g[i])) * u[i]);
-}
-
 // MASKED: the M rows are E experts x m_max slots; only the first masked_m[e] slots of expert e are quantised
 // (the others are neither read nor written), and the scale of slot i of expert e sits at e*se + i*sm + g*sg.
 template <int DT, int GROUP, int KIND, int SEG, bool ROWFAST, bool FUSE, bool MASKED>

@@ -48,6 +48,17 @@ struct Raw8<FP8K_F32> {
   }
 };
 
+// silu_and_mul in front of the quantisation: T( T(silu(gate)) * up ) with gate = x[m, c], up = x[m, K + c] of an
+// input row of 2K elements - what silu_and_mul would have written to memory, bit for bit (same two roundings).
+template <int DT>
+__device__ __forceinline__ void silu_mul8(const Raw8<DT>& gate, const Raw8<DT>& up, float (&a)[8]) {
+  float g[8], u[8];
+  gate.unpack(g);
+  up.unpack(u);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a[i] = round_to<DT>(round_to<DT>(silu_f32(g[i])) * u[i]);
+}
+
 // eps as the torch-native formula sees it: amax is clamped in the input dtype, so bf16 sees eps rounded to bf16
 inline float quant_eps(float eps, int in_dtype) {
   if (in_dtype != FP8K_BF16) return eps;

@@ -444,6 +444,39 @@ def test_grouped_gemm_short_k_runs_exact(dev, T, E, topk, N, K, block):
                 assert torch.equal(got[slots], ref.bfloat16().float())
 
 
+@pytest.mark.parametrize("T,E,topk,N,K,block", [(1, 8, 2, 264, 128, 16), (40, 40, 3, 2056, 384, 16), (64, 24, 4, 3080, 1024, 16), (90, 8, 4, 1160, 256, 32),
+                                                (130, 16, 6, 1032, 640, 32), (50, 64, 8, 2048, 1024, 32)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_grouped_gemm_with_activation_and_quant_inside(dev, T, E, topk, N, K, block, dt):
+    """The second GEMM of the experts on the first one's 16-bit output: bit for bit silu_and_mul + group quant + grouped GEMM; fewer and
+    more tiles than workgroups, one to eight groups per row, part-filled blocks, ids of -1, routed weights or none."""
+    from sglang_amd._lib import BF16, F16, check, lib, stream_ptr
+    from sglang_amd.fused_moe import moe_align_block_size
+    from sglang_amd.sgl_kernel import moe_block_gemm
+    from sglang_amd.fp8_kernel import sglang_per_token_group_quant_fp8
+
+    g = torch.Generator().manual_seed(K + T)
+    x = torch.randn((T * topk, 2 * K), generator=g).to(dt).to(dev)
+    x[T // 2] *= 1e-6
+    w = torch.randn((E, N, K), generator=g).to(dev).to(torch.float8_e4m3fn)
+    ws = torch.rand((E, (N + 127) // 128, K // 128), generator=g).to(dev)
+    ids = torch.rand((T, E), generator=g).argsort(dim=1)[:, :topk].int()
+    ids[:T // 3, 0] = 1
+    ids[torch.rand(ids.shape, generator=g) < 0.05] = -1
+    tw = torch.rand((T, topk), generator=g).to(dev)
+    sorted_ids, expert_ids, npad = moe_align_block_size(ids.to(dev), block, E)
+    q, s = sglang_per_token_group_quant_fp8(x, 128, column_major_scales=True, fuse_silu_and_mul=True)
+    assert lib.fp8k_moe_act_block_gemm_takes(block, N, K, K) == 1
+    for weigh in (False, True):
+        want, got = (torch.full((T * topk, N), 7.0, dtype=dt, device=dev) for _ in range(2))
+        moe_block_gemm(q, w, want, s, ws, tw, sorted_ids, expert_ids, npad, weigh, 1, block, ids.numel())
+        check(lib.fp8k_moe_act_block_gemm(x.data_ptr(), w.data_ptr(), ws.data_ptr(), got.data_ptr(), sorted_ids.data_ptr(), expert_ids.data_ptr(),
+                                          npad.data_ptr(), tw.data_ptr() if weigh else None, sorted_ids.numel(), block, ids.numel(), E, N, K, 2 * K,
+                                          N * K, K, *ws.stride(), N, 1e-10, BF16 if dt == torch.bfloat16 else F16, stream_ptr(dev)))
+        torch.cuda.synchronize()
+        assert torch.equal(want, got)
+
+
 def test_grouped_gemm_random_routings_exact(dev):
     """Forty seeded random routings (1..600 tokens, 2..40 experts, top-1..6, every block size, skewed and absent
     experts, ids of -1) on integer data with power-of-two scales: exact, with per-token and with sorted scales."""
