@@ -253,6 +253,14 @@ int fp8k_moe_align_block_size(const void* topk_ids, int ids_are_int64, int64_t n
                               int64_t block_size, int32_t* sorted_token_ids, int64_t sorted_capacity,
                               int32_t* expert_ids, int64_t expert_capacity, int32_t* num_tokens_post_pad,
                               int32_t* cumsum_buffer, int pad_sorted_token_ids, void* stream);
+/*
+ * fp8k_moe_align_block_size (with padding) and fp8k_group_quant of the layer's input x [M, K] (16-bit, group 128, float scales) in
+ * one launch where both are small, otherwise in theirs: the tables, bytes and scales of the two calls.
+ */
+int fp8k_moe_align_quant(const void* topk_ids, int ids_are_int64, int64_t numel, int64_t num_buckets, int64_t block_size,
+                         int32_t* sorted_token_ids, int64_t sorted_capacity, int32_t* expert_ids, int64_t expert_capacity,
+                         int32_t* num_tokens_post_pad, int32_t* cumsum_buffer, const void* x, void* q, float* s, int64_t M, int64_t K,
+                         float eps, int dtype, int64_t s_stride_m, int64_t s_stride_g, void* stream);
 
 /*
  * Grouped block-scaled FP8 GEMM with expert indirection:

@@ -94,6 +94,8 @@ SIGNATURES = {
         _c_int,
         [_c_ptr, _c_int, _c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr],
     ),
+    "fp8k_moe_align_quant": (_c_int, [_c_ptr, _c_int] + [_c_i64] * 3 + [_c_ptr, _c_i64, _c_ptr, _c_i64] + [_c_ptr] * 5 + [_c_i64] * 2
+                             + [_c_f32, _c_int] + [_c_i64] * 2 + [_c_ptr]),
     "fp8k_moe_block_gemm": (_c_int, [_c_ptr] * 9 + [_c_i64] * 16 + [_c_int, _c_int, _c_ptr]),
     "fp8k_moe_block_gemm_ue8m0": (_c_int, [_c_ptr] * 9 + [_c_i64] * 16 + [_c_int, _c_int, _c_ptr]),
     "fp8k_moe_balance_blocks": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr]),

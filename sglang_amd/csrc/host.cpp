@@ -491,13 +491,13 @@ PyObject* fused_experts(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const float* twp = tw.data_ptr<float>();
   void* st = c.stream;
 
-  check(fp8k_moe_align_block_size(ids.data_ptr(), ids64, slots, E + 1, bm, sorted_ids, cap, block_expert, blocks, padded, cumsum, 1, st));
+  // small blocks read their scales column-major per token, large ones get them gathered into slot order
+  check(fp8k_moe_align_quant(ids.data_ptr(), ids64, slots, E + 1, bm, sorted_ids, cap, block_expert, blocks, padded, cumsum, x.data_ptr(), q1,
+                             s1, T, H, kEps, dc, sorted ? kb1 : 1, sorted ? 1 : T, st));
   if (balanced) {
     check(fp8k_moe_balance_blocks(sorted_ids, block_expert, padded, cap, bm, slots, E, even_ids, st));
     sorted_ids = even_ids;
   }
-  // small blocks read their scales column-major per token, large ones get them gathered into slot order
-  check(fp8k_group_quant(x.data_ptr(), q1, s1, T, H, 128, kEps, -448.f, 448.f, dc, sorted ? kb1 : 1, sorted ? 1 : T, FP8K_SCALE_F32, st));
   if (sorted) check(fp8k_moe_sort_scales(s1, ss1, sorted_ids, padded, cap, kb1, topk, slots, kb1, 1, st));
   auto gemm = [&](const void* A, const Tensor& W, const Tensor& Ws, const float* As, int64_t as_m, int64_t as_k, void* C, bool weigh,
                   int64_t per_row) {

@@ -19,6 +19,8 @@ namespace fp8k {
 constexpr int kAlignThreads = 1024;
 constexpr int kAlignMaxBuckets = 4096;
 constexpr int64_t kAlignFusedMax = 8192;  // ids up to which one workgroup does the whole job
+constexpr int64_t kAlignQuantMax = 4 << 20;  // elements that are quantised in the alignment's launch: beyond, the 48 KB of LDS that
+                                             // its workgroups come with keep the quantisation from filling the CUs
 
 template <typename IdT>
 __device__ __forceinline__ int bucket_of(const IdT* ids, int64_t i, int nb) {
@@ -97,12 +99,11 @@ __global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const IdT* __r
   place_ids(ids, first, last, nb, counts, sorted);
 }
 
-template <typename IdT, bool SCATTER, bool PRECOUNTED = false>
-__global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(const IdT* __restrict__ ids, int64_t numel, int nb,
-                                                                  int block, int32_t* __restrict__ sorted,
-                                                                  int32_t* __restrict__ expert_ids,
-                                                                  int32_t* __restrict__ post_pad,
-                                                                  int32_t* __restrict__ cumsum, int pad_ids) {
+// the work of one workgroup of kAlignThreads threads
+template <typename IdT, bool SCATTER, bool PRECOUNTED>
+__device__ __forceinline__ void align_ids(const IdT* __restrict__ ids, int64_t numel, int nb, int block, int32_t* __restrict__ sorted,
+                                          int32_t* __restrict__ expert_ids, int32_t* __restrict__ post_pad, int32_t* __restrict__ cumsum,
+                                          int pad_ids) {
   __shared__ int32_t counts[kAlignMaxBuckets];
   __shared__ int32_t prefix[kAlignMaxBuckets + 1];
   __shared__ int32_t cursor[kAlignMaxBuckets];
@@ -161,6 +162,45 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(const IdT* __r
   if (SCATTER) {
     __syncthreads();
     place_ids(ids, 0, numel, nb, cursor, sorted);
+  }
+}
+
+template <typename IdT, bool SCATTER, bool PRECOUNTED = false>
+__global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(const IdT* __restrict__ ids, int64_t numel, int nb, int block,
+                                                                  int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids,
+                                                                  int32_t* __restrict__ post_pad, int32_t* __restrict__ cumsum, int pad_ids) {
+  align_ids<IdT, SCATTER, PRECOUNTED>(ids, numel, nb, block, sorted, expert_ids, post_pad, cumsum, pad_ids);
+}
+
+// The alignment and the group quantisation of the layer's input know nothing of each other and each leave most of the chip idle:
+// workgroup 0 aligns, the others quantise (group 128, a group per 16 lanes, group_quant_kernel's arithmetic), in one launch.
+template <typename IdT, int DT>
+__global__ __launch_bounds__(kAlignThreads) void moe_align_quant_kernel(const IdT* __restrict__ ids, int64_t numel, int nb, int block,
+                                                                        int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids,
+                                                                        int32_t* __restrict__ post_pad, int32_t* __restrict__ cumsum,
+                                                                        const void* __restrict__ x, uint8_t* __restrict__ q,
+                                                                        float* __restrict__ s, int64_t groups, int row_groups, int64_t sm,
+                                                                        int64_t sg, float eps) {
+  if (blockIdx.x == 0) {
+    align_ids<IdT, true, false>(ids, numel, nb, block, sorted, expert_ids, post_pad, cumsum, 1);
+    return;
+  }
+  const int64_t g = (int64_t)(blockIdx.x - 1) * (kAlignThreads / 16) + (threadIdx.x >> 4);
+  if (g >= groups) return;
+  const int64_t at = g * 128 + (threadIdx.x & 15) * 8;
+  Raw8<DT> raw;
+  raw.load(x, at);
+  float a[8];
+  raw.unpack(a);
+  const float amax = fmaxf(group_max<16>(absmax8(a)), eps);
+  const float sc = div448<true>(amax);
+  bool redo;
+  uint2 o = quant8_bracket<true>(a, sc, amax, redo);
+  if (__builtin_expect(redo, 0)) o = quant8_divide(a, sc);
+  *reinterpret_cast<uint2*>(q + at) = o;
+  if ((threadIdx.x & 15) == 0) {
+    const int64_t row = g / row_groups;
+    s[row * sm + (g - row * row_groups) * sg] = sc;
   }
 }
 
@@ -284,11 +324,8 @@ static unsigned stream_grid(int64_t work_items) {
 
 using namespace fp8k;
 
-extern "C" int fp8k_moe_align_block_size(const void* topk_ids, int ids_are_int64, int64_t numel, int64_t num_buckets,
-                                         int64_t block_size, int32_t* sorted_token_ids, int64_t sorted_capacity,
-                                         int32_t* expert_ids, int64_t expert_capacity, int32_t* num_tokens_post_pad,
-                                         int32_t* cumsum_buffer, int pad_sorted_token_ids, void* stream) {
-  clear_error();
+static int align_checks(const void* topk_ids, int64_t numel, int64_t num_buckets, int64_t block_size, const int32_t* sorted_token_ids,
+                        int64_t sorted_capacity, const int32_t* expert_ids, int64_t expert_capacity, const int32_t* num_tokens_post_pad) {
   FP8K_REQUIRE(numel >= 0 && numel < 0x7fffffffLL, "moe_align_block_size: bad number of ids (%lld)", (long long)numel);
   FP8K_REQUIRE(num_buckets >= 1 && num_buckets <= kAlignMaxBuckets,
                "moe_align_block_size: num_experts must be in [1, %d] (got %lld)", kAlignMaxBuckets, (long long)num_buckets);
@@ -303,6 +340,17 @@ extern "C" int fp8k_moe_align_block_size(const void* topk_ids, int ids_are_int64
                (long long)(worst / block_size));
   FP8K_REQUIRE(sorted_token_ids && expert_ids && num_tokens_post_pad, "moe_align_block_size: null output pointer");
   FP8K_REQUIRE(numel == 0 || topk_ids, "moe_align_block_size: null topk_ids");
+  return FP8K_OK;
+}
+
+extern "C" int fp8k_moe_align_block_size(const void* topk_ids, int ids_are_int64, int64_t numel, int64_t num_buckets,
+                                         int64_t block_size, int32_t* sorted_token_ids, int64_t sorted_capacity,
+                                         int32_t* expert_ids, int64_t expert_capacity, int32_t* num_tokens_post_pad,
+                                         int32_t* cumsum_buffer, int pad_sorted_token_ids, void* stream) {
+  clear_error();
+  const int rc = align_checks(topk_ids, numel, num_buckets, block_size, sorted_token_ids, sorted_capacity, expert_ids, expert_capacity,
+                              num_tokens_post_pad);
+  if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   // one workgroup does everything up to kAlignFusedMax ids (and whenever the caller gives no scratch table); more ids
   // are counted and placed by one workgroup per kAlignChunk ids
@@ -330,6 +378,43 @@ extern "C" int fp8k_moe_align_block_size(const void* topk_ids, int ids_are_int64
   else FP8K_ALIGN(int32_t);
 #undef FP8K_ALIGN
   return check_launch("moe_align_block_size");
+}
+
+extern "C" int fp8k_moe_align_quant(const void* topk_ids, int ids_are_int64, int64_t numel, int64_t num_buckets, int64_t block_size,
+                                    int32_t* sorted_token_ids, int64_t sorted_capacity, int32_t* expert_ids, int64_t expert_capacity,
+                                    int32_t* num_tokens_post_pad, int32_t* cumsum_buffer, const void* x, void* q, float* s, int64_t M,
+                                    int64_t K, float eps, int dtype, int64_t s_stride_m, int64_t s_stride_g, void* stream) {
+  clear_error();
+  const char* op = "moe_align_quant";
+  FP8K_REQUIRE(M > 0 && K > 0 && K % 128 == 0 && M * (K / 128) < 0x7fffffffLL && (dtype == FP8K_F16 || dtype == FP8K_BF16), "%s: bad activations", op);
+  FP8K_REQUIRE(x && q && s && aligned(x, 16) && aligned(q, 8) && aligned(s, 4), "%s: x must be 16-byte, q 8-byte aligned", op);
+  FP8K_REQUIRE(s_stride_m > 0 && s_stride_g > 0, "%s: scale strides must be positive", op);
+  // more ids than one workgroup takes, or activations that fill the chip on their own: the two calls
+  if (numel < 1 || numel > kAlignFusedMax || M * K > kAlignQuantMax) {
+    const int rc = fp8k_moe_align_block_size(topk_ids, ids_are_int64, numel, num_buckets, block_size, sorted_token_ids, sorted_capacity,
+                                             expert_ids, expert_capacity, num_tokens_post_pad, cumsum_buffer, 1, stream);
+    return rc ? rc
+              : fp8k_group_quant(x, q, s, M, K, 128, eps, -448.f, 448.f, dtype, s_stride_m, s_stride_g, FP8K_SCALE_F32, stream);
+  }
+  const int rc = align_checks(topk_ids, numel, num_buckets, block_size, sorted_token_ids, sorted_capacity, expert_ids, expert_capacity,
+                              num_tokens_post_pad);
+  if (rc) return rc;
+  const int64_t groups = M * (K / 128);
+  const dim3 grid((unsigned)(1 + (groups + kAlignThreads / 16 - 1) / (kAlignThreads / 16)));
+  hipStream_t st = (hipStream_t)stream;
+#define FP8K_AQ(T, DT)                                                                                                            \
+  hipLaunchKernelGGL((moe_align_quant_kernel<T, DT>), grid, dim3(kAlignThreads), 0, st, (const T*)topk_ids, numel, (int)num_buckets, \
+                     (int)block_size, sorted_token_ids, expert_ids, num_tokens_post_pad, cumsum_buffer, x, (uint8_t*)q, s, groups,    \
+                     (int)(K / 128), s_stride_m, s_stride_g, quant_eps(eps, dtype))
+  if (ids_are_int64) {
+    if (dtype == FP8K_BF16) FP8K_AQ(int64_t, FP8K_BF16);
+    else FP8K_AQ(int64_t, FP8K_F16);
+  } else {
+    if (dtype == FP8K_BF16) FP8K_AQ(int32_t, FP8K_BF16);
+    else FP8K_AQ(int32_t, FP8K_F16);
+  }
+#undef FP8K_AQ
+  return check_launch(op);
 }
 
 namespace fp8k {

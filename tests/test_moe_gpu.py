@@ -444,6 +444,40 @@ def test_grouped_gemm_short_k_runs_exact(dev, T, E, topk, N, K, block):
                 assert torch.equal(got[slots], ref.bfloat16().float())
 
 
+@pytest.mark.parametrize("T,E,topk,K,block", [(1, 8, 1, 128, 16), (37, 64, 3, 7168, 16), (100, 32, 6, 640, 32), (1024, 128, 8, 4096, 256),
+                                              (1025, 8, 8, 128, 256), (3000, 16, 2, 1536, 64)])
+@pytest.mark.parametrize("id_dtype", [torch.int32, torch.int64])
+def test_align_and_quant_in_one_launch(dev, T, E, topk, K, block, id_dtype):
+    """The largest and the first too large number of ids and of activations among them: the table is the alignment's (slots of an
+    expert in any order), bytes and scales are the group quant's, both scale layouts."""
+    from sglang_amd._lib import BF16, check, lib, stream_ptr
+    from sglang_amd.fp8_kernel import sglang_per_token_group_quant_fp8
+    from sglang_amd.fused_moe import moe_align_block_size
+
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn((T, K), generator=g).bfloat16().to(dev)
+    ids = torch.randint(-1, E, (T, topk), generator=g).to(id_dtype).to(dev)
+    want = [v.cpu() for v in moe_align_block_size(ids, block, E)]
+    n = ids.numel()
+    cap = n + (E + 1) * (block - 1)
+    for column in (False, True):
+        wq, wscale = sglang_per_token_group_quant_fp8(x, 128, column_major_scales=column)
+        sorted_ids, cumsum = torch.zeros(cap, dtype=torch.int32, device=dev), torch.zeros(E + 2, dtype=torch.int32, device=dev)
+        experts, npad = torch.zeros(-(-cap // block), dtype=torch.int32, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
+        q, s = torch.empty_like(wq), torch.empty_like(wscale)
+        check(lib.fp8k_moe_align_quant(ids.data_ptr(), id_dtype == torch.int64, n, E + 1, block, sorted_ids.data_ptr(), cap, experts.data_ptr(),
+                                       experts.numel(), npad.data_ptr(), cumsum.data_ptr(), x.data_ptr(), q.data_ptr(), s.data_ptr(), T, K, 1e-10,
+                                       BF16, *s.stride(), stream_ptr(dev)))
+        torch.cuda.synchronize()
+        assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8)) and torch.equal(s, wscale)
+        used = int(npad)
+        assert used == int(want[2]) and torch.equal(experts.cpu()[:used // block], want[1][:used // block])
+        got, ref, start = sorted_ids.cpu()[:used], want[0][:used], 0
+        for e, count in zip(*want[1][:used // block].unique_consecutive(return_counts=True)):
+            assert torch.equal(got[start:start + count * block].sort()[0], ref[start:start + count * block].sort()[0])
+            start += int(count) * block
+
+
 @pytest.mark.parametrize("T,E,topk,N,K,block", [(1, 8, 2, 264, 128, 16), (40, 40, 3, 2056, 384, 16), (64, 24, 4, 3080, 1024, 16), (90, 8, 4, 1160, 256, 32),
                                                 (130, 16, 6, 1032, 640, 32), (50, 64, 8, 2048, 1024, 32)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
