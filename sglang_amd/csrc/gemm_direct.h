@@ -2,22 +2,28 @@
 //
 // With so few activation rows the GEMM is an HBM stream of the weight matrix (2*TM FLOP per weight byte, far under
 // the chip's ridge), so everything is arranged around the weight loads.  A wavefront owns 16 weight rows and keeps
-// eight K blocks (16 KB) of them in flight in registers: two non-temporal 16-byte loads per lane and K block, each
-// instruction covering 8 whole 128-byte lines (lane l: row l/8, 16-byte chunk l%8) - whole-line requests measured
-// 25 % more HBM bandwidth here than the half-line requests that loading straight into the matrix-core operand
-// layout would make.  The move into that layout (operand "A" of v_mfma_f32_16x16x128_f8f6f4: lane l holds 32 bytes
+// eight K blocks (16 KB; four in the grouped GEMM) of them in flight in registers: two non-temporal 16-byte loads per
+// lane and K block, each instruction covering 8 whole 128-byte lines (lane l: row l/8, 16-byte chunk l%8) - whole-line
+// requests measured 25 % more HBM bandwidth here than the half-line requests that loading straight into the matrix-core
+// operand layout would make.  The move into that layout (operand "A" of v_mfma_f32_16x16x128_f8f6f4: lane l holds 32 bytes
 // of row l%16) is a round trip through a 2 KB LDS slot private to the wave: LDS operations of one wave execute in
 // order, so it needs no barrier and no wait beyond the register dependency.  The matrix core only sums over K, so
 // the K order inside a 128-byte block is free as long as both operands agree: lane (row, q = l/16) takes chunks
 // q and 4+q of the block.
 //
 // The activation rows (shared by the 8 waves = 128 weight rows of a workgroup) are staged through LDS in chunks
-// of 8 K blocks: registers -> ds_write one chunk ahead, one barrier per chunk (an LDS-only barrier: the weight
+// of as many K blocks: registers -> ds_write one chunk ahead, one barrier per chunk (an LDS-only barrier: the weight
 // loads stay in flight across it), rows padded by 16 bytes so the 16 rows of an operand fetch fall into different
 // banks.  In block mode the chunk also carries as[m,kb]*bs[nb,kb] (a workgroup spans exactly one 128-row weight
 // scale block), zero past the K range, so the K tail needs no branch.  (Every wave re-reads all activation rows
 // of the block from LDS, which is why blocks of 64 and 128 rows measured slower here than through
 // gemm_stream_kernel.)
+//
+// The grouped GEMM keeps four K blocks in flight instead of eight: 112 registers and 50 KB of LDS let two workgroups
+// share a CU (eight took 174 registers: one), so the start and the write-out of one block hide behind the stream of
+// another, and a short K (an expert's intermediate size) pads to less.  Bytes in flight per CU stay the same.  Measured
+// on the whole layer with 32-row blocks: 128 experts x 4096 x 256 at 384 slots 1.05x, x 1024 1.05x, 64 x 7168 x 1024
+// 1.03x; with 16-row blocks 1.00 .. 1.05x.  The linears keep eight: their grid leaves one workgroup per CU.
 #pragma once
 
 #include "gemm_kernels.h"
@@ -25,7 +31,7 @@
 namespace fp8k {
 
 constexpr int kDirTileN = 128;                   // 8 waves x 16 weight rows
-constexpr int kDirDepth = 8;                     // weight prefetch depth in K blocks = K blocks per activation chunk
+constexpr int kDirDepth = 8;                     // of a linear: weight prefetch depth in K blocks = K blocks per activation chunk
 constexpr uint32_t kOutOfRange = 0xF0000000u;    // buffer offset past every descriptor range: reads zero
 
 __device__ __forceinline__ v4f mfma_16x16x128(v8i a, v8i b, v4f c) {
@@ -45,12 +51,10 @@ __device__ __forceinline__ v8i join(v4i lo, v4i hi) {
 }
 
 template <int TM, int MODE, int OUT_DT, int BIAS_DT, bool SPLIT, bool MOE>
-__global__ __launch_bounds__(512, 2) void gemm_direct_kernel(const GemmArgs p) {
+__global__ __launch_bounds__(512, MOE ? 4 : 2) void gemm_direct_kernel(const GemmArgs p) {
   static_assert(TM == 16 || TM == 32, "gemm_direct_kernel: 16 or 32 rows per block (more rows are LDS-read bound here)");
   constexpr int MS = TM / 16;                 // 16-row activation sub-tiles
-  constexpr int KC = kDirDepth;               // K blocks per activation chunk
-  constexpr int DEPTH = kDirDepth;
-  constexpr int U = DEPTH / KC;               // chunks per trip of the unrolled loop
+  constexpr int KC = MOE ? kDirDepth / 2 : kDirDepth;  // K blocks per activation chunk = weight prefetch depth
   constexpr int RB = KC * kTileK;             // bytes of one activation row in a chunk
   constexpr int XROW = RB + 16;               // LDS row stride
   constexpr int LPR = RB / 16;                // lanes per staged row
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(512, 2) void gemm_direct_kernel(const GemmArgs p) {
   const uint32_t wst1 = (uint32_t)((wrow + 8) * kTileK + ((wc ^ (((wrow + 8) >> 1) & 7)) << 4));
   const uint32_t wrd0 = (uint32_t)(r * kTileK + ((kq ^ ((r >> 1) & 7)) << 4));
   const uint32_t wrd1 = (uint32_t)(r * kTileK + (((4 + kq) ^ ((r >> 1) & 7)) << 4));
-  v4i wreg[DEPTH][2];
+  v4i wreg[KC][2];
   auto load_w = [&](int slot, int kb) {
     const bool ok = kb < nkb;
     wreg[slot][0] = buf_load16_stream(rW, ok ? voW0 + (uint32_t)kb * kTileK : kOutOfRange);
@@ -197,7 +201,7 @@ __global__ __launch_bounds__(512, 2) void gemm_direct_kernel(const GemmArgs p) {
   stage_load(1);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) load_w(d, d);
+  for (int d = 0; d < KC; ++d) load_w(d, d);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < XI; ++j)
@@ -205,34 +209,29 @@ __global__ __launch_bounds__(512, 2) void gemm_direct_kernel(const GemmArgs p) {
   if (stager) scs[0][skb][sm] = s0x * s0w;
 
   const uint32_t xrd = (uint32_t)(r * XROW + kq * 16);
-  for (int c0 = 0; c0 < nch; c0 += U) {
+  for (int c = 0; c < nch; ++c) {
+    const int buf = c & 1;
+    lds_barrier();                // chunk c is visible; every wave is done with chunk c-1 (weight loads stay in flight)
+    stage_store(buf ^ 1);         // chunk c+1
+    stage_load(c + 2);
+    // memory operations retire in order: the staging loads must stay OLDER than this trip's weight loads, or
+    // the wait for them at the next barrier would drain the weight prefetch
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int c = c0 + u;         // a chunk past the K range holds zeros and zero scales
-      const int buf = c & 1;
-      lds_barrier();                // chunk c is visible; every wave is done with chunk c-1 (weight loads stay in flight)
-      stage_store(buf ^ 1);         // chunk c+1
-      stage_load(c + 2);
-      // memory operations retire in order: the staging loads must stay OLDER than this trip's weight loads, or
-      // the wait for them at the next barrier would drain the weight prefetch
-      __builtin_amdgcn_sched_barrier(0);
+    for (int kbl = 0; kbl < KC; ++kbl) {
+      const v8i wa = weight_operand(kbl);
+      load_w(kbl, (c + 1) * KC + kbl);
 #pragma unroll
-      for (int kbl = 0; kbl < KC; ++kbl) {
-        const int slot = u * KC + kbl;
-        const v8i wa = weight_operand(slot);
-        load_w(slot, c * KC + kbl + DEPTH);
+      for (int ms = 0; ms < MS; ++ms) {
+        const uint8_t* xp = &xs[buf][ms * 16 * XROW + xrd + kbl * kTileK];
+        const v8i xa = join(*reinterpret_cast<const v4i*>(xp), *reinterpret_cast<const v4i*>(xp + 64));
+        if (MODE == kModeBlock) {
+          const v4f t = mfma_16x16x128(wa, xa, v4f{0.f, 0.f, 0.f, 0.f});
+          const float sc = scs[buf][kbl][ms * 16 + r];
 #pragma unroll
-        for (int ms = 0; ms < MS; ++ms) {
-          const uint8_t* xp = &xs[buf][ms * 16 * XROW + xrd + kbl * kTileK];
-          const v8i xa = join(*reinterpret_cast<const v4i*>(xp), *reinterpret_cast<const v4i*>(xp + 64));
-          if (MODE == kModeBlock) {
-            const v4f t = mfma_16x16x128(wa, xa, v4f{0.f, 0.f, 0.f, 0.f});
-            const float sc = scs[buf][kbl][ms * 16 + r];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[ms][i] = __builtin_fmaf(t[i], sc, acc[ms][i]);
-          } else {
-            acc[ms] = mfma_16x16x128(wa, xa, acc[ms]);
-          }
+          for (int i = 0; i < 4; ++i) acc[ms][i] = __builtin_fmaf(t[i], sc, acc[ms][i]);
+        } else {
+          acc[ms] = mfma_16x16x128(wa, xa, acc[ms]);
         }
       }
     }

@@ -51,14 +51,16 @@ def get_default_config(M: int, E: int, topk: int) -> Dict[str, int]:
 
     Measured on MI355X with 256 experts, top-8 and near-balanced routing: while the layer streams every expert's
     weights for a handful of rows each, the register-streaming kernel with 16- or 32-row blocks wins (up to about 22
-    rows per expert: 1.95 ms against 2.02 ms at 512 tokens); from there on the 256-row kernel, which walks its items
-    with the weight stream running on across them, skips the slot groups that are padding and forms the activation and
-    the requantisation in the write-out of GEMM 1 (2.06 ms against 2.13 ms with 64-row blocks at 768 tokens, 2.21
-    against 2.29 with 128-row blocks at 1536, 2.48 against 2.65 at 3072).  The 64- and 128-row forms of the streaming
-    kernel remain for callers that pass their own BLOCK_SIZE_M.
+    rows per expert: 1.95 ms against 2.02 ms at 512 tokens): 16 rows while an average expert still fits one such block
+    with room for uneven routing (at 6 rows per expert 86 us against 96 with an intermediate size of 256 and a hidden
+    size of 2048, 137 against 181 with 64 experts of 2048 x 2048, 254 either way with 7168 x 256), 32 beyond.
+    From 22 on the 256-row kernel, which walks its items with the weight stream running on across them, skips the slot
+    groups that are padding and forms the activation and the requantisation in the write-out of GEMM 1 (2.06 ms against
+    2.13 ms with 64-row blocks at 768 tokens, 2.21 against 2.29 with 128-row blocks at 1536, 2.48 against 2.65 at 3072).
+    The 64- and 128-row forms of the streaming kernel remain for callers that pass their own BLOCK_SIZE_M.
     """
     per_expert = (M * topk + E - 1) // max(E, 1)
-    if per_expert <= 4:
+    if per_expert <= 7:
         bm = 16
     elif per_expert <= 22:
         bm = 32
