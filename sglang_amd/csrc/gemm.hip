@@ -304,8 +304,8 @@ static int launch_tiles(const GemmArgs& a0, const Plan& pl, hipStream_t st) {
   const int ncu8 = std::max(8, num_cu() / 8 * 8);
   const int tail_units = (ntiles - pl.tail_first) * (pl.halves ? 2 : pl.splits);
   unsigned nwg;
-  if (pl.tail_first > ncu8) {
-    // more whole tiles than CUs: one walking workgroup per CU, which also takes a unit of the tail at the end
+  if (pl.tail_first >= ncu8) {
+    // at least as many whole tiles as CUs: one walking workgroup per CU, which also takes a unit of the tail at the end
     a.walkers = ncu8;
     a.tail_shared = 1;
     nwg = (unsigned)std::max(ncu8, tail_units);
