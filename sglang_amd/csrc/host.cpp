@@ -147,20 +147,36 @@ class Scratch {
   size_t used_ = 0;
 };
 
-// the call's device made current, and its stream
+// What allocates or launches runs without the interpreter lock: a launch into a full queue and an allocation that has to free
+// cached blocks wait for the device, and other Python threads, one of which the device may be waiting for, must not wait with it.
+class WithoutGil {
+ public:
+  WithoutGil() : state_(PyEval_SaveThread()) {}
+  ~WithoutGil() { PyEval_RestoreThread(state_); }
+  WithoutGil(const WithoutGil&) = delete;
+  WithoutGil& operator=(const WithoutGil&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
+// the part of a call that works on the device: no interpreter lock, the call's device made current, and its stream
 struct Call {
   explicit Call(const Tensor& t)
       : guard(t.device()), device(t.get_device()), stream(c10::hip::getCurrentHIPStream(t.get_device()).stream()) {}
+  WithoutGil unlocked;  // first: taken back last
   c10::DeviceGuard guard;
   int device;
   hipStream_t stream;
 };
 
-// the GEMM workspace of the current stream (sgl_kernel._workspace): nullptr and false when the Python side raised
-bool stream_workspace(const Tensor& like, hipStream_t st, int64_t need, void*& p, int64_t& bytes) {
+// the GEMM workspace of the current stream (sgl_kernel._workspace): nullptr and false when the Python side raised.  Asked for
+// with the interpreter lock; what it returns is never released.
+bool stream_workspace(const Tensor& like, int64_t need, void*& p, int64_t& bytes) {
   p = nullptr;
   bytes = 0;
   if (need <= 0) return true;
+  const hipStream_t st = c10::hip::getCurrentHIPStream(like.get_device()).stream();
   PyObject* key = Py_BuildValue("(iK)", (int)like.get_device(), (unsigned long long)(uintptr_t)st);
   if (!key) return false;
   PyObject* buf = PyDict_GetItem(g_workspaces, key);  // borrowed
@@ -184,6 +200,15 @@ bool stream_workspace(const Tensor& like, hipStream_t st, int64_t need, void*& p
   return true;
 }
 
+// Threads that share a stream share its workspace: the launches of one product (copy of the scales, GEMM, reduction) go onto the
+// stream together.  One lock per workspace, so a thread waits for launches onto its own stream only; taken without the interpreter lock.
+std::mutex& workspace_lock(const void* workspace) {
+  static std::mutex mutex;
+  static auto* const locks = new std::map<const void*, std::mutex>;  // as many as there are workspaces; both live as long as the process
+  std::lock_guard<std::mutex> lock(mutex);
+  return (*locks)[workspace];
+}
+
 #define DECLINE Py_RETURN_NONE
 
 // ---------------------------------------------------------------------------------------------- group quant
@@ -205,29 +230,31 @@ PyObject* group_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (group <= 0 || width % group != 0 || K % group != 0 || K == 0 || (fuse && (width % 2 != 0 || group != 128))) DECLINE;
   const int64_t M = x.numel() / width, G = K / group;
 
-  Call c(x);
-  c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
-  shape.back() = K;
-  Tensor q = empty(shape, ScalarType::Float8_e4m3fn, x.device());
-  Tensor s;
-  int64_t sm, sg;
-  if (ue8m0) {
-    sm = 1;
-    sg = ceil_to(M, 4);
-    s = empty_column_major(M, ceil_div(G, 4), sg, ScalarType::Int, x.device());
-  } else if (column) {
-    sm = 1;
-    sg = tma ? ceil_to(M, 4) : M;
-    s = empty_column_major(M, G, sg, ScalarType::Float, x.device());
-  } else {
-    shape.back() = G;
-    s = empty(shape, ScalarType::Float, x.device());
-    sm = G;
-    sg = 1;
+  Tensor q, s;
+  {
+    Call c(x);
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = K;
+    q = empty(shape, ScalarType::Float8_e4m3fn, x.device());
+    int64_t sm, sg;
+    if (ue8m0) {
+      sm = 1;
+      sg = ceil_to(M, 4);
+      s = empty_column_major(M, ceil_div(G, 4), sg, ScalarType::Int, x.device());
+    } else if (column) {
+      sm = 1;
+      sg = tma ? ceil_to(M, 4) : M;
+      s = empty_column_major(M, G, sg, ScalarType::Float, x.device());
+    } else {
+      shape.back() = G;
+      s = empty(shape, ScalarType::Float, x.device());
+      sm = G;
+      sg = 1;
+    }
+    check((fuse ? fp8k_silu_mul_group_quant : fp8k_group_quant)(
+        x.data_ptr(), q.data_ptr(), s.data_ptr(), M, K, group, eps, -448.f, 448.f, code(dt), sm, sg,
+        ue8m0 ? FP8K_SCALE_UE8M0_PACKED : FP8K_SCALE_F32, c.stream));
   }
-  check((fuse ? fp8k_silu_mul_group_quant : fp8k_group_quant)(
-      x.data_ptr(), q.data_ptr(), s.data_ptr(), M, K, group, eps, -448.f, 448.f, code(dt), sm, sg,
-      ue8m0 ? FP8K_SCALE_UE8M0_PACKED : FP8K_SCALE_F32, c.stream));
   PyObject* out = PyTuple_New(2);
   if (!out) return nullptr;
   PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(q)));
@@ -253,14 +280,17 @@ PyObject* block_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!tensor_arg(a[4], bias) || !plain(bias, dev) || bias.dim() != 1 || bias.size(0) != N || bias.scalar_type() != dt || !bias.is_contiguous()) DECLINE;
   }
 
-  Call c(x);
-  c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
-  shape.back() = N;
-  Tensor out = empty(shape, dt, x.device());
-  const int64_t wsb = fp8k_linear_workspace_bytes(M, N, K, 1);
-  Scratch mem(wsb, c.stream);
-  check(fp8k_block_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(), M,
-                          N, K, K, ws.stride(0), ws.stride(1), N, kEps, code(dt), wsb ? mem.take(wsb) : nullptr, wsb, c.stream));
+  Tensor out;
+  {
+    Call c(x);
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = N;
+    out = empty(shape, dt, x.device());
+    const int64_t wsb = fp8k_linear_workspace_bytes(M, N, K, 1);
+    Scratch mem(wsb, c.stream);
+    check(fp8k_block_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), bias.defined() ? bias.data_ptr() : nullptr, out.data_ptr(), M,
+                            N, K, K, ws.stride(0), ws.stride(1), N, kEps, code(dt), wsb ? mem.take(wsb) : nullptr, wsb, c.stream));
+  }
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -289,17 +319,22 @@ PyObject* block_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
     DECLINE;
   }
 
-  Call c(x);
-  Tensor out = empty({M, N}, dt, x.device());
   void* work;
   int64_t bytes;
-  if (!stream_workspace(x, c.stream, fp8k_block_gemm_workspace_bytes(M, N, K), work, bytes)) return nullptr;
-  if (packed)
-    check(fp8k_block_gemm_ue8m0(x.data_ptr(), w.data_ptr(), xs.data_ptr<int32_t>(), ws.data_ptr<float>(), out.data_ptr(), M, N, K, K,
-                                K, xs.stride(0), xs.stride(1), ws.stride(0), ws.stride(1), N, code(dt), work, bytes, c.stream));
-  else
-    check(fp8k_block_gemm(x.data_ptr(), w.data_ptr(), xs.data_ptr<float>(), ws.data_ptr<float>(), out.data_ptr(), M, N, K, K, K,
-                          xs.stride(0), xs.stride(1), ws.stride(0), ws.stride(1), N, code(dt), work, bytes, c.stream));
+  if (!stream_workspace(x, fp8k_block_gemm_workspace_bytes(M, N, K), work, bytes)) return nullptr;
+  Tensor out;
+  {
+    Call c(x);
+    out = empty({M, N}, dt, x.device());
+    std::unique_lock<std::mutex> together;
+    if (work) together = std::unique_lock<std::mutex>(workspace_lock(work));
+    if (packed)
+      check(fp8k_block_gemm_ue8m0(x.data_ptr(), w.data_ptr(), xs.data_ptr<int32_t>(), ws.data_ptr<float>(), out.data_ptr(), M, N, K, K,
+                                  K, xs.stride(0), xs.stride(1), ws.stride(0), ws.stride(1), N, code(dt), work, bytes, c.stream));
+    else
+      check(fp8k_block_gemm(x.data_ptr(), w.data_ptr(), xs.data_ptr<float>(), ws.data_ptr<float>(), out.data_ptr(), M, N, K, K, K,
+                            xs.stride(0), xs.stride(1), ws.stride(0), ws.stride(1), N, code(dt), work, bytes, c.stream));
+  }
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -325,15 +360,18 @@ PyObject* token_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (bias.scalar_type() != dt && bias.scalar_type() != ScalarType::Float) DECLINE;
   }
 
-  Call c(x);
-  c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
-  shape.back() = N;
-  Tensor out = empty(shape, dt, x.device());
-  const int64_t wsb = fp8k_linear_workspace_bytes(M, N, K, 0);
-  Scratch mem(wsb, c.stream);
-  check(fp8k_token_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), ws.numel() == 1 ? 0 : 1, bias.defined() ? bias.data_ptr() : nullptr,
-                          bias.defined() ? code(bias.scalar_type()) : FP8K_F32, out.data_ptr(), M, N, K, N > 1 ? w.stride(1) : K, N, code(dt),
-                          wsb ? mem.take(wsb) : nullptr, wsb, c.stream));
+  Tensor out;
+  {
+    Call c(x);
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = N;
+    out = empty(shape, dt, x.device());
+    const int64_t wsb = fp8k_linear_workspace_bytes(M, N, K, 0);
+    Scratch mem(wsb, c.stream);
+    check(fp8k_token_linear(x.data_ptr(), w.data_ptr(), ws.data_ptr<float>(), ws.numel() == 1 ? 0 : 1, bias.defined() ? bias.data_ptr() : nullptr,
+                            bias.defined() ? code(bias.scalar_type()) : FP8K_F32, out.data_ptr(), M, N, K, N > 1 ? w.stride(1) : K, N, code(dt),
+                            wsb ? mem.take(wsb) : nullptr, wsb, c.stream));
+  }
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -366,11 +404,15 @@ PyObject* mla_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const ScalarType dt = x.scalar_type();
   if (!plain(x, dev) || !plain(s, dev) || x.dim() != 3 || x.stride(2) != 1 || x.numel() == 0) DECLINE;
   if (!(is_half(dt) || dt == ScalarType::Float) || s.scalar_type() != ScalarType::Float || s.dim() != 1 || s.size(0) != 1) DECLINE;
-  Call c(x);
-  Tensor q = empty(x.sizes(), ScalarType::Float8_e4m3fn, x.device());
-  int32_t* const sync = fp8k_tensor_quant_mla_takes_sync(x.numel()) ? stream_sync(x, c.stream) : nullptr;
-  check(fp8k_tensor_quant_mla_sync(x.data_ptr(), q.data_ptr(), s.data_ptr<float>(), x.size(0), x.size(1), x.size(2), x.stride(0),
-                                   x.stride(1), (float)PyFloat_AS_DOUBLE(a[2]), code(dt), sync, c.stream));
+  const float eps = (float)PyFloat_AS_DOUBLE(a[2]);
+  Tensor q;
+  {
+    Call c(x);
+    q = empty(x.sizes(), ScalarType::Float8_e4m3fn, x.device());
+    int32_t* const sync = fp8k_tensor_quant_mla_takes_sync(x.numel()) ? stream_sync(x, c.stream) : nullptr;
+    check(fp8k_tensor_quant_mla_sync(x.data_ptr(), q.data_ptr(), s.data_ptr<float>(), x.size(0), x.size(1), x.size(2), x.stride(0),
+                                     x.stride(1), eps, code(dt), sync, c.stream));
+  }
   return THPVariable_Wrap(std::move(q));
   END_HANDLE_TH_ERRORS
 }
@@ -389,11 +431,14 @@ PyObject* bmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t b = A.size(0), m = A.size(1), k = A.size(2), nn = B.size(2);
   if (A.stride(2) != 1 || B.stride(1) != 1 || k % 128 != 0 || nn % 8 != 0) DECLINE;
   if (as.numel() != 1 || bs.numel() != 1 || as.scalar_type() != ScalarType::Float || bs.scalar_type() != ScalarType::Float) DECLINE;
-  Call c(A);
-  Tensor out = empty({b, m, nn}, dt, A.device());
-  check(fp8k_bmm_fp8_tensor_scales(A.data_ptr(), B.data_ptr(), as.data_ptr<float>(), bs.data_ptr<float>(), out.data_ptr(), b, m, nn, k,
-                     b > 1 ? A.stride(0) : m * k, m > 1 ? A.stride(1) : k, b > 1 ? B.stride(0) : nn * k, nn > 1 ? B.stride(2) : k,
-                     m * nn, nn, code(dt), c.stream));
+  Tensor out;
+  {
+    Call c(A);
+    out = empty({b, m, nn}, dt, A.device());
+    check(fp8k_bmm_fp8_tensor_scales(A.data_ptr(), B.data_ptr(), as.data_ptr<float>(), bs.data_ptr<float>(), out.data_ptr(), b, m, nn, k,
+                       b > 1 ? A.stride(0) : m * k, m > 1 ? A.stride(1) : k, b > 1 ? B.stride(0) : nn * k, nn > 1 ? B.stride(2) : k,
+                       m * nn, nn, code(dt), c.stream));
+  }
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -411,13 +456,19 @@ PyObject* fused_gate(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const ScalarType dt = x.scalar_type();
   if (!plain(x, dev) || !plain(bias, dev) || x.dim() != 2 || bias.dim() != 1 || bias.size(0) != x.size(1) || x.size(0) == 0) DECLINE;
   if (bias.scalar_type() != dt || !(is_half(dt) || dt == ScalarType::Float) || !x.is_contiguous() || !bias.is_contiguous()) DECLINE;
-  const int64_t rows = x.size(0), topk = PyLong_AsLongLong(a[4]);
+  const int64_t rows = x.size(0), groups = PyLong_AsLongLong(a[2]), topk_group = PyLong_AsLongLong(a[3]);
+  const int64_t topk = PyLong_AsLongLong(a[4]), shared = PyLong_AsLongLong(a[5]);
+  const double scaling = PyFloat_AS_DOUBLE(a[6]);
+  const bool scale_output = truth(a[7]);
   if (topk <= 0) DECLINE;
-  Call c(x);
-  Tensor w = empty({rows, topk}, ScalarType::Float, x.device()), ids = empty({rows, topk}, ScalarType::Int, x.device());
-  check(fp8k_moe_fused_gate(x.data_ptr(), bias.data_ptr(), w.data_ptr<float>(), ids.data_ptr<int32_t>(), rows, x.size(1),
-                            PyLong_AsLongLong(a[2]), PyLong_AsLongLong(a[3]), topk, PyLong_AsLongLong(a[5]),
-                            PyFloat_AS_DOUBLE(a[6]), truth(a[7]) ? 1 : 0, code(dt), c.stream));
+  Tensor w, ids;
+  {
+    Call c(x);
+    w = empty({rows, topk}, ScalarType::Float, x.device());
+    ids = empty({rows, topk}, ScalarType::Int, x.device());
+    check(fp8k_moe_fused_gate(x.data_ptr(), bias.data_ptr(), w.data_ptr<float>(), ids.data_ptr<int32_t>(), rows, x.size(1), groups,
+                              topk_group, topk, shared, scaling, scale_output ? 1 : 0, code(dt), c.stream));
+  }
   PyObject* out = PyTuple_New(2);
   if (!out) return nullptr;
   PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(w)));
@@ -465,63 +516,67 @@ PyObject* fused_experts(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t kb1 = H / 128, kb2 = I / 128;
   const bool act_gemm2 = !fuse && fp8k_moe_act_block_gemm_takes(bm, H, I, I);  // silu_and_mul and requantisation inside GEMM 2
   const bool sorted = bm >= 64;  // blocks of 64 slots and more read their activation scales in slot order
-  Call c(x);
-  Tensor out = inplace ? x : empty(x.sizes(), dt, x.device());
-  const int64_t b_ids = cap * 4, b_q1 = T * H, b_s1 = T * kb1 * 4, b_ss1 = cap * kb1 * 4, b_mid = slots * N * 2, b_q2 = slots * I,
-                b_s2 = slots * kb2 * 4, b_ss2 = cap * kb2 * 4, b_out = slots * H * 2;
-  using S = Scratch;
-  Scratch mem(2 * S::room(b_ids) + S::room(blocks * 4) + S::room(4) + S::room((E + 2) * 4) + S::room(b_q1) + S::room(b_s1) +
-                  (sorted ? S::room(b_ss1) + S::room(b_ss2) : 0) + (fuse ? 0 : S::room(b_mid) + S::room(b_s2)) + S::room(b_q2) +
-                  S::room(b_out),
-              c.stream);
-  int32_t* sorted_ids = mem.take<int32_t>(b_ids);
-  int32_t* even_ids = mem.take<int32_t>(b_ids);
-  int32_t* block_expert = mem.take<int32_t>(blocks * 4);
-  int32_t* padded = mem.take<int32_t>(4);
-  int32_t* cumsum = mem.take<int32_t>((E + 2) * 4);
-  void* q1 = mem.take(b_q1);
-  float* s1 = mem.take<float>(b_s1);
-  void* q2 = mem.take(b_q2);
-  void* down = mem.take(b_out);
-  float* ss1 = sorted ? mem.take<float>(b_ss1) : nullptr;
-  float* ss2 = sorted ? mem.take<float>(b_ss2) : nullptr;
-  void* mid = fuse ? nullptr : mem.take(b_mid);
-  float* sm2 = fuse ? nullptr : mem.take<float>(b_s2);
-  const int dc = code(dt);
-  const float* twp = tw.data_ptr<float>();
-  void* st = c.stream;
+  const float scaling = (float)PyFloat_AS_DOUBLE(a[11]);
+  Tensor out;
+  {
+    Call c(x);
+    out = inplace ? x : empty(x.sizes(), dt, x.device());
+    const int64_t b_ids = cap * 4, b_q1 = T * H, b_s1 = T * kb1 * 4, b_ss1 = cap * kb1 * 4, b_mid = slots * N * 2, b_q2 = slots * I,
+                  b_s2 = slots * kb2 * 4, b_ss2 = cap * kb2 * 4, b_out = slots * H * 2;
+    using S = Scratch;
+    Scratch mem(2 * S::room(b_ids) + S::room(blocks * 4) + S::room(4) + S::room((E + 2) * 4) + S::room(b_q1) + S::room(b_s1) +
+                    (sorted ? S::room(b_ss1) + S::room(b_ss2) : 0) + (fuse ? 0 : S::room(b_mid) + S::room(b_s2)) + S::room(b_q2) +
+                    S::room(b_out),
+                c.stream);
+    int32_t* sorted_ids = mem.take<int32_t>(b_ids);
+    int32_t* even_ids = mem.take<int32_t>(b_ids);
+    int32_t* block_expert = mem.take<int32_t>(blocks * 4);
+    int32_t* padded = mem.take<int32_t>(4);
+    int32_t* cumsum = mem.take<int32_t>((E + 2) * 4);
+    void* q1 = mem.take(b_q1);
+    float* s1 = mem.take<float>(b_s1);
+    void* q2 = mem.take(b_q2);
+    void* down = mem.take(b_out);
+    float* ss1 = sorted ? mem.take<float>(b_ss1) : nullptr;
+    float* ss2 = sorted ? mem.take<float>(b_ss2) : nullptr;
+    void* mid = fuse ? nullptr : mem.take(b_mid);
+    float* sm2 = fuse ? nullptr : mem.take<float>(b_s2);
+    const int dc = code(dt);
+    const float* twp = tw.data_ptr<float>();
+    void* st = c.stream;
 
-  // small blocks read their scales column-major per token, large ones get them gathered into slot order
-  check(fp8k_moe_align_quant(ids.data_ptr(), ids64, slots, E + 1, bm, sorted_ids, cap, block_expert, blocks, padded, cumsum, x.data_ptr(), q1,
-                             s1, T, H, kEps, dc, sorted ? kb1 : 1, sorted ? 1 : T, st));
-  if (balanced) {
-    check(fp8k_moe_balance_blocks(sorted_ids, block_expert, padded, cap, bm, slots, E, even_ids, st));
-    sorted_ids = even_ids;
+    // small blocks read their scales column-major per token, large ones get them gathered into slot order
+    check(fp8k_moe_align_quant(ids.data_ptr(), ids64, slots, E + 1, bm, sorted_ids, cap, block_expert, blocks, padded, cumsum, x.data_ptr(), q1,
+                               s1, T, H, kEps, dc, sorted ? kb1 : 1, sorted ? 1 : T, st));
+    if (balanced) {
+      check(fp8k_moe_balance_blocks(sorted_ids, block_expert, padded, cap, bm, slots, E, even_ids, st));
+      sorted_ids = even_ids;
+    }
+    if (sorted) check(fp8k_moe_sort_scales(s1, ss1, sorted_ids, padded, cap, kb1, topk, slots, kb1, 1, st));
+    auto gemm = [&](const void* A, const Tensor& W, const Tensor& Ws, const float* As, int64_t as_m, int64_t as_k, void* C, bool weigh,
+                    int64_t per_row) {
+      check(fp8k_moe_block_gemm(A, W.data_ptr(), As, Ws.data_ptr<float>(), C, sorted_ids, block_expert, padded, weigh ? twp : nullptr, cap_used,
+                                bm, slots, per_row, E, W.size(1), W.size(2), W.size(2), as_m, as_k, W.stride(0), W.stride(1), Ws.stride(0),
+                                Ws.stride(1), Ws.stride(2), W.size(1), dc, (sorted ? 1 : 0) | (balanced ? 2 : 0), st));
+    };
+    if (fuse) {
+      check(fp8k_moe_block_gemm_silu_quant(q1, w13.data_ptr(), ss1, s13.data_ptr<float>(), q2, ss2, sorted_ids, block_expert, padded, cap,
+                                           slots, topk, E, N, H, H, cap, w13.stride(0), w13.stride(1), s13.stride(0), s13.stride(1),
+                                           s13.stride(2), I, cap, kEps, dc, balanced ? 1 : 0, st));
+    } else {
+      gemm(q1, w13, s13, sorted ? ss1 : s1, 1, sorted ? cap : T, mid, on_input, topk);
+    }
+    if (act_gemm2) {
+      check(fp8k_moe_act_block_gemm(mid, w2.data_ptr(), s2.data_ptr<float>(), down, sorted_ids, block_expert, padded, on_input ? nullptr : twp,
+                                    cap_used, bm, slots, E, H, I, N, w2.stride(0), I, s2.stride(0), s2.stride(1), s2.stride(2), H, kEps, dc, st));
+    } else if (!fuse) {
+      check(fp8k_silu_mul_group_quant(mid, q2, sm2, slots, I, 128, kEps, -448.f, 448.f, dc, sorted ? kb2 : 1, sorted ? 1 : slots,
+                                      FP8K_SCALE_F32, st));
+      if (sorted) check(fp8k_moe_sort_scales(sm2, ss2, sorted_ids, padded, cap, kb2, 1, slots, kb2, 1, st));
+    }
+    if (!act_gemm2) gemm(q2, w2, s2, sorted ? ss2 : sm2, 1, sorted ? cap : slots, down, !on_input, 1);
+    check(fp8k_moe_sum_reduce(down, out.data_ptr(), T, topk, H, topk * H, H, H, scaling, dc, st));
   }
-  if (sorted) check(fp8k_moe_sort_scales(s1, ss1, sorted_ids, padded, cap, kb1, topk, slots, kb1, 1, st));
-  auto gemm = [&](const void* A, const Tensor& W, const Tensor& Ws, const float* As, int64_t as_m, int64_t as_k, void* C, bool weigh,
-                  int64_t per_row) {
-    check(fp8k_moe_block_gemm(A, W.data_ptr(), As, Ws.data_ptr<float>(), C, sorted_ids, block_expert, padded, weigh ? twp : nullptr, cap_used,
-                              bm, slots, per_row, E, W.size(1), W.size(2), W.size(2), as_m, as_k, W.stride(0), W.stride(1), Ws.stride(0),
-                              Ws.stride(1), Ws.stride(2), W.size(1), dc, (sorted ? 1 : 0) | (balanced ? 2 : 0), st));
-  };
-  if (fuse) {
-    check(fp8k_moe_block_gemm_silu_quant(q1, w13.data_ptr(), ss1, s13.data_ptr<float>(), q2, ss2, sorted_ids, block_expert, padded, cap,
-                                         slots, topk, E, N, H, H, cap, w13.stride(0), w13.stride(1), s13.stride(0), s13.stride(1),
-                                         s13.stride(2), I, cap, kEps, dc, balanced ? 1 : 0, st));
-  } else {
-    gemm(q1, w13, s13, sorted ? ss1 : s1, 1, sorted ? cap : T, mid, on_input, topk);
-  }
-  if (act_gemm2) {
-    check(fp8k_moe_act_block_gemm(mid, w2.data_ptr(), s2.data_ptr<float>(), down, sorted_ids, block_expert, padded, on_input ? nullptr : twp,
-                                  cap_used, bm, slots, E, H, I, N, w2.stride(0), I, s2.stride(0), s2.stride(1), s2.stride(2), H, kEps, dc, st));
-  } else if (!fuse) {
-    check(fp8k_silu_mul_group_quant(mid, q2, sm2, slots, I, 128, kEps, -448.f, 448.f, dc, sorted ? kb2 : 1, sorted ? 1 : slots,
-                                    FP8K_SCALE_F32, st));
-    if (sorted) check(fp8k_moe_sort_scales(sm2, ss2, sorted_ids, padded, cap, kb2, 1, slots, kb2, 1, st));
-  }
-  if (!act_gemm2) gemm(q2, w2, s2, sorted ? ss2 : sm2, 1, sorted ? cap : slots, down, !on_input, 1);
-  check(fp8k_moe_sum_reduce(down, out.data_ptr(), T, topk, H, topk * H, H, H, (float)PyFloat_AS_DOUBLE(a[11]), dc, st));
   if (inplace) {
     Py_INCREF(a[0]);
     return a[0];

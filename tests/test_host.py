@@ -3,6 +3,10 @@
 They must decline - return None before launching anything - whatever they do not take as it is, so that the dispatcher path
 decides; and where they do take a call, its result is that of the dispatcher path, bit for bit.
 """
+import sys
+import threading
+import time
+
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -215,3 +219,52 @@ def test_bmm_tile_edges(dev, b, m, n, k):
     ref = (A[:, :m] @ B.transpose(1, 2)) * 0.125
     assert torch.equal(out[:, :m, :n].float().cpu(), ref.half().float())
     assert not out[:, m:].any() and not out[:, :, n:].any()
+
+
+def _calls(dev):
+    """One call per native function, of arguments it takes."""
+    x, (w, s) = _randn((40, 512)), _weight(256, 512)
+    q, xs = fp8_kernel.sglang_per_token_group_quant_fp8(x, 128)
+    h, e = _randn((20, 4, 128)).transpose(0, 1), 8
+    wb, wbs = fp8_utils.input_to_float8(_randn((4, 256, 128), seed=3))
+    qh, hs = fp8_kernel.per_tensor_quant_mla_fp8(h, torch.zeros((1,), device=dev))
+    logits, bias = _randn((40, e), torch.float32), _randn((e,), torch.float32)
+    tw, ids = fused_moe.biased_grouped_topk(x, logits, bias, 2, True, 4, 2)
+    w13, s13 = w.repeat(e, 1, 1).contiguous(), s.repeat(e, 1, 1).contiguous()
+    w2, s2 = [t.repeat(e, 1, 1).contiguous() for t in _weight(512, 128)]
+    return {
+        "group_quant": (x, 128, 1e-10, False, False, False, False),
+        "block_linear": (x, w, BLOCK, s, None),
+        "block_matmul": (q, w, xs, s, BLOCK, torch.bfloat16, False),
+        "token_linear": (x, w.t(), torch.ones((256, 1), device=dev), None, True),
+        "mla_quant": (h, torch.zeros((1,), device=dev), 1e-12),
+        "bmm": (qh, wb.transpose(1, 2), hs, wbs, torch.bfloat16),
+        "fused_gate": (logits, bias, 4, 2, 2, 0, 0.0, False),
+        "fused_experts": (x, w13, w2, s13, s2, tw, ids, 16, False, False, False, 1.0, False),
+    }
+
+
+@pytest.mark.gpu
+def test_other_threads_run_during_the_calls(dev):
+    """With a switch interval that nothing here reaches, another thread gets the interpreter only where a call gives it up."""
+    calls, ticks, stop = _calls(dev), [0], threading.Event()
+
+    def count():
+        while not stop.is_set():
+            ticks[0] += 1
+            time.sleep(0)
+
+    thread, interval = threading.Thread(target=count), sys.getswitchinterval()
+    sys.setswitchinterval(60.0)
+    try:
+        thread.start()
+        for name, args in calls.items():
+            fn, results, before = getattr(_host, name), [], ticks[0]  # kept: freeing a tensor gives the interpreter up as well
+            while len(results) < 5000 and ticks[0] == before:
+                results.append(fn(*args))
+            assert ticks[0] != before and all(r is not None for r in results), name
+    finally:
+        stop.set()
+        sys.setswitchinterval(interval)
+        thread.join()
+    torch.cuda.synchronize()
