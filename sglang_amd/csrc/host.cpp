@@ -6,11 +6,12 @@
 // torch's caching allocator in one piece and makes the C ABI calls back to back: 5 to 8 us for a linear.
 //
 // Every function returns None, before anything has been launched, for operands that it does not take as they are: tensors of
-// a dispatch mode or a subclass (tracing, fake tensors), inputs that want gradients, unusual types and layouts, and everything
+// a mode or a subclass (of the dispatcher's - tracing, fake tensors - or with a __torch_function__), inputs that want gradients, unusual types and layouts, and everything
 // that is an error.  The Python caller then goes through the dispatcher ops, which know all cases and word the errors.
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/grad_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
@@ -38,12 +39,15 @@ using c10::ScalarType;
 
 constexpr float kEps = 1e-10f;
 
+PyObject* g_has_torch_function = nullptr;  // torch.overrides.has_torch_function_unary
 PyObject* g_workspaces = nullptr;     // sgl_kernel._workspaces: (device index, stream) -> the buffer of that stream
 PyObject* g_grow_workspace = nullptr; // sgl_kernel._workspace
 
 // ---------------------------------------------------------------------------------------------- operands
-// A dispatch mode is active (tracing, fake tensors, functionalisation, vmap): the dispatcher has to see the ops.
+// A mode is active that has to see the ops: a torch function mode, or one of the dispatcher (tracing, fake tensors,
+// functionalisation, vmap).
 bool modes_active() {
+  if (at::impl::torch_function_mode_enabled()) return true;
   constexpr DispatchKeySet modes({DispatchKey::Python, DispatchKey::PythonTLSSnapshot, DispatchKey::Functionalize,
                                   DispatchKey::FuncTorchDynamicLayerFrontMode, DispatchKey::FuncTorchBatched,
                                   DispatchKey::Tracer});
@@ -60,8 +64,16 @@ bool plain(const Tensor& t, int device) {
   return !(t.requires_grad() && at::GradMode::is_enabled());
 }
 
+// a tensor whose class has no say in what is done with it: a subclass may have a __torch_function__ without being a dispatcher
+// subclass; parameters and subclasses that switch theirs off have none
 bool tensor_arg(PyObject* o, Tensor& t) {
-  if (!THPVariable_Check(o)) return false;
+  if (!THPVariable_CheckExact(o)) {  // neither a Tensor nor a Parameter
+    if (!THPVariable_Check(o)) return false;
+    PyObject* const has = PyObject_CallFunctionObjArgs(g_has_torch_function, o, nullptr);
+    if (!has) throw python_error();
+    Py_DECREF(has);  // True or False
+    if (has != Py_False) return false;
+  }
   t = THPVariable_Unpack(o);
   return true;
 }
@@ -606,4 +618,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "native calls of the layer
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host(void) {
+  PyObject* const overrides = PyImport_ImportModule("torch.overrides");
+  if (!overrides) return nullptr;
+  g_has_torch_function = PyObject_GetAttrString(overrides, "has_torch_function_unary");
+  Py_DECREF(overrides);
+  return g_has_torch_function ? PyModule_Create(&module) : nullptr;
+}

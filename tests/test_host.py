@@ -10,6 +10,7 @@ import time
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.overrides import TorchFunctionMode
 
 from sglang_amd import _host, fp8_kernel, fp8_utils, fused_moe, sgl_kernel
 
@@ -268,3 +269,58 @@ def test_other_threads_run_during_the_calls(dev):
         sys.setswitchinterval(interval)
         thread.join()
     torch.cuda.synchronize()
+
+
+class _Sub(torch.Tensor):
+    """A subclass without __torch_dispatch__: its key set is that of a plain tensor."""
+
+
+class _Quiet(torch.Tensor):
+    __torch_function__ = torch._C._disabled_torch_function_impl
+
+
+class _Record(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.gpu
+def test_function_subclasses_and_modes_are_seen(dev, dispatcher):
+    """Every native call declines a tensor of a class with a __torch_function__, in any place, and all of them under a function
+    mode; parameters and classes that switch theirs off are taken."""
+    for name, args in _calls(dev).items():
+        fn, places = getattr(_host, name), [i for i, a in enumerate(args) if isinstance(a, torch.Tensor)]
+
+        def with_class(i, cls):
+            return [a.as_subclass(cls) if j == i else a for j, a in enumerate(args)]
+
+        for i in places:
+            assert fn(*with_class(i, _Sub)) is None, (name, i)
+            assert fn(*with_class(i, _Quiet)) is not None, (name, i)
+            if args[i].is_floating_point() and args[i].element_size() > 1:
+                param = [torch.nn.Parameter(a, requires_grad=False) if j == i else a for j, a in enumerate(args)]
+                assert fn(*param) is not None, (name, i)
+        with torch._C.DisableTorchFunctionSubclass():
+            assert fn(*with_class(places[0], _Sub)) is not None
+        with _Record():
+            assert fn(*args) is None, name
+    # through the entry points: what comes back and what a mode sees are the dispatcher path's
+    x, (w, s) = _randn((40, 512)), _weight(256, 512)
+    sub = x.as_subclass(_Sub)
+    for call in (lambda: fp8_utils.w8a8_block_fp8_linear(sub, w, BLOCK, s),
+                 lambda: fp8_utils.w8a8_block_fp8_linear(x, w.as_subclass(_Sub), BLOCK, s),
+                 lambda: fp8_utils.apply_fp8_linear(sub, w.t(), torch.ones((256, 1), device=dev), use_per_token_if_dynamic=True),
+                 lambda: fp8_kernel.sglang_per_token_group_quant_fp8(sub, 128)[0]):
+        got, want = call(), dispatcher(call)
+        assert type(got) is type(want) and _same(got.as_subclass(torch.Tensor), want.as_subclass(torch.Tensor))
+        seen = []
+        for run in (call, lambda: dispatcher(call)):
+            with _Record() as mode:
+                run()
+            seen.append(mode.seen)
+        assert seen[0] == seen[1] and any("fp8k" in f for f in seen[0])
