@@ -14,6 +14,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/grad_mode.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPCachingAllocator.h>
@@ -27,6 +28,7 @@
 #include <initializer_list>
 #include <map>
 #include <mutex>
+#include <vector>
 
 #include "../../include/fp8k.h"
 
@@ -221,6 +223,9 @@ std::mutex& workspace_lock(const void* workspace) {
   return (*locks)[workspace];
 }
 
+// A record of the call for torch's profiler and other observers, as the dispatcher keeps one of an op: for the rest of the scope.
+#define OBSERVED(name, ...) RECORD_FUNCTION("fp8k::" name, (std::vector<c10::IValue>{__VA_ARGS__}))
+
 #define DECLINE Py_RETURN_NONE
 
 // ---------------------------------------------------------------------------------------------- group quant
@@ -245,6 +250,7 @@ PyObject* group_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor q, s;
   {
     Call c(x);
+    OBSERVED("group_quant", x);
     c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = K;
     q = empty(shape, ScalarType::Float8_e4m3fn, x.device());
@@ -295,6 +301,7 @@ PyObject* block_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor out;
   {
     Call c(x);
+    OBSERVED("block_linear", x, w, ws, bias);
     c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = N;
     out = empty(shape, dt, x.device());
@@ -337,6 +344,7 @@ PyObject* block_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor out;
   {
     Call c(x);
+    OBSERVED("block_matmul", x, w, xs, ws);
     out = empty({M, N}, dt, x.device());
     std::unique_lock<std::mutex> together;
     if (work) together = std::unique_lock<std::mutex>(workspace_lock(work));
@@ -375,6 +383,7 @@ PyObject* token_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor out;
   {
     Call c(x);
+    OBSERVED("token_linear", x, w, ws, bias);
     c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = N;
     out = empty(shape, dt, x.device());
@@ -420,6 +429,7 @@ PyObject* mla_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor q;
   {
     Call c(x);
+    OBSERVED("mla_quant", x, s);
     q = empty(x.sizes(), ScalarType::Float8_e4m3fn, x.device());
     int32_t* const sync = fp8k_tensor_quant_mla_takes_sync(x.numel()) ? stream_sync(x, c.stream) : nullptr;
     check(fp8k_tensor_quant_mla_sync(x.data_ptr(), q.data_ptr(), s.data_ptr<float>(), x.size(0), x.size(1), x.size(2), x.stride(0),
@@ -446,6 +456,7 @@ PyObject* bmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor out;
   {
     Call c(A);
+    OBSERVED("bmm", A, B, as, bs);
     out = empty({b, m, nn}, dt, A.device());
     check(fp8k_bmm_fp8_tensor_scales(A.data_ptr(), B.data_ptr(), as.data_ptr<float>(), bs.data_ptr<float>(), out.data_ptr(), b, m, nn, k,
                        b > 1 ? A.stride(0) : m * k, m > 1 ? A.stride(1) : k, b > 1 ? B.stride(0) : nn * k, nn > 1 ? B.stride(2) : k,
@@ -476,6 +487,7 @@ PyObject* fused_gate(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor w, ids;
   {
     Call c(x);
+    OBSERVED("fused_gate", x, bias);
     w = empty({rows, topk}, ScalarType::Float, x.device());
     ids = empty({rows, topk}, ScalarType::Int, x.device());
     check(fp8k_moe_fused_gate(x.data_ptr(), bias.data_ptr(), w.data_ptr<float>(), ids.data_ptr<int32_t>(), rows, x.size(1), groups,
@@ -532,6 +544,7 @@ PyObject* fused_experts(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor out;
   {
     Call c(x);
+    OBSERVED("fused_experts", x, w13, w2, s13, s2, tw, ids);
     out = inplace ? x : empty(x.sizes(), dt, x.device());
     const int64_t b_ids = cap * 4, b_q1 = T * H, b_s1 = T * kb1 * 4, b_ss1 = cap * kb1 * 4, b_mid = slots * N * 2, b_q2 = slots * I,
                   b_s2 = slots * kb2 * 4, b_ss2 = cap * kb2 * 4, b_out = slots * H * 2;

@@ -324,3 +324,17 @@ def test_function_subclasses_and_modes_are_seen(dev, dispatcher):
                 run()
             seen.append(mode.seen)
         assert seen[0] == seen[1] and any("fp8k" in f for f in seen[0])
+
+
+@pytest.mark.gpu
+def test_profiler_sees_the_calls(dev):
+    """A record per native call, with the shapes of its tensors, where the dispatcher keeps one of an op."""
+    calls = _calls(dev)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=True) as prof:
+        for name, args in calls.items():
+            getattr(_host, name)(*args)
+    records = {e.name: e for e in prof.events() if e.name.startswith("fp8k::")}
+    assert set(records) == {"fp8k::" + name for name in calls}
+    for name, args in calls.items():
+        shapes = [list(a.shape) for a in args if isinstance(a, torch.Tensor) and a.dim()]
+        assert [s for s in records["fp8k::" + name].input_shapes if s] == shapes, name
