@@ -398,10 +398,15 @@ PyObject* token_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---------------------------------------------------------------------------------------------- absorbed products
-// Three zeroed int32 per (device, stream) for fp8k_tensor_quant_mla_sync, made on first use and kept: at most kMaxSync of them, other
-// streams (and calls under graph capture, whose replays may run on any stream) get none and take the two launches.
+// Three zeroed int32 per (device, stream) for fp8k_tensor_quant_mla_sync, made on first use and kept: at most kMaxSync of them.  What
+// makes one stream of a handle are torch's own streams, which live as long as the process.  A stream that came in from outside (its
+// id is its handle) may be destroyed and its handle given to another while launches are queued, and hipStreamPerThread is one handle
+// for a stream of every thread.  Those get none and take the two launches, as do calls under graph capture, whose replays may
+// run on any stream.
 constexpr size_t kMaxSync = 64;
-int32_t* stream_sync(const Tensor& like, hipStream_t st) {
+int32_t* stream_sync(const Tensor& like, const c10::hip::HIPStream& stream) {
+  const hipStream_t st = stream.stream();
+  if (st && (uint64_t)stream.id() == (uint64_t)(uintptr_t)st) return nullptr;
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return nullptr;
   static std::mutex mutex;
@@ -431,7 +436,7 @@ PyObject* mla_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Call c(x);
     OBSERVED("mla_quant", x, s);
     q = empty(x.sizes(), ScalarType::Float8_e4m3fn, x.device());
-    int32_t* const sync = fp8k_tensor_quant_mla_takes_sync(x.numel()) ? stream_sync(x, c.stream) : nullptr;
+    int32_t* const sync = fp8k_tensor_quant_mla_takes_sync(x.numel()) ? stream_sync(x, c10::hip::getCurrentHIPStream(dev)) : nullptr;
     check(fp8k_tensor_quant_mla_sync(x.data_ptr(), q.data_ptr(), s.data_ptr<float>(), x.size(0), x.size(1), x.size(2), x.stride(0),
                                      x.stride(1), eps, code(dt), sync, c.stream));
   }

@@ -170,6 +170,24 @@ def test_mla_quant_in_one_launch(dev, dispatcher, heads, m, k):
 
 
 @pytest.mark.gpu
+def test_mla_quant_keeps_nothing_for_streams_from_outside(dev):
+    """The counters of the one-launch form belong to a stream that torch made; under a handle that may come to mean another stream, or
+    means one per thread, the two launches run."""
+    x = _randn((64, 32, 128)).transpose(0, 1)
+    want = fp8_kernel.per_tensor_quant_mla_fp8(x, torch.zeros((1,), device=dev))
+    own, before = torch.cuda.Stream(), torch.cuda.memory_allocated()
+    per_thread = 2  # hipStreamPerThread
+    for stream in (torch.cuda.ExternalStream(own.cuda_stream), torch.cuda.ExternalStream(per_thread)):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            got = fp8_kernel.per_tensor_quant_mla_fp8(x, torch.zeros((1,), device=dev))
+        torch.cuda.synchronize()
+        assert _same(got, want)
+        del got
+        assert torch.cuda.memory_allocated() == before
+
+
+@pytest.mark.gpu
 def test_mla_quant_in_one_launch_ends_its_wait(dev):
     """A count that never comes out (set from the host): every workgroup gives up its bounded wait and finds the maximum for itself."""
     from sglang_amd._lib import BF16, check, lib, stream_ptr
