@@ -449,10 +449,14 @@ __global__ __launch_bounds__(1024) void rows_tensor_quant_small_kernel(const voi
 // sync[1], counts itself in at sync[0], waits until all have, and quantises what it still holds - the tensor is read once, and the
 // host pays for one launch (4.2 us of an absorbed product's 18.7 with its zeroed scale).  The counting costs a queue at one line per
 // workgroup, so they are few and large: 256 of 256 threads took 6 us longer than 64 of 1024 at 2 MB.  The wait is bounded: an idle
-// chip holds all of them at once, but work of other streams may keep CUs, so a workgroup that has waited kMlaSpins polls takes the
-// maximum of the whole tensor for itself and goes on; nobody depends on another one's progress.  The last to leave writes the
-// scale and zeroes the three words for the next launch on them, which must be on the same stream.
-constexpr int kMlaOnceHold = 4, kMlaOnceGroups = 64, kMlaSpins = 4096;
+// chip with a CU for each holds all of them at once, but work of other streams may keep CUs, so a workgroup that has waited kMlaSpins
+// polls takes the maximum of the whole tensor for itself and goes on; nobody depends on another one's progress.  The last to leave
+// writes the scale and zeroes the three words for the next launch on them, which must be on the same stream.
+// What the wait may cost: a poll takes 0.12 us and the maximum of the whole tensor 22 / 60 / 128 us at 0.5 / 2 / 4 MB, so it ends about
+// where going on alone would have cost as much: 52 / 90 / 156 us in all for a count that never comes out (485 / 522 / 576 with 4096
+// polls).  Beside 256x256 GEMMs of another stream that hold every CU for 470 us each, 58 calls come through in 60 GEMMs' time (29 of
+// the two launches, each of which waits for a gap) and the GEMMs take no longer, 27.3 ms; with 64 polls they take 31.2.
+constexpr int kMlaOnceHold = 4, kMlaOnceGroups = 64, kMlaSpins = 256;
 template <int DT>
 __global__ __launch_bounds__(1024) void rows_tensor_quant_once_kernel(const void* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ s,
                                                                      uint32_t total, uint32_t chunks, uint32_t S, int64_t stride_h,
