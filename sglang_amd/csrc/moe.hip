@@ -911,6 +911,7 @@ extern "C" int fp8k_moe_sum(const void* x, void* out, int64_t tokens, int64_t to
 // moe_fused_gate: grouped top-k routing with a selection bias (DeepSeek-V3 style), one token per sub-group of
 // TPR = num_expert_group lanes, VPT = experts / groups values per lane (a lane holds one whole expert group).
 //   score  = T(sigmoid(x));  choice = T(score + bias)                       (arithmetic in the input type T)
+//   A choice that is no number ranks with -inf, below every number (gate_choice), in both forms of the kernel.
 //   group weight = T(top1 + top2 of choice inside the group); the groups with the smallest weight are dropped
 //   one at a time until topk_group remain (ties: the higher group goes), then the topk best choices among the
 //   remaining groups are taken one at a time (ties: the lower expert wins).  Weights are the un-biased scores,
@@ -922,6 +923,19 @@ __device__ __forceinline__ float gate_load(const void* p, int64_t i) {
   if (DT == FP8K_F32) return ((const float*)p)[i];
   if (DT == FP8K_BF16) return __uint_as_float((uint32_t)((const u16*)p)[i] << 16);
   return f16_bits_to_f32(((const u16*)p)[i]);
+}
+
+// Comparisons with a NaN are all false: which of two values it hides would depend on how a kernel lays out its reductions.
+template <int DT>
+__device__ __forceinline__ float gate_choice(float score, float bias) {
+  const float c = round_to<DT>(score + bias);
+  return c == c ? c : -__builtin_inff();
+}
+// weight of a group from its two largest choices; of +inf and -inf it is +inf
+template <int DT>
+__device__ __forceinline__ float gate_group_weight(float m1, float m2) {
+  const float s = round_to<DT>(m1 + m2);
+  return s == s ? s : m1;
 }
 
 template <int DT, int VPT>
@@ -965,11 +979,13 @@ __global__ __launch_bounds__(256) void moe_fused_gate_kernel(const void* __restr
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       score[i] = round_to<DT>(1.0f / (1.0f + expf(-xin[i])));
-      choice[i] = round_to<DT>(score[i] + bin[i]);
+      choice[i] = gate_choice<DT>(score[i], bin[i]);
     }
   }
 
-  // drop the weakest groups: a group's weight does not change while other groups are dropped
+  // drop the weakest groups: dropping the smallest weight (of equal ones the highest group) until topk_group remain keeps the
+  // first topk_group in the order of (larger weight, lower group)
+  bool dropped;
   {
     float m1 = -__builtin_inff(), m2 = -__builtin_inff();
 #pragma unroll
@@ -978,18 +994,13 @@ __global__ __launch_bounds__(256) void moe_fused_gate_kernel(const void* __restr
       if (v > m1) { m2 = m1; m1 = v; }
       else if (v > m2) m2 = v;
     }
-    const float gsum = VPT > 1 ? round_to<DT>(m1 + m2) : m1;
-    bool dropped = false;
-    for (int k = 0; k < tpr - topk_group; ++k) {
-      float sum = dropped ? kCleared : gsum;
-      int grp = lane_in_row;
-      for (int mask = tpr >> 1; mask > 0; mask >>= 1) {
-        const float osum = __shfl_xor(sum, mask, tpr);
-        const int ogrp = __shfl_xor(grp, mask, tpr);
-        if (sum > osum || (osum == sum && ogrp > grp)) { sum = osum; grp = ogrp; }
-      }
-      dropped = dropped || lane_in_row == grp;
+    const float gsum = VPT > 1 ? gate_group_weight<DT>(m1, m2) : m1;
+    int rank = 0;
+    for (int g = 0; g < tpr; ++g) {
+      const float o = __shfl(gsum, g, tpr);
+      rank += (o > gsum || (o == gsum && g < lane_in_row)) ? 1 : 0;
     }
+    dropped = rank >= topk_group;
     if (dropped) {
 #pragma unroll
       for (int i = 0; i < VPT; ++i) choice[i] = kCleared;
@@ -1020,7 +1031,7 @@ __global__ __launch_bounds__(256) void moe_fused_gate_kernel(const void* __restr
     }
     float best = tv[0];
     int idx = ti[0];
-    if (choice[0] == kCleared) { best = -__builtin_inff(); idx = first; }
+    if (dropped && choice[0] == kCleared) { best = -__builtin_inff(); idx = first; }
     for (int mask = tpr >> 1; mask > 0; mask >>= 1) {
       const float obest = __shfl_xor(best, mask, tpr);
       const int oidx = __shfl_xor(idx, mask, tpr);
@@ -1096,7 +1107,7 @@ __global__ __launch_bounds__(256) void moe_fused_gate_wave_kernel(const void* __
 #pragma unroll
   for (int i = 0; i < EPL; ++i) {
     score[i] = round_to<DT>(1.0f / (1.0f + expf(-gate_load<DT>(input, row * experts + first + i))));
-    choice[i] = round_to<DT>(score[i] + gate_load<DT>(bias, first + i));
+    choice[i] = gate_choice<DT>(score[i], gate_load<DT>(bias, first + i));
   }
   // group weight: the two largest choices of the group; equal ones count twice
   bool group0_gone;
@@ -1112,9 +1123,7 @@ __global__ __launch_bounds__(256) void moe_fused_gate_wave_kernel(const void* __
       m2 = fmaxf(fminf(m1, o1), fmaxf(m2, o2));
       m1 = fmaxf(m1, o1);
     }
-    const float gsum = lpg * EPL > 1 ? round_to<DT>(m1 + m2) : m1;
-    // dropping the smallest weight (of equal ones the highest group) until topk_group remain keeps the first topk_group in
-    // the order of (larger weight, lower group)
+    const float gsum = lpg * EPL > 1 ? gate_group_weight<DT>(m1, m2) : m1;
     int rank = 0;
     const int group = lane / lpg;
     for (int g = 0; g < groups; ++g) {

@@ -936,6 +936,47 @@ def test_moe_fused_gate_forms_agree(dev, params, dtype):
             assert torch.equal(many[0][-77:], few[0]) and torch.equal(many[1][-77:], few[1])
 
 
+@pytest.mark.parametrize("params", [(64, 8, 3, 6), (64, 4, 1, 16), (128, 8, 4, 8), (128, 16, 16, 20), (64, 16, 2, 4)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_moe_fused_gate_of_what_is_no_number(dev, params, dtype):
+    """NaN logits (the first and the last of a group, a whole group, a whole row, one value anywhere) and infinite biases route alike in
+    both forms; a NaN ranks below every number, so the others of its row are routed as without it."""
+    from sglang_amd.sgl_kernel import moe_fused_gate
+
+    E, G, tg, topk = params
+    g = torch.Generator().manual_seed(E + G)
+    x = (torch.randperm(8197 * E, generator=g).reshape(8197, E).float() / (8197 * E) - 0.5).to(dtype)
+    bias = torch.randn((E,), generator=g) * 0.1
+    per, tail = E // G, x[-77:]
+    tail[0::7, :: per] = float("nan")
+    tail[1::7, per - 1 :: per] = float("nan")
+    tail[2::7, :per] = float("nan")
+    tail[3::7] = float("nan")
+    tail[4::7, 5] = float("nan")
+    tail[5::7, E - per :] = float("nan")
+    forced = bias.clone()
+    forced[::per], forced[3] = float("inf"), -float("inf")
+    same = lambda a, b: torch.equal(torch.nan_to_num(a, nan=-1.0), torch.nan_to_num(b, nan=-1.0))  # noqa: E731
+    for b in (bias, forced):
+        for shared, scale_out in ((0, True), (1, False)):
+            many = moe_fused_gate(x.to(dev), b.to(dtype).to(dev), G, tg, topk, shared, 2.5, scale_out)
+            few = moe_fused_gate(tail.to(dev), b.to(dtype).to(dev), G, tg, topk, shared, 2.5, scale_out)
+            assert same(many[0][-77:], few[0]) and torch.equal(many[1][-77:], few[1])
+            assert int(few[1].min()) >= 0 and int(few[1].max()) < E + shared
+    if dtype == torch.float32:
+        ids = moe_fused_gate(tail.to(dev), bias.to(dev), G, tg, topk)[1].cpu()
+        choice = torch.nan_to_num(torch.sigmoid(tail) + bias, nan=-float("inf"))
+        for r in range(77):
+            groups = choice[r].reshape(G, per)
+            weight = groups.topk(min(2, per), dim=1).values.sum(dim=1)
+            kept = weight.sort(descending=True, stable=True).indices[:tg]
+            left = torch.full_like(groups, -float("inf"))
+            left[kept] = groups[kept]
+            finite = int(torch.isfinite(left).sum())
+            if finite >= topk:
+                assert ids[r].tolist() == left.reshape(-1).sort(descending=True, stable=True).indices[:topk].tolist()
+
+
 def test_biased_grouped_topk_is_the_gate_kernel_and_matches_the_tensor_op_restatement(dev):
     """The layer-level routing entry point runs the fused gate kernel; on well-separated float32 logits its expert sets
     and weights are those of the tensor-op restatement of topk.py:665-738 kept with the tests.  Shapes the kernel does
