@@ -1,5 +1,5 @@
 // Grouped FP8 GEMM of 16- or 32-slot blocks with a short K (the second GEMM of experts whose intermediate size is sharded or
-// small: K = 256 .. 2048), gfx950.
+// small: K = 256 .. 1280), gfx950.
 //
 // It is a stream of the hit experts' weights, but in tiles of 128 weight rows x K bytes = 32 .. 128 KB: a workgroup per tile
 // (gemm_direct_kernel) spends most of its life on what comes before the stream - block table, slot table, activation rows,
@@ -8,7 +8,7 @@
 // of ALL of K and their scales in LDS, and its weight stream runs on across tiles and blocks: every wave owns 16 weight rows of
 // each tile of the run and keeps D K blocks of them in flight in registers, the next tile's following this tile's last.
 // Finished rows are stored without a barrier; the waves meet only where the block changes.  Two workgroups share a CU, so one
-// streams while the other changes blocks.
+// streams while the other changes blocks; that takes LDS for two, which K = 2048 with 32 slots (84 KB) does not leave.
 //
 // Whole layer, before -> now: 128 experts, H = 4096, top 6, 128 tokens, I = 256 176 -> 113 us, I = 512 224 -> 191; 256 experts,
 // H = 7168, I = 512, 865 tokens 739 -> 578 (its second GEMM, 940 MB of weights, 372 -> 211 us).
@@ -25,8 +25,13 @@
 
 namespace fp8k {
 
-constexpr int kMoeShortKMax = 2048;
+constexpr int kLdsBytes = 160 * 1024;  // of a CU
+constexpr int kMoeShortKMax = 1280, kMoeShortKFew = 512, kMoeShortKAct = 1024;  // with 32 and 16 slots per block (rule: moe.hip); ACT
 __host__ __device__ constexpr int moe_shortk_row(int K) { return K + 16; }  // LDS row: rows of an operand fetch fall into different banks
+constexpr int moe_shortk_lds(int slots, int K) {  // a workgroup's: activation rows, the waves' weight slots, scales
+  return slots * moe_shortk_row(K) + 8 * 16 * kTileK + kMoeShortKMax / kTileK * slots * 4;
+}
+static_assert(2 * moe_shortk_lds(32, kMoeShortKMax) <= kLdsBytes, "two workgroups share a CU, and the grid has two for each");
 
 template <int TM, int OUT_DT, bool ACT>
 __global__ __launch_bounds__(512, 4) void moe_shortk_kernel(const GemmArgs p) {

@@ -589,12 +589,16 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
   hipStream_t st = (hipStream_t)stream;
 #define FP8K_MOE_DIRECT(TM, O) \
   hipLaunchKernelGGL((gemm_direct_kernel<TM, kModeBlock, O, FP8K_F32, false, true>), dim3((unsigned)nwg), dim3(512), 0, st, a)
-  // Short K: a run of tiles per workgroup, where there are more tiles than workgroups (two per CU) to make runs of.  With 16
-  // slots a tile is all weight stream, and from 16 K blocks on a workgroup per tile with eight K blocks in flight is level or
-  // 2 % ahead (128 experts, H = 4096, 8 .. 64 tokens, K = 2048); with 32 slots the run is ahead at every K that fits.
+  // Short K: a run of tiles per workgroup, where there are more tiles than workgroups (two per CU) to make runs of.  The longer the
+  // K, the less of a tile's time is the set-up that a run saves.  With 32 slots a run is 3 - 13 % ahead of a workgroup per tile up
+  // to K = 1152, 1 % behind to 9 % ahead at 1280 and behind with half-full blocks from 1408 on (5 % at 1536, 7 at 1920; 256 experts,
+  // 7168 weight rows, 256 tokens, K = 1152 / 1280 / 1920 379 / 421 / 614 us against 397 / 424 / 573).  With 16 slots a tile is
+  // all weight stream: level at K = 512, 6 - 10 % behind from 768 on (100 tokens, K = 512 / 1024 161 / 311 us against 158 / 282).
+  // At K = 2048 with 32 slots, where one workgroup fits a CU, whole layers took 1 - 26 % longer as runs: 256 experts, H = 7168,
+  // 256 / 512 / 700 tokens 1807 / 1900 / 2020 us against 1738 / 1852 / 2010, 64 experts, H = 2048, 150 tokens 186 against 149.
   const int64_t blocks_max = moe_blocks_in_use(num_valid_tokens, num_experts, block_m, a.m_blocks);
   const int64_t most = 2 * (int64_t)num_cu() / 8 * 8;
-  if (direct && K <= (block_m == 16 ? kMoeShortKMax / 2 : kMoeShortKMax) && blocks_max * a.tiles_n > most && N * ldb < (1LL << 31)) {
+  if (direct && K <= (block_m == 16 ? kMoeShortKFew : kMoeShortKMax) && blocks_max * a.tiles_n > most && N * ldb < (1LL << 31)) {
     const dim3 grid((unsigned)most), block(512);
     const unsigned lds = (unsigned)(block_m * moe_shortk_row((int)K));
 #define FP8K_SHORTK(TM, O) hipLaunchKernelGGL((moe_shortk_kernel<TM, O, false>), grid, block, lds, st, a)
@@ -688,7 +692,7 @@ extern "C" int fp8k_moe_block_gemm_ue8m0(const void* A, const void* B, const flo
 }
 
 extern "C" int fp8k_moe_act_block_gemm_takes(int64_t block_m, int64_t N, int64_t K, int64_t ldb) {
-  return (block_m == 16 || block_m == 32) && K > 0 && K % kTileK == 0 && K <= kMoeShortKMax / 2 && N > 0 && N % 8 == 0 && N * ldb < (1LL << 31);
+  return (block_m == 16 || block_m == 32) && K > 0 && K % kTileK == 0 && K <= kMoeShortKAct && N > 0 && N % 8 == 0 && N * ldb < (1LL << 31);
 }
 
 extern "C" int fp8k_moe_act_block_gemm(const void* x, const void* B, const float* Bs, void* C, const int32_t* sorted_token_ids,
@@ -699,7 +703,7 @@ extern "C" int fp8k_moe_act_block_gemm(const void* x, const void* B, const float
   clear_error();
   const char* op = "moe_act_block_gemm";
   FP8K_REQUIRE(fp8k_moe_act_block_gemm_takes(block_m, N, K, ldb), "%s: block_m 16 or 32, K a multiple of 128 up to %d, N of 8 (got %lld, %lld, %lld)",
-               op, kMoeShortKMax / 2, (long long)block_m, (long long)K, (long long)N);
+               op, kMoeShortKAct, (long long)block_m, (long long)K, (long long)N);
   FP8K_REQUIRE(dtype == FP8K_F16 || dtype == FP8K_BF16, "%s: the activation type must be Half or BFloat16", op);
   FP8K_REQUIRE(num_experts > 0 && num_valid_tokens >= 0 && num_valid_tokens < 0x7fffffffLL && sorted_capacity >= 0 && sorted_capacity < 0x7fffffffLL,
                "%s: bad shape", op);

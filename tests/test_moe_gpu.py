@@ -412,10 +412,11 @@ def test_grouped_gemm_256_slot_blocks_every_group_count(dev):
 
 
 @pytest.mark.parametrize("T,E,topk,N,K,block", [(64, 40, 2, 2056, 128, 16), (70, 24, 3, 3080, 384, 16), (33, 40, 1, 2048, 1024, 16),
-                                                (90, 64, 4, 1160, 640, 32), (200, 8, 4, 2568, 2048, 32), (130, 96, 6, 1032, 256, 32)])
+                                                (90, 64, 4, 1160, 640, 32), (200, 8, 4, 2568, 2048, 32), (200, 8, 4, 2568, 1280, 32), (64, 40, 2, 2056, 512, 16),
+                                                (130, 96, 6, 1032, 256, 32)])
 def test_grouped_gemm_short_k_runs_exact(dev, T, E, topk, N, K, block):
     """More tiles than workgroups, so that each takes a run of them: runs that start and end inside a block, blocks of one slot and
-    full ones, one to 16 K blocks, a last tile of 8 weight rows, ids of -1 (stored as zeros); exact on integer data."""
+    full ones, one to ten K blocks and K that is left to a workgroup per tile, a last tile of 8 weight rows, ids of -1 (stored as zeros); exact on integer data."""
     from sglang_amd.fused_moe import moe_align_block_size
     from sglang_amd.sgl_kernel import moe_block_gemm
 
