@@ -80,7 +80,12 @@ bool tensor_arg(PyObject* o, Tensor& t) {
   return true;
 }
 
-bool truth(PyObject* o) { return o == Py_True || (o != Py_False && PyObject_IsTrue(o) == 1); }
+bool truth(PyObject* o) {
+  if (o == Py_True || o == Py_False) return o == Py_True;
+  const int is = PyObject_IsTrue(o);
+  if (is < 0) throw python_error();
+  return is == 1;
+}
 
 bool is_fp8(const Tensor& t) { return t.scalar_type() == ScalarType::Float8_e4m3fn; }
 bool is_half(ScalarType t) { return t == ScalarType::BFloat16 || t == ScalarType::Half; }
@@ -226,7 +231,12 @@ std::mutex& workspace_lock(const void* workspace) {
 // A record of the call for torch's profiler and other observers, as the dispatcher keeps one of an op: for the rest of the scope.
 #define OBSERVED(name, ...) RECORD_FUNCTION("fp8k::" name, (std::vector<c10::IValue>{__VA_ARGS__}))
 
-#define DECLINE Py_RETURN_NONE
+// an argument that did not convert is the dispatcher path's to word as well
+#define DECLINE     \
+  do {              \
+    PyErr_Clear();  \
+    Py_RETURN_NONE; \
+  } while (0)
 
 // ---------------------------------------------------------------------------------------------- group quant
 // group_quant(x, group_size, eps, column_major, tma_aligned, ue8m0, fuse_silu) -> (q, scales) or None
@@ -488,7 +498,7 @@ PyObject* fused_gate(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t topk = PyLong_AsLongLong(a[4]), shared = PyLong_AsLongLong(a[5]);
   const double scaling = PyFloat_AS_DOUBLE(a[6]);
   const bool scale_output = truth(a[7]);
-  if (topk <= 0) DECLINE;
+  if (topk <= 0 || PyErr_Occurred()) DECLINE;
   Tensor w, ids;
   {
     Call c(x);

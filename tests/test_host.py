@@ -30,6 +30,14 @@ def test_declines_what_it_does_not_take():
         assert _host.group_quant(f, 128, 1e-10, False, False, False, False) is None
 
 
+def test_declines_numbers_that_do_not_convert():
+    """A number too large for the check is declined like any other, without an error left behind."""
+    x, w, s = torch.zeros((4, 256), dtype=torch.bfloat16), torch.zeros((128, 256), dtype=torch.float8_e4m3fn), torch.ones((1, 2))
+    assert _host.block_linear(x, w, [2**100, 128], s, None) is None
+    with pytest.raises(RuntimeError, match="only block_size"):
+        fp8_kernel.w8a8_block_fp8_matmul(w, w, s, s, [2**100, 128])
+
+
 @pytest.fixture
 def dispatcher(monkeypatch):
     """Calls fn() with every native call declining."""
