@@ -124,16 +124,6 @@ int fp8k_block_gemm(const void* A, const void* B, const float* As, const float* 
                     int64_t workspace_bytes, void* stream);
 
 /*
- * fp8k_block_gemm followed by `+ bias` (the two statements of the reference's linear, fp8_utils.py:220-226), in the
- * kernel's write-out: the product is rounded to out_dtype, then bias[n] (out_dtype, [N], may be NULL) is added in float32
- * and the sum rounded again, so the result is the elementwise addition's bit for bit.
- */
-int fp8k_block_gemm_bias(const void* A, const void* B, const float* As, const float* Bs, const void* bias, void* C,
-                         int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t as_stride_m,
-                         int64_t as_stride_k, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, int out_dtype,
-                         void* workspace, int64_t workspace_bytes, void* stream);
-
-/*
  * The same product with power-of-two scales that the matrix core applies itself (no float promote per K block):
  * As_packed int32 words of four UE8M0 exponent bytes, as fp8k_group_quant writes them with FP8K_SCALE_UE8M0_PACKED
  * (row m, K blocks 4j..4j+3 in the word at As_packed[m*as_stride_m + j*as_stride_w]); Bs float32, every value a power of
@@ -175,21 +165,16 @@ int fp8k_block_gemm_noalloc(const void* A, const void* B, const float* As, const
 int fp8k_scaled_mm(const void* A, const void* B, const float* sa, const float* sb, const void* bias, void* C,
                    int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int out_dtype,
                    int bias_dtype, void* workspace, int64_t workspace_bytes, void* stream);
-/*
- * fp8k_scaled_mm with strides for the two scale vectors: 1 as above, 0 for one scale that holds for every row / column
- * (a per-tensor scale needs no broadcast copy).  Same workspace.
- */
-int fp8k_scaled_mm_strided(const void* A, const void* B, const float* sa, int64_t sa_stride, const float* sb,
-                           int64_t sb_stride, const void* bias, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
-                           int64_t ldb, int64_t ldc, int out_dtype, int bias_dtype, void* workspace,
-                           int64_t workspace_bytes, void* stream);
 int64_t fp8k_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
  * A whole linear on 16-bit activations x [M, K] (contiguous): the group quantisation (fp8k_group_quant, group 128, float
- * scales; K a multiple of 128) or the per-token one (fp8k_token_quant; K a multiple of 16), then fp8k_block_gemm_bias resp.
- * fp8k_scaled_mm_strided; the results are those of the two calls bit for bit.  A few rows (the sizes for which
- * fp8k_linear_fuses_quant returns 1) take one launch.  dtype: of x and C.  Workspace: 256-byte aligned, fp8k_linear_workspace_bytes of it (0 possible), nothing in it has to be initialised.
+ * scales; K a multiple of 128) or the per-token one (fp8k_token_quant; K a multiple of 16), then fp8k_block_gemm resp.
+ * fp8k_scaled_mm, whose results are the linear's bit for bit.  sb_stride 1: sb [N]; 0: one scale for the whole weight.
+ * bias [N] or NULL.  fp8k_block_linear adds one of type dtype as the reference's linear does (fp8_utils.py:220-226): to the
+ * product rounded to dtype, in float32, and rounds again; fp8k_token_linear as fp8k_scaled_mm does.  A few rows (the sizes for
+ * which fp8k_linear_fuses_quant returns 1) take one launch.  dtype: of x and C.  Workspace: 256-byte aligned,
+ * fp8k_linear_workspace_bytes of it (0 possible), nothing in it has to be initialised.
  */
 int fp8k_linear_fuses_quant(int64_t M, int64_t N, int64_t K);
 int64_t fp8k_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int block_mode);

@@ -61,10 +61,6 @@ SIGNATURES = {
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr] + [_c_i64] * 10 + [_c_int, _c_ptr, _c_i64, _c_ptr],
     ),
-    "fp8k_block_gemm_bias": (
-        _c_int,
-        [_c_ptr] * 6 + [_c_i64] * 10 + [_c_int, _c_ptr, _c_i64, _c_ptr],
-    ),
     "fp8k_block_gemm_ue8m0": (
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr] + [_c_i64] * 10 + [_c_int, _c_ptr, _c_i64, _c_ptr],
@@ -74,10 +70,6 @@ SIGNATURES = {
     "fp8k_scaled_mm": (
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr] + [_c_i64] * 6 + [_c_int, _c_int, _c_ptr, _c_i64, _c_ptr],
-    ),
-    "fp8k_scaled_mm_strided": (
-        _c_int,
-        [_c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr] + [_c_i64] * 6 + [_c_int, _c_int, _c_ptr, _c_i64, _c_ptr],
     ),
     "fp8k_scaled_mm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "fp8k_linear_fuses_quant": (_c_int, [_c_i64] * 3),

@@ -434,7 +434,7 @@ extern "C" void fp8k_tune_force_gemm_plan(int kind, int splits) {
 extern "C" int64_t fp8k_block_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) { return block_gemm_workspace_bytes(M, N, K); }
 extern "C" int64_t fp8k_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) { return workspace_bytes(M, N, K); }
 
-static int block_gemm_impl(const void* A, const void* B, const float* As, const float* Bs, const void* bias, void* C, int64_t M, int64_t N,
+static int block_gemm_impl(const void* A, const void* B, const float* As, const float* Bs, void* C, int64_t M, int64_t N,
                            int64_t K, int64_t lda, int64_t ldb, int64_t as_stride_m, int64_t as_stride_k,
                            int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, int out_dtype, void* workspace,
                            int64_t workspace_bytes_given, void* stream) {
@@ -454,7 +454,7 @@ static int block_gemm_impl(const void* A, const void* B, const float* As, const 
     return fail(FP8K_ERR_WORKSPACE, "fp8_blockwise_scaled_mm: workspace of %lld bytes required, %lld given",
                 (long long)need, (long long)(workspace ? workspace_bytes_given : 0));
   GemmArgs a{};
-  a.X = (const uint8_t*)A; a.W = (const uint8_t*)B; a.sx = As; a.sw = Bs; a.bias = bias; a.C = C;
+  a.X = (const uint8_t*)A; a.W = (const uint8_t*)B; a.sx = As; a.sw = Bs; a.bias = nullptr; a.C = C;
   a.partial = (float*)workspace;
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = lda; a.ldw = ldb; a.ldc = ldc;
   a.sx_m = as_stride_m; a.sx_k = as_stride_k; a.sw_n = bs_stride_n; a.sw_k = bs_stride_k;
@@ -476,16 +476,7 @@ extern "C" int fp8k_block_gemm(const void* A, const void* B, const float* As, co
                                int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, int out_dtype, void* workspace,
                                int64_t workspace_bytes_given, void* stream) {
   clear_error();
-  return block_gemm_impl(A, B, As, Bs, nullptr, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
-                         out_dtype, workspace, workspace_bytes_given, stream);
-}
-
-extern "C" int fp8k_block_gemm_bias(const void* A, const void* B, const float* As, const float* Bs, const void* bias, void* C,
-                                    int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t as_stride_m,
-                                    int64_t as_stride_k, int64_t bs_stride_n, int64_t bs_stride_k, int64_t ldc, int out_dtype,
-                                    void* workspace, int64_t workspace_bytes_given, void* stream) {
-  clear_error();
-  return block_gemm_impl(A, B, As, Bs, bias, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
+  return block_gemm_impl(A, B, As, Bs, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
                          out_dtype, workspace, workspace_bytes_given, stream);
 }
 
@@ -546,7 +537,7 @@ extern "C" int fp8k_block_gemm_noalloc(const void* A, const void* B, const float
   }
   // nothing in the buffer has to start at zero: every float partial and every copied scale that a launch reads was
   // written by the same call
-  return block_gemm_impl(A, B, As, Bs, nullptr, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
+  return block_gemm_impl(A, B, As, Bs, C, M, N, K, lda, ldb, as_stride_m, as_stride_k, bs_stride_n, bs_stride_k, ldc,
                          out_dtype, ws, need > 0 ? kStaticScratchBytes : 0, stream);
 }
 
@@ -585,22 +576,13 @@ extern "C" int fp8k_block_gemm_ue8m0(const void* A, const void* B, const int32_t
 extern "C" int fp8k_scaled_mm(const void* A, const void* B, const float* sa, const float* sb, const void* bias, void* C,
                               int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int out_dtype,
                               int bias_dtype, void* workspace, int64_t workspace_bytes_given, void* stream) {
-  return fp8k_scaled_mm_strided(A, B, sa, 1, sb, 1, bias, C, M, N, K, lda, ldb, ldc, out_dtype, bias_dtype, workspace,
-                                workspace_bytes_given, stream);
-}
-
-extern "C" int fp8k_scaled_mm_strided(const void* A, const void* B, const float* sa, int64_t sa_stride, const float* sb,
-                                      int64_t sb_stride, const void* bias, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
-                                      int64_t ldb, int64_t ldc, int out_dtype, int bias_dtype, void* workspace,
-                                      int64_t workspace_bytes_given, void* stream) {
   clear_error();
   int rc = common_checks("fp8_scaled_mm", A, B, C, M, N, K, lda, ldb, ldc, out_dtype);
   if (rc) return rc;
   if (M == 0 || N == 0) return FP8K_OK;
   FP8K_REQUIRE(K > 0, "fp8_scaled_mm: K must be positive");
   FP8K_REQUIRE(sa && sb, "fp8_scaled_mm: null scale pointer");
-  FP8K_REQUIRE((sa_stride == 0 || sa_stride == 1) && (sb_stride == 0 || sb_stride == 1), "fp8_scaled_mm: scale strides must be 0 or 1");
-  FP8K_REQUIRE(sb_stride == 0 || aligned(sb, 16), "fp8_scaled_mm: scales_b must be 16-byte aligned");
+  FP8K_REQUIRE(aligned(sb, 16), "fp8_scaled_mm: scales_b must be 16-byte aligned");
   if (bias)
     FP8K_REQUIRE(bias_dtype == FP8K_F32 || bias_dtype == FP8K_F16 || bias_dtype == FP8K_BF16,
                  "fp8_scaled_mm: bias dtype must be float32, float16 or bfloat16");
@@ -613,7 +595,7 @@ extern "C" int fp8k_scaled_mm_strided(const void* A, const void* B, const float*
   a.X = (const uint8_t*)A; a.W = (const uint8_t*)B; a.sx = sa; a.sw = sb; a.bias = bias; a.C = C;
   a.partial = (float*)workspace;
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = lda; a.ldw = ldb; a.ldc = ldc;
-  a.sx_m = sa_stride; a.sw_n = sb_stride;
+  a.sx_m = a.sw_n = 1;
   hipStream_t st = (hipStream_t)stream;
   const int bd = bias ? bias_dtype : FP8K_F32;
 #define FP8K_SMM(O, B) launch<kModeRow, O, B>(a, pl, st)

@@ -31,6 +31,16 @@ def test_library_exports_every_declared_symbol():
     assert _lib.lib.fp8k_abi_version() == _lib.ABI_VERSION
 
 
+def test_every_entry_point_has_a_caller():
+    """What the package itself does not call is an interface for others that the header says so of, or a query about a plan."""
+    package = os.path.join(ROOT, "sglang_amd")
+    files = [p for ext in ("py", "cpp") for p in glob.glob(os.path.join(package, "**", "*." + ext), recursive=True)]
+    text = "".join(open(p).read().split("def _load", 1)[-1] for p in files)  # of _lib.py what follows its table of symbols
+    product = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "fp8k.h")).read(), flags=re.S)
+    unused = {s for s in re.findall(r"\b(fp8k_[a-z0-9_]+)\s*\(", product) if not re.search(r"\b%s\b" % s, text)}
+    assert unused == {"fp8k_block_gemm_noalloc", "fp8k_linear_fuses_quant"}
+
+
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     import importlib
 
