@@ -57,6 +57,20 @@ def _run(cmd: list[str]) -> None:
         sys.stderr.write(err + "\n")
 
 
+def _host_stale() -> bool:
+    """Whether _host.so has to be built: older than its sources, or built for another torch, whose C++ interface it uses."""
+    import torch
+
+    if _stale(HOST, [os.path.join(HERE, HOST_SRC), os.path.abspath(__file__), os.path.join(HERE, "..", "..", "include", "fp8k.h")]):
+        return True
+    with open(HOST, "rb") as f:
+        return _torch_mark(torch.__version__).encode() not in f.read()
+
+
+def _torch_mark(version: str) -> str:
+    return "built for torch %s;" % version
+
+
 def _host_command() -> list[str]:
     """Host code only: the native side of the layer-level calls, against torch's C++ API."""
     import sysconfig
@@ -67,7 +81,8 @@ def _host_command() -> list[str]:
     inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
            sysconfig.get_paths()["include"]]
     return [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
-            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-Wno-deprecated-declarations"] + [
+            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-Wno-deprecated-declarations",
+            '-DFP8K_TORCH_MARK="%s"' % _torch_mark(torch.__version__)] + [
         "-isystem" + d for d in inc] + [HOST_SRC, "-o", HOST, "-L" + HERE, "-lfp8k", "-L" + os.path.join(root, "lib"),
                                         "-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lc10",
                                         "-Wl,-rpath,$ORIGIN/csrc"]
@@ -92,7 +107,7 @@ def build(force: bool = False, jobs: int = 4, verbose: bool = True) -> str:
         _run([cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
         if verbose:
             print("[fp8k] linked", LIB, flush=True)
-    if force or _stale(HOST, [os.path.join(HERE, HOST_SRC), os.path.abspath(__file__), hdrs[-2]]):
+    if force or _host_stale():
         _run(_host_command())
         if verbose:
             print("[fp8k] linked", HOST, flush=True)

@@ -651,5 +651,8 @@ PyMODINIT_FUNC PyInit__host(void) {
   if (!overrides) return nullptr;
   g_has_torch_function = PyObject_GetAttrString(overrides, "has_torch_function_unary");
   Py_DECREF(overrides);
-  return g_has_torch_function ? PyModule_Create(&module) : nullptr;
+  if (!g_has_torch_function) return nullptr;
+  PyObject* const m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch", FP8K_TORCH_MARK) < 0) return nullptr;
+  return m;
 }

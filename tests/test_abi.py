@@ -41,6 +41,21 @@ def test_every_entry_point_has_a_caller():
     assert unused == {"fp8k_block_gemm_noalloc", "fp8k_linear_fuses_quant"}
 
 
+def test_host_extension_belongs_to_one_torch(monkeypatch):
+    """_host.so uses torch's C++ interface: under another torch it is built again, and refused if it was not."""
+    import torch
+
+    import sglang_amd
+    from sglang_amd.csrc import build
+
+    monkeypatch.setattr(build, "_stale", lambda target, deps: False)
+    assert not build._host_stale()
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    assert build._host_stale()
+    with pytest.raises(ImportError, match="built for torch"):
+        sglang_amd._check_host()
+
+
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     import importlib
 
