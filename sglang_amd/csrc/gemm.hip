@@ -41,9 +41,9 @@ static Plan plan_tile128(int64_t M, int64_t N, int kb, int splits) {
   return pl;
 }
 
-// decode-sized, up to 32 rows: weights go HBM -> registers -> matrix core.  K is cut so that about 512 workgroups
-// (two per CU, one round) stream at once, at least 8 K blocks each, while the float partials stay a small fraction
-// of the weight bytes
+// decode-sized, up to 32 rows: weights go HBM -> registers -> matrix core.  K is cut into about 512 workgroups (two per CU, one
+// round, up to 16 rows; above, the LDS of the activations leaves one per CU and they run in two) of at least 8 K blocks each, while
+// the float partials stay a small fraction of the weight bytes
 static Plan plan_direct(int64_t M, int64_t N, int64_t K) {
   Plan pl{3, 1, 0, 0, 0, 0};
   const int kb = (int)(K / kTileK);

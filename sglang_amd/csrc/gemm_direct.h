@@ -19,7 +19,7 @@
 // of the block from LDS, which is why blocks of 64 and 128 rows measured slower here than through
 // gemm_stream_kernel.)
 //
-// The grouped GEMM keeps four K blocks in flight instead of eight: 112 registers and 50 KB of LDS let two workgroups
+// The grouped GEMM keeps four K blocks in flight instead of eight: at most 109 registers and 50 KB of LDS let two workgroups
 // share a CU (eight took 174 registers: one), so the start and the write-out of one block hide behind the stream of
 // another, and a short K (an expert's intermediate size) pads to less.  Bytes in flight per CU stay the same.  Measured
 // on the whole layer with 32-row blocks: 128 experts x 4096 x 256 at 384 slots 1.05x, x 1024 1.05x, 64 x 7168 x 1024

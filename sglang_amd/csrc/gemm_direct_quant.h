@@ -8,9 +8,10 @@
 // The price is the quantisation once per workgroup, about 6 vector instructions per element: kQuantFuseMax says up to which
 // M * K it stays under the launch it replaces.
 //
-// Whole linear, bf16, before -> now: M = 1: 4608 x 7168 13.5 -> 8.7 us (33 MB: 5.3 us at the read ceiling), 6144 x 4096 10.9 ->
-// 7.4, 7168 x 18432 28.9 -> 22.1, 1024 x 1024 9.7 -> 5.2 (the host's time for one launch); M = 8, at the limit of M * K:
-// 6144 x 4096 11.7 -> 8.8, per-token 11.1 -> 9.1.
+// Whole linear, bf16, two launches -> this one, one weight: M = 1: 4608 x 7168 13.5 -> 8.7 us (33 MB: 5.3 us at the read ceiling),
+// 6144 x 4096 10.9 -> 7.4, 7168 x 18432 28.9 -> 22.1, 1024 x 1024 9.7 -> 5.2 (the host's time for one launch); M = 8, at the limit
+// of M * K: 6144 x 4096 11.7 -> 8.8, per-token 11.1 -> 9.1.  With the weights rotated over 600 MB, so that none comes out of the
+// memory-side cache: 9.4, 8.2, 22.4, 5.3; 9.6, 9.9.
 //
 // Split of the work, K order, LDS re-layout of the weights and summation are gemm_wavek_kernel's, and the quantisation is
 // that of group_quant_kernel (block mode) or token_quant_kernel (row mode), so results are those of the two launches bit for

@@ -10,12 +10,16 @@
 // Finished rows are stored without a barrier; the waves meet only where the block changes.  Two workgroups share a CU, so one
 // streams while the other changes blocks; that takes LDS for two, which K = 2048 with 32 slots (84 KB) does not leave.
 //
-// Whole layer, before -> now: 128 experts, H = 4096, top 6, 128 tokens, I = 256 176 -> 113 us, I = 512 224 -> 191; 256 experts,
-// H = 7168, I = 512, 865 tokens 739 -> 578 (its second GEMM, 940 MB of weights, 372 -> 211 us).
+// GEMM alone, a workgroup per tile with eight K blocks in flight / with four and two workgroups per CU / here: 128 experts, 4096
+// rows, 128 tokens of top 6, K = 256 91 / 47 / 28 us, 16 slots 58 / 38 / 26; 256 experts, 7168 rows, 865 tokens of top 6, K = 512
+// (940 MB) 367 / 228 / 224.  Up to which K it is ahead of the second: moe.hip.
 //
 // ACT: the rows come as the 16-bit output [slots, 2 K] of the first GEMM, and a workgroup forms silu_and_mul and the group
 // quantisation of its block's rows when it puts them into LDS - bit for bit the bytes and scales of the kernel that does it
-// between the two GEMMs (4.7 us and a launch).  A block is staged by the few workgroups whose runs it spans, padding rows cost nothing.
+// between the two GEMMs (4.1 - 4.8 us at up to 128 tokens, and a launch).  Whole layers without / with it: 64 experts, H = 2048,
+// I = 256 .. 768 1.03 .. 1.11 times, 128 experts, H = 4096, and 256, H = 7168, up to I = 512 1.01 .. 1.08 (128 experts, I = 256,
+// 140 tokens 96 -> 92 us); at I = 1024 64 experts still gain 1 - 6 %, the others lose up to 7 % beyond a few tokens (288 -> 268
+// without).  A block is staged by the few workgroups whose runs it spans, padding rows cost nothing.
 //
 // Operand layouts, the LDS round trip of the weights and the order of the K sums are gemm_direct_kernel's.
 #pragma once

@@ -18,8 +18,8 @@
 // an operand fetch over all banks.  At the end the KS partial sums meet in LDS in ascending order, as in gemm_wavek_kernel.
 //
 // GEMM alone, bf16, against what ran before (K cut across workgroups with partials, or across the waves of one whose lanes fetched
-// their own activations): 32 x 4096 x 4096 10.7 -> 7.4 us, 24 x 7168 x 16384 30.6 -> 24.6 (117 MB: 4.8 TB/s), 64 x 4096 x 4096
-// 14.4 -> 9.3, 13 x 12224 x 3968 18.9 -> 11.0, 128 x 4096 x 4096 16.4 -> 14.3.
+// their own activations), weights rotated over 600 MB: 32 x 4096 x 4096 10.6 -> 7.6 us, 24 x 7168 x 16384 32.4 -> 26.7 (117 MB: 4.4
+// TB/s), 64 x 4096 x 4096 15.2 -> 10.3, 13 x 12224 x 3968 19.4 -> 11.8, 128 x 4096 x 4096 17.9 -> 15.6, 96 x 8192 x 4096 22.6 -> 16.1.
 #pragma once
 
 #include "gemm_direct.h"

@@ -1080,10 +1080,9 @@ __global__ __launch_bounds__(256) void moe_fused_gate_kernel(const void* __restr
 
 // The same with a whole wavefront per token: lane l holds the EPL = experts / 64 experts from l * EPL on (64 / groups lanes per
 // expert group).  The routing is a serial chain - sigmoid, group weights, then one arg-max after the other - and the form above
-// walks a group's VPT values inside one lane at every link of it: 13.8 us for one token of 256 experts, 3.8 here (4096 tokens 14.9,
-// 6.8 here; 512 experts, top 16 25.2 -> 6.5).  Here a link is a
-// reduction over the lanes (six DPP steps, a ballot that finds the lowest lane of the maximum) around at most EPL values, and
-// the groups that stay are found by rank instead of by dropping one after the other.
+// walks a group's VPT values inside one lane at every link of it: 13.6 us for one token of 256 experts in eight groups, 4.1 here
+// (4096 tokens 14.6, 7.1 here; 512 experts in 16 groups, top 16 27.6, 6.9 here for one token).  Here a link is a reduction over
+// the lanes (six DPP steps, a ballot that finds the lowest lane of the maximum) around at most EPL values.
 __device__ __forceinline__ float wave_max(float v) {  // of all 64 lanes, in every lane
   v = fmaxf(v, dpp_f<kDppXor1>(v));
   v = fmaxf(v, dpp_f<kDppXor2>(v));
@@ -1212,8 +1211,10 @@ extern "C" int fp8k_moe_fused_gate(const void* input, const void* bias, float* t
   FP8K_REQUIRE(aligned(input, 16) && aligned(bias, 16), "%s: input and bias must be 16-byte aligned", op);
   hipStream_t st = (hipStream_t)stream;
   // A wavefront per token where the experts fill its lanes and every pick has a lane of its own: latency is what a routing of up
-  // to some thousand tokens costs.  Above that the lanes count, of which the other form takes an eighth: it is 10 - 20 % ahead
-  // at 16384 tokens of 64 or 128 experts in eight groups, but not with 32 experts per group (18.6 against 19.7 us) or many groups.
+  // to some thousand tokens costs.  Above that the lanes count, of which the other form takes an eighth: eight groups of 64 / 128 experts
+  // take 7.3 / 9.0 us here against 7.3 / 10.4 at 8192 tokens and 11.8 / 15.3 against 8.3 / 12.9 at 16384.  With 32 experts per group or
+  // more than 16 groups this form is ahead or level up to 16384 (256 experts, 8 / 32 groups: 19.0 / 22.8 against 19.3 / 26.0) and at
+  // 32768 10 % behind (34.9 against 31.5) / 6 % ahead.
   if (num_experts >= 64 && num_experts <= 512 && topk <= 64 && (num_rows <= 8192 || vpt > 16 || num_expert_group > 16)) {
     const dim3 grid((unsigned)((num_rows + 3) / 4)), block(256);
 #define FP8K_GATEW2(DT, V)                                                                                                  \
