@@ -418,17 +418,24 @@ int32_t* stream_sync(const Tensor& like, const c10::hip::HIPStream& stream) {
   const hipStream_t st = stream.stream();
   if (st && (uint64_t)stream.id() == (uint64_t)(uintptr_t)st) return nullptr;
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return nullptr;
+  if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
+    (void)hipGetLastError();  // the launches report what is wrong with the stream, not this question
+    return nullptr;
+  }
+  if (capturing != hipStreamCaptureStatusNone) return nullptr;
   static std::mutex mutex;
   static auto* const words = new std::map<std::pair<int, hipStream_t>, Tensor>;  // lives as long as the process
-  std::lock_guard<std::mutex> lock(mutex);
   const auto key = std::make_pair((int)like.get_device(), st);
-  auto it = words->find(key);
-  if (it == words->end()) {
+  {
+    std::lock_guard<std::mutex> lock(mutex);
+    const auto it = words->find(key);
+    if (it != words->end()) return it->second.data_ptr<int32_t>();
     if (words->size() >= kMaxSync) return nullptr;
-    it = words->emplace(key, at::zeros({3}, like.options().dtype(ScalarType::Int))).first;  // on the current stream, which is st
   }
-  return it->second.data_ptr<int32_t>();
+  // outside the lock, as it may wait for the device; of two threads on one stream the first to come back decides
+  Tensor fresh = at::zeros({3}, like.options().dtype(ScalarType::Int));  // on the current stream, which is st
+  std::lock_guard<std::mutex> lock(mutex);
+  return words->emplace(key, std::move(fresh)).first->second.data_ptr<int32_t>();
 }
 
 // mla_quant(x, x_s, eps) -> x_q or None
