@@ -384,3 +384,32 @@ def test_profiler_sees_the_calls(dev):
     for name, args in calls.items():
         shapes = [list(a.shape) for a in args if isinstance(a, torch.Tensor) and a.dim()]
         assert [s for s in records["fp8k::" + name].input_shapes if s] == shapes, name
+
+
+@pytest.mark.gpu
+def test_threads_that_share_a_stream_share_its_workspace(dev):
+    """Products with K cut through float partials, of two threads on one stream at once: the launches of one do not come between
+    those of the other."""
+    from sglang_amd._lib import lib
+
+    m, n, k = 128, 1024, 8192
+    assert lib.fp8k_block_gemm_workspace_bytes(m, n, k) > m * n * 8  # partials of two and more K ranges
+    w, s = _weight(n, k)
+    jobs = [fp8_kernel.sglang_per_token_group_quant_fp8(_randn((m, k), seed=seed), 128, column_major_scales=True) for seed in (1, 2)]
+    want = [fp8_kernel.w8a8_block_fp8_matmul(q, w, xs, s, BLOCK, torch.bfloat16) for q, xs in jobs]
+    torch.cuda.synchronize()
+    got, start = [None, None], threading.Barrier(2)
+
+    def work(i):
+        q, xs = jobs[i]
+        start.wait()
+        got[i] = [_host.block_matmul(q, w, xs, s, BLOCK, torch.bfloat16, False) for _ in range(500)]
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(out, want[i]) for out in got[i])
