@@ -34,22 +34,12 @@ constexpr int kDirTileN = 128;                   // 8 waves x 16 weight rows
 constexpr int kDirDepth = 8;                     // of a linear: weight prefetch depth in K blocks = K blocks per activation chunk
 constexpr uint32_t kOutOfRange = 0xF0000000u;    // buffer offset past every descriptor range: reads zero
 
-__device__ __forceinline__ v4f mfma_16x16x128(v8i a, v8i b, v4f c) {
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
-}
 __device__ __forceinline__ v4i buf_load16(rsrc_t r, uint32_t voff) {
   return __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0);
 }
 __device__ __forceinline__ v4i buf_load16_stream(rsrc_t r, uint32_t voff) {  // non-temporal: used once
   return __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 2);
 }
-__device__ __forceinline__ v8i join(v4i lo, v4i hi) {
-  v8i r;
-  r[0] = lo[0]; r[1] = lo[1]; r[2] = lo[2]; r[3] = lo[3];
-  r[4] = hi[0]; r[5] = hi[1]; r[6] = hi[2]; r[7] = hi[3];
-  return r;
-}
-
 template <int TM, int MODE, int OUT_DT, int BIAS_DT, bool SPLIT, bool MOE>
 __global__ __launch_bounds__(512, MOE ? 4 : 2) void gemm_direct_kernel(const GemmArgs p) {
   static_assert(TM == 16 || TM == 32, "gemm_direct_kernel: 16 or 32 rows per block (more rows are LDS-read bound here)");

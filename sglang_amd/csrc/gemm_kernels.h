@@ -8,6 +8,7 @@
 #pragma once
 
 #include <type_traits>
+#include <utility>
 
 #include "fp8k_common.h"
 
@@ -72,6 +73,41 @@ __device__ __forceinline__ v16f mfma_32x32x64(v8i a, v8i b, v16f c) {
 // elements that this lane holds of its A row / B column
 __device__ __forceinline__ v16f mfma_32x32x64_scaled(v8i a, v8i b, v16f c, int scale_a, int scale_b) {
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, scale_a, 0, scale_b);
+}
+
+// 16 x 16 x 128: a whole K block of the scales per instruction.  A lane holds 32 K bytes of one row of each operand (lane & 15);
+// which ones is free as long as both operands agree.  Result: column lane & 15 (activation row), rows (lane >> 4) * 4 + i.
+__device__ __forceinline__ v4f mfma_16x16x128(v8i a, v8i b, v4f c) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+}
+__device__ __forceinline__ v4f mfma_16x16x128_scaled(v8i a, v8i b, v4f c, int scale_a, int scale_b) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, scale_a, 0, scale_b);
+}
+__device__ __forceinline__ v8i join(v4i lo, v4i hi) {
+  v8i r;
+  r[0] = lo[0]; r[1] = lo[1]; r[2] = lo[2]; r[3] = lo[3];
+  r[4] = hi[0]; r[5] = hi[1]; r[6] = hi[2]; r[7] = hi[3];
+  return r;
+}
+// lane L of the 16 lanes of a row, in all of them
+template <int L>
+__device__ __forceinline__ float row_broadcast(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + L, 0xf, 0xf, true));
+}
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+// lane l holds the value of row l: out[g] holds, in every lane, that of row 16 g + (l & 15)
+__device__ __forceinline__ void spread_rows(uint32_t v, uint32_t (&out)[4]) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(v, v, false, false);  // rows 0 .. 31 twice, rows 32 .. 63 twice
+  const auto lo = __builtin_amdgcn_permlane16_swap(halves[0], halves[0], false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(halves[1], halves[1], false, false);
+  out[0] = lo[0]; out[1] = lo[1]; out[2] = hi[0]; out[3] = hi[1];
 }
 
 template <int OUT_DT>
@@ -196,7 +232,12 @@ __device__ __forceinline__ void load_bias8(const void* bias, int64_t n, float (&
 
 // ------------------------------------------------------------------------------------------------
 // 256(n) x 256(m) x 128(k) workgroup tile, 8 wavefronts (2 along n x 4 along m), wave tile
-// 128(n) x 64(m) = 4 x 2 MFMA tiles of 32x32, K step 128 = two v_mfma_f32_32x32x64_f8f6f4.
+// 128(n) x 64(m) = 8 x 4 MFMA tiles of 16x16, K step 128 = one v_mfma_f32_16x16x128_f8f6f4.
+//
+// Bound: the matrix cores under the chip's power limit.  A bare loop of MFMAs on quantised normal data reaches 4.56 PFLOP/s in
+// the 16x16x128 form and 4.19 in the 32x32x64 form (4.94 both on zeros), with the same rounding error of a K block; the kernel
+// with 32x32x64 tiles took 447 us at 4096 x 18432 x 7168 (block scales) where this one takes 426, 377 against 361 at 8192^3
+// (row scales), 200 against 193 at 2000 x 7168 x 18432 (UE8M0), 106 against 104 at 4096 x 32768 x 512.
 //
 // LDS: three weight stages and two activation stages of 256 rows x 128 B each = 160 KB, filled by
 // buffer_load_dwordx4 ... lds (no register staging; rows past the matrix edge are out of the
@@ -212,16 +253,15 @@ __device__ __forceinline__ void load_bias8(const void* bias, int64_t n, float (&
 // last four MFMAs of block it still run.  A wave's loads retire in order and are issued as
 // activations, scales, weights: the wait in front of the barrier leaves its four weight loads in
 // flight, so the weights - whose lines come from HBM or the memory-side cache, where the
-// activations mostly hit the L2 - have two barrier intervals to arrive.  Operand
-// fetches are issued two MFMA groups ahead of their use; the eight 1 KB global loads of a wave are
-// spread over the first half of the interval, two per group, because the texture-address path
-// moves 64 B/clk per CU and a burst would stall the issuing wave.  The loop body is branch-free
-// (loads past the last K block are out of range or unread), which keeps the compiler from sinking
-// the scale FMAs to the loop latch.
+// activations mostly hit the L2 - have two barrier intervals to arrive.  The eight 1 KB global loads
+// of a wave are spread over the first half of the interval, one behind an MFMA, because the
+// texture-address path moves 64 B/clk per CU and a burst would stall the issuing wave.  The loop body
+// is branch-free (loads past the last K block are out of range or unread), which keeps the compiler
+// from sinking the scale FMAs to the loop latch.
 //
-// Block mode keeps two short-lived accumulators: t = W.X over one K block, then
-// acc += t * (as[m,kb] * bs[nb,kb]), with the 16 FMAs of group g-1 split around the two MFMAs of
-// group g; row mode accumulates in place and scales in the epilogue.
+// Block mode: t = W.X over one K block into one of four short-lived accumulators, then
+// acc += t * (as[m,kb] * bs[nb,kb]), the four FMAs of an MFMA four MFMAs later; row mode accumulates
+// in place and scales in the epilogue.  Up to 251 registers, nothing spilled.
 // ------------------------------------------------------------------------------------------------
 constexpr int kTileN = 256, kTileM = 256, kTileK = 128;
 
@@ -346,23 +386,12 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
     }
     const uint32_t soW = (uint32_t)(w * 32 * p.ldw), soX = (uint32_t)(w * 32 * p.ldx);
     const uint32_t stepW = (uint32_t)(8 * p.ldw), stepX = (uint32_t)(8 * p.ldx);
-    const int lr = ln & 31, h = ln >> 5;
-    const int swz = (lr >> 1) & 7;
-    // lane part of an operand fetch address: row lr of a 32-row group, 16-byte chunk (ks, j) at its swizzled place.
-    // Stage, wave position and group are uniform and reach the address through scalar registers, so weights and
-    // activations share these four registers.
-    uint32_t fa[2][2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) fa[ks][j] = (uint32_t)(lr * kTileK + (((ks * 4 + h * 2 + j) ^ swz) << 4));
-    auto frag = [&](const uint8_t* grp, int ks) -> v8i {  // grp: first row of the 32-row group inside its stage (uniform)
-      const v4i lo = *reinterpret_cast<const v4i*>(grp + fa[ks][0]);
-      const v4i hi = *reinterpret_cast<const v4i*>(grp + fa[ks][1]);
-      v8i r;
-      r[0] = lo[0]; r[1] = lo[1]; r[2] = lo[2]; r[3] = lo[3];
-      r[4] = hi[0]; r[5] = hi[1]; r[6] = hi[2]; r[7] = hi[3];
-      return r;
+    const int lr = ln & 15, kq = ln >> 4;
+    // lane part of an operand fetch address: row lr of a 16-row group, 16-byte chunks kq and kq + 4 at their swizzled places.
+    // Stage, wave position and group are uniform, so weights and activations share these two registers.
+    const uint32_t fa0 = (uint32_t)(lr * kTileK + ((kq ^ ((lr >> 1) & 7)) << 4)), fa1 = fa0 ^ 64u;
+    auto frag = [&](const uint8_t* grp) -> v8i {  // grp: first row of the 16-row group inside its stage (uniform)
+      return join(*reinterpret_cast<const v4i*>(grp + fa0), *reinterpret_cast<const v4i*>(grp + fa1));
     };
 
     // ---- global -> LDS through buffer loads: descriptor at the tile's first row, rows past the matrix edge are out
@@ -392,7 +421,6 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
     const int kb_end = is_split ? min(p.K / kTileK, kb_begin + p.kb_per_split) : p.K / kTileK;
     const int nkb = kb_end - kb_begin;
 
-    auto slot_at = [&](int i) -> int { return m0 + i; };
     tile_rsrcs(rW, rX, t, half, is_half, kb_begin, kb_end);
     // the item after this one: with three and more K blocks here its first blocks are requested by this item's last trips
     Item next;
@@ -422,66 +450,80 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
     auto wst = [&](int b) -> int { return (gw0 + b) % 3; };
     auto xst = [&](int b) -> int { return (gx0 + b) & 1; };
 
-    // ---- scales (block mode)
-    // activation rows whose scales this lane applies (any valid row for padding lanes)
-    const int mrow0 = min(m0 + wm * 64 + lr, p.M - 1);
-    const int mrow1 = min(m0 + wm * 64 + 32 + lr, p.M - 1);
-    // element offsets of this lane's two scale rows (32 bits: the host checks M * K/128 against 2^31)
-    const uint32_t sxo0 = (uint32_t)((int64_t)mrow0 * p.sx_m + (int64_t)kb_begin * p.sx_k);
-    const uint32_t sxo1 = (uint32_t)((int64_t)mrow1 * p.sx_m + (int64_t)kb_begin * p.sx_k);
+    // ---- scales: lane l fetches that of activation row l of the wave's 64 (a valid row for padding lanes) and hands it to the
+    // lanes that apply it (spread_rows).  Element offset in 32 bits: the host checks M * K/128 against 2^31.
+    const uint32_t sxo = (uint32_t)((int64_t)min(m0 + wm * 64 + ln, p.M - 1) * p.sx_m);
     const uint32_t sxk = (uint32_t)p.sx_k;
     const int nb = min(n0 + wn * 128, p.N - 1) >> 7;
     const float* swp = p.sw + (int64_t)nb * p.sw_n + (int64_t)kb_begin * p.sw_k;
-    // scaled mode: sx points at int32 words of four UE8M0 bytes (K blocks 4j..4j+3 of a row), sx_k = word stride
-    const uint32_t* sqp = reinterpret_cast<const uint32_t*>(p.sx);
-    const uint32_t sqo0 = (uint32_t)((int64_t)mrow0 * p.sx_m), sqo1 = (uint32_t)((int64_t)mrow1 * p.sx_m);
-    int sq[2] = {127, 127}, sqw = 127;      // exponent bytes of the block the current MFMAs belong to
-    uint32_t q0n = 0, q1n = 0;              // words holding the next block's activation exponents
-
-    v16f acc[4][2];
+    // block mode: floats; scaled mode: int32 words of four UE8M0 bytes (K blocks 4j..4j+3 of a row), sx_k = word stride
+    uint32_t sxr = 0;
+    float swr = 0.f;
+    auto request_scales = [&](int b) {
+      if (MODE == kModeRow) return;
+      const int kn = min(b, nkb - 1);
+      const uint32_t k = (uint32_t)(MODE == kModeScaled ? (kb_begin + kn) >> 2 : kb_begin + kn);
+      sxr = reinterpret_cast<const uint32_t*>(p.sx)[sxo + k * sxk];
+      swr = swp[(int64_t)kn * p.sw_k];
+    };
+    // block mode: scn[g] = as * bs of row 16 g + lr; scaled mode: the exponents (byte 0 of each word) for the matrix core
+    uint32_t sc[4] = {127, 127, 127, 127}, scn[4] = {127, 127, 127, 127};
+    int sqw = 127, sqwn = 127;
+    auto take_scales = [&](int b) {  // the requested scales, which are block b's, into scn / sqwn
+      if (MODE == kModeRow) return;
+      if (MODE == kModeBlock) spread_rows(__float_as_uint(__uint_as_float(sxr) * swr), scn);
+      else spread_rows(sxr >> (((kb_begin + b) & 3) * 8), scn);
+      sqwn = (int)(__float_as_uint(swr) >> 23);
+      // formed here, in front of the next request: moved behind it, the copy of its registers would wait for it
+      asm volatile("" : "+v"(scn[0]), "+v"(scn[1]), "+v"(scn[2]), "+v"(scn[3]));
+      if (MODE == kModeScaled) asm volatile("" : "+v"(sqwn));
+    };
+    auto use_scales = [&] {
+      if (MODE == kModeRow) return;
 #pragma unroll
-    for (int ns = 0; ns < 4; ++ns)
-#pragma unroll
-      for (int ms = 0; ms < 2; ++ms)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[ns][ms][r] = 0.f;
+      for (int g = 0; g < 4; ++g) sc[g] = scn[g];
+      sqw = sqwn;
+    };
 
-    // Operand registers: X[ms][ks] the four activation fragments of a K block, W[ks] the two fragments of ONE weight
-    // group.  A K block is walked as four steps, one per weight group ns, each step the MFMAs (ms, ks) = (0,0) (1,0)
-    // (0,1) (1,1): W[0] is free after the second and W[1] after the fourth, and each is refilled in place with the
-    // next group's fragment two MFMAs before its first use.  (A second set of weight registers would push the block
-    // mode past 256 registers, and scratch reloads inside the K loop cannot coexist with its partial vmcnt waits.)
-    v8i X[2][2], W[2];
-    v16f tq[2];
-    float sc[2] = {0.f, 0.f}, scn[2] = {0.f, 0.f};
-    float s0n = 0.f, s1n = 0.f, sbn = 0.f;
+    v4f acc[8][4];
+#pragma unroll
+    for (int ns = 0; ns < 8; ++ns)
+#pragma unroll
+      for (int ms = 0; ms < 4; ++ms) acc[ns][ms] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    auto RW = [&](int ks, const uint8_t* st, int ns) { W[ks] = frag(st + (wn * 128 + ns * 32) * kTileK, ks); };
-    auto RX = [&](int ms, int ks, const uint8_t* st) { X[ms][ks] = frag(st + (wm * 64 + ms * 32) * kTileK, ks); };
-    // one MFMA of step ns.  Block mode: the products of a step gather in tq[ms] (K half 0 starts from zero, K half 1
-    // adds), to be folded into acc[ns][ms] with the block's scale during the next step; the other modes accumulate
-    // in place.
-    auto M = [&](int ms, int ks, int ns) {
+    // Operand registers: X[ms] the four activation fragments of a K block, W[ns & 3] the weight fragments of two pairs of 16-row
+    // groups.  A K block is walked as four pairs, each of eight MFMAs: the four activation groups against the pair's first weight
+    // group, then against its second (four MFMAs in a row that share an operand: against two the order costs 0.5 - 1 %).  The
+    // weights of a pair are fetched during the pair before; X[ms] is refilled behind its last MFMA of a block.
+    v8i X[4], W[4];
+    v4f tq[4];
+    auto RW = [&](const uint8_t* st, int ns) { W[ns & 3] = frag(st + (wn * 128 + ns * 16) * kTileK); };
+    auto RX = [&](const uint8_t* st, int ms) { X[ms] = frag(st + (wm * 64 + ms * 16) * kTileK); };
+    // MFMA k of a K block: weight group k / 4, activation group k % 4.  Block mode: the product waits in tq[k % 4] and is folded into
+    // its accumulator with the block's scale in front of MFMA k + 4; the other modes accumulate in place.
+    auto F = [&](int k) {
       if (MODE == kModeBlock) {
-        if (ks == 0) {
-          v16f z;
+        const int ns = k >> 2, ms = k & 3;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) z[r] = 0.f;
-          tq[ms] = mfma_32x32x64(W[0], X[ms][0], z);
-        } else {
-          tq[ms] = mfma_32x32x64(W[1], X[ms][1], tq[ms]);
-        }
-      } else if (MODE == kModeScaled) {
-        acc[ns][ms] = mfma_32x32x64_scaled(W[ks], X[ms][ks], acc[ns][ms], sqw, sq[ms]);
-      } else {
-        acc[ns][ms] = mfma_32x32x64(W[ks], X[ms][ks], acc[ns][ms]);
+        for (int i = 0; i < 4; ++i) acc[ns][ms][i] = __builtin_fmaf(tq[ms][i], __uint_as_float(sc[ms]), acc[ns][ms][i]);
       }
     };
-    // the 16 scale-FMAs that fold a finished product into its accumulator (block mode only)
-    auto F = [&](v16f& a, const v16f& tt, float sv) {
-      if (MODE == kModeBlock) {
+    auto M = [&](int k) {
+      const int ns = k >> 2, ms = k & 3;
+      if (MODE == kModeBlock) tq[ms] = mfma_16x16x128(W[ns & 3], X[ms], v4f{0.f, 0.f, 0.f, 0.f});
+      else if (MODE == kModeScaled) acc[ns][ms] = mfma_16x16x128_scaled(W[ns & 3], X[ms], acc[ns][ms], sqw, (int)sc[ms]);
+      else acc[ns][ms] = mfma_16x16x128(W[ns & 3], X[ms], acc[ns][ms]);
+    };
+    // one pair; `pending`: the last four MFMAs of the pair before have yet to be folded.  between(i) comes behind MFMA i of the pair
+    auto pair = [&](int pr, bool pending, auto&& between) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) a[r] = __builtin_fmaf(tt[r], sv, a[r]);
+      for (int i = 0; i < 8; ++i) {
+        if (pending || i >= 4) F((pr * 8 + i + 28) & 31);
+        SB();
+        M(pr * 8 + i);
+        SB();
+        between(i);
+        SB();
       }
     };
 
@@ -526,63 +568,37 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
 #pragma unroll
       for (int j = 0; j < 4; ++j) LW(j, 1, wst(1));
     }
-    if (MODE == kModeBlock) { sc[0] = p.sx[sxo0]; sc[1] = p.sx[sxo1]; const float sb = swp[0]; sc[0] *= sb; sc[1] *= sb; }
-    auto exponents = [&](uint32_t w0, uint32_t w1, float sb, int kb_abs) {  // -> sq, sqw for K block kb_abs
-      const int sh = (kb_abs & 3) * 8;
-      sq[0] = (int)(w0 >> sh);
-      sq[1] = (int)(w1 >> sh);
-      sqw = (int)(__float_as_uint(sb) >> 23);
-    };
-    if (MODE == kModeScaled) exponents(sqp[sqo0 + (uint32_t)(kb_begin >> 2) * sxk], sqp[sqo1 + (uint32_t)(kb_begin >> 2) * sxk], swp[0], kb_begin);
+    request_scales(0);
     wait_vm0();
     __syncthreads();
-    // scales of block 1, then activations of block 1, weights of blocks 1 and 2: the order the loop keeps, so that at
+    take_scales(0);
+    use_scales();
+    // activations of block 1, scales of block 1, weights of block 2: the order the loop keeps, so that at
     // a barrier only a wave's four youngest loads - weights for the block after next - may still be in flight
-    if (MODE == kModeBlock) { const int kn = min(1, nkb - 1); s0n = p.sx[sxo0 + (uint32_t)kn * sxk]; s1n = p.sx[sxo1 + (uint32_t)kn * sxk]; sbn = swp[(int64_t)kn * p.sw_k]; }
-    if (MODE == kModeScaled) {
-      const int kn = min(1, nkb - 1);
-      q0n = sqp[sqo0 + (uint32_t)((kb_begin + kn) >> 2) * sxk]; q1n = sqp[sqo1 + (uint32_t)((kb_begin + kn) >> 2) * sxk]; sbn = swp[(int64_t)kn * p.sw_k];
-    }
-    SB();
 #pragma unroll
     for (int j = 0; j < 4; ++j) LX(j, 1, xst(1));
+    request_scales(1);
+    SB();
 #pragma unroll
     for (int j = 0; j < 4; ++j) LW(j, 2, wst(2));
-    const uint8_t* const stW0 = smem + wst(0) * kWStage;
-    const uint8_t* const stX0 = smem + kXBase + xst(0) * kXStage;
-    RX(0, 0, stX0); RX(1, 0, stX0); RW(0, stW0, 0);
-    RX(0, 1, stX0); RX(1, 1, stX0); RW(1, stW0, 0);
-    SB();
-    // steps 0..2 of block 0
-    M(0, 0, 0); SB();
-    M(1, 0, 0); SB();
-    RW(0, stW0, 1); SB();
-    M(0, 1, 0); SB();
-    M(1, 1, 0); SB();
-    RW(1, stW0, 1); SB();
-    F(acc[0][0], tq[0], sc[0]); SB();
-    M(0, 0, 1); SB();
-    F(acc[0][1], tq[1], sc[1]); SB();
-    M(1, 0, 1); SB();
-    RW(0, stW0, 2); SB();
-    M(0, 1, 1); SB();
-    M(1, 1, 1); SB();
-    RW(1, stW0, 2); SB();
-    F(acc[1][0], tq[0], sc[0]); SB();
-    M(0, 0, 2); SB();
-    F(acc[1][1], tq[1], sc[1]); SB();
-    M(1, 0, 2); SB();
-    RW(0, stW0, 3); SB();
-    M(0, 1, 2); SB();
-    M(1, 1, 2); SB();
-    RW(1, stW0, 3); SB();
-    // pending: F(acc[2][0], tq[0], sc[0]), F(acc[2][1], tq[1], sc[1])
+    {
+      const uint8_t* const stW = smem + wst(0) * kWStage;
+      const uint8_t* const stX = smem + kXBase + xst(0) * kXStage;
+      RW(stW, 0); RW(stW, 1); RX(stX, 0); RX(stX, 1); RX(stX, 2); RX(stX, 3);
+      SB();
+#pragma unroll
+      for (int pr = 0; pr < 3; ++pr)
+        pair(pr, pr > 0, [&](int i) {
+          if (i == 1) RW(stW, 2 * pr + 2);
+          if (i == 3) RW(stW, 2 * pr + 3);
+        });
+    }
 
     int w_ld = wst(0), w_rd = wst(1);  // weight stages: the one block it left (refilled with block it+3), the one of block it+1
     for (int it = 0; it < nkb - 1; ++it) {
-      const uint8_t* stW = smem + w_rd * kWStage;                     // block it+1
-      const uint8_t* stX = smem + kXBase + xst(it + 1) * kXStage;
-      const int xl = xst(it);                                         // activation stage block it left
+      const uint8_t* const stW = smem + w_rd * kWStage;                     // block it+1
+      const uint8_t* const stX = smem + kXBase + xst(it + 1) * kXStage;
+      const int xl = xst(it);                                               // activation stage block it left
       lds_barrier<4>();  // block it+1 has landed; the weights of block it+2 may still be on their way
       SB();
       // Two waves share a SIMD's matrix pipe.  Left to the arbiter, one of them is served first whenever both are ready,
@@ -590,72 +606,43 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
       // alone cannot keep the pipe busy (its products wait for their own scale FMAs).  The issue priority therefore falls
       // with a wave's progress through the trip: whoever is behind goes first, and the two stay interleaved.
       __builtin_amdgcn_s_setprio(3);
-      // ---- step 3 of block it; every operand register is refilled from block it+1 after its last use
-      F(acc[2][0], tq[0], sc[0]); SB();
-      M(0, 0, 3); SB();
-      RX(0, 0, stX); LX(0, it + 2, xl); LX(1, it + 2, xl); SB();
-      F(acc[2][1], tq[1], sc[1]); SB();
-      M(1, 0, 3); SB();
-      RX(1, 0, stX); RW(0, stW, 0); LX(2, it + 2, xl); LX(3, it + 2, xl); SB();
-      M(0, 1, 3); SB();
-      RX(0, 1, stX); SB();
-      M(1, 1, 3); SB();
-      RX(1, 1, stX); RW(1, stW, 0); SB();
+      // ---- last pair of block it; every operand register is refilled from block it+1 after its last use
+      pair(3, true, [&](int i) {
+        if (i == 0) RW(stW, 0);
+        if (i == 2) RW(stW, 1);
+        if (i >= 4) RX(stX, i - 4);
+        if (i < 4) LX(i, it + 2, xl);
+      });
       __builtin_amdgcn_s_setprio(2);
-      if (MODE == kModeBlock) { scn[0] = s0n * sbn; scn[1] = s1n * sbn; }
-      // ---- step 0 of block it+1; the pending products still belong to block it
-      F(acc[3][0], tq[0], sc[0]); SB();
-      if (MODE == kModeScaled) exponents(q0n, q1n, sbn, kb_begin + it + 1);  // the MFMAs from here on are block it+1's
-      M(0, 0, 0); SB();
-      F(acc[3][1], tq[1], sc[1]); SB();
-      M(1, 0, 0); SB();
-      // the scales of block it+2 are requested after the activation loads and before the weight loads: the wait in
-      // front of their use then leaves exactly the weight loads in flight
-      if (MODE == kModeBlock) {
-        sc[0] = scn[0]; sc[1] = scn[1];
-        const int kn = min(it + 2, nkb - 1);
-        s0n = p.sx[sxo0 + (uint32_t)kn * sxk]; s1n = p.sx[sxo1 + (uint32_t)kn * sxk]; sbn = swp[(int64_t)kn * p.sw_k];
-      }
-      if (MODE == kModeScaled) {
-        const int kn = min(it + 2, nkb - 1);
-        q0n = sqp[sqo0 + (uint32_t)((kb_begin + kn) >> 2) * sxk]; q1n = sqp[sqo1 + (uint32_t)((kb_begin + kn) >> 2) * sxk]; sbn = swp[(int64_t)kn * p.sw_k];
-      }
-      SB();
-      RW(0, stW, 1); LW(0, it + 3, w_ld); LW(1, it + 3, w_ld); SB();
-      M(0, 1, 0); SB();
-      M(1, 1, 0); SB();
-      RW(1, stW, 1); LW(2, it + 3, w_ld); LW(3, it + 3, w_ld); SB();
+      // ---- block it+1; the products still pending belong to block it.  The scales of block it+2 are requested after the
+      // activation loads and before the weight loads.
+      take_scales(it + 1);
+      if (MODE == kModeScaled) use_scales();
+      pair(0, true, [&](int i) {
+        if (i == 0) request_scales(it + 2);
+        if (i == 1) RW(stW, 2);
+        if (i == 3) RW(stW, 3);
+        if (i == 3 && MODE == kModeBlock) use_scales();
+        if (i == 2 || i == 4 || i == 6) LW(i / 2 - 1, it + 3, w_ld);
+      });
       __builtin_amdgcn_s_setprio(1);
-      // ---- steps 1 and 2 of block it+1
-      F(acc[0][0], tq[0], sc[0]); SB();
-      M(0, 0, 1); SB();
-      F(acc[0][1], tq[1], sc[1]); SB();
-      M(1, 0, 1); SB();
-      RW(0, stW, 2); SB();
-      M(0, 1, 1); SB();
-      M(1, 1, 1); SB();
-      RW(1, stW, 2); SB();
+      pair(1, true, [&](int i) {
+        if (i == 0) LW(3, it + 3, w_ld);
+        if (i == 1) RW(stW, 4);
+        if (i == 3) RW(stW, 5);
+      });
       __builtin_amdgcn_s_setprio(0);
-      F(acc[1][0], tq[0], sc[0]); SB();
-      M(0, 0, 2); SB();
-      F(acc[1][1], tq[1], sc[1]); SB();
-      M(1, 0, 2); SB();
-      RW(0, stW, 3); SB();
-      M(0, 1, 2); SB();
-      M(1, 1, 2); SB();
-      RW(1, stW, 3); SB();
+      pair(2, true, [&](int i) {
+        if (i == 1) RW(stW, 6);
+        if (i == 3) RW(stW, 7);
+      });
       w_ld = w_rd;
       w_rd = w_rd == 2 ? 0 : w_rd + 1;
     }
-    // ---- step 3 of the last block
-    F(acc[2][0], tq[0], sc[0]); SB();
-    M(0, 0, 3); SB();
-    F(acc[2][1], tq[1], sc[1]); SB();
-    M(1, 0, 3); SB();
-    M(0, 1, 3); SB();
-    M(1, 1, 3); SB();
-    F(acc[3][0], tq[0], sc[0]);
-    F(acc[3][1], tq[1], sc[1]);
+    // ---- last pair of the last block
+    pair(3, true, [](int) {});
+#pragma unroll
+    for (int k = 28; k < 32; ++k) F(k);
 
     // Finished tiles leave through LDS so that every store instruction writes whole 256-byte row segments
     // (the accumulator layout alone gives 8 bytes per row per lane: 32 partial lines per instruction).
@@ -681,22 +668,37 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
       SB();
     }
 
-    const auto col_of = [&](int ns, int rg) { return n0 + wn * 128 + ns * 32 + rg * 8 + h * 4; };
+    const auto col_of = [&](int ns) { return n0 + wn * 128 + ns * 16 + kq * 4; };
+    // Row mode: scales and bias.  The 16 lanes of a row (equal kq) own the same 32 columns: each fetches two of them, and the one a
+    // value needs is broadcast along the row inside the multiplication.  (All 32 in every lane, beside the accumulators, spill.)
+    float sa[4] = {1.f, 1.f, 1.f, 1.f}, sbv[2] = {1.f, 1.f}, biasv[2] = {0.f, 0.f};
+    const bool has_bias = MODE == kModeRow && p.bias != nullptr;
     if (MODE == kModeRow && !is_split) {
-      float sa[2];
 #pragma unroll
-      for (int ms = 0; ms < 2; ++ms) {
-        const int m = slot_at(wm * 64 + ms * 32 + lr);
+      for (int ms = 0; ms < 4; ++ms) {
+        const int m = m0 + wm * 64 + ms * 16 + lr;
         sa[ms] = m < nrows ? row_scale(p, m) : 1.f;
       }
-      finish_rows<16, 2, BIAS_DT>(p, sa, [&](int j) { return col_of(j >> 2, j & 3); },
-                                  [&](int j, int ms, int q, auto f) { acc[j >> 2][ms][(j & 3) * 4 + q] = f(acc[j >> 2][ms][(j & 3) * 4 + q]); });
-    }
-    // value (ns, rg) of row slot ms of this lane, packed to two 16-bit pairs
-    auto out_pair = [&](int ns, int ms, int rg) -> uint2 {
-      float v[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = acc[ns][ms][rg * 4 + q];
+      for (int j = 0; j < 2; ++j) {
+        const int col = min(col_of(j * 4 + (lr >> 2)) + (lr & 3), p.N - 1);
+        sbv[j] = p.sw[(int64_t)col * p.sw_n];
+        if (has_bias) biasv[j] = load_scalar<BIAS_DT>(p.bias, col);
+      }
+    }
+    // the four columns ns of row group ms of this lane, packed to two 16-bit pairs
+    auto out_pair = [&](auto ns_c, int ms) -> uint2 {
+      constexpr int ns = decltype(ns_c)::value;
+      v4f v = acc[ns][ms];
+      if (MODE == kModeRow) {
+        const float s = sbv[ns >> 2], b = biasv[ns >> 2];
+        constexpr int l0 = (ns & 3) * 4;
+        v[0] = v[0] * row_broadcast<l0>(s) * sa[ms]; v[1] = v[1] * row_broadcast<l0 + 1>(s) * sa[ms];
+        v[2] = v[2] * row_broadcast<l0 + 2>(s) * sa[ms]; v[3] = v[3] * row_broadcast<l0 + 3>(s) * sa[ms];
+        if (has_bias) {
+          v[0] += row_broadcast<l0>(b); v[1] += row_broadcast<l0 + 1>(b); v[2] += row_broadcast<l0 + 2>(b); v[3] += row_broadcast<l0 + 3>(b);
+        }
+      }
       uint2 o;
       if (OUT_DT == FP8K_BF16) {
         o.x = pack_bf16x2(v[0], v[1]);
@@ -713,12 +715,12 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
       if (MODE == kModeBlock && p.bias) load_bias8<BIAS_DT>(p.bias, min(n0 + wn * 128 + ((ln & 15) << 3), p.N - 8), bias8);
       uint8_t* ep = smem + (w < 4 ? ews * kWStage + w * 8192 : kXBase + exs * kXStage + (w - 4) * 8192);  // 32 rows x 256 B per pass
 #pragma unroll
-      for (int ms = 0; ms < 2; ++ms) {
+      for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll
-        for (int ns = 0; ns < 4; ++ns)
-#pragma unroll
-          for (int rg = 0; rg < 4; ++rg)
-            *reinterpret_cast<uint2*>(ep + lr * 256 + (((ns * 4 + rg) ^ (lr & 15)) << 4) + h * 8) = out_pair(ns, ms, rg);
+        for (int g = 0; g < 2; ++g)
+          static_for<8>([&](auto ns) {
+            *reinterpret_cast<uint2*>(ep + (g * 16 + lr) * 256 + (((ns * 2 + (kq >> 1)) ^ lr) << 4) + (kq & 1) * 8) = out_pair(ns, pass * 2 + g);
+          });
         __builtin_amdgcn_wave_barrier();  // one wave's LDS accesses complete in order: no wait needed
         const int rr = ln >> 4, pc = ln & 15;
 #pragma unroll
@@ -726,7 +728,7 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
           const int r = i * 4 + rr;
           uint4 o = *reinterpret_cast<const uint4*>(ep + r * 256 + ((pc ^ (r & 15)) << 4));
           if (MODE == kModeBlock && p.bias) o = add_bias8<OUT_DT>(o, bias8);
-          const int m = slot_at(wm * 64 + ms * 32 + r);
+          const int m = m0 + wm * 64 + pass * 32 + r;
           const int n = n0 + wn * 128 + (pc << 3);  // consecutive lanes store consecutive 16-byte chunks
           if (m < nrows && n < p.N) *reinterpret_cast<uint4*>((u16*)p.C + (int64_t)m * p.ldc + n) = o;
         }
@@ -734,33 +736,24 @@ __global__ __launch_bounds__(512, 1) void gemm_tile256_kernel(const GemmArgs p) 
       }
     } else {
 #pragma unroll
-      for (int ms = 0; ms < 2; ++ms) {
-        const int ml = wm * 64 + ms * 32 + lr;  // row inside the tile
-        const int m = slot_at(ml);               // output row
-        if (m >= nrows) continue;
-#pragma unroll
-        for (int ns = 0; ns < 4; ++ns) {
-#pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
-            const int n = n0 + wn * 128 + ns * 32 + rg * 8 + h * 4;
-            if (n >= p.N) continue;
-            if (is_split) {
-              float* tile_part = p.partial + ((int64_t)(t - p.tail_first) * p.splits + split) * (kTileM * kTileN);
-              *reinterpret_cast<float4*>(tile_part + ml * kTileN + (n - n0)) =
-                  make_float4(acc[ns][ms][rg * 4], acc[ns][ms][rg * 4 + 1], acc[ns][ms][rg * 4 + 2], acc[ns][ms][rg * 4 + 3]);
-            } else {
-              if (MODE == kModeBlock && p.bias) {
-                float v[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] = acc[ns][ms][rg * 4 + q];
-                finish4<MODE, OUT_DT, BIAS_DT>(p, n, 1.f, v);
-                store4<OUT_DT>(p.C, (int64_t)m * p.ldc + n, v[0], v[1], v[2], v[3]);
-              } else {
-                *reinterpret_cast<uint2*>((u16*)p.C + (int64_t)m * p.ldc + n) = out_pair(ns, ms, rg);
-              }
-            }
+      for (int ms = 0; ms < 4; ++ms) {
+        const int ml = wm * 64 + ms * 16 + lr, m = m0 + ml;  // row inside the tile, output row
+        static_for<8>([&](auto ns) {
+          const int n = col_of(ns);
+          const uint2 o = out_pair(ns, ms);  // by all lanes: its broadcasts read lanes that store nothing
+          if (m >= nrows || n >= p.N) return;
+          const v4f v4 = acc[ns][ms];
+          if (is_split) {
+            float* tile_part = p.partial + ((int64_t)(t - p.tail_first) * p.splits + split) * (kTileM * kTileN);
+            *reinterpret_cast<float4*>(tile_part + ml * kTileN + (n - n0)) = make_float4(v4[0], v4[1], v4[2], v4[3]);
+          } else if (MODE == kModeBlock && p.bias) {
+            float v[4] = {v4[0], v4[1], v4[2], v4[3]};
+            finish4<MODE, OUT_DT, BIAS_DT>(p, n, 1.f, v);
+            store4<OUT_DT>(p.C, (int64_t)m * p.ldc + n, v[0], v[1], v[2], v[3]);
+          } else {
+            *reinterpret_cast<uint2*>((u16*)p.C + (int64_t)m * p.ldc + n) = o;
           }
-        }
+        });
       }
     }
     if (!has_next) {

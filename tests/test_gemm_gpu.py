@@ -169,6 +169,38 @@ def test_block_gemm_last_round_in_half_tiles_exact(dev, M):
     np.testing.assert_array_equal(c, O.w8a8_block_fp8_matmul(xq, wq, xs, ws, out_dtype="bf16", acc=np.float64))
 
 
+@pytest.mark.parametrize("M,N,K", [(300, 264, 128), (513, 520, 256), (250, 1032, 640)])
+@pytest.mark.parametrize("bias_dtype", [None, torch.float32, torch.bfloat16, torch.float16])
+def test_tile256_row_scales_and_bias_exact(dev, M, N, K, bias_dtype):
+    """256x256 tiles with row scales: every lane of the write-out gets its columns' scales and biases from other lanes, in the
+    16-byte stores and in the 8-byte ones of an ldc that is no multiple of 8.  Integers, power-of-two scales: exact in float16."""
+    from sglang_amd._lib import check, lib, stream_ptr
+
+    rng = np.random.default_rng(M + K)
+    xv, wv = rng.integers(-1, 2, (M, K)), rng.integers(-1, 2, (N, K))
+    sa, sb = 2.0 ** rng.integers(-2, 2, M), 2.0 ** rng.integers(-2, 2, N)
+    ref = (xv @ wv.T) * sb * sa[:, None]
+    bias = None if bias_dtype is None else torch.from_numpy(rng.integers(-16, 17, N).astype(np.float32)).to(dev, bias_dtype)
+    if bias is not None:
+        ref = ref + bias.float().cpu().numpy()
+    A, B = (fp8_tensor(O.f32_to_e4m3fn(v.astype(np.float32)), dev) for v in (xv, wv))
+    sa_t, sb_t = (torch.from_numpy(v.astype(np.float32)).to(dev) for v in (sa, sb))
+    try:
+        lib.fp8k_tune_force_gemm_plan(1, 0)
+        need = lib.fp8k_scaled_mm_workspace_bytes(M, N, K)
+        work = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+        for ldc in (N, N + 4):
+            C = torch.full((M, ldc), 7.0, dtype=torch.float16, device=dev)
+            check(lib.fp8k_scaled_mm(A.data_ptr(), B.data_ptr(), sa_t.data_ptr(), sb_t.data_ptr(), bias.data_ptr() if bias is not None else None,
+                                     C.data_ptr(), M, N, K, K, K, ldc, 1, {None: 0, torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[bias_dtype],
+                                     work.data_ptr(), need, stream_ptr(dev)))
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(C[:, :N].float().cpu().numpy(), ref.astype(np.float16).astype(np.float32))
+            assert bool((C[:, N:] == 7.0).all())
+    finally:
+        lib.fp8k_tune_force_gemm_plan(-1, 0)
+
+
 def test_block_gemm_scale_layouts_agree(dev):
     xq, xs, wq, ws = _quantised_problem(200, 512, 1024, 9)
     a = _run_block(xq, xs, wq, ws, dev, col_major_as=False)
