@@ -16,11 +16,11 @@ namespace fp8k {
 
 struct Plan {
   int kind;    // 0 = generic, 1 = tile256, 2 = weight-streaming through LDS (33..128 rows), 3 = direct (<= 32 rows),
-               // 4 = tile128, 5 = direct with K cut across the waves of a workgroup (<= 16 rows, N below 16 K), 7 = skinny
-               // strips over all of K (<= 128 rows, N up to 16 K)
+               // 4 = tiles of 128 weight rows, 5 = direct with K cut across the waves of a workgroup (<= 16 rows, N below 16 K),
+               // 7 = skinny strips over all of K (<= 128 rows, N up to 16 K)
   int splits;  // >1: split-K through the float workspace
   int kb_per_split;
-  int tm;      // rows per block of the streaming kernels
+  int tm;      // rows per block of the streaming kernels, activation rows of a tile (kind 4)
   int tail_first;   // tile256: first tile that is cut along K or into halves (== number of tiles when none is)
   int halves;       // tile256: the tiles from tail_first on are computed as two 128-row halves; kinds 5, 7: waves along n
   int64_t ws_bytes; // float workspace the plan needs
@@ -31,8 +31,9 @@ struct Plan {
 static thread_local int g_force_kind = -1, g_force_splits = 0;
 static thread_local int g_tail_halves = 1;  // tuning aid: 0 keeps the last round of 256x256 tiles whole
 
-static Plan plan_tile128(int64_t M, int64_t N, int kb, int splits) {
+static Plan plan_tile128(int64_t M, int64_t N, int kb, int splits, int tm) {
   Plan pl{4, 1, 0, 0, 0, 0};
+  pl.tm = tm;
   if (splits > kb) splits = kb;
   if (splits < 1) splits = 1;
   pl.kb_per_split = (kb + splits - 1) / splits;
@@ -75,7 +76,7 @@ static Plan plan_direct(int64_t M, int64_t N, int64_t K) {
 // (nothing goes through the workspace); kb_per_split is the K range of one wave, tm reuses the row-count slot, and
 // the number of waves along n travels in `halves`.
 constexpr int64_t kWaveKMaxN = 16384;
-static Plan plan_wavek(int64_t M, int64_t N, int64_t K) {
+static Plan plan_wavek(int64_t M, int64_t N, int64_t K, int cu) {
   Plan pl{5, 1, 0, 0, 0, 0};
   const int kb = (int)(K / kTileK);
   pl.tm = 16;
@@ -86,8 +87,8 @@ static Plan plan_wavek(int64_t M, int64_t N, int64_t K) {
   int64_t best_rows = -1;
   for (int cand = 1; cand <= 4; cand *= 2) {
     const int64_t wgs = (N + 16 * cand - 1) / (16 * cand);
-    if (wgs > 2 * (int64_t)num_cu() && cand < 4) continue;
-    const int64_t rows = (wgs + num_cu() - 1) / num_cu() * 16 * cand;
+    if (wgs > 2 * (int64_t)cu && cand < 4) continue;
+    const int64_t rows = (wgs + cu - 1) / cu * 16 * cand;
     const int per_wave = (kb + 8 / cand - 1) / (8 / cand);
     if (best_rows < 0 || rows < best_rows || (rows == best_rows && per_wave <= 16)) { best_rows = rows; nw = cand; }
   }
@@ -99,29 +100,31 @@ static Plan plan_wavek(int64_t M, int64_t N, int64_t K) {
 }
 // Up to 128 rows: the strips of weight rows that one workgroup each runs over all of K are as narrow as leaves every CU one.
 constexpr int64_t kSkinnyMaxN = 16384;
-static Plan plan_skinny(int64_t M, int64_t N, int64_t K) {
+static Plan plan_skinny(int64_t M, int64_t N, int64_t K, int cu) {
   Plan pl{7, 1, 0, 0, 0, 0};
   pl.tm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
-  pl.halves = N <= 16 * num_cu() ? 1 : N <= 32 * num_cu() ? 2 : 4;
+  pl.halves = N <= 16 * cu ? 1 : N <= 32 * cu ? 2 : 4;
   if (g_force_kind == 7 && (g_force_splits == 1 || g_force_splits == 2 || g_force_splits == 4)) pl.halves = g_force_splits;  // tuning aid
   if (pl.tm == 128) pl.halves = 2;
   return pl;
 }
 // Where it is ahead (M = 4 .. 64 x 16 widths up to 20480 x 9 depths up to 18432, timed against the other decode kernels and the
-// 128-row tiles under every K cut: what the rule takes is within 1 % of the best on average up to 32 rows, 4 % above):
+// 64-row tiles under every K cut):
 //  * more than 64 weight rows per CU's strip cost more activation traffic than a K cut costs partials, from 9 rows on;
-//  * that traffic grows with rows x K: above 32 rows a K of more than 8192 is left to the 128-row tiles with a K cut, and with
-//    64-row strips, whose waves have little of the LDS traffic to hide it behind, K of more than 4096 unless they fill the chip;
 //  * 17 .. 32 rows in 64-row strips that leave a quarter of the CUs idle: up to K = 6144;
-//  * 65 .. 128 rows, in 32-row strips only: a middle range of K, 3 - 37 % ahead inside it.
-static bool prefers_skinny(int64_t M, int64_t N, int64_t K) {
+//  * 33 .. 64 rows: that traffic grows with rows x K, so up to a K where the 64-row tiles are level (370 shapes, weights out of HBM;
+//    time over the tiles': up to 4096 weight rows 0.63 at K = 1536 .. 3072, 0.75 at 5120, 0.92 at 7168, 1.04 at 10240; up to 8192
+//    0.71, 0.89, 0.94 at 6144, 1.05 at 8192), and in 64-row strips from K = 1664 (0.82 - 0.95; level below) to 4608, or 10240
+//    where the strips fill the chip.
+static bool prefers_skinny(int64_t M, int64_t N, int64_t K, int cu) {
   if (M > kSkinnyMaxM || N > kSkinnyMaxN) return false;
-  const bool wide = N > 32 * num_cu(), fills = N >= 48 * num_cu();
+  const bool wide = N > 32 * cu, fills = N >= 48 * cu;
   if (M <= 8) return K <= 9216;  // above: the wave-cut kernel, whose waves keep all of their K range in flight
   if (M <= 16) return true;
   if (M <= 32) return !wide || fills || K <= 6144;
-  if (M > 64) return !wide && K >= 1536 && K <= (N >= 16 * num_cu() ? 4608 : 3072);
-  return wide ? K >= 1024 && K <= (fills ? 10240 : 4096) : K <= 8192;
+  if (M > 64) return !wide && K >= 1536 && K <= (N >= 16 * cu ? 4608 : 3072);
+  if (wide) return K > 1536 && K <= (fills ? 10240 : 4608);
+  return K <= (N <= 16 * cu ? 7168 : 6144);
 }
 // Activations few enough for every workgroup to quantise them for itself (gemm_wavek_quant_kernel): up to 16 rows of at most
 // kQuantFuseMax elements together.  The share of the quantisation grows with M * K while the launch it saves does not (the gain
@@ -149,99 +152,111 @@ static Plan plan_stream(int64_t M, int64_t N, int64_t K) {
 
 // One workgroup (one CU) per 256x256 tile.  The tiles of the last, partial round over the CUs are cut along K
 // so that the round keeps every CU busy for 1/splits of a tile time (>= 4 K blocks per piece).
-static Plan plan_tile256(int64_t M, int64_t N, int64_t K) {
+static Plan plan_tile256(int64_t M, int64_t N, int64_t K, int cu) {
   Plan pl{1, 1, 0, 0, 0, 0};
   const int kb = (int)(K / kTileK);
   const int64_t tiles = ((M + kTileM - 1) / kTileM) * ((N + kTileN - 1) / kTileN);
-  const int64_t rest = tiles % num_cu();
-  int splits = rest ? (int)(num_cu() / rest) : 1;
+  const int64_t rest = tiles % cu;
+  int splits = rest ? (int)(cu / rest) : 1;
   if (splits > kb / 4) splits = kb / 4;
   if (splits < 1) splits = 1;
   // With at least one full round before it, the cut only pays when the tile time it saves (about 2 us per K block)
   // outweighs writing and re-reading the float partials (256 KB per piece): measured break-even.
-  if (tiles > num_cu() && kb * (splits - 1) * 8 <= rest * splits * splits) splits = 1;
+  if (tiles > cu && kb * (splits - 1) * 8 <= rest * splits * splits) splits = 1;
   pl.kb_per_split = (kb + splits - 1) / splits;
   pl.splits = (kb + pl.kb_per_split - 1) / pl.kb_per_split;
   pl.tail_first = (int)(pl.splits > 1 ? tiles - rest : tiles);
   pl.ws_bytes = pl.splits > 1 ? rest * pl.splits * (int64_t)(kTileM * kTileN) * 4 : 0;
   // A last round that fills at most half the CUs and is not worth a K cut: its tiles run as two 128-row halves, one
   // workgroup each (half the matrix-core time per K block, nothing to reduce).
-  if (pl.splits == 1 && tiles > num_cu() && rest > 0 && rest <= num_cu() / 2 && M > kTileM / 2 && g_tail_halves) {
+  if (pl.splits == 1 && tiles > cu && rest > 0 && rest <= cu / 2 && M > kTileM / 2 && g_tail_halves) {
     pl.halves = 1;
     pl.tail_first = (int)(tiles - rest);
   }
   return pl;
 }
 
-// the plan without the 128x128 tile kernel: direct / streaming / 256x256 tiles by the number of rows
-static Plan plan_base(int64_t M, int64_t N, int64_t K) {
+// the plan without the 128-row tiles: skinny / direct / streaming / 256x256 tiles by the number of rows
+static Plan plan_base(int64_t M, int64_t N, int64_t K, int cu) {
   const bool fits32 = M * K < (1LL << 31);
   if (g_force_kind == 3 && M <= 32 && fits32) return plan_direct(M, N, K);
-  if (g_force_kind == 5 && M <= 16 && fits32) return plan_wavek(M, N, K);
-  if (g_force_kind == 7 && M <= kSkinnyMaxM && fits32) return plan_skinny(M, N, K);
+  if (g_force_kind == 5 && M <= 16 && fits32) return plan_wavek(M, N, K, cu);
+  if (g_force_kind == 7 && M <= kSkinnyMaxM && fits32) return plan_skinny(M, N, K, cu);
   if (g_force_kind == 2 && M <= 128 && fits32) return plan_stream(M, N, K);
-  if (g_force_kind == 1) return plan_tile256(M, N, K);
-  if (fits32 && few_activations(M, N, K)) return plan_wavek(M, N, K);
-  if (fits32 && prefers_skinny(M, N, K)) return plan_skinny(M, N, K);
-  if (fits32 && M <= 8 && N < kWaveKMaxN) return plan_wavek(M, N, K);
+  if (g_force_kind == 1) return plan_tile256(M, N, K, cu);
+  if (fits32 && few_activations(M, N, K)) return plan_wavek(M, N, K, cu);
+  if (fits32 && prefers_skinny(M, N, K, cu)) return plan_skinny(M, N, K, cu);
+  if (fits32 && M <= 8 && N < kWaveKMaxN) return plan_wavek(M, N, K, cu);
   if (M <= 32 && fits32) return plan_direct(M, N, K);
   if (M <= 128 && fits32) return plan_stream(M, N, K);
-  return plan_tile256(M, N, K);
+  return plan_tile256(M, N, K, cu);
 }
 
-
-// Rough device-time models in microseconds, fitted to sweeps over M = 48..2048 on the DeepSeek-V3 and Llama
-// projection shapes; they only have to rank the two candidates where the gap is large.
-//  * 128x128 tiles: a workgroup spends 0.42 us per K block when its operands come out of the L2, up to 0.72 us
-//    when every CU streams lines that are new to the chip (the share of such lines falls with the number of
-//    tiles that share a weight or activation tile); first loads + tile write-out 2.5 us per round of tiles,
-//    launch 1 us; more than two rounds are left to the 256x256 kernel, two rounds measure about 15 % over the
-//    model; a K cut adds the reduction launch (4 us) and the float partials (written and read back at about
-//    5 TB/s).
-//  * streaming kernel: 10-11 us fixed, the weights once at 5.5 TB/s, its partials at about 8 TB/s.
-//  * 256x256 tiles: 1.6 us per K block and tile, 8 us fixed, 6 us + partials (8 TB/s) for a cut last round.
-static double est_tile128(int64_t M, int64_t N, int kb, int* best_splits) {
-  const int64_t tm = (M + kT128 - 1) / kT128, tn = (N + kT128 - 1) / kT128;
-  const int64_t tiles = tm * tn;
-  const double cold = std::min(1.0, 1.0 / (double)tm + 1.0 / (double)tn);
+// Device-time models in microseconds of the two tile kernels, fitted to 2500 shapes (M = 33 .. 2400, N = 512 .. 24576, K = 512 .. 18432,
+// block scales, weights out of HBM, every K cut; rms error 6 and 5 %).  Over those with more than 128 rows the choice they make
+// is 0.4 % behind the best of all plans on average, 14 % at worst.
+//  * tiles of 128 weight rows and TM = 128 or 64 activation rows: 0.43 (0.34) per K block - the serial chain of a trip more than its
+//    work - and a little more when the weights are new to the chip and the chip is full; 3 us of first loads and write-out per
+//    round of tiles, at most two rounds; a K cut adds the reduction launch and the float partials.  Below 12 us a cut gains nothing
+//    where the host makes the launches one by one: it takes 4 us for each (134 x 1280 x 2944 as a linear: 17 - 18 us with three
+//    K ranges, which are the quicker product by 0.4, and 15 without).
+//  * 256x256 tiles: 1.5 per K block on a full chip (0.7 for a workgroup alone), 4.4 per tile, 15 us + partials for a cut last round.
+static double est_tile128(int64_t M, int64_t N, int kb, int cu, int* best_splits, int* best_tm) {
   double best = 1e30;
-  for (int s = 1; s <= 8; ++s) {
-    if (s > 1 && (s > kb / 4 || tiles * s > 256)) break;  // a K cut stays within one round of workgroups
-    const int64_t wgs = tiles * s;
-    const int64_t rounds = (wgs + num_cu() - 1) / num_cu();
-    if (rounds > 2) break;
-    const int kbps = (kb + s - 1) / s;
-    const double tb = 0.42 + 0.30 * cold * std::min(1.0, (double)wgs / num_cu());
-    double t = 1.0 + (double)rounds * (kbps * tb + 2.5);
-    if (rounds == 2) t *= 1.15;
-    if (s > 1) t += 4.0 + (double)s * M * N * 8.0 / 5e6;
-    if (t < best) { best = t; *best_splits = s; }
+  const int64_t tn = (N + kT128 - 1) / kT128;
+  for (int rows = 64; rows <= (M > 64 ? 128 : 64); rows += 64) {
+    const int64_t tm = (M + rows - 1) / rows;
+    for (int s = 1; s <= 8; ++s) {
+      const int64_t wgs = tm * tn * s, rounds = (wgs + cu - 1) / cu;
+      if (rounds > 2 || (s > 1 && (rounds > 1 || s > kb / 3))) break;  // a K cut stays within one round of workgroups
+      const double fill = std::min(1.0, (double)wgs / cu), cold = 1.0 / (double)tm;
+      const double tb = rows == 64 ? 0.342 + 0.048 * cold + fill * (0.159 * cold + 0.008) : 0.433 + 0.018 * cold + fill * (0.056 * cold + 0.065);
+      double t = 1.4 + (double)rounds * ((kb + s - 1) / s * tb + (rows == 64 ? 2.8 : 3.4));
+      if (rounds == 2) t *= 0.985;
+      if (s > 1) t += 3.1 + (double)s * M * N * 8.0 / 4.15e6;
+      t = std::max(t, s > 1 ? 12.0 : 8.0);
+      if (t < best) { best = t; *best_splits = s; *best_tm = rows; }
+    }
   }
   return best;
 }
 
-static double est_base(const Plan& pl, int64_t M, int64_t N, int64_t K) {
-  const int kb = (int)(K / kTileK);
-  if (pl.kind == 2)
-    return (M <= 64 ? 10.0 : 11.0) + (double)N * K / 5.5e6 + (pl.splits > 1 ? (double)pl.splits * M * N * 8.0 / 8e6 : 0.0);
-  const int64_t tiles = ((M + kTileM - 1) / kTileM) * ((N + kTileN - 1) / kTileN);
-  if (pl.splits == 1) return 8.0 + (double)((tiles + num_cu() - 1) / num_cu()) * kb * 1.6;
-  const int64_t rest = tiles % num_cu();
-  return 8.0 + (double)(tiles / num_cu()) * kb * 1.6 + pl.kb_per_split * 1.6 + 6.0 +
-         (double)rest * pl.splits * (kTileM * kTileN * 4) * 2.0 / 8e6;
+static double est_tile256(const Plan& pl, int64_t M, int64_t N, int kb, int cu) {
+  const int64_t tiles = ((M + kTileM - 1) / kTileM) * ((N + kTileN - 1) / kTileN), rest = tiles % cu;
+  auto per_kb = [&](int64_t wgs) { return 0.68 + 0.87 * std::min(1.0, (double)wgs / cu); };
+  if (pl.splits == 1) {
+    const double rounds = pl.halves ? (double)(tiles / cu) + 0.6 : (double)((tiles + cu - 1) / cu);
+    return 4.7 + rounds * (kb * per_kb(tiles) + 4.4);
+  }
+  return 4.7 + (double)(tiles / cu) * (kb * per_kb(cu) + 4.4) + pl.kb_per_split * per_kb(rest * pl.splits) + 15.4 +
+         (double)rest * pl.splits * 0.0205;
 }
 
 static Plan make_plan(int64_t M, int64_t N, int64_t K) {
   Plan pl{0, 1, 0, 0, 0, 0};
   if (K % kTileK != 0 || N % 4 != 0) return pl;
-  const int kb = (int)(K / kTileK);
-  if (g_force_kind == 4 && N % 8 == 0) return plan_tile128(M, N, kb, g_force_splits);
-  pl = plan_base(M, N, K);
-  if (g_force_kind >= 0 || M <= 32 || N % 8 != 0 || (pl.kind != 1 && pl.kind != 2)) return pl;
-  // a few hundred rows, or fewer 256x256 tiles than CUs: the 128x128 tile kernel when the model puts it ahead
-  int s128 = 1;
-  const double t128 = est_tile128(M, N, kb, &s128);
-  if (t128 < 0.92 * est_base(pl, M, N, K)) return plan_tile128(M, N, kb, s128);
+  const int kb = (int)(K / kTileK), cu = num_cu();  // once: asking the runtime for the device costs more than all of the arithmetic
+  // tuning aid: the K cut in the low byte, 256 for tiles of 64 activation rows
+  if (g_force_kind == 4 && N % 8 == 0) return plan_tile128(M, N, kb, g_force_splits & 255, g_force_splits & 256 ? 64 : 128);
+  pl = plan_base(M, N, K, cu);
+  if (g_force_kind >= 0 || N % 8 != 0 || M <= 16) return pl;
+  int splits = 1, rows = 0;
+  if (pl.kind == 1) {
+    if (est_tile128(M, N, kb, cu, &splits, &rows) < est_tile256(pl, M, N, kb, cu)) return plan_tile128(M, N, kb, splits, rows);
+  } else if (pl.kind == 2) {
+    // The streaming kernel keeps 256-row tiles x 2 - 3 K ranges where 128-row tiles are a little more than half a chip and a K cut
+    // would be a second round: 97 x 18240 x 15104 70 us against 79, 97 x 17152 x 8192 41 against 45; 122 x 20288 x 6400 42 against 39,
+    // 106 x 23040 x 5760 41 against 35.  Everywhere else the tiles are ahead, up to twice (108 x 15616 x 1024 8.2 against 19.3).
+    if (!(N > 64 * cu && N <= 80 * cu && K >= 8192)) {
+      est_tile128(M, N, kb, cu, &splits, &rows);
+      if (rows) return plan_tile128(M, N, kb, splits, rows);
+    }
+  } else if (pl.kind == 3 && N > 32 * cu && N < 48 * cu && K > 6144) {
+    // 17 .. 32 rows of weights too wide for one 32-row strip per CU and too narrow for 64-row strips: 64-row tiles with a K cut
+    // (us, against the direct kernel: 26 x 8768 x 6400 17.3 / 23.7, 18 x 8640 x 9984 21.6 / 25.8, 23 x 10688 x 14208 31.9 / 36.4)
+    est_tile128(M, N, kb, cu, &splits, &rows);
+    return plan_tile128(M, N, kb, splits, rows);
+  }
   return pl;
 }
 
@@ -283,16 +298,20 @@ static int launch_tiles(const GemmArgs& a0, const Plan& pl, hipStream_t st) {
   a.splits = pl.splits;
   a.kb_per_split = pl.kb_per_split;
   if (pl.kind == 4) {
-    a.tiles_m = (a.M + kT128 - 1) / kT128;
+    a.tiles_m = (a.M + pl.tm - 1) / pl.tm;
     a.tiles_n = (a.N + kT128 - 1) / kT128;
     const unsigned nwg = (unsigned)(((int64_t)a.tiles_m * a.tiles_n * pl.splits + 7) / 8 * 8);
+#define FP8K_T128(SPLIT, TM) hipLaunchKernelGGL((gemm_tile128_kernel<MODE, OUT_DT, BIAS_DT, SPLIT, TM>), dim3(nwg), dim3(512), 0, st, a)
     if (pl.splits == 1) {
-      hipLaunchKernelGGL((gemm_tile128_kernel<MODE, OUT_DT, BIAS_DT, false>), dim3(nwg), dim3(512), 0, st, a);
-      return check_launch("gemm_tile128");
+      if (pl.tm == 64) FP8K_T128(false, 64);
+      else FP8K_T128(false, 128);
+    } else {
+      if (pl.tm == 64) FP8K_T128(true, 64);
+      else FP8K_T128(true, 128);
     }
-    hipLaunchKernelGGL((gemm_tile128_kernel<MODE, OUT_DT, BIAS_DT, true>), dim3(nwg), dim3(512), 0, st, a);
+#undef FP8K_T128
     int rc = check_launch("gemm_tile128");
-    if (rc) return rc;
+    if (rc || pl.splits == 1) return rc;
     const int64_t quads = (int64_t)a.M * (a.N / 4);
     hipLaunchKernelGGL((splitk_reduce_kernel<MODE, OUT_DT, BIAS_DT>), dim3((unsigned)((quads + 255) / 256)), dim3(256),
                        0, st, a);
@@ -554,9 +573,11 @@ extern "C" int fp8k_block_gemm_ue8m0(const void* A, const void* B, const int32_t
   FP8K_REQUIRE(As_packed && Bs, "%s: null scale pointer", op);
   FP8K_REQUIRE(as_stride_m >= 0 && as_stride_w >= 0 && bs_stride_n >= 0 && bs_stride_k >= 0, "%s: negative scale stride", op);
   FP8K_REQUIRE((M - 1) * as_stride_m + ((K + kTileK - 1) / kTileK / 4) * as_stride_w < (1LL << 31), "%s: scales span more than 2^31 elements", op);
-  const Plan pl = make_plan(M, N, K);
+  Plan pl = make_plan(M, N, K);
   // the matrix core applies the scales only in the tile kernels; smaller problems take the float-scale
   // entry point with the exponents expanded to floats
+  if (g_force_kind < 0 && M > 32 && K % kTileK == 0 && N % 8 == 0 && pl.kind != 1 && pl.kind != 4)
+    pl = plan_tile128(M, N, (int)(K / kTileK), 1, M <= 64 ? 64 : 128);
   FP8K_REQUIRE(pl.kind == 1 || pl.kind == 4, "%s: built for M > 128 with K a multiple of 128 (got M=%lld, K=%lld); expand the scales "
                "and call fp8k_block_gemm", op, (long long)M, (long long)K);
   const int64_t need = pl.ws_bytes;
@@ -671,7 +692,7 @@ static int quant_linear(const char* op, bool block_mode, const void* x, const vo
    : dtype == FP8K_BF16 ? FP8K_QL(FN, FP8K_BF16, __VA_ARGS__)                                                                     \
                         : FP8K_QL(FN, FP8K_F16, __VA_ARGS__))
   if (fuses_quant(M, N, K)) {
-    const Plan pl = plan_wavek(M, N, K);
+    const Plan pl = plan_wavek(M, N, K, num_cu());
     a.q_eps = quant_eps(eps, dtype);
     a.wk_nw = pl.halves; a.kb_per_split = pl.kb_per_split;
     return FP8K_LINEAR(launch_quant_linear, a, st);
@@ -757,9 +778,9 @@ static int bmm_impl(const void* A, const void* B, const float* sa, const float* 
   a.kb_per_split = (int)(K / kTileK);
   const unsigned nwg = (unsigned)(((int64_t)a.tiles_m * a.tiles_n + 7) / 8 * 8);
   if (out_dtype == FP8K_BF16)
-    hipLaunchKernelGGL((gemm_tile128_kernel<kModeRow, FP8K_BF16, FP8K_F32, false>), dim3(nwg, (unsigned)batch), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((gemm_tile128_kernel<kModeRow, FP8K_BF16, FP8K_F32, false, 128>), dim3(nwg, (unsigned)batch), dim3(512), 0, st, a);
   else
-    hipLaunchKernelGGL((gemm_tile128_kernel<kModeRow, FP8K_F16, FP8K_F32, false>), dim3(nwg, (unsigned)batch), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((gemm_tile128_kernel<kModeRow, FP8K_F16, FP8K_F32, false, 128>), dim3(nwg, (unsigned)batch), dim3(512), 0, st, a);
   return check_launch(op);
 }
 

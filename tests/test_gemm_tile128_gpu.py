@@ -127,3 +127,44 @@ def test_automatic_plan_matches_pinned_kernels(dev):
             assert _rel_err(auto, other) <= REL_TOL
     finally:
         lib.fp8k_tune_force_gemm_plan(-1, 0)
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("M,N,kb", [(1, 128, 1), (64, 136, 2), (65, 520, 4), (130, 264, 5), (100, 392, 7), (257, 128, 9), (63, 1032, 14)])
+def test_tiles_of_64_activation_rows_exact(dev, tile128, M, N, kb, splits):
+    """The half-height tiles on integers with power-of-two scales: every remainder of the four K blocks whose scales come together,
+    with and without a K cut that starts inside such a group; float scales in both layouts, then row scales with a bias."""
+    from sglang_amd.sgl_kernel import fp8_scaled_mm
+
+    K = kb * 128
+    rng = np.random.default_rng(M * kb)
+    xq, wq = (O.f32_to_e4m3fn(rng.integers(-4, 5, (n, K)).astype(np.float32)) for n in (M, N))
+    xs = (2.0 ** rng.integers(-3, 4, (M, kb))).astype(np.float32)
+    ws = (2.0 ** rng.integers(-3, 4, ((N + 127) // 128, kb))).astype(np.float32)
+    ref = O.w8a8_block_fp8_matmul(xq, wq, xs, ws, out_dtype="bf16", acc=np.float64)
+    tile128(256 + splits)
+    for col_major in (False, True):
+        np.testing.assert_array_equal(_run_block(xq, xs, wq, ws, dev, col_major_as=col_major), ref)
+    sa, sb = ((2.0 ** rng.integers(-3, 3, (n,))).astype(np.float32) for n in (M, N))
+    bias = rng.integers(-8, 9, (N,)).astype(np.float32)
+    got = fp8_scaled_mm(fp8_tensor(xq, dev), fp8_tensor(wq, dev).t(), torch.from_numpy(sa).to(dev), torch.from_numpy(sb).to(dev),
+                        torch.bfloat16, torch.from_numpy(bias).to(dev)).float().cpu().numpy()
+    np.testing.assert_array_equal(got, O.fp8_scaled_mm(xq, wq, sa, sb, out_dtype="bf16", bias=bias))
+
+
+@pytest.mark.parametrize("splits", [1, 2])
+@pytest.mark.parametrize("M,N,K", [(129, 256, 256), (300, 520, 1152)])
+def test_tiles_of_64_activation_rows_ue8m0(dev, tile128, M, N, K, splits):
+    """Packed UE8M0 exponents: a word holds those of four K blocks, and a K cut may start anywhere in it."""
+    from sglang_amd.fp8_kernel import sglang_per_token_group_quant_fp8, w8a8_block_fp8_matmul
+    from sglang_amd.sgl_kernel import mark_ue8m0
+
+    x = torch.from_numpy(O.make_activation(M, K, seed=M)).to(dev).to(torch.bfloat16)
+    wq, ws = O.block_quant_weight(O.make_weight(N, K, seed=N))
+    B, Bs = fp8_tensor(wq, dev), mark_ue8m0(torch.from_numpy(O.ceil_to_ue8m0(ws)).to(dev))
+    xq, xs = sglang_per_token_group_quant_fp8(x, 128, column_major_scales=True, scale_tma_aligned=True, scale_ue8m0=True)
+    tile128(splits)
+    a = w8a8_block_fp8_matmul(xq, B, xs, Bs, [128, 128], torch.bfloat16)
+    tile128(256 + splits)
+    b = w8a8_block_fp8_matmul(xq, B, xs, Bs, [128, 128], torch.bfloat16)
+    assert torch.equal(a, b)  # the same sums in the same order as the 128-row tiles, which the tests above hold against the oracle
