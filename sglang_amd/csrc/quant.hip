@@ -177,11 +177,15 @@ __global__ __launch_bounds__(256) void group_quant_kernel(const void* __restrict
   }
 }
 
-template <int DT, int GROUP, int KIND, bool FUSE = false, bool MASKED = false>
-static int launch_group_quant(const void* x, void* q, void* s, int64_t M, int64_t K, float eps, int64_t sm, int64_t sg,
-                              hipStream_t st, const int32_t* masked_m = nullptr, int m_max = 1, int64_t se = 0) {
+// Segments per wave: four keep enough bytes in flight to stream a large input; up to a wave per wave slot of the chip (8192 segments,
+// 4 M elements) what counts is that the latency of one segment, not of four, stands in front of the product.  Whole linears,
+// quantisation and product, us, four / one: 32 x 4096 x 4096 10.7 / 9.5, 64 x 4096 x 4096 13.5 / 12.6, 200 x 7168 x 2304 15.0 / 14.1,
+// 128 x 7168 x 16384 43.2 / 42.4, 1000 x 24576 x 1536 50.6 / 49.8; level above (2048 x 7168 x 2304 41.2 / 41.2).
+constexpr int64_t kFewSegments = 8192;
+template <int DT, int GROUP, int KIND, int SEG, bool FUSE, bool MASKED>
+static int launch_group_quant_seg(const void* x, void* q, void* s, int64_t M, int64_t K, float eps, int64_t sm, int64_t sg,
+                                  hipStream_t st, const int32_t* masked_m, int m_max, int64_t se) {
   constexpr int GPW = 64 / (GROUP / 8);
-  constexpr int SEG = 4;
   const int G = (int)(K / GROUP);
   const int nseg_row = (G + GPW - 1) / GPW;
   const int64_t total = M * nseg_row;
@@ -196,6 +200,15 @@ static int launch_group_quant(const void* x, void* q, void* s, int64_t M, int64_
     hipLaunchKernelGGL((group_quant_kernel<DT, GROUP, KIND, SEG, false, FUSE, MASKED>), grid, block, 0, st, x, (uint8_t*)q, s,
                        (int)M, G, K, nseg_row, eps, sm, sg, masked_m, m_max, se);
   return check_launch("group_quant");
+}
+template <int DT, int GROUP, int KIND, bool FUSE = false, bool MASKED = false>
+static int launch_group_quant(const void* x, void* q, void* s, int64_t M, int64_t K, float eps, int64_t sm, int64_t sg,
+                              hipStream_t st, const int32_t* masked_m = nullptr, int m_max = 1, int64_t se = 0) {
+  if constexpr (GROUP == 128 && DT != FP8K_F32 && !MASKED) {
+    if (M * ((K / GROUP + 3) / 4) <= kFewSegments)
+      return launch_group_quant_seg<DT, GROUP, KIND, 1, FUSE, MASKED>(x, q, s, M, K, eps, sm, sg, st, masked_m, m_max, se);
+  }
+  return launch_group_quant_seg<DT, GROUP, KIND, 4, FUSE, MASKED>(x, q, s, M, K, eps, sm, sg, st, masked_m, m_max, se);
 }
 
 template <int DT, int KIND>

@@ -59,6 +59,14 @@ def test_group_quant_sweep_4096(dev, seed, layout):
     _check(x, dev, 128, layout)
 
 
+@pytest.mark.parametrize("layout", _layouts())
+@pytest.mark.parametrize("M,K", [(8192, 512), (8193, 384), (2731, 1664), (911, 4224), (1171, 3456)])
+def test_group_quant_on_both_sides_of_the_segment_rule(dev, M, K, layout):
+    """Up to 8192 segments of 512 elements a wave takes one, above four: 8192 and 8193, and ragged last segments and rows above."""
+    x = O.make_activation(M, K, seed=M)
+    _check(x, dev, 128, layout)
+
+
 @pytest.mark.parametrize("layout", [(False, False, False), (True, False, False), (True, True, True)])
 @pytest.mark.parametrize("seed", [0, 1, 2, 3, 4])
 @pytest.mark.parametrize("M", [1, 64, 512])
