@@ -791,8 +791,12 @@ struct MoeItem {
   int tile_n;
   int expert;
 };
+// Tables of the launch that no kernel writes while it reads them, for scalar loads: in a kernel that also stores, the
+// compiler takes vector loads for them otherwise, and those return in order behind every weight load in flight.
+typedef const int32_t __attribute__((address_space(4)))* const_ints;
+__device__ __forceinline__ const_ints as_const_ints(const int32_t* p) { return (const_ints)(uintptr_t)p; }
 // blocks in use (a device-side count: the host sizes the grid for the worst case)
-__device__ __forceinline__ int moe_blocks_used(const GemmArgs& p) { return min(p.num_post_pad[0] / p.block_m, p.m_blocks); }
+__device__ __forceinline__ int moe_blocks_used(const GemmArgs& p) { return min(as_const_ints(p.num_post_pad)[0] / p.block_m, p.m_blocks); }
 __device__ __forceinline__ MoeItem moe_work_item(const GemmArgs& p, int bid, int used) {
   constexpr int kWin = 4;
   MoeItem it{-1, 0, -1};
@@ -805,7 +809,7 @@ __device__ __forceinline__ MoeItem moe_work_item(const GemmArgs& p, int bid, int
   const int w0 = pos & ~(kWin - 1);                   // first position of the window
   int e[kWin];
 #pragma unroll
-  for (int i = 0; i < kWin; ++i) e[i] = first_blk + w0 + i < end_blk ? p.expert_ids[first_blk + w0 + i] : -2 - i;
+  for (int i = 0; i < kWin; ++i) e[i] = first_blk + w0 + i < end_blk ? as_const_ints(p.expert_ids)[first_blk + w0 + i] : -2 - i;
   const int pi = pos - w0;
   int a = 0, b = kWin, ex = e[0];                     // group [a, b) of the window that holds position pi
 #pragma unroll

@@ -12,8 +12,13 @@
 //   (groups wm, wm + 2, wm + 4, wm + 6), so that a block that is half padding still loads both rows of waves evenly;
 //   2 x 4 MFMA tiles of 32x32 each (24 KB of LDS operands per 16 MFMAs); groups without real slots skip their MFMAs.
 //   A workgroup can walk several items: the two stage rings run on across items, the last two trips of an item
-//   request the first two weight blocks of the next one, and the item is written out through the stages its last
-//   block used while the next item's first blocks travel.
+//   request the first two weight blocks of the next one, and the item is written out through the activation stage of
+//   its last block (FUSE: that and the weight stage) while the next item's first blocks travel.  Between two items no
+//   load stands in front of the write-out: slot ids come with the last trip's scale loads or through the scalar cache,
+//   routed weights with the item's first trip, the next scales are under way, and weight block 2 follows the stores.
+//   With these as chained vector loads, each behind the weight blocks in flight, an item cost 3 - 4 us more.  Whole
+//   layers, us, before / after: 64 experts, 7168 x 256, top 4, 1600 tokens 199 / 186; 64 experts, 4096 x 512, top 4, 1600
+//   176 / 169; 256 experts, top 8, 7168 x 256, 1024 418 / 405, 7168 x 2048, 4096 2627 / 2599.
 // Load order inside a K block is scales, activations, weights, so that at the next barrier only the four
 // youngest weight loads of each wave may still be in flight (memory operations retire in order).
 #pragma once
@@ -80,9 +85,10 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
       }
     }
   };
+  const int used = moe_blocks_used(p);
   auto fetch_item = [&](int& jj) -> MoeItem {  // first item at or after jj that has a GEMM to do (or the end)
     for (;;) {
-      const MoeItem it = moe_work_item(p, jj * 8 + xcd);
+      const MoeItem it = moe_work_item(p, jj * 8 + xcd, used);
       if (it.mb < 0 || it.expert >= 0) return it;
       zero_fill(it);
       jj += jstep;
@@ -96,6 +102,8 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
   const rsrc_t rS = make_rsrc(p.sx, (uint32_t)(((xrows - 1) * p.sx_m + nkb) * 4));  // used by the paired loads only
   // through a buffer descriptor: a 32-bit lane offset and a uniform offset, no 64-bit address per lane and group
   const rsrc_t rSall = make_rsrc(p.sx, 0xFFFFFFFFu);
+  const rsrc_t rIds = make_rsrc(p.sorted_ids, (uint32_t)p.m_blocks * (uint32_t)(TM * 4));
+  const const_ints ids = as_const_ints(p.sorted_ids);
 
   // ---- global -> LDS: a wave load covers 8 rows (lane: row lane/8, 16-byte chunk lane%8, stored at chunk
   // position c ^ ((row>>1)&7)); whole offsets travel in the bounds-checked per-lane operand
@@ -143,53 +151,123 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
     const int rowsW = min(kTileN, p.N - nn);
     return make_rsrc(Wb + (int64_t)nn * p.ldw, (uint32_t)((rowsW - 1) * p.ldw + p.K));
   };
-  // Entering an item: its activation block 0 goes into its first activation stage (the weights of its blocks 0 and 1
+  // Scales.  PAIRS: sxp[ms] holds the activation scales of an even K block and the odd one after it, fetched with
+  // one 8-byte load every other trip; with row-major scales the rows of a block are gathered, so every lane's load is
+  // a cache line of its own whatever the layout, and what counts is the number of load instructions and that a
+  // row's line is met again on the following trips.  Otherwise sxn[ms] / sbn hold the scales of the NEXT K block,
+  // requested one trip ahead in front of that trip's stage loads: at the next barrier everything older than the
+  // four youngest weight loads has landed, the scales among it.  SORTED: the last trip of an item has no next block, and
+  // its loads fetch the block's slot ids for the write-out in place of scales (same lanes, same groups).
+  constexpr bool pairs = PAIRS;
+  v2f sxp[MS];
+  float sxn[MS], sbn = 0.f;
+  float sba = 0.f, sbb = 0.f;  // PAIRS: weight scales of the even / odd block in flight
+  uint32_t sxo[MS];            // element offsets into the activation scales (the host checks they fit 32 bits); SORTED: byte offset of the lane's row, [0] only
+  int nact = 0;                // the wave's 32-slot groups (wm, wm + 2, wm + 4, wm + 6) that hold real slots: a prefix, real slots come first
+  const float* swp = nullptr;
+  int idp[2] = {0, 0};         // SORTED, not FUSE: slot ids of the groups h and 2 + h (h: half of the wave), for the routed weights
+  auto load_sb = [&](float& sb, int kb) { sb = swp[(int64_t)min(kb, nkb - 1) * p.sw_k]; };
+  auto load_sx = [&](int kb) {
+    if constexpr (SORTED) {
+      const bool last = kb >= nkb;
+      const rsrc_t r = last ? rIds : rSall;
+      const uint32_t step = last ? 1u : (uint32_t)p.sx_m;
+      const uint32_t row0 = (uint32_t)(slot0 + wm * 32) * step + (last ? 0u : (uint32_t)kb * (uint32_t)p.sx_k);
+      const uint32_t vo = sxo[0] * step;
+#pragma unroll
+      for (int ms = 0; ms < MS; ++ms)
+        sxn[ms] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)vo, (int)((row0 + (uint32_t)ms * 64u * step) * 4u), 0));
+    } else {
+      const uint32_t ko = (uint32_t)(min(kb, nkb - 1) * (int)p.sx_k);
+#pragma unroll
+      for (int ms = 0; ms < MS; ++ms)
+        sxn[ms] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rSall, (int)(sxo[ms] * 4u), (int)(ko * 4u), 0));
+    }
+  };
+  auto load_sx_pair = [&](int kb) {  // kb even: blocks kb and kb+1 (past the tensor: zero)
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms)
+      sxp[ms] = __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(rS, (int)((sxo[ms] + (uint32_t)kb) * 4u), 0, 0));
+  };
+  // Entering an item: its first scales and its activation block 0 are requested (the weights of its blocks 0 and 1
   // were requested in the last two trips of the item before it, or below for a workgroup's first item).  For every
-  // item but the first this runs in front of the previous item's write-out, which keeps to the weight and
-  // activation stages that item used last - the ones no request in flight points at.  The lane id is taken anew
-  // (from the execution mask): lane-derived values that stayed live across the K loops would be parked in scratch
-  // and reloaded inside them, and scratch reloads count against the partial vmcnt waits.
-  auto start_item = [&](const MoeItem& it, bool first) {
+  // item but the first this runs in front of the previous item's write-out, which keeps to the stages that item used
+  // last - the ones no request in flight points at.  Vector loads return in order, so a vector load here arrives behind
+  // the weight blocks in flight, a full memory latency later, and each one that depends on another adds a round trip to
+  // the time in which the weight stream stands still: the slot ids come through the scalar cache, and nothing here waits
+  // for a vector load (SORTED).  The lane id is taken anew (from the execution mask): lane-derived values that stayed
+  // live across the K loops would be parked in scratch and reloaded inside them, and scratch reloads count against the
+  // partial vmcnt waits.
+  auto enter = [&](const MoeItem& it) {
     int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     asm volatile("" : "+v"(ln));
-    const int rl = ln >> 3, cp = ln & 7;
+    const int rl = ln >> 3, cp = ln & 7, lr = ln & 31, h = ln >> 5;
     slot0 = it.mb * TM;
     n0 = it.tile_n * (FUSE ? 128 : kTileN);
     expert = it.expert;
-    // slot table first, weights behind it: loads retire in order, so the table arrives without waiting for the
-    // weights, and the weights do not wait for the table
-    int sid[LW];
+    // the wave's 64 weight rows lie inside one 128-row block (FUSE: gate rows for wn 0, 1, up rows for wn 2, 3)
+    const int nb = FUSE ? ((wn < 2 ? n0 : half_n + n0) >> 7) : (min(n0 + wn * 64, p.N - 1) >> 7);
+    swp = p.sw + (int64_t)expert * p.sw_expert_stride + (int64_t)nb * p.sw_n;
+    nact = 0;
 #pragma unroll
-    for (int q = 0; q < LW; ++q) sid[q] = p.sorted_ids[slot0 + (w * LW + q) * 8 + rl];
-    if (first) {
-      // the wave's 8-row groups g = 4w + q: groups q and q + 2 differ by 16 rows and share the chunk swizzle, so two
-      // lane offsets serve the four weight loads (the 16-row step is uniform and joins the K offset)
+    for (int ms = 0; ms < MS; ++ms) nact += ids[slot0 + (ms * 2 + wm) * 32] < nrows ? 1 : 0;
+    if constexpr (SORTED) {
+      sxo[0] = (uint32_t)lr * 4u;
+      load_sx(0);
+      load_sb(sbn, 0);
+      if constexpr (!FUSE) {
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int g = w * LW + q;  // 8-row group, 0..31, of both tiles
-        const int c = cp ^ (((g & 1) << 2) + (rl >> 1));
-        voW[q] = (uint32_t)((g * 8 + rl) * p.ldw + c * 16);
+        for (int i = 0; i < 2; ++i)
+          idp[i] = __builtin_amdgcn_raw_buffer_load_b32(rIds, (h * 64 + lr) * 4, (slot0 + wm * 32 + i * 128) * 4, 0);
       }
-      w16 = (uint32_t)(16 * p.ldw);
-      rW = weights_of(it);
-      __builtin_amdgcn_sched_barrier(0);
-      issue_w(rW, 0, 0);
-      issue_w(rW, 1, 1);
-      __builtin_amdgcn_sched_barrier(0);
     }
+    xreal = ids[slot0 + w * (LW * 8)] < nrows;  // the first row of the wave's first group: a prefix
 #pragma unroll
     for (int q = 0; q < LW; ++q) {
-      const int g = w * LW + q;
+      const int g = w * LW + q;  // 8-row group, 0..31
       const int c = cp ^ (((g & 1) << 2) + (rl >> 1));
-      const int sd = sid[q];
+      int sd = ids[slot0 + g * 8];
+#pragma unroll
+      for (int r = 1; r < 8; ++r) {
+        const int s = ids[slot0 + g * 8 + r];
+        sd = rl == r ? s : sd;
+      }
       voX[q] = sd < nrows ? (uint32_t)((int64_t)(sd / p.top_k) * p.ldx + c * 16) : 0xF0000000u;  // padding reads zeros
     }
-    xreal = __builtin_amdgcn_ballot_w64(sid[0] < nrows) != 0;  // the first row of the wave's first group: a prefix
     issue_x(0, gx0);
   };
-  start_item(item, true);
+  // Whether weight block 2 of an item is requested behind the write-out in front of it (its stage is free by then), not
+  // in the item's first trip.
+  // (Asked anew from the scalar nkb at each place: as one value across the K loops it is parked in scratch.)
+  auto early = [&]() -> bool {
+    int n = nkb;
+    asm volatile("" : "+s"(n));
+    return SORTED && !FUSE && n >= 3;
+  };
+  {
+    int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(ln));
+    const int rl = ln >> 3, cp = ln & 7;
+    // the wave's 8-row groups g = 4w + q: groups q and q + 2 differ by 16 rows and share the chunk swizzle, so two
+    // lane offsets serve the four weight loads (the 16-row step is uniform and joins the K offset)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int g = w * LW + q;  // 8-row group, 0..31, of both tiles
+      const int c = cp ^ (((g & 1) << 2) + (rl >> 1));
+      voW[q] = (uint32_t)((g * 8 + rl) * p.ldw + c * 16);
+    }
+    w16 = (uint32_t)(16 * p.ldw);
+  }
+  rW = weights_of(item);
+  issue_w(rW, 0, 0);
+  issue_w(rW, 1, 1);
+  enter(item);
+  __builtin_amdgcn_sched_barrier(0);
+  if (early()) issue_w(rW, 2, 2);
+  __builtin_amdgcn_sched_barrier(0);
 
   for (;;) {
+    asm volatile("" : "+v"(voW[0]), "+v"(voW[1]));  // sums with them stay out of the way of the K loops' registers
     int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     asm volatile("" : "+v"(ln));
     const int lr = ln & 31, h = ln >> 5;
@@ -212,21 +290,6 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
       return r;
     };
 
-    // ---- scales: activation scale rows follow the activation rows
-    uint32_t sxo[MS];  // element offsets into the activation scales (the host checks they fit 32 bits)
-    int nact = 0;      // the wave's 32-slot groups (wm, wm + 2, wm + 4, wm + 6) that hold real slots: a prefix, real slots come first
-#pragma unroll
-    for (int ms = 0; ms < MS; ++ms) {
-      const int s = p.sorted_ids[slot0 + (ms * 2 + wm) * 32 + lr];
-      nact += __builtin_amdgcn_readfirstlane(s) < nrows ? 1 : 0;
-      sxo[ms] = SORTED ? (uint32_t)((int64_t)(slot0 + wm * 32 + lr) * p.sx_m)  // + ms * 64 rows, added as a uniform
-                       : (s < nrows ? (uint32_t)((int64_t)(s / p.top_k) * p.sx_m) : 0u);
-    }
-    const uint32_t sx32 = SORTED ? (uint32_t)(64 * p.sx_m) : 0u;  // step between the scale rows of two of the wave's groups
-    // the wave's 64 weight rows lie inside one 128-row block (FUSE: gate rows for wn 0, 1, up rows for wn 2, 3)
-    const int nb = FUSE ? ((wn < 2 ? n0 : half_n + n0) >> 7) : (min(n0 + wn * 64, p.N - 1) >> 7);
-    const float* swp = p.sw + (int64_t)expert * p.sw_expert_stride + (int64_t)nb * p.sw_n;
-
     v16f acc[NS][MS];
 #pragma unroll
     for (int ns = 0; ns < NS; ++ns)
@@ -235,36 +298,32 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[ns][ms][r] = 0.f;
 
-    // Scales.  PAIRS: sxp[ms] holds the activation scales of an even K block and the odd one after it, fetched with
-    // one 8-byte load every other trip; with row-major scales the rows of a block are gathered, so every lane's load is
-    // a cache line of its own whatever the layout, and what counts is the number of load instructions and that a
-    // row's line is met again on the following trips.  Otherwise sxn[ms] / sbn hold the scales of the NEXT K block,
-    // requested one trip ahead in front of that trip's stage loads: at the next barrier everything older than the
-    // four youngest weight loads has landed, the scales among it.
-    constexpr bool pairs = PAIRS;
-    v2f sxp[MS];
-    float sxn[MS], sbn = 0.f;
-    float sba = 0.f, sbb = 0.f;  // PAIRS: weight scales of the even / odd block in flight
-    auto load_sb = [&](float& sb, int kb) { sb = swp[(int64_t)min(kb, nkb - 1) * p.sw_k]; };
-    auto load_sx = [&](int kb) {
-      const uint32_t ko = (uint32_t)(min(kb, nkb - 1) * (int)p.sx_k);
+    if constexpr (!SORTED) {  // activation scale rows follow the activation rows
 #pragma unroll
-      for (int ms = 0; ms < MS; ++ms)
-        sxn[ms] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rSall, (int)(sxo[SORTED ? 0 : ms] * 4u),
-                                                                                (int)((ko + (uint32_t)ms * sx32) * 4u), 0));
-    };
-    auto load_sx_pair = [&](int kb) {  // kb even: blocks kb and kb+1 (past the tensor: zero)
-#pragma unroll
-      for (int ms = 0; ms < MS; ++ms)
-        sxp[ms] = __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(rS, (int)((sxo[ms] + (uint32_t)kb) * 4u), 0, 0));
-    };
-    if (pairs) { load_sx_pair(0); load_sb(sba, 0); load_sb(sbb, 1); }
-    else { load_sx(0); load_sb(sbn, 0); }
+      for (int ms = 0; ms < MS; ++ms) {
+        const int s = p.sorted_ids[slot0 + (ms * 2 + wm) * 32 + lr];
+        sxo[ms] = s < nrows ? (uint32_t)((int64_t)(s / p.top_k) * p.sx_m) : 0u;
+      }
+      if (pairs) { load_sx_pair(0); load_sb(sba, 0); load_sb(sbb, 1); }
+      else { load_sx(0); load_sb(sbn, 0); }
+    }
     // the item after this one, looked up while the first blocks arrive
     int jn = j + jstep;
     const MoeItem next = fetch_item(jn);
     rWn = weights_of(next);
-    wait_vm0();  // the first trip's partial wait assumes the in-loop order of loads; the previous item's stores are out
+    // the first trip's partial wait counts on four weight loads as the youngest requests
+    if (!early()) wait_vm0();
+    float rsp[2] = {1.f, 1.f};  // SORTED, not FUSE: routed weights of the groups h and 2 + h; requested in the first trip
+    auto load_rs = [&]() {
+      if constexpr (SORTED && !FUSE) {
+        const float* tw = p.topk_w;
+        asm volatile("" : "+s"(tw));
+        if (tw) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) rsp[i] = tw[min(idp[i], nrows - 1)];  // padding slots are never stored
+        }
+      }
+    };
 
     // one K block; its scales sit in sxp[.][parity] and sb on entry; the odd trips reload both blocks' activation
     // scales in the paired form
@@ -389,7 +448,8 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
       int ex[MS], ew = 127;      // exponent bytes of the block in work
       int exd = 127, ewd = 127;  // ... of the deferred group
       // barrier of trip `it`, the exponents of its block, the next scales and the stage loads
-      auto open = [&](int it) {
+      auto open = [&](int it, auto first_c) {
+        constexpr bool FIRST = decltype(first_c)::value;
         lds_barrier<LW>();  // everything but the wave's loads of weight block it+1 has landed
         SB();
 #pragma unroll
@@ -397,11 +457,12 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
         ew = (int)(__float_as_uint(sbn) >> 23);
         load_sx(it + 1);
         load_sb(sbn, it + 1);
+        if constexpr (FIRST) load_rs();
         SB();  // scales, then activations, then weights
         issue_x(it + 1, (gx0 + it + 1) & 1);
         const int k2 = it + 2;
         const bool nx = k2 >= nkb;
-        issue_w(nx ? rWn : rW, nx ? k2 - nkb : k2, (gw0 + k2) % WST);
+        if (!FIRST || !early()) issue_w(nx ? rWn : rW, nx ? k2 - nkb : k2, (gw0 + k2) % WST);
         SB();
       };
       // the last group of the previous block (fragments xa / xb, exponents exd / ewd); REFILL: the fragments of block
@@ -441,7 +502,7 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
         exd = ex[NA > 0 ? NA - 1 : 0];
         ewd = ew;
       };
-      open(0);
+      open(0, yes{});
       if constexpr (NA > 0) {
         const uint8_t* sw_ = smem + (gw0 % WST) * WBYTES;
         const uint8_t* sx_ = smem + XBASE + (gx0 & 1) * XBYTES;
@@ -455,8 +516,9 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
         SB();
         groups(sx_);
       }
+      if (early()) wait_vm0();  // weight block 2 is older than activation block 1
       auto trip = [&](int it) {
-        open(it);
+        open(it, no{});
         if constexpr (NA > 0) {
           const uint8_t* sw_ = smem + ((gw0 + it) % WST) * WBYTES;
           const uint8_t* sx_ = smem + XBASE + ((gx0 + it) & 1) * XBYTES;
@@ -506,7 +568,8 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
           issue_w1(i - 4, nx ? rWn : rW, nx ? k2 - nkb : k2, (gw0 + k2) % WST);
         }
       };
-      auto open = [&](int it, auto all_loads) {
+      auto open = [&](int it, auto all_loads, auto first_c) {
+        constexpr bool FIRST = decltype(first_c)::value;
         lds_barrier<LW>();  // everything but the wave's loads of weight block it+1 has landed
         SB();
         sd0 = sc[L2];
@@ -515,11 +578,16 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
         for (int ms = 0; ms < MS; ++ms) sc[ms] = sxn[ms] * sbn;
         load_sx(it + 1);
         load_sb(sbn, it + 1);
+        if constexpr (FIRST) load_rs();
         SB();  // scales, then activations, then weights
         ld_it = it;
         if constexpr (decltype(all_loads)::value) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) ld(i);
+          for (int i = 0; i < 4; ++i) ld(i);
+          if (!FIRST || !early()) {
+#pragma unroll
+            for (int i = 4; i < 8; ++i) ld(i);
+          }
         }
         SB();
       };
@@ -571,7 +639,7 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
         if constexpr (NA >= 3) step(yes{}, std::integral_constant<int, 0>{}, sc[0], fill_x{}, smem, sx_ + ((2 * 2 + wm) * 32) * kTileK);
         if constexpr (NA >= 4) step(yes{}, std::integral_constant<int, 1>{}, sc[1], fill_x{}, smem, sx_ + ((3 * 2 + wm) * 32) * kTileK);
       };
-      open(0, yes{});
+      open(0, yes{}, yes{});
       if constexpr (NA > 0) {
         const uint8_t* sw_ = smem + (gw0 % WST) * WBYTES;
         const uint8_t* sx_ = smem + XBASE + (gx0 & 1) * XBYTES;
@@ -585,8 +653,9 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
         SB();
         groups(yes{}, sx_);
       }
+      if (early()) wait_vm0();  // weight block 2 is older than activation block 1
       for (int it = 1; it < nkb; ++it) {
-        open(it, std::integral_constant<bool, NA == 0>{});
+        open(it, std::integral_constant<bool, NA == 0>{}, no{});
         if constexpr (NA > 0) {
           const uint8_t* sw_ = smem + ((gw0 + it) % WST) * WBYTES;
           const uint8_t* sx_ = smem + XBASE + ((gx0 + it) & 1) * XBYTES;
@@ -645,21 +714,31 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
         default: run(std::integral_constant<int, 0>{}); break;
       }
     }
-    // output rows and routed weights, fetched while the stages drain (lane id taken anew, as above)
+    // output rows and routed weights (lane id taken anew, as above)
     const bool wide = (p.ldc & 7) == 0 && (reinterpret_cast<uintptr_t>(p.C) & 15) == 0;
     int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     asm volatile("" : "+v"(lane_e));
     const int lr_e = lane_e & 31, h_e = lane_e >> 5;
     const int er = lane_e >> 3, ec = lane_e & 7;  // store loop: row inside a group of 8, 16-byte chunk of the wave's 128 bytes
-    const int eslot0 = slot0, en0 = n0;
-    int oslots[MS], srow[16];
+    const int eslot0 = slot0, en0 = n0, enact = nact;
+    int oslots[MS];
     float rsw[MS];
+    if constexpr (SORTED) {
 #pragma unroll
-    for (int ms = 0; ms < MS; ++ms) oslots[ms] = p.sorted_ids[eslot0 + (ms * 2 + wm) * 32 + lr_e];
+      for (int ms = 0; ms < MS; ++ms) oslots[ms] = __builtin_bit_cast(int, sxn[ms]);  // what the last trip fetched
 #pragma unroll
-    for (int i = 0; i < 16; ++i) srow[i] = (wide && !FUSE) ? p.sorted_ids[eslot0 + ((i >> 2) * 2 + wm) * 32 + (i & 3) * 8 + er] : 0;
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t v = __builtin_bit_cast(uint32_t, rsp[i]);
+        const auto halves = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        rsw[2 * i] = __builtin_bit_cast(float, (uint32_t)halves[0]);
+        rsw[2 * i + 1] = __builtin_bit_cast(float, (uint32_t)halves[1]);
+      }
+    } else {
 #pragma unroll
-    for (int ms = 0; ms < MS; ++ms) rsw[ms] = (p.topk_w && oslots[ms] < nrows) ? p.topk_w[oslots[ms]] : 1.f;
+      for (int ms = 0; ms < MS; ++ms) oslots[ms] = p.sorted_ids[eslot0 + (ms * 2 + wm) * 32 + lr_e];
+#pragma unroll
+      for (int ms = 0; ms < MS; ++ms) rsw[ms] = (p.topk_w && oslots[ms] < nrows) ? p.topk_w[oslots[ms]] : 1.f;
+    }
     lds_barrier();  // every wave has left the item's last stages; the requests in flight point at the other ones
     const int ews = (gw0 + nkb - 1) % WST, exs = (gx0 + nkb - 1) & 1;  // the stages of the item's last block
     gw0 = (gw0 + nkb) % WST;
@@ -667,7 +746,7 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
     const bool has_next = next.mb >= 0;
     if (has_next) {
       rW = rWn;
-      start_item(next, false);  // its first activation block travels while this item is written out
+      enter(next);  // its scales and its first activation block travel while this item is written out
     }
 
     if constexpr (FUSE) {
@@ -703,7 +782,7 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
 #pragma unroll
         for (int it4 = 0; it4 < 4; ++it4) {
           const int r = it4 * 16 + (lane_e >> 2);
-          qrow[it4] = p.sorted_ids[eslot0 + ((MINE + 2 * (r >> 5)) * 2 + wm) * 32 + (r & 31)];
+          qrow[it4] = __builtin_amdgcn_ds_bpermute((r & 31) * 4, oslots[MINE + 2 * (it4 >> 1)]);
         }
         // a group holds real slots iff its first slot is real (wave-uniform)
         bool real_mine[2], real_send[2];
@@ -805,51 +884,44 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
       continue;
     }
 
-    // ---- write-out through LDS, in two passes of 64 slots.  A wave re-lays 64 slots x 64 n of its block out in a
-    // private 8 KB slot inside the weight / activation stage of the item's last block (128 B per row, 16-byte chunk c
-    // of row r at position c ^ ((r >> 1) & 7), so that the accumulator-shaped 8-byte writes and the 16-byte reads
-    // spread over all banks): no workgroup barrier, and every store instruction writes eight whole 128-byte lines.
-    uint8_t* const ep = smem + (w < 4 ? ews * WBYTES + w * 8192 : XBASE + exs * XBYTES + (w - 4) * 8192);
+    // ---- write-out through LDS, in passes of 32 slots.  A wave re-lays 32 slots x 64 n of its block out in a private 4 KB
+    // of the activation stage of the item's last block (128 B per row, 16-byte chunk c of row r at position
+    // c ^ ((r >> 1) & 7), so that the accumulator-shaped 8-byte writes and the 16-byte reads spread over all banks): no
+    // workgroup barrier, every store instruction writes eight whole 128-byte lines, and the weight stage is left alone.
+    uint8_t* const ep = smem + XBASE + exs * XBYTES + w * 4096;
 #pragma unroll
-    for (int ph = 0; ph < 2; ++ph) {
-      if (ph * 2 >= nact) break;  // the wave's remaining slot groups are all padding (real slots come first): nothing to store
+    for (int ms = 0; ms < MS; ++ms) {
+      if (ms >= enact) break;  // the wave's remaining slot groups are all padding (real slots come first): nothing to store
+      const int oslot = oslots[ms];
+      const bool ok = oslot < nrows;
+      const float rs = rsw[ms];
 #pragma unroll
-      for (int mh = 0; mh < 2; ++mh) {
-        const int ms = ph * 2 + mh;
-        if (ms >= nact) continue;
-        const int row = mh * 32 + lr_e;  // inside the pass's 64 slots
-        const int oslot = oslots[ms];
-        const bool ok = oslot < nrows;
-        const float rs = rsw[ms];
+      for (int nr = 0; nr < NS * 4; ++nr) {
+        const int ns = nr >> 2, rg = nr & 3;
+        float v[4];
 #pragma unroll
-        for (int nr = 0; nr < NS * 4; ++nr) {
-          const int ns = nr >> 2, rg = nr & 3;
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = acc[ns][ms][rg * 4 + r] * rs;
-          if (wide) {
-            uint2 o;
-            if (OUT_DT == FP8K_BF16) {
-              o.x = pack_bf16x2(v[0], v[1]);
-              o.y = pack_bf16x2(v[2], v[3]);
-            } else {
-              o.x = f32_to_f16_bits(v[0]) | (f32_to_f16_bits(v[1]) << 16);
-              o.y = f32_to_f16_bits(v[2]) | (f32_to_f16_bits(v[3]) << 16);
-            }
-            *reinterpret_cast<uint2*>(ep + row * 128 + ((nr ^ ((row >> 1) & 7)) << 4) + h_e * 8) = o;
+        for (int r = 0; r < 4; ++r) v[r] = acc[ns][ms][rg * 4 + r] * rs;
+        if (wide) {
+          uint2 o;
+          if (OUT_DT == FP8K_BF16) {
+            o.x = pack_bf16x2(v[0], v[1]);
+            o.y = pack_bf16x2(v[2], v[3]);
           } else {
-            const int n = en0 + wn * 64 + nr * 8 + h_e * 4;
-            if (ok && n < p.N) store4<OUT_DT>(p.C, (int64_t)oslot * p.ldc + n, v[0], v[1], v[2], v[3]);
+            o.x = f32_to_f16_bits(v[0]) | (f32_to_f16_bits(v[1]) << 16);
+            o.y = f32_to_f16_bits(v[2]) | (f32_to_f16_bits(v[3]) << 16);
           }
+          *reinterpret_cast<uint2*>(ep + lr_e * 128 + ((nr ^ ((lr_e >> 1) & 7)) << 4) + h_e * 8) = o;
+        } else {
+          const int n = en0 + wn * 64 + nr * 8 + h_e * 4;
+          if (ok && n < p.N) store4<OUT_DT>(p.C, (int64_t)oslot * p.ldc + n, v[0], v[1], v[2], v[3]);
         }
       }
       if (wide) {
         __builtin_amdgcn_wave_barrier();  // one wave's LDS accesses complete in order: no wait needed
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if (ph * 2 + (i >> 2) >= nact) continue;
+        for (int i = 0; i < 4; ++i) {
           const int row = i * 8 + er;
-          const int s = srow[ph * 8 + i];
+          const int s = __builtin_amdgcn_ds_bpermute(row * 4, oslot);
           const int n = en0 + wn * 64 + (ec << 3);
           const uint4 o = *reinterpret_cast<const uint4*>(ep + row * 128 + ((ec ^ ((row >> 1) & 7)) << 4));
           if (s < nrows && n < p.N) *reinterpret_cast<uint4*>((u16*)p.C + (int64_t)s * p.ldc + n) = o;
@@ -861,6 +933,9 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
       wait_vm0();  // the out-of-range requests of the last trips still point at the stages: let them retire before the LDS goes back
       return;
     }
+    __builtin_amdgcn_sched_barrier(0);
+    if (early()) issue_w(rW, 2, ews);  // the youngest requests in front of the first trip's barrier
+    __builtin_amdgcn_sched_barrier(0);
     item = next;
     j = jn;
   }

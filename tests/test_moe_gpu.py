@@ -411,6 +411,43 @@ def test_grouped_gemm_256_slot_blocks_every_group_count(dev):
             assert torch.equal(outs[0], C)
 
 
+@pytest.mark.parametrize("T,E,topk,N,K,pow2", [(900, 40, 6, 2568, 128, False), (900, 40, 6, 2568, 256, False), (700, 24, 5, 4616, 384, False),
+                                               (700, 24, 5, 4616, 512, True), (1500, 8, 2, 8712, 640, False), (1500, 8, 2, 8712, 384, True)])
+def test_grouped_gemm_walks_of_256_slot_blocks_exact(dev, T, E, topk, N, K, pow2):
+    """More tiles than workgroups, so that the entry into an item runs beside the write-out of the one before it: one to five K
+    blocks, partly filled and absent blocks, a last tile of 8 weight rows, up to and above 192 slots per expert, activation scales
+    with and without a row stride of one, routed weights on and off; exact on integer data with power-of-two scales."""
+    from sglang_amd.fused_moe import moe_align_block_size
+    from sglang_amd.sgl_kernel import moe_balance_blocks, moe_block_gemm, moe_sort_scales
+
+    g = torch.Generator().manual_seed(K + T)
+    powers = lambda *s: 2.0 ** torch.randint(-3, 3, s, generator=g).float()  # noqa: E731
+    x, w = (torch.randint(-4, 5, s, generator=g).float() for s in ((T, K), (E, N, K)))
+    xs, ws = powers(T, K // 128), powers(E, (N + 127) // 128, K // 128)
+    ids = torch.rand((T, E), generator=g).argsort(dim=1)[:, :topk].int()
+    ids[: T // 3, 0] = 1                   # one expert with more than a block
+    ids[ids == 2] = -1                     # an expert of another rank
+    tw = powers(T, topk)
+    slots = ids.numel()
+    sorted_ids, expert_ids, npad = moe_align_block_size(ids.to(dev), 256, E)
+    balanced = slots > 192 * E
+    if balanced:
+        sorted_ids = moe_balance_blocks(sorted_ids, expert_ids, npad, 256, slots, E)
+    A, B, wsd, twd = x.to(dev).to(torch.float8_e4m3fn), w.to(dev).to(torch.float8_e4m3fn), ws.to(dev), tw.to(dev)
+    sorted_scales = moe_sort_scales(xs.to(dev), sorted_ids, npad, topk, slots)
+    want = torch.zeros((slots, N))
+    for e in range(E):
+        at = (ids.flatten() == e).nonzero().flatten()
+        rows = x[at // topk] * xs[at // topk].repeat_interleave(128, 1)
+        want[at] = rows @ (w[e] * ws[e].repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)).t()
+    for sc, weigh in ((sorted_scales, True), (sorted_scales, False), (sorted_scales.contiguous(), True)):
+        C = torch.full((slots, N), float("nan"), dtype=torch.bfloat16, device=dev)
+        moe_block_gemm(A, B, C, sc, wsd, twd, sorted_ids, expert_ids, npad, weigh, topk, 256, slots, scales_sorted=True,
+                       pow2_scales=pow2, balanced=balanced)
+        ref = want * tw.flatten()[:, None] if weigh else want
+        assert torch.equal(C.float().cpu(), ref.bfloat16().float())
+
+
 @pytest.mark.parametrize("T,E,topk,N,K,block", [(64, 40, 2, 2056, 128, 16), (70, 24, 3, 3080, 384, 16), (33, 40, 1, 2048, 1024, 16),
                                                 (90, 64, 4, 1160, 640, 32), (200, 8, 4, 2568, 2048, 32), (200, 8, 4, 2568, 1280, 32), (64, 40, 2, 2056, 512, 16),
                                                 (130, 96, 6, 1032, 256, 32)])
