@@ -271,8 +271,9 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00020000);
 }
 // 16 bytes per lane from buffer + voff (per lane) + soff (uniform) straight into LDS at lds_base + lane*16
+template <bool NT = false>  // NT: non-temporal, for bytes that one workgroup reads once
 __device__ __forceinline__ void buf_load16_to_lds(rsrc_t r, uint32_t voff, uint32_t soff, uint8_t* lds_base) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds_base, 16, (int)voff, (int)soff, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds_base, 16, (int)voff, (int)soff, 0, NT ? 2 : 0);
 }
 // 4 bytes per lane into LDS at lds_base + lane*4 (inactive lanes write nothing)
 __device__ __forceinline__ void buf_load4_to_lds(rsrc_t r, uint32_t voff, uint32_t soff, uint8_t* lds_base) {

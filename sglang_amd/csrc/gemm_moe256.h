@@ -42,10 +42,16 @@ namespace fp8k {
 // SCALED (sorted scales only): both scale tensors hold powers of two (UE8M0 checkpoints with UE8M0-rounded activation
 // scales) and the matrix core applies them itself (v_mfma_scale_f32_32x32x64_f8f6f4 takes the two exponent bytes):
 // the products accumulate in place, the float promote and its second accumulator disappear.
-template <int OUT_DT, bool PAIRS, bool SORTED, bool FUSE = false, bool SCALED = false>
+// ONCE (sorted scales only): the host expects one block per expert, so that no other workgroup reads an item's weight tile.
+// The weights are then loaded non-temporally, and leave the L2 to the activation rows, which every n tile of the block reads
+// again; the result rows too are stored past it.  Whole layers, us, plain / ONCE: 256 experts, 7168 x 2048, top 8: 1024 tokens
+// 2105 / 1959, 4096 2622 / 2565; 7168 x 512: 1024 641 / 611, 3200 821 / 785; 64 experts, 7168 x 256, top 4, 1600 tokens
+// 187 / 184.  With several blocks per expert they share the tile in L2: 64 experts, 7168 x 2048, top 8, 2400 tokens 1248 / 1271.
+template <int OUT_DT, bool PAIRS, bool SORTED, bool FUSE = false, bool SCALED = false, bool ONCE = false>
 __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p) {
   static_assert(!FUSE || (SORTED && !PAIRS), "the fused write-out is built for sorted activation scales");
   static_assert(!SCALED || (SORTED && !PAIRS && !FUSE), "hardware scaling is built for sorted activation scales");
+  static_assert(!ONCE || SORTED, "built for sorted activation scales");
   constexpr int TM = 256, WST = 3, XST = 2, MS = 4, NS = 2, LW = 4;  // LW: wave loads per tile per stage
   constexpr int WBYTES = kTileN * kTileK, XBYTES = TM * kTileK;
   constexpr int XBASE = WST * WBYTES;
@@ -125,7 +131,7 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
     uint8_t* base = smem + stage * WBYTES + w * (LW * 1024);
     const uint32_t ko = (uint32_t)kblk * kTileK;
 #pragma unroll
-    for (int q = 0; q < LW; ++q) buf_load16_to_lds(r, voW[q & 1] + (ko + (q >> 1) * w16), wsoff, base + q * 1024);
+    for (int q = 0; q < LW; ++q) buf_load16_to_lds<ONCE>(r, voW[q & 1] + (ko + (q >> 1) * w16), wsoff, base + q * 1024);
   };
   auto issue_x = [&](int kblk, int stage) {
     uint8_t* base = smem + XBASE + stage * XBYTES + w * (LW * 1024);
@@ -135,7 +141,8 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
   };
   // the same, one wave load at a time (q = 0 .. LW-1)
   auto issue_w1 = [&](int q, const rsrc_t& r, int kblk, int stage) {
-    buf_load16_to_lds(r, voW[q & 1] + ((uint32_t)kblk * kTileK + (q >> 1) * w16), wsoff, smem + stage * WBYTES + w * (LW * 1024) + q * 1024);
+    buf_load16_to_lds<ONCE>(r, voW[q & 1] + ((uint32_t)kblk * kTileK + (q >> 1) * w16), wsoff,
+                            smem + stage * WBYTES + w * (LW * 1024) + q * 1024);
   };
   auto issue_x1 = [&](int q, int kblk, int stage) {
     buf_load16_to_lds(rX, voX[q] + (uint32_t)kblk * kTileK, 0, smem + XBASE + stage * XBYTES + w * (LW * 1024) + q * 1024);
@@ -923,8 +930,12 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
           const int row = i * 8 + er;
           const int s = __builtin_amdgcn_ds_bpermute(row * 4, oslot);
           const int n = en0 + wn * 64 + (ec << 3);
-          const uint4 o = *reinterpret_cast<const uint4*>(ep + row * 128 + ((ec ^ ((row >> 1) & 7)) << 4));
-          if (s < nrows && n < p.N) *reinterpret_cast<uint4*>((u16*)p.C + (int64_t)s * p.ldc + n) = o;
+          const v4i o = *reinterpret_cast<const v4i*>(ep + row * 128 + ((ec ^ ((row >> 1) & 7)) << 4));
+          if (s < nrows && n < p.N) {
+            v4i* const dst = reinterpret_cast<v4i*>((u16*)p.C + (int64_t)s * p.ldc + n);
+            if (ONCE) __builtin_nontemporal_store(o, dst);
+            else *dst = o;
+          }
         }
         __builtin_amdgcn_wave_barrier();
       }

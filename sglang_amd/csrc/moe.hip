@@ -526,8 +526,10 @@ extern "C" int fp8k_moe_sort_scales(const float* As, float* out, const int32_t* 
 
 // whether the 256-slot grouped kernel runs as one walking workgroup per CU (the walk hands the weight stream on two K
 // blocks ahead, so K must have them)
+// Up to 192 slots per expert on average most experts are one block of 256
+static bool moe256_once(int64_t num_valid_tokens, int64_t num_experts) { return num_valid_tokens <= num_experts * 192; }
 static bool moe256_walks(int64_t num_valid_tokens, int64_t num_experts, int64_t K, bool balanced) {
-  return (balanced || num_valid_tokens <= num_experts * 192) && K >= 2 * kTileK;
+  return (balanced || moe256_once(num_valid_tokens, num_experts)) && K >= 2 * kTileK;
 }
 
 // blocks that can be in use: every one holds a slot, and only an expert's last (or that of the slots without one) is not full
@@ -638,10 +640,13 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
     // row-major activation scales (what fused_experts_impl produces for 256-slot blocks) take the form that fetches
     // two K blocks per load
     const bool pairs = !as_sorted && as_stride_k == 1 && (as_stride_m & 1) == 0 && aligned(As, 8);  // 129..256 and more slots per expert: both 128-row halves on one weight stage
+    const bool once = moe256_once(num_valid_tokens, num_experts);
 #define FP8K_MOE256(O) \
   do { \
     if (pairs) hipLaunchKernelGGL((moe_stream256_kernel<O, true, false>), dim3((unsigned)nwg), dim3(512), 0, st, a); \
+    else if (as_sorted && pow2_scales && once) hipLaunchKernelGGL((moe_stream256_kernel<O, false, true, false, true, true>), dim3((unsigned)nwg), dim3(512), 0, st, a); \
     else if (as_sorted && pow2_scales) hipLaunchKernelGGL((moe_stream256_kernel<O, false, true, false, true>), dim3((unsigned)nwg), dim3(512), 0, st, a); \
+    else if (as_sorted && once) hipLaunchKernelGGL((moe_stream256_kernel<O, false, true, false, false, true>), dim3((unsigned)nwg), dim3(512), 0, st, a); \
     else if (as_sorted) hipLaunchKernelGGL((moe_stream256_kernel<O, false, true>), dim3((unsigned)nwg), dim3(512), 0, st, a); \
     else hipLaunchKernelGGL((moe_stream256_kernel<O, false, false>), dim3((unsigned)nwg), dim3(512), 0, st, a); \
   } while (0)
@@ -797,8 +802,15 @@ extern "C" int fp8k_moe_block_gemm_silu_quant(const void* A, const void* B, cons
   const int64_t nwg = walk ? std::min<int64_t>(per_xcd * 8 * a.tiles_n, std::max(8, num_cu() / 8 * 8)) : per_xcd * 8 * a.tiles_n;
   FP8K_REQUIRE(nwg < 0x7fffffffLL, "%s: grid too large", op);
   hipStream_t st = (hipStream_t)stream;
-  if (act_dtype == FP8K_BF16) hipLaunchKernelGGL((moe_stream256_kernel<FP8K_BF16, false, true, true>), dim3((unsigned)nwg), dim3(512), 0, st, a);
-  else hipLaunchKernelGGL((moe_stream256_kernel<FP8K_F16, false, true, true>), dim3((unsigned)nwg), dim3(512), 0, st, a);
+#define FP8K_MOE256_ACT(O, ONCE) hipLaunchKernelGGL((moe_stream256_kernel<O, false, true, true, false, ONCE>), dim3((unsigned)nwg), dim3(512), 0, st, a)
+  if (moe256_once(num_valid_tokens, num_experts)) {
+    if (act_dtype == FP8K_BF16) FP8K_MOE256_ACT(FP8K_BF16, true);
+    else FP8K_MOE256_ACT(FP8K_F16, true);
+  } else {
+    if (act_dtype == FP8K_BF16) FP8K_MOE256_ACT(FP8K_BF16, false);
+    else FP8K_MOE256_ACT(FP8K_F16, false);
+  }
+#undef FP8K_MOE256_ACT
   return check_launch(op);
 }
 
