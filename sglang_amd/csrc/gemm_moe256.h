@@ -42,7 +42,8 @@ namespace fp8k {
 // SCALED (sorted scales only): both scale tensors hold powers of two (UE8M0 checkpoints with UE8M0-rounded activation
 // scales) and the matrix core applies them itself (v_mfma_scale_f32_32x32x64_f8f6f4 takes the two exponent bytes):
 // the products accumulate in place, the float promote and its second accumulator disappear.
-// ONCE (sorted scales only): the host expects one block per expert, so that no other workgroup reads an item's weight tile.
+// ONCE (sorted scales only): the host expects one block per expert, so that no other workgroup reads an item's weight tile, and
+// weights that outgrow the last-level cache (moe256_once()).
 // The weights are then loaded non-temporally, and leave the L2 to the activation rows, which every n tile of the block reads
 // again; the result rows too are stored past it.  Whole layers, us, plain / ONCE: 256 experts, 7168 x 2048, top 8: 1024 tokens
 // 2105 / 1959, 4096 2622 / 2565; 7168 x 512: 1024 641 / 611, 3200 821 / 785; 64 experts, 7168 x 256, top 4, 1600 tokens

@@ -524,12 +524,20 @@ extern "C" int fp8k_moe_sort_scales(const float* As, float* out, const int32_t* 
   return check_launch(op);
 }
 
+// Up to 192 slots per expert on average most experts are one block of 256
+static bool moe256_one_block(int64_t num_valid_tokens, int64_t num_experts) { return num_valid_tokens <= num_experts * 192; }
+// Whether the 256-slot kernel loads its weights non-temporally (ONCE): one block per expert, so that no other workgroup reads the
+// tile, and weights that the 256 MB last-level cache cannot hold until the next call.  GEMM 1 counts the weights of GEMM 2 (half
+// as many) to its own: what GEMM 1 leaves alone, GEMM 2 finds again.  Whole layers, us, plain / this rule: 402 MB (64 experts,
+// 2048 x 1024, top 4, 512 tokens) 114 / 100, 352 MB (64 experts, 7168 x 256, 1600 tokens) 186 / 178; non-temporal all the same
+// at 201 MB (64 experts, 4096 x 256, 512 tokens) 73 / 93, at 100 MB (64 experts, 2048 x 256, 512 tokens) 50 / 56.
+static bool moe256_once(int64_t num_valid_tokens, int64_t num_experts, int64_t weight_bytes) {
+  return moe256_one_block(num_valid_tokens, num_experts) && weight_bytes > (256LL << 20);
+}
 // whether the 256-slot grouped kernel runs as one walking workgroup per CU (the walk hands the weight stream on two K
 // blocks ahead, so K must have them)
-// Up to 192 slots per expert on average most experts are one block of 256
-static bool moe256_once(int64_t num_valid_tokens, int64_t num_experts) { return num_valid_tokens <= num_experts * 192; }
 static bool moe256_walks(int64_t num_valid_tokens, int64_t num_experts, int64_t K, bool balanced) {
-  return (balanced || moe256_once(num_valid_tokens, num_experts)) && K >= 2 * kTileK;
+  return (balanced || moe256_one_block(num_valid_tokens, num_experts)) && K >= 2 * kTileK;
 }
 
 // blocks that can be in use: every one holds a slot, and only an expert's last (or that of the slots without one) is not full
@@ -640,7 +648,7 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
     // row-major activation scales (what fused_experts_impl produces for 256-slot blocks) take the form that fetches
     // two K blocks per load
     const bool pairs = !as_sorted && as_stride_k == 1 && (as_stride_m & 1) == 0 && aligned(As, 8);  // 129..256 and more slots per expert: both 128-row halves on one weight stage
-    const bool once = moe256_once(num_valid_tokens, num_experts);
+    const bool once = moe256_once(num_valid_tokens, num_experts, num_experts * N * K);
 #define FP8K_MOE256(O) \
   do { \
     if (pairs) hipLaunchKernelGGL((moe_stream256_kernel<O, true, false>), dim3((unsigned)nwg), dim3(512), 0, st, a); \
@@ -803,7 +811,7 @@ extern "C" int fp8k_moe_block_gemm_silu_quant(const void* A, const void* B, cons
   FP8K_REQUIRE(nwg < 0x7fffffffLL, "%s: grid too large", op);
   hipStream_t st = (hipStream_t)stream;
 #define FP8K_MOE256_ACT(O, ONCE) hipLaunchKernelGGL((moe_stream256_kernel<O, false, true, true, false, ONCE>), dim3((unsigned)nwg), dim3(512), 0, st, a)
-  if (moe256_once(num_valid_tokens, num_experts)) {
+  if (moe256_once(num_valid_tokens, num_experts, num_experts * N * K / 2 * 3)) {
     if (act_dtype == FP8K_BF16) FP8K_MOE256_ACT(FP8K_BF16, true);
     else FP8K_MOE256_ACT(FP8K_F16, true);
   } else {

@@ -412,11 +412,12 @@ def test_grouped_gemm_256_slot_blocks_every_group_count(dev):
 
 
 @pytest.mark.parametrize("T,E,topk,N,K,pow2", [(900, 40, 6, 2568, 128, False), (900, 40, 6, 2568, 256, False), (700, 24, 5, 4616, 384, False),
-                                               (700, 24, 5, 4616, 512, True), (1500, 8, 2, 8712, 640, False), (1500, 8, 2, 8712, 384, True)])
+                                               (700, 24, 5, 4616, 512, True), (1500, 8, 2, 8712, 640, False), (1500, 8, 2, 8712, 384, True),
+                                               (150, 64, 4, 8200, 512, False), (150, 64, 4, 8200, 512, True)])
 def test_grouped_gemm_walks_of_256_slot_blocks_exact(dev, T, E, topk, N, K, pow2):
     """More tiles than workgroups, so that the entry into an item runs beside the write-out of the one before it: one to five K
-    blocks, partly filled and absent blocks, a last tile of 8 weight rows, up to and above 192 slots per expert, activation scales
-    with and without a row stride of one, routed weights on and off; exact on integer data with power-of-two scales."""
+    blocks, partly filled and absent blocks, a last tile of 8 weight rows, up to and above 192 slots per expert, weights below and
+    above the 256 MB from which they are loaded non-temporally, activation scales with and without a row stride of one, routed weights on and off; exact on integer data with power-of-two scales."""
     from sglang_amd.fused_moe import moe_align_block_size
     from sglang_amd.sgl_kernel import moe_balance_blocks, moe_block_gemm, moe_sort_scales
 
