@@ -230,47 +230,50 @@ static int dispatch_group(const void* x, void* q, void* s, int64_t M, int64_t K,
 }
 
 // ------------------------------------------------------------------------------------------------
-// per-token quant: one workgroup per row, row held in registers between the amax and the cast
+// per-token quant: WPR waves to a row, the row held in registers between the amax and the cast
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ float block_max_256(float v, float* red) {
-  v = group_max<64>(v);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) red[w] = v;
-  __syncthreads();
-  v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  __syncthreads();
-  return v;
-}
-
-template <int DT>
+// Bound by the latency of one row: load, maximum, store (large inputs by HBM: 8192 x 4096 runs at 5.9 TB/s).  The loads of a row
+// are all in flight together; issued one by one behind the use of the one before, as conditional loads are, a row of 14336
+// columns waited for memory seven times.  HOLD is what the row needs, no more: empty turns cost up to 30 % on short rows.
+template <int DT, int WPR, int HOLD>
 __global__ __launch_bounds__(256) void token_quant_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
-                                                          float* __restrict__ s, int64_t K) {
-  constexpr int HOLD = 8;  // 8 chunks x 256 threads x 8 elements = 16384 columns stay in registers
+                                                          float* __restrict__ s, int M, int64_t K) {
+  static_assert(WPR == 1 || WPR == 4, "a wave or a workgroup to a row");
+  constexpr int LANES = WPR * 64;  // HOLD chunks x LANES x 8 elements stay in registers
   __shared__ float red[4];
-  const int64_t row = blockIdx.x;
-  const int nchunk = (int)(K / 8);
+  const int tid = (int)threadIdx.x % LANES;
+  const int64_t row = (int64_t)blockIdx.x * (4 / WPR) + (int)threadIdx.x / LANES;
+  const int nchunk = row < M ? (int)(K / 8) : 0;  // lanes of a row past the end take part in the barrier only
   Raw8<DT> raw[HOLD];
+  // every load of the row is on its way before the first value is looked at
+#pragma unroll
+  for (int c = 0; c < HOLD; ++c) {
+    const int ch = c * LANES + tid;
+    raw[c].zero();
+    if (ch < nchunk) raw[c].load(x, row * K + (int64_t)ch * 8);
+  }
   float m = 0.f;
 #pragma unroll
   for (int c = 0; c < HOLD; ++c) {
-    const int ch = c * 256 + threadIdx.x;
-    if (ch < nchunk) {
-      raw[c].load(x, row * K + (int64_t)ch * 8);
-      float a[8];
-      raw[c].unpack(a);
-      m = fmaxf(m, absmax8(a));
-    }
+    float a[8];
+    raw[c].unpack(a);
+    m = fmaxf(m, absmax8(a));
   }
-  for (int ch = HOLD * 256 + threadIdx.x; ch < nchunk; ch += 256) {
+  for (int ch = HOLD * LANES + tid; ch < nchunk; ch += LANES) {
     Raw8<DT> t;
     t.load(x, row * K + (int64_t)ch * 8);
     float a[8];
     t.unpack(a);
     m = fmaxf(m, absmax8(a));
   }
-  m = block_max_256(m, red);
+  m = group_max<64>(m);
+  if constexpr (WPR > 1) {
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  }
   const float sc = m / kFp8Max;
-  if (threadIdx.x == 0) s[row] = sc;
+  if (tid == 0 && row < M) s[row] = sc;
   const float inv = (sc == 0.f) ? 0.f : 1.0f / sc;
   auto emit = [&](const float(&a)[8], int ch) {
     float y[8];
@@ -283,20 +286,47 @@ __global__ __launch_bounds__(256) void token_quant_kernel(const void* __restrict
   };
 #pragma unroll
   for (int c = 0; c < HOLD; ++c) {
-    const int ch = c * 256 + threadIdx.x;
+    const int ch = c * LANES + tid;
     if (ch < nchunk) {
       float a[8];
       raw[c].unpack(a);
       emit(a, ch);
     }
   }
-  for (int ch = HOLD * 256 + threadIdx.x; ch < nchunk; ch += 256) {
+  for (int ch = HOLD * LANES + tid; ch < nchunk; ch += LANES) {
     Raw8<DT> t;
     t.load(x, row * K + (int64_t)ch * 8);
     float a[8];
     t.unpack(a);
     emit(a, ch);
   }
+}
+
+// A wave to a row where that fills its lanes with two chunks, four with many rows; else a workgroup.  us, one workgroup with eight
+// conditional loads (before) / a workgroup / a wave: 1 x 4096 2.35 / 2.10 / 2.66, 200 x 18432 6.18 / 5.02 / -, 2048 x 4096 6.66 / 6.03
+// / 6.55, 500 x 2048 2.56 / 2.37 / 2.52, 8192 x 2048 11.86 / 11.15 / 10.16, 64 x 1024 2.38 / 2.17 / 2.12, 8192 x 1024 8.60 / 7.78
+// / 6.06, 4096 x 512 4.73 / 4.41 / 3.14.
+template <int DT>
+static void launch_token_quant(const void* x, uint8_t* q, float* s, int64_t M, int64_t K, hipStream_t st) {
+#define FP8K_TOKEN(WPR, HOLD) \
+  hipLaunchKernelGGL((token_quant_kernel<DT, WPR, HOLD>), dim3((unsigned)((M + 4 / WPR - 1) / (4 / WPR))), dim3(256), 0, st, x, q, s, (int)M, K)
+  if (K <= 1024) FP8K_TOKEN(1, 2);
+  else if (K <= 2048 && M >= 1024) FP8K_TOKEN(1, 4);
+  else if (K <= 2048) FP8K_TOKEN(4, 1);
+  else if (K <= 4096) FP8K_TOKEN(4, 2);
+  else if (K <= 8192) FP8K_TOKEN(4, 4);
+  else FP8K_TOKEN(4, 8);
+#undef FP8K_TOKEN
+}
+
+__device__ __forceinline__ float block_max_256(float v, float* red) {
+  v = group_max<64>(v);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) red[w] = v;
+  __syncthreads();
+  v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  __syncthreads();
+  return v;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -564,9 +594,8 @@ int quant_for_linear(bool groups, const void* x, void* q, float* s, int64_t M, i
   if (groups)
     return bf ? launch_group_quant<FP8K_BF16, 128, FP8K_SCALE_F32>(x, q, s, M, K, quant_eps(eps, dtype), 1, M, st)
               : launch_group_quant<FP8K_F16, 128, FP8K_SCALE_F32>(x, q, s, M, K, quant_eps(eps, dtype), 1, M, st);
-  const dim3 grid((unsigned)M), block(256);
-  if (bf) hipLaunchKernelGGL(token_quant_kernel<FP8K_BF16>, grid, block, 0, st, x, (uint8_t*)q, s, K);
-  else hipLaunchKernelGGL(token_quant_kernel<FP8K_F16>, grid, block, 0, st, x, (uint8_t*)q, s, K);
+  if (bf) launch_token_quant<FP8K_BF16>(x, (uint8_t*)q, s, M, K, st);
+  else launch_token_quant<FP8K_F16>(x, (uint8_t*)q, s, M, K, st);
   return check_launch("token_quant");
 }
 
@@ -699,11 +728,10 @@ extern "C" int fp8k_token_quant(const void* x, void* q, float* s, int64_t M, int
   FP8K_REQUIRE(x && q && s, "token_quant: null pointer");
   FP8K_REQUIRE(aligned(x, 16) && aligned(q, 8), "token_quant: x must be 16-byte, q 8-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid((unsigned)M), block(256);
   switch (in_dtype) {
-    case FP8K_BF16: hipLaunchKernelGGL(token_quant_kernel<FP8K_BF16>, grid, block, 0, st, x, (uint8_t*)q, s, K); break;
-    case FP8K_F16: hipLaunchKernelGGL(token_quant_kernel<FP8K_F16>, grid, block, 0, st, x, (uint8_t*)q, s, K); break;
-    default: hipLaunchKernelGGL(token_quant_kernel<FP8K_F32>, grid, block, 0, st, x, (uint8_t*)q, s, K); break;
+    case FP8K_BF16: launch_token_quant<FP8K_BF16>(x, (uint8_t*)q, s, M, K, st); break;
+    case FP8K_F16: launch_token_quant<FP8K_F16>(x, (uint8_t*)q, s, M, K, st); break;
+    default: launch_token_quant<FP8K_F32>(x, (uint8_t*)q, s, M, K, st); break;
   }
   return check_launch("token_quant");
 }

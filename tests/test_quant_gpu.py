@@ -273,6 +273,23 @@ def test_per_token_quant(dev, M, K):
     np.testing.assert_array_equal(u8(q), q_ref)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K", [(3, 8), (5, 1024), (6, 1032), (1023, 2048), (1025, 2040), (2, 2056), (2, 4096), (3, 4104), (3, 8192), (2, 8200),
+                                 (2, 16384), (3, 18440)])
+def test_per_token_quant_row_forms(dev, M, K, dtype):
+    """Both sides of every line between the forms (a wave or a workgroup to a row, one to eight chunks held, more than are held),
+    rows that leave a workgroup's last waves idle, a row of zeros."""
+    from sglang_amd.fp8_kernel import sglang_per_token_quant_fp8
+
+    x = torch.from_numpy(O.make_activation(M, K, seed=M + K)).to(dtype)
+    x[1] = 0
+    x[M - 1, K - 1] = 3e4  # the last value of the last row decides its scale
+    q, s = sglang_per_token_quant_fp8(x.to(dev))
+    q_ref, s_ref = O.per_token_quant_fp8(x.float().numpy())
+    np.testing.assert_array_equal(s.cpu().numpy(), s_ref)
+    np.testing.assert_array_equal(u8(q), q_ref)
+
+
 @pytest.mark.parametrize("numel", [8, 1000, 4096 * 7168 + 5])
 def test_per_tensor_quant(dev, numel):
     from sglang_amd.fp8_kernel import scaled_fp8_quant
