@@ -168,3 +168,24 @@ def test_tiles_of_64_activation_rows_ue8m0(dev, tile128, M, N, K, splits):
     tile128(256 + splits)
     b = w8a8_block_fp8_matmul(xq, B, xs, Bs, [128, 128], torch.bfloat16)
     assert torch.equal(a, b)  # the same sums in the same order as the 128-row tiles, which the tests above hold against the oracle
+
+
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("M,N", [(65, 136), (128, 1032)])
+def test_every_count_of_k_runs_exact(dev, tile128, M, N, splits):
+    """The reduction takes four K runs at a time: every remainder behind none, one and two of them, on integers with power-of-two
+    scales and a bias."""
+    from sglang_amd.sgl_kernel import fp8_scaled_mm
+
+    K = 128 * (2 * splits + 1)
+    rng = np.random.default_rng(M + splits)
+    xq, wq = (O.f32_to_e4m3fn(rng.integers(-4, 5, (n, K)).astype(np.float32)) for n in (M, N))
+    xs = (2.0 ** rng.integers(-3, 4, (M, K // 128))).astype(np.float32)
+    ws = (2.0 ** rng.integers(-3, 4, ((N + 127) // 128, K // 128))).astype(np.float32)
+    tile128(splits)
+    np.testing.assert_array_equal(_run_block(xq, xs, wq, ws, dev), O.w8a8_block_fp8_matmul(xq, wq, xs, ws, out_dtype="bf16", acc=np.float64))
+    sa, sb = ((2.0 ** rng.integers(-3, 3, (n,))).astype(np.float32) for n in (M, N))
+    bias = rng.integers(-8, 9, (N,)).astype(np.float32)
+    got = fp8_scaled_mm(fp8_tensor(xq, dev), fp8_tensor(wq, dev).t(), torch.from_numpy(sa).to(dev), torch.from_numpy(sb).to(dev),
+                        torch.bfloat16, torch.from_numpy(bias).to(dev)).float().cpu().numpy()
+    np.testing.assert_array_equal(got, O.fp8_scaled_mm(xq, wq, sa, sb, out_dtype="bf16", bias=bias))
