@@ -257,6 +257,35 @@ def test_moe_sum_reduce_exact(dev, T, topk, H, scale):
     np.testing.assert_array_equal(out.float().cpu().numpy(), O.moe_sum_reduce(x, scale))
 
 
+@pytest.mark.parametrize("T,topk,H", [(3, 2, 64), (5, 3, 136), (2, 5, 2048), (7, 6, 72), (3, 7, 1024), (2, 9, 128), (2340, 8, 7168)])
+def test_moe_sum_reduce_every_remainder_exact(dev, T, topk, H):
+    """Four experts' rows at a time with every remainder, and one at a time where the input is larger than 256 MB (2340 x 8 x 7168)."""
+    from sglang_amd.sgl_kernel import moe_sum_reduce
+
+    x = torch.randint(-8, 9, (T, topk, H), generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
+    out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
+    moe_sum_reduce(x.to(dev), out, 0.5)
+    assert torch.equal(out.float().cpu(), (x.float().sum(1) * 0.5).bfloat16().float())
+
+
+@pytest.mark.parametrize("T,E,topk,kb", [(300, 8, 2, 1), (70, 5, 3, 7), (64, 4, 2, 8), (200, 6, 1, 9), (40, 8, 2, 56)])
+def test_moe_sort_scales_exact(dev, T, E, topk, kb):
+    """Eight K blocks per lane: none, one and more groups of them, with remainders; padding positions are zero."""
+    from sglang_amd.fused_moe import moe_align_block_size
+    from sglang_amd.sgl_kernel import moe_sort_scales
+
+    g = torch.Generator().manual_seed(kb)
+    ids = torch.rand((T, E), generator=g).argsort(dim=1)[:, :topk].int()
+    As = torch.rand((T, kb), generator=g)
+    sorted_ids, _, npad = moe_align_block_size(ids.to(dev), 64, E)
+    for scales in (As.to(dev), As.to(dev).t().contiguous().t()):
+        got = moe_sort_scales(scales, sorted_ids, npad, topk, T * topk).cpu()
+        n = int(npad[0])
+        slot = sorted_ids.cpu()[:n].long()
+        want = torch.where((slot < T * topk)[:, None], As[(slot // topk).clamp(max=T - 1)], torch.zeros(()))
+        assert torch.equal(got[:n], want)
+
+
 @pytest.mark.parametrize("topk", [1, 2, 3, 4, 8])
 def test_moe_sum_exact(dev, topk):
     from sglang_amd.sgl_kernel import moe_sum
