@@ -17,7 +17,7 @@ extern "C" {
  * Tuning and test aid (no counterpart in the reference): pins the kernel family that the dense GEMM entry points
  * pick for later calls made by the calling thread (the setting is thread-local; other threads keep the automatic
  * choice).  kind -1: automatic (the default).  kind 4: the 128x128 tile kernel with K
- * cut into `splits` runs (0 or 1: none).  kind 0: the choice by the number of rows alone, without the 128x128
+ * cut into `splits` runs (0 or 1: none; | 256: the form with 64 activation rows).  kind 0: the choice by the number of rows alone, without the 128x128
  * kernel.  kind 1: 256x256 tiles; kind 2: the streaming kernel (up to 128 rows); kind 3: the direct kernel (up to 32
  * rows, `splits` > 0 pins its K cut too); kind 5: the direct kernel that cuts K across the waves of a workgroup (up to
  * 32 rows); where a pinned family cannot take the shape, the choice by rows stands.
@@ -60,7 +60,8 @@ int fp8k_tune_stream_read_write(const void* src, int64_t bytes, void* dst, int64
 /*
  * Measurement aid: the bare matrix-core rate.  One workgroup of 8 wavefronts per CU; every wavefront loads six operand
  * fragments (2 KB each) of the caller's bytes once and then issues iters x 8 independent
- * v_mfma_f32_32x32x64 (e4m3 x e4m3) products of them with nothing else in the loop.  *flops receives the number of
+ * v_mfma_f32_32x32x64 (e4m3 x e4m3) products of them with nothing else in the loop.  (The 16x16x128 products that the dense
+ * tile kernels use reach 4.56 PFLOP/s on quantised-weight bytes where these reach 4.19, and as much on zeros.)  *flops receives the number of
  * floating-point operations the launch performs (2 x 32 x 32 x 64 per instruction); timed by the caller it gives the
  * rate the matrix cores sustain on this machine for THESE operand bytes - the power management clocks the chip by what
  * the data toggles, so random FP8 bytes and all-zero bytes give different ceilings.  sink receives one float per lane
@@ -71,8 +72,9 @@ int fp8k_tune_mfma_peak(const void* operands, int64_t bytes, int64_t iters, floa
 
 /*
  * Measurement aid (no counterpart in the reference): the K loop of the 256x256 block-scaled tile kernel built up from the
- * bare MFMA loop of fp8k_tune_mfma_peak one ingredient at a time, on operands that never change, in the tile kernel's
- * instruction order (16 MFMAs per wave and K block, 8 waves per CU).  form 1: the block-scaled product form (two MFMAs
+ * bare MFMA loop of fp8k_tune_mfma_peak one ingredient at a time, on operands that never change, on 32x32x64 products
+ * (16 per wave and K block, 8 waves per CU; the tile kernel itself takes 16x16x128 products, with the same operand
+ * bytes, FMAs and loads per K block).  form 1: the block-scaled product form (two MFMAs
  * into a short-lived accumulator, 16 scale FMAs fold it into the long-lived one); form 2: + the operand fragments
  * refilled from LDS behind their last use; form 3: + one LDS-only workgroup barrier per K block; form 4: + the eight
  * 1 KB global -> LDS stage loads per wave and K block (from the first 16 MiB of `operands`, cache-resident) and the

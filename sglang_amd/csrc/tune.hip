@@ -198,7 +198,7 @@ namespace fp8k {
 //           hardware-scaled modes of the tile kernel
 //   FORM 6  form 5 with 16 multiplies per 32x32 tile and K block in the place of the FMAs: what a loop would issue that
 //           accumulates in place and multiplies the accumulators by the ratio of two consecutive blocks' scales
-// The instruction order is the tile kernel's (steps 3, 0, 1, 2 of its loop).
+// On 32x32x64 products; the tile kernel takes 16x16x128 ones, with the same operand bytes, FMAs and loads per K block.
 template <int FORM>
 __global__ __launch_bounds__(512, 1) void mfma_loop_kernel(const uint8_t* __restrict__ operands, int64_t bytes, int iters,
                                                            float* __restrict__ sink) {
