@@ -49,14 +49,15 @@ def moe_align_block_size(
 def get_default_config(M: int, E: int, topk: int) -> Dict[str, int]:
     """Rows per block of the grouped GEMM (the reference's BLOCK_SIZE_M, fused_moe_triton_config.py).
 
-    Measured on MI355X with 256 experts, top-8 and near-balanced routing: while the layer streams every expert's
-    weights for a handful of rows each, the register-streaming kernel with 16- or 32-row blocks wins (up to about 22
-    rows per expert: 1.95 ms against 2.02 ms at 512 tokens): 16 rows while an average expert still fits one such block
-    with room for uneven routing (at 6 rows per expert 86 us against 96 with an intermediate size of 256 and a hidden
-    size of 2048, 137 against 181 with 64 experts of 2048 x 2048, 254 either way with 7168 x 256), 32 beyond.
-    From 22 on the 256-row kernel, which walks its items with the weight stream running on across them, skips the slot
-    groups that are padding and forms the activation and the requantisation in the write-out of GEMM 1 (2.06 ms against
-    2.13 ms with 64-row blocks at 768 tokens, 2.21 against 2.29 with 128-row blocks at 1536, 2.48 against 2.65 at 3072).
+    Measured on MI355X with near-balanced routing: while the layer streams every expert's weights for a handful of rows
+    each, the register-streaming kernel with 16- or 32-row blocks wins, up to about 22 rows per expert: 16 rows while an
+    average expert still fits one such block with room for uneven routing (at 6 rows per expert 86 us against 96 with an
+    intermediate size of 256 and a hidden size of 2048, 137 against 181 with 64 experts of 2048 x 2048, 254 either way with
+    7168 x 256), 32 beyond.  From 22 on the 256-row kernel, which walks its items with the weight stream running on across
+    them, skips the slot groups that are padding and forms the activation and the requantisation in the write-out of GEMM 1
+    (256 experts of 7168 x 2048, top-8: 1.87 ms against 2.11 ms with 64-row blocks at 768 tokens, 2.00 against 2.29 with
+    128-row blocks at 1536, 2.27 against 2.69 at 3072).  The line is one for all sizes: at 20 rows per expert the 256-row
+    kernel is 22 % behind with 64 experts of 7168 x 256, level with 7168 x 512 and 5 % ahead with 256 of 7168 x 2048.
     The 64- and 128-row forms of the streaming kernel remain for callers that pass their own BLOCK_SIZE_M.
     """
     per_expert = (M * topk + E - 1) // max(E, 1)
