@@ -7,9 +7,9 @@ on the current torch stream of the tensor's device and never synchronises.
 """
 from __future__ import annotations
 
+import threading
 import weakref
 from typing import Optional
-
 
 import torch
 
@@ -22,6 +22,7 @@ FP8_MIN = -448.0
 
 _workspaces: dict = {}   # (device index, stream handle) -> the buffer handed out on that stream
 _retired: list = []      # every buffer ever handed out and since outgrown: kept alive for the life of the process
+_publish = threading.RLock()  # which buffer of a stream is handed out: decided by one thread at a time
 
 
 def _workspace(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
@@ -32,17 +33,26 @@ def _workspace(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
     replays write partials there.  When a later call needs more, a larger buffer takes its place for new launches and
     the old one is parked in `_retired`.  Growth is geometric (at least double, at least 32 MiB), so a process parks
     a handful of buffers at most.  Allocation under stream capture goes through torch's allocator like the GEMM's
-    output tensor does, into the capturing graph's pool; `reserve_workspace` sizes the buffer ahead of a capture."""
+    output tensor does, into the capturing graph's pool; `reserve_workspace` sizes the buffer ahead of a capture.
+
+    Threads that need or outgrow a stream's buffer at once each allocate one, without a lock as that may wait for the
+    device, and the first to come back decides: another finds its buffer (or retires it, if it is too small) and drops
+    its own, which nobody has seen.  A buffer stored over one that is already in use would release that one, and its
+    memory could become the output of the very product that works in it."""
     if nbytes <= 0:
         return None
     key = (device.index, torch.cuda.current_stream(device).cuda_stream)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         size = max(nbytes, 32 << 20, 2 * buf.numel() if buf is not None else 0)
-        if buf is not None:
-            _retired.append(buf)
-        buf = torch.empty(size, dtype=torch.uint8, device=device)
-        _workspaces[key] = buf
+        fresh = torch.empty(size, dtype=torch.uint8, device=device)
+        with _publish:
+            buf = _workspaces.get(key)
+            if buf is None or buf.numel() < nbytes:
+                _workspaces[key] = fresh
+                if buf is not None:
+                    _retired.append(buf)
+                buf = fresh
     return buf
 
 

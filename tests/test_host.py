@@ -6,6 +6,7 @@ decides; and where they do take a call, its result is that of the dispatcher pat
 import sys
 import threading
 import time
+import types
 
 import pytest
 import torch
@@ -413,3 +414,38 @@ def test_threads_that_share_a_stream_share_its_workspace(dev):
     torch.cuda.synchronize()
     for i in range(2):
         assert all(torch.equal(out, want[i]) for out in got[i])
+
+
+@pytest.mark.parametrize("held", [0, 1 << 20])
+@pytest.mark.parametrize("needs", [(40 << 20, 40 << 20), (40 << 20, 100 << 20)])
+def test_no_workspace_handed_out_is_released(monkeypatch, held, needs):
+    """Threads that first need, or outgrow, the workspace of one stream at the same moment: what each of them is given is large
+    enough and stays alive, in use or retired."""
+    buffers, retired, real = {}, [], torch.empty
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(cuda_stream=7))
+    if held:
+        buffers[None, 7] = real(held, dtype=torch.uint8)
+    monkeypatch.setattr(sgl_kernel, "_workspaces", buffers)
+    monkeypatch.setattr(sgl_kernel, "_retired", retired)
+    met = threading.Barrier(2)
+
+    def empty(*args, **kwargs):
+        met.wait(timeout=30)  # neither thread has stored its buffer when the other has decided to make one
+        return real(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    got = [None, None]
+
+    def work(i):
+        got[i] = sgl_kernel._workspace(torch.device("cpu"), needs[i])
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    kept = [*buffers.values(), *retired]
+    for buf, need in zip(got, needs):
+        assert buf.numel() >= need and any(buf is k for k in kept)
+    assert len({id(k) for k in kept}) == len(kept)
+    assert buffers[None, 7].numel() >= max(needs)
