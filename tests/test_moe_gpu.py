@@ -297,6 +297,25 @@ def test_moe_sum_exact(dev, topk):
     np.testing.assert_array_equal(out.float().cpu().numpy(), O.moe_sum(x))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("topk", [2, 3, 4])
+def test_moe_sum_both_sides_of_the_batch_rule(dev, topk, dtype):
+    """The last token count whose rows are all requested together and the first that walks them one by one: the sums of the element
+    type, one rounding per addition, either way."""
+    from sglang_amd.sgl_kernel import moe_sum
+
+    H = 7168
+    most = (256 << 20) // (2 * (topk + 1) * H)
+    for T in (most, most + 1):
+        x = torch.randn((T, topk, H), device=dev).to(dtype)
+        out = torch.empty((T, H), device=dev, dtype=dtype)
+        moe_sum(x, out)
+        want = x[:, 0]
+        for k in range(1, topk):
+            want = want + x[:, k]
+        assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("seed", [0, 1, 2])
 def test_grouped_gemm_hardware_scaled_is_exact_on_integer_data(dev, seed):
     """fp8k_moe_block_gemm_ue8m0 (256-slot blocks, sorted power-of-two scales): on small integers with power-of-two
