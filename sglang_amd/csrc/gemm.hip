@@ -573,13 +573,11 @@ extern "C" int fp8k_block_gemm_ue8m0(const void* A, const void* B, const int32_t
   FP8K_REQUIRE(As_packed && Bs, "%s: null scale pointer", op);
   FP8K_REQUIRE(as_stride_m >= 0 && as_stride_w >= 0 && bs_stride_n >= 0 && bs_stride_k >= 0, "%s: negative scale stride", op);
   FP8K_REQUIRE((M - 1) * as_stride_m + ((K + kTileK - 1) / kTileK / 4) * as_stride_w < (1LL << 31), "%s: scales span more than 2^31 elements", op);
-  Plan pl = make_plan(M, N, K);
-  // the matrix core applies the scales only in the tile kernels, so 33 and more rows take one whatever the plan of their float form;
-  // smaller problems take the float-scale entry point with the exponents expanded to floats
-  if (g_force_kind < 0 && M > 32 && K % kTileK == 0 && N % 8 == 0 && pl.kind != 1 && pl.kind != 4)
-    pl = plan_tile128(M, N, (int)(K / kTileK), 1, M <= 64 ? 64 : 128);
-  FP8K_REQUIRE(pl.kind == 1 || pl.kind == 4, "%s: built for M > 128 with K a multiple of 128 (got M=%lld, K=%lld); expand the scales "
-               "and call fp8k_block_gemm", op, (long long)M, (long long)K);
+  // the matrix core applies the scales only in the tile kernels, and every plan for more than 128 rows and whole K blocks is one of
+  // them; smaller problems take the float-scale entry point with the exponents expanded to floats
+  const Plan pl = make_plan(M, N, K);
+  FP8K_REQUIRE(M > 128 && (pl.kind == 1 || pl.kind == 4), "%s: built for M > 128 with K a multiple of 128 (got M=%lld, K=%lld); expand the "
+               "scales and call fp8k_block_gemm", op, (long long)M, (long long)K);
   const int64_t need = pl.ws_bytes;
   if (need > 0 && (!workspace || workspace_bytes_given < need))
     return fail(FP8K_ERR_WORKSPACE, "%s: workspace of %lld bytes required, %lld given", op, (long long)need,

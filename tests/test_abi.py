@@ -139,3 +139,14 @@ def test_scale_layout_factory_matches_reference_shapes():
     assert s.shape == (45, 14) and s.stride() == (1, 48) and s.dtype == torch.int32
     s = mk((45, 640), "cpu", 128, True, True, True)
     assert s.shape == (45, 2)
+
+
+def test_packed_scales_are_refused_up_to_128_rows():
+    """Whatever kernel the float form of such a problem would take: the exponents are applied in the tile kernels only."""
+    from sglang_amd import _lib
+
+    buf = ctypes.create_string_buffer(4096)
+    p = (ctypes.addressof(buf) + 255) // 256 * 256
+    for M, N, K in ((24, 8768, 6400), (64, 1024, 16384), (100, 512, 512), (128, 4608, 1536), (129, 256, 144)):
+        rc = _lib.lib.fp8k_block_gemm_ue8m0(p, p, p, p, p, M, N, K, K, K, 1, M, K // 128, 1, N, _lib.BF16, p, 1 << 40, None)
+        assert rc == 1 and b"M > 128" in _lib.lib.fp8k_last_error(), (M, N, K)
