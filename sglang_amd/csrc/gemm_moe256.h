@@ -333,8 +333,8 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
       }
     };
 
-    // one K block; its scales sit in sxp[.][parity] and sb on entry; the odd trips reload both blocks' activation
-    // scales in the paired form
+    // The loop of the forms whose scales follow the activation rows (paired or not).  One K block; its scales sit in
+    // sxp[.][parity] and sb, or sxn and sbn, on entry; the odd trips reload both blocks' activation scales in the paired form
     auto trip = [&](auto na, int it, int parity, float& sb) {
       constexpr int NA = decltype(na)::value;  // 32-slot groups of the wave's half with real slots
       lds_barrier<LW>();  // everything but the wave's loads of weight block it+1 has landed
@@ -342,8 +342,7 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
       // the scale loads of the previous trip with them, and loads return in order - that wait would also be one for
       // the weight block requested before those scales
       __builtin_amdgcn_sched_barrier(0);
-      float sc[MS];  // SCALED: the exponent byte of the activation scale, as bits
-      int sc_w = 127;  // SCALED: exponent byte of the weight scale
+      float sc[MS];
       if (pairs) {
 #pragma unroll
         for (int ms = 0; ms < MS; ++ms) sc[ms] = sxp[ms][parity] * sb;
@@ -351,8 +350,7 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
         load_sb(sb, it + 2);
       } else {
 #pragma unroll
-        for (int ms = 0; ms < MS; ++ms) sc[ms] = SCALED ? __uint_as_float(__float_as_uint(sxn[ms]) >> 23) : sxn[ms] * sbn;
-        if (SCALED) sc_w = (int)(__float_as_uint(sbn) >> 23);
+        for (int ms = 0; ms < MS; ++ms) sc[ms] = sxn[ms] * sbn;
         load_sx(it + 1);
         load_sb(sbn, it + 1);
       }
@@ -377,24 +375,10 @@ __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p)
       v16f z;
 #pragma unroll
       for (int r = 0; r < 16; ++r) z[r] = 0.f;
-      if constexpr (SCALED) {
-#pragma unroll
-        for (int ms = 0; ms < NA; ++ms) {
-          const v8i x0 = frag(sx_ + ((ms * 2 + wm) * 32) * kTileK, 0);
-          const v8i x1 = frag(sx_ + ((ms * 2 + wm) * 32) * kTileK, 1);
-          const int ex = (int)__float_as_uint(sc[ms]);
-#pragma unroll
-          for (int ns = 0; ns < NS; ++ns) {
-            acc[ns][ms] = mfma_32x32x64_scaled(wf[ns][0], x0, acc[ns][ms], sc_w, ex);
-            acc[ns][ms] = mfma_32x32x64_scaled(wf[ns][1], x1, acc[ns][ms], sc_w, ex);
-          }
-        }
-      } else if constexpr (NA <= 3 || (SORTED && !FUSE)) {
+      if constexpr (NA <= 3) {
         // two products in flight: the 16 scale-FMAs of one 32x32 product issue while the matrix core works on the
         // next (with one product at a time the wave sits out the matrix core's latency in front of every group of
-        // FMAs, and with two waves per SIMD nobody else fills it).  The four-group copy of the other scale forms has
-        // no registers for it; the sorted form's pays four scratch accesses per two trips and still gains (16384
-        // tokens: 8.62 -> 8.48 ms).
+        // FMAs, and with two waves per SIMD nobody else fills it).  The four-group copy has no registers for it.
         v16f tq[2];
         v8i x0 = frag(sx_ + (wm * 32) * kTileK, 0);
         v8i x1 = frag(sx_ + (wm * 32) * kTileK, 1);
