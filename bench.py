@@ -259,26 +259,23 @@ def hbm_tile_read_gbs(torch, dev, pitch, gib=4, runs=5):
 
 
 def mfma_ceiling_tflops(torch, dev, iters=40000, runs=3):
-    """Rate of a bare v_mfma_f32_32x32x64 (e4m3) loop on this machine (fp8k_tune_mfma_peak: 8 waves per CU, operands in
-    registers, nothing else in the loop) on operand bytes taken from a quantised headline weight ("random") and on
+    """Rate of a bare v_mfma_f32_16x16x128 (e4m3) loop, the instruction of the dense tile kernels, on this machine
+    (fp8k_tune_mfma_peak: 8 waves per CU, operands in registers, nothing else in the loop) on operand bytes taken from a
+    quantised headline weight ("random") and on
     all-zero bytes ("zeros"); best of `runs` after a settling launch.  The power management clocks the chip by what the
-    data toggles: the random-data figure is the ceiling of FP8 products of this shape on real data (16x16x128 products reach
-    9 % more), and its ratio to the zero-data figure separates that limit from kernel quality."""
-    import ctypes
-
-    from sglang_amd._lib import check, lib, stream_ptr
-
+    data toggles: the random-data figure is the ceiling of FP8 products on real data, and its ratio to the zero-data
+    figure separates that limit from kernel quality."""
     ncu = torch.cuda.get_device_properties(dev).multi_processor_count
     wq, _ = _block_quant_weight(torch, 4096, 4096, 0, dev)
     sink = torch.empty(ncu * 512, dtype=torch.float32, device=dev)
     out = {}
     for name, ops in (("random", wq.view(torch.uint8)), ("zeros", torch.zeros_like(wq.view(torch.uint8)))):
-        out[name] = _mfma_probe(torch, dev, ops, sink, 0, iters, runs)
+        out[name] = _mfma_probe(torch, dev, ops, sink, None, iters, runs)
     return out
 
 
 def _mfma_probe(torch, dev, ops, sink, form, iters, runs):
-    """TFLOP/s of one form of the MFMA probes (0: fp8k_tune_mfma_peak, 1..4: fp8k_tune_mfma_loop), best of `runs`."""
+    """TFLOP/s of one form of the MFMA probes (None: fp8k_tune_mfma_peak, 0..6: fp8k_tune_mfma_loop), best of `runs`."""
     import ctypes
 
     from sglang_amd._lib import check, lib, stream_ptr
@@ -288,7 +285,7 @@ def _mfma_probe(torch, dev, ops, sink, form, iters, runs):
     for r in range(runs + 1):
         a, b = _events(torch, 2)
         a.record()
-        if form == 0:
+        if form is None:
             check(lib.fp8k_tune_mfma_peak(ops.data_ptr(), ops.numel(), iters, sink.data_ptr(), sink.numel(),
                                           ctypes.byref(flops), stream_ptr(dev)))
         else:
@@ -301,11 +298,12 @@ def _mfma_probe(torch, dev, ops, sink, form, iters, runs):
     return round(flops.value / best / 1e9, 1)
 
 
-MFMA_LOOP_FORMS = ("bare MFMA loop", "+ block-scaled product form (16 scale FMAs per two MFMAs)",
-                   "+ operand fragments refilled from LDS", "+ one workgroup barrier per K block",
-                   "+ eight 1 KB stage loads per wave and K block",
-                   "the complete loop without the scale FMAs (products accumulate in place)",
-                   "the same with 16 multiplies per tile and K block (accumulators rescaled between K blocks)")
+MFMA_LOOP_FORMS = ((None, "bare loop of 16x16x128 products"), (1, "+ block-scaled product form (four scale FMAs per MFMA)"),
+                   (2, "+ operand fragments refilled from LDS"), (3, "+ one workgroup barrier per K block, falling wave priority"),
+                   (4, "+ eight 1 KB stage loads per wave and K block"),
+                   (5, "the complete loop without the scale FMAs (products accumulate in place)"),
+                   (6, "the same with four multiplies per MFMA (accumulators rescaled between K blocks)"),
+                   (0, "bare loop of 32x32x64 products"))
 
 
 def mfma_loop_lines(torch, dev, iters=40000, runs=3):
@@ -316,10 +314,10 @@ def mfma_loop_lines(torch, dev, iters=40000, runs=3):
     sink = torch.empty(ncu * 512, dtype=torch.float32, device=dev)
     rnd, zer = wq.view(torch.uint8), torch.zeros_like(wq.view(torch.uint8))
     lines = ["| form | TFLOP/s on quantised-weight bytes | of 5 PFLOP/s | TFLOP/s on zeros | of 5 PFLOP/s |", "|---|---|---|---|---|"]
-    for form, name in enumerate(MFMA_LOOP_FORMS):
+    for form, name in MFMA_LOOP_FORMS:
         a = _mfma_probe(torch, dev, rnd, sink, form, iters, runs)
         b = _mfma_probe(torch, dev, zer, sink, form, iters, runs)
-        lines.append("| %d: %s | %.0f | %.2f | %.0f | %.2f |" % (form, name, a, a / PEAK_FP8_TFLOPS, b, b / PEAK_FP8_TFLOPS))
+        lines.append("| %s: %s | %.0f | %.2f | %.0f | %.2f |" % ("-" if form is None else form, name, a, a / PEAK_FP8_TFLOPS, b, b / PEAK_FP8_TFLOPS))
     # the stage loads above walk 16 MiB (more than one XCD's 4 MB L2: most come from the memory-side cache); the same with
     # a 2 MiB range, every load an L2 hit
     a = _mfma_probe(torch, dev, rnd[:2 << 20], sink, 4, iters, runs)
@@ -837,7 +835,7 @@ def main() -> int:
         return 0
     if args.mfma_ceiling:
         c = mfma_ceiling_tflops(torch, dev)
-        print("bare v_mfma_f32_32x32x64 e4m3 loop, 8 waves per CU: %.0f TFLOP/s on quantised-weight bytes (%.2f of 5 PFLOP/s), "
+        print("bare v_mfma_f32_16x16x128 e4m3 loop, 8 waves per CU: %.0f TFLOP/s on quantised-weight bytes (%.2f of 5 PFLOP/s), "
               "%.0f TFLOP/s on all-zero bytes (%.2f)" % (c["random"], c["random"] / PEAK_FP8_TFLOPS, c["zeros"],
                                                         c["zeros"] / PEAK_FP8_TFLOPS))
         return 0

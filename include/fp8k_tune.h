@@ -58,11 +58,11 @@ int fp8k_tune_stream_read_write(const void* src, int64_t bytes, void* dst, int64
                                 int64_t stores_per_wave, void* stream);
 
 /*
- * Measurement aid: the bare matrix-core rate.  One workgroup of 8 wavefronts per CU; every wavefront loads six operand
- * fragments (2 KB each) of the caller's bytes once and then issues iters x 8 independent
- * v_mfma_f32_32x32x64 (e4m3 x e4m3) products of them with nothing else in the loop.  (The 16x16x128 products that the dense
- * tile kernels use reach 4.56 PFLOP/s on quantised-weight bytes where these reach 4.19, and as much on zeros.)  *flops receives the number of
- * floating-point operations the launch performs (2 x 32 x 32 x 64 per instruction); timed by the caller it gives the
+ * Measurement aid: the bare matrix-core rate.  One workgroup of 8 wavefronts per CU; every wavefront loads eight operand
+ * fragments (2 KB each) of the caller's bytes once and then issues iters x 16 independent
+ * v_mfma_f32_16x16x128 (e4m3 x e4m3) products of them, the instruction of the dense tile kernels, with nothing else in the
+ * loop.  *flops receives the number of
+ * floating-point operations the launch performs (2 x 16 x 16 x 128 per instruction); timed by the caller it gives the
  * rate the matrix cores sustain on this machine for THESE operand bytes - the power management clocks the chip by what
  * the data toggles, so random FP8 bytes and all-zero bytes give different ceilings.  sink receives one float per lane
  * (CUs x 512) so that the loop cannot be optimised away.
@@ -72,15 +72,17 @@ int fp8k_tune_mfma_peak(const void* operands, int64_t bytes, int64_t iters, floa
 
 /*
  * Measurement aid (no counterpart in the reference): the K loop of the 256x256 block-scaled tile kernel built up from the
- * bare MFMA loop of fp8k_tune_mfma_peak one ingredient at a time, on operands that never change, on 32x32x64 products
- * (16 per wave and K block, 8 waves per CU; the tile kernel itself takes 16x16x128 products, with the same operand
- * bytes, FMAs and loads per K block).  form 1: the block-scaled product form (two MFMAs
- * into a short-lived accumulator, 16 scale FMAs fold it into the long-lived one); form 2: + the operand fragments
- * refilled from LDS behind their last use; form 3: + one LDS-only workgroup barrier per K block; form 4: + the eight
+ * bare MFMA loop of fp8k_tune_mfma_peak one ingredient at a time, on operands that never change (32 products of 16x16x128
+ * per wave and K block, 8 waves per CU).  form 1: the block-scaled product form (every MFMA into one of four short-lived
+ * accumulators, four scale FMAs fold it into a long-lived one); form 2: + the operand fragments
+ * refilled from LDS behind their last use; form 3: + one LDS-only workgroup barrier per K block and the falling wave priority;
+ * form 4: + the eight
  * 1 KB global -> LDS stage loads per wave and K block (from the first 16 MiB of `operands`, cache-resident) and the
  * partial wait for them at the barrier; form 5: form 4 without the scale FMAs (the products accumulate in place, as in the
- * row-scaled and hardware-scaled modes); form 6: form 5 with 16 multiplies per 32x32 tile and K block in the place of
- * the FMAs (a loop that accumulates in place and rescales the accumulators between K blocks).  `iters` K blocks; *flops receives the matrix FLOPs of the launch.  Timed by the
+ * row-scaled and hardware-scaled modes); form 6: form 5 with four multiplies per MFMA in the place of
+ * the FMAs (a loop that accumulates in place and rescales the accumulators between K blocks).  form 0: the bare loop in
+ * v_mfma_f32_32x32x64 products, the instruction of the 256-slot grouped kernel (16 per count of iters).  `iters` K blocks; *flops
+ * receives the matrix FLOPs of the launch.  Timed by the
  * caller, the steps down from form to form are what each ingredient costs the matrix cores.
  * operands 32-byte aligned, bytes >= 1 MiB; sink: CUs x 512 floats.
  */

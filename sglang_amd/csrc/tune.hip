@@ -144,14 +144,50 @@ extern "C" int fp8k_tune_stream_read_write(const void* src, int64_t bytes, void*
 
 
 namespace fp8k {
-// Bare matrix-core loop: every wave keeps two weight-side and four activation-side operand fragments of the caller's
-// bytes in registers and issues the eight independent products of them, `iters` times over, into eight accumulators -
-// no loads, no LDS, no barriers inside the loop.  One workgroup of 8 waves per CU (two waves per SIMD, the occupancy
-// of the tile kernels).  The accumulators are folded into `sink` at the end so that the loop stays.
+// Bare matrix-core loop in the product the dense tile kernels issue: every wave keeps four weight-side and four activation-side
+// operand fragments of the caller's bytes in registers and issues the sixteen independent 16x16x128 products of them,
+// `iters` times over, into sixteen accumulators - no loads, no LDS, no barriers inside the loop.  One workgroup of 8
+// waves per CU (two waves per SIMD, the occupancy of the tile kernels).  The accumulators are folded into `sink` at the end so that
+// the loop stays.
 __global__ __launch_bounds__(512, 1) void mfma_peak_kernel(const uint8_t* __restrict__ operands, int64_t bytes, int iters,
                                                            float* __restrict__ sink) {
   const int lane = threadIdx.x & 63;
-  const int64_t frag0 = ((int64_t)blockIdx.x * 8 + (threadIdx.x >> 6)) * 6;  // 6 fragments of 64 lanes x 32 bytes per wave
+  const int64_t frag0 = ((int64_t)blockIdx.x * 8 + (threadIdx.x >> 6)) * 8;  // 8 fragments of 64 lanes x 32 bytes per wave
+  const int64_t nfrag = bytes / 2048;
+  v8i a[4], b[4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const v8i v = *reinterpret_cast<const v8i*>(operands + ((frag0 + i) % nfrag) * 2048 + lane * 32);
+    if (i < 4) a[i] = v;
+    else b[i - 4] = v;
+  }
+  v4f acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int it = 0; it < iters; ++it) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = mfma_16x16x128(a[i], b[j], acc[i][j]);
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s += acc[i][j][r];
+  sink[(int64_t)blockIdx.x * 512 + threadIdx.x] = s;
+}
+
+// The same in the product of the 256-slot grouped kernel: two weight-side and four activation-side fragments, eight independent
+// 32x32x64 products.
+__global__ __launch_bounds__(512, 1) void mfma_peak_32x32x64_kernel(const uint8_t* __restrict__ operands, int64_t bytes, int iters,
+                                                                    float* __restrict__ sink) {
+  const int lane = threadIdx.x & 63;
+  const int64_t frag0 = ((int64_t)blockIdx.x * 8 + (threadIdx.x >> 6)) * 6;
   const int64_t nfrag = bytes / 2048;
   v8i a[2], b[4];
 #pragma unroll
@@ -188,17 +224,15 @@ namespace fp8k {
 // The K loop of the 256x256 block-scaled tile kernel built up from the bare MFMA loop, one ingredient at a time, on
 // operands that never change (LDS filled once, the stage loads fetch a small cache-resident range), so that what each
 // ingredient costs the matrix cores can be read off:
-//   FORM 1  the block-scaled product form: two MFMAs into a short-lived accumulator, folded into the long-lived one by 16
-//           scale FMAs placed behind the first MFMAs of the next product (8 products = 16 MFMAs per K block, as a wave of
-//           the tile kernel has them)
+//   FORM 1  the block-scaled product form: every MFMA into one of four short-lived accumulators, folded into a long-lived one by
+//           four scale FMAs four MFMAs later (32 MFMAs of 16x16x128 per K block, as a wave of the tile kernel has them)
 //   FORM 2  + the operand fragments refilled from LDS behind their last use (24 ds_read_b128 per wave and K block)
-//   FORM 3  + one LDS-only workgroup barrier per K block
+//   FORM 3  + one LDS-only workgroup barrier per K block, and the falling wave priority between two of them
 //   FORM 4  + the eight 1 KB stage loads per wave and K block (global -> LDS) and the partial vmcnt wait at the barrier
 //   FORM 5  form 4 without the scale FMAs: the products accumulate in place, as in the row-scaled and the
 //           hardware-scaled modes of the tile kernel
-//   FORM 6  form 5 with 16 multiplies per 32x32 tile and K block in the place of the FMAs: what a loop would issue that
-//           accumulates in place and multiplies the accumulators by the ratio of two consecutive blocks' scales
-// On 32x32x64 products; the tile kernel takes 16x16x128 ones, with the same operand bytes, FMAs and loads per K block.
+//   FORM 6  form 5 with four multiplies per MFMA in the place of the FMAs: what a loop would issue that accumulates in place and
+//           multiplies the accumulators by the ratio of two consecutive blocks' scales
 template <int FORM>
 __global__ __launch_bounds__(512, 1) void mfma_loop_kernel(const uint8_t* __restrict__ operands, int64_t bytes, int iters,
                                                            float* __restrict__ sink) {
@@ -218,62 +252,64 @@ __global__ __launch_bounds__(512, 1) void mfma_loop_kernel(const uint8_t* __rest
   // a fragment = 64 lanes x 32 bytes, kept as two conflict-free 1 KB halves; a weight stage holds 16 of them, an
   // activation stage 16
   auto frag = [&](const uint8_t* base) -> v8i {
-    const v4i lo = *reinterpret_cast<const v4i*>(base + lane * 16);
-    const v4i hi = *reinterpret_cast<const v4i*>(base + 1024 + lane * 16);
-    v8i f;
-    f[0] = lo[0]; f[1] = lo[1]; f[2] = lo[2]; f[3] = lo[3];
-    f[4] = hi[0]; f[5] = hi[1]; f[6] = hi[2]; f[7] = hi[3];
-    return f;
+    return join(*reinterpret_cast<const v4i*>(base + lane * 16), *reinterpret_cast<const v4i*>(base + 1024 + lane * 16));
   };
-  v8i X[2][2], W[2];
-  v16f acc[4][2], tq[2], z;
+  v8i X[4], W[4];
+  v4f acc[8][4], tq[4];
 #pragma unroll
-  for (int q = 0; q < 16; ++q) { z[q] = 0.f; tq[0][q] = 0.f; tq[1][q] = 0.f; }
+  for (int q = 0; q < 4; ++q) tq[q] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int ns = 0; ns < 4; ++ns)
+  for (int ns = 0; ns < 8; ++ns)
 #pragma unroll
-    for (int ms = 0; ms < 2; ++ms)
+    for (int ms = 0; ms < 4; ++ms) acc[ns][ms] = v4f{0.f, 0.f, 0.f, 0.f};
+  const float sc[4] = {1.0f + lane * 1e-9f, 1.0f - lane * 1e-9f, 1.0f + lane * 2e-9f, 1.0f - lane * 2e-9f};
 #pragma unroll
-      for (int q = 0; q < 16; ++q) acc[ns][ms][q] = 0.f;
-  float sc[2] = {1.0f + lane * 1e-9f, 1.0f - lane * 1e-9f};
-  W[0] = frag(smem + (wn * 8) * 2048); W[1] = frag(smem + (wn * 8 + 1) * 2048);
-#pragma unroll
-  for (int ms = 0; ms < 2; ++ms)
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) X[ms][ks] = frag(smem + 3 * 32768 + (wm * 4 + ms * 2 + ks) * 2048);
+  for (int i = 0; i < 4; ++i) {
+    W[i] = frag(smem + (wn * 8 + i) * 2048);
+    X[i] = frag(smem + 3 * 32768 + (wm * 4 + i) * 2048);
+  }
   // without the refills the operands would be loop constants, and the products with them: the register is passed through
   // an empty asm statement instead, which the compiler cannot see through
-  auto RW = [&](int ks, const uint8_t* st, int ns) {
+  auto refill = [&](v8i& f, const uint8_t* from) {
     if (FORM >= 2) {
-      W[ks] = frag(st + (wn * 8 + ns * 2 + ks) * 2048);
+      f = frag(from);
     } else {
-      int t = W[ks][0];
+      int t = f[0];
       asm volatile("" : "+v"(t));
-      W[ks][0] = t;
+      f[0] = t;
     }
   };
-  auto RX = [&](int ms, int ks, const uint8_t* st) { if (FORM >= 2) X[ms][ks] = frag(st + (wm * 4 + ms * 2 + ks) * 2048); };
+  auto RW = [&](const uint8_t* st, int ns) { refill(W[ns & 3], st + (wn * 8 + ns) * 2048); };
+  auto RX = [&](const uint8_t* st, int ms) { refill(X[ms], st + (wm * 4 + ms) * 2048); };
   constexpr bool kFold = FORM != 5 && FORM != 6;
-  int step_ns = 0;  // the accumulator row the in-place form is working on (a constant after unrolling)
-  auto M = [&](int ms, int ks) {
-    if (!kFold) acc[step_ns][ms] = mfma_32x32x64(W[ks], X[ms][ks], acc[step_ns][ms]);
-    else if (ks == 0) tq[ms] = mfma_32x32x64(W[0], X[ms][0], z);
-    else tq[ms] = mfma_32x32x64(W[1], X[ms][1], tq[ms]);
-  };
-  auto F = [&](v16f& a, const v16f& t, float sv) {
-    if (FORM == 6) {
+  auto F = [&](int k) {
+    const int ns = k >> 2, ms = k & 3;
 #pragma unroll
-      for (int q = 0; q < 16; ++q) a[q] = a[q] * sv;
-      return;
+    for (int i = 0; i < 4; ++i) {
+      if (FORM == 6) acc[ns][ms][i] *= sc[ms];
+      else if (kFold) acc[ns][ms][i] = __builtin_fmaf(tq[ms][i], sc[ms], acc[ns][ms][i]);
     }
-    if (!kFold) return;
+  };
+  auto M = [&](int k) {
+    const int ns = k >> 2, ms = k & 3;
+    if (kFold) tq[ms] = mfma_16x16x128(W[ns & 3], X[ms], v4f{0.f, 0.f, 0.f, 0.f});
+    else acc[ns][ms] = mfma_16x16x128(W[ns & 3], X[ms], acc[ns][ms]);
+  };
+  auto pair = [&](int pr, auto&& between) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) a[q] = __builtin_fmaf(t[q], sv, a[q]);
+    for (int i = 0; i < 8; ++i) {
+      F((pr * 8 + i + 28) & 31);
+      SB();
+      M(pr * 8 + i);
+      SB();
+      between(i);
+      SB();
+    }
   };
   int w_ld = 0, w_rd = 1;
   for (int it = 0; it < iters; ++it) {
-    const uint8_t* stW = smem + w_rd * 32768;
-    const uint8_t* stX = smem + 3 * 32768 + ((it + 1) & 1) * 32768;
+    const uint8_t* const stW = smem + w_rd * 32768;
+    const uint8_t* const stX = smem + 3 * 32768 + ((it + 1) & 1) * 32768;
     uint8_t* const ldX = smem + 3 * 32768 + (it & 1) * 32768 + w * 4096;
     uint8_t* const ldW = smem + w_ld * 32768 + w * 4096;
     const uint32_t go = (uint32_t)(((blockIdx.x * 3 + it) * 65536) % span) + w * 4096 + lane * 16;
@@ -282,55 +318,41 @@ __global__ __launch_bounds__(512, 1) void mfma_loop_kernel(const uint8_t* __rest
     if (FORM >= 4) lds_barrier<4>();
     else if (FORM == 3) lds_barrier();
     SB();
-    step_ns = 3;
-    F(acc[2][0], tq[0], sc[0]); SB();
-    M(0, 0); SB();
-    RX(0, 0, stX); LX(0); LX(1); SB();
-    F(acc[2][1], tq[1], sc[1]); SB();
-    M(1, 0); SB();
-    RX(1, 0, stX); RW(0, stW, 0); LX(2); LX(3); SB();
-    M(0, 1); SB();
-    RX(0, 1, stX); SB();
-    M(1, 1); SB();
-    RX(1, 1, stX); RW(1, stW, 0); SB();
-    step_ns = 0;
-    F(acc[3][0], tq[0], sc[0]); SB();
-    M(0, 0); SB();
-    F(acc[3][1], tq[1], sc[1]); SB();
-    M(1, 0); SB();
-    RW(0, stW, 1); LW(0); LW(1); SB();
-    M(0, 1); SB();
-    M(1, 1); SB();
-    RW(1, stW, 1); LW(2); LW(3); SB();
-    step_ns = 1;
-    F(acc[0][0], tq[0], sc[0]); SB();
-    M(0, 0); SB();
-    F(acc[0][1], tq[1], sc[1]); SB();
-    M(1, 0); SB();
-    RW(0, stW, 2); SB();
-    M(0, 1); SB();
-    M(1, 1); SB();
-    RW(1, stW, 2); SB();
-    step_ns = 2;
-    F(acc[1][0], tq[0], sc[0]); SB();
-    M(0, 0); SB();
-    F(acc[1][1], tq[1], sc[1]); SB();
-    M(1, 0); SB();
-    RW(0, stW, 3); SB();
-    M(0, 1); SB();
-    M(1, 1); SB();
-    RW(1, stW, 3); SB();
+    if (FORM >= 3) __builtin_amdgcn_s_setprio(3);
+    pair(3, [&](int i) {
+      if (i == 0) RW(stW, 0);
+      if (i == 2) RW(stW, 1);
+      if (i >= 4) RX(stX, i - 4);
+      if (i < 4) LX(i);
+    });
+    if (FORM >= 3) __builtin_amdgcn_s_setprio(2);
+    pair(0, [&](int i) {
+      if (i == 1) RW(stW, 2);
+      if (i == 3) RW(stW, 3);
+      if (i == 2 || i == 4 || i == 6) LW(i / 2 - 1);
+    });
+    if (FORM >= 3) __builtin_amdgcn_s_setprio(1);
+    pair(1, [&](int i) {
+      if (i == 0) LW(3);
+      if (i == 1) RW(stW, 4);
+      if (i == 3) RW(stW, 5);
+    });
+    if (FORM >= 3) __builtin_amdgcn_s_setprio(0);
+    pair(2, [&](int i) {
+      if (i == 1) RW(stW, 6);
+      if (i == 3) RW(stW, 7);
+    });
     w_ld = w_rd;
     w_rd = w_rd == 2 ? 0 : w_rd + 1;
   }
   wait_vm0();
-  float sum = tq[0][0] + tq[1][0];
+  float sum = tq[0][0] + tq[1][0] + tq[2][0] + tq[3][0];
 #pragma unroll
-  for (int ns = 0; ns < 4; ++ns)
+  for (int ns = 0; ns < 8; ++ns)
 #pragma unroll
-    for (int ms = 0; ms < 2; ++ms)
+    for (int ms = 0; ms < 4; ++ms)
 #pragma unroll
-      for (int q = 0; q < 16; ++q) sum += acc[ns][ms][q];
+      for (int q = 0; q < 4; ++q) sum += acc[ns][ms][q];
   sink[(int64_t)blockIdx.x * 512 + threadIdx.x] = sum;
 }
 }  // namespace fp8k
@@ -342,14 +364,15 @@ extern "C" int fp8k_tune_mfma_loop(const void* operands, int64_t bytes, int64_t 
   FP8K_REQUIRE(operands && aligned(operands, 32), "%s: operands must be a 32-byte aligned device pointer", op);
   FP8K_REQUIRE(bytes >= (1 << 20) && bytes < (1LL << 40), "%s: at least 1 MiB of operand bytes is needed", op);
   FP8K_REQUIRE(iters >= 1 && iters <= (1 << 24), "%s: iters must be in [1, 2^24]", op);
-  FP8K_REQUIRE(form >= 1 && form <= 6, "%s: form must be 1..6", op);
+  FP8K_REQUIRE(form >= 0 && form <= 6, "%s: form must be 0..6", op);
   const int ncu = num_cu();
   FP8K_REQUIRE(sink && sink_floats >= (int64_t)ncu * 512, "%s: sink must hold %lld floats", op, (long long)ncu * 512);
-  if (flops) *flops = (int64_t)ncu * 8 * iters * 16 * (2LL * 32 * 32 * 64);
+  if (flops) *flops = (int64_t)ncu * 8 * iters * 32 * (2LL * 16 * 16 * 128);
   const dim3 grid((unsigned)ncu), block(512);
   hipStream_t st = (hipStream_t)stream;
   const uint8_t* o = (const uint8_t*)operands;
   switch (form) {
+    case 0: hipLaunchKernelGGL(mfma_peak_32x32x64_kernel, grid, block, 0, st, o, bytes, (int)iters * 2, sink); break;
     case 1: hipLaunchKernelGGL(mfma_loop_kernel<1>, grid, block, 0, st, o, bytes, (int)iters, sink); break;
     case 2: hipLaunchKernelGGL(mfma_loop_kernel<2>, grid, block, 0, st, o, bytes, (int)iters, sink); break;
     case 3: hipLaunchKernelGGL(mfma_loop_kernel<3>, grid, block, 0, st, o, bytes, (int)iters, sink); break;
@@ -369,7 +392,7 @@ extern "C" int fp8k_tune_mfma_peak(const void* operands, int64_t bytes, int64_t 
   FP8K_REQUIRE(iters >= 1 && iters <= (1 << 24), "%s: iters must be in [1, 2^24]", op);
   const int ncu = num_cu();
   FP8K_REQUIRE(sink && sink_floats >= (int64_t)ncu * 512, "%s: sink must hold %lld floats", op, (long long)ncu * 512);
-  if (flops) *flops = (int64_t)ncu * 8 * iters * 8 * (2LL * 32 * 32 * 64);
+  if (flops) *flops = (int64_t)ncu * 8 * iters * 16 * (2LL * 16 * 16 * 128);
   hipLaunchKernelGGL(mfma_peak_kernel, dim3((unsigned)ncu), dim3(512), 0, (hipStream_t)stream, (const uint8_t*)operands, bytes,
                      (int)iters, sink);
   return check_launch(op);

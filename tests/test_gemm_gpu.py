@@ -509,6 +509,24 @@ def test_stream_read_write_probe_writes_its_pattern_and_checks_its_arguments(dev
     assert rc != 0 and b"dst holds" in lib.fp8k_last_error()
 
 
+def test_mfma_probe_of_the_grouped_kernels_product(dev):
+    """Form 0 of fp8k_tune_mfma_loop, the bare loop of 32x32x64 products: on ones each of a lane's 8 x 16 sums is 64 x 2 iters."""
+    import ctypes
+
+    from sglang_amd._lib import lib, stream_ptr
+
+    ncu = torch.cuda.get_device_properties(dev).multi_processor_count
+    sink = torch.empty((ncu * 512,), dtype=torch.float32, device=dev)
+    ones = torch.full((1 << 20,), 0x38, dtype=torch.uint8, device=dev)
+    flops, iters = ctypes.c_int64(0), 3
+    rc = lib.fp8k_tune_mfma_loop(ones.data_ptr(), ones.numel(), iters, 0, sink.data_ptr(), sink.numel(), ctypes.byref(flops),
+                                 stream_ptr(dev))
+    assert rc == 0, lib.fp8k_last_error()
+    torch.cuda.synchronize()
+    assert flops.value == ncu * 8 * 2 * iters * 8 * 2 * 32 * 32 * 64
+    assert (sink == 128 * 64.0 * 2 * iters).all()
+
+
 def test_mfma_probes_compute_what_they_claim_and_check_their_arguments(dev):
     """The measurement aids fp8k_tune_mfma_peak / fp8k_tune_mfma_loop: on operand bytes 0x38 (1.0 in e4m3) every one of the
     bare loop's 8 x 16 accumulator values per lane is 64 x iters, on all-zero bytes every form sums to zero; the FLOP
