@@ -170,6 +170,49 @@ def test_tiles_of_64_activation_rows_ue8m0(dev, tile128, M, N, K, splits):
     assert torch.equal(a, b)  # the same sums in the same order as the 128-row tiles, which the tests above hold against the oracle
 
 
+@pytest.mark.parametrize("mode", ["block", "row", "packed"])
+@pytest.mark.parametrize("tile_rows,splits", [(64, 1), (64, 2), (128, 1)])
+@pytest.mark.parametrize("M,N,kb", [(193, 264, 5), (257, 392, 7)])
+def test_write_out_forms_exact(dev, tile128, M, N, kb, tile_rows, splits, mode):
+    """Both heights of the tiles, both output types, output rows that take the 16-byte and (a stride that is no multiple of eight
+    elements) the 8-byte stores; float, row and packed power-of-two scales.  Integers and powers of two: the oracle's values bit
+    for bit, and nothing written beside them."""
+    from sglang_amd._lib import BF16, F16, F32, check, lib, stream_ptr
+
+    K = kb * 128
+    rng = np.random.default_rng(M + kb)
+    xq, wq = (O.f32_to_e4m3fn(rng.integers(-4, 5, (n, K)).astype(np.float32)) for n in (M, N))
+    A, B = fp8_tensor(xq, dev), fp8_tensor(wq, dev)
+    # scales up to 1: float16 holds every sum
+    xs = (2.0 ** rng.integers(-3, 1, (M, 1 if mode == "row" else kb))).astype(np.float32)
+    ws = (2.0 ** rng.integers(-3, 1, (N,) if mode == "row" else ((N + 127) // 128, kb))).astype(np.float32)
+    if mode == "packed":
+        words = torch.from_numpy(O.pack_ue8m0_scales(xs)).to(dev)
+        As = torch.empty_strided(words.shape, (1, (M + 3) // 4 * 4), dtype=torch.int32, device=dev).copy_(words)
+    else:
+        As = torch.from_numpy(xs).to(dev)
+    Bs = torch.from_numpy(ws).to(dev)
+    tile128((256 if tile_rows == 64 else 0) + splits)
+    need = max(lib.fp8k_block_gemm_workspace_bytes(M, N, K), 1)
+    work = torch.empty(need, dtype=torch.uint8, device=dev)
+    st = stream_ptr(dev)
+    for dtype, code, name in ((torch.bfloat16, BF16, "bf16"), (torch.float16, F16, "f16")):
+        ref = O.fp8_scaled_mm(xq, wq, xs.reshape(-1), ws, name) if mode == "row" else \
+            O.w8a8_block_fp8_matmul(xq, wq, xs, ws, out_dtype=name, acc=np.float64)
+        for ldc in (N, N + 4):
+            C = torch.full((M, ldc), 7.0, dtype=dtype, device=dev)
+            if mode == "row":
+                check(lib.fp8k_scaled_mm(A.data_ptr(), B.data_ptr(), As.data_ptr(), Bs.data_ptr(), None, C.data_ptr(), M, N, K, K, K, ldc,
+                                         code, F32, work.data_ptr(), need, st))
+            else:
+                fn = lib.fp8k_block_gemm if mode == "block" else lib.fp8k_block_gemm_ue8m0
+                check(fn(A.data_ptr(), B.data_ptr(), As.data_ptr(), Bs.data_ptr(), C.data_ptr(), M, N, K, K, K, As.stride(0), As.stride(1),
+                         Bs.stride(0), Bs.stride(1), ldc, code, work.data_ptr(), need, st))
+            got = C.float().cpu().numpy()
+            np.testing.assert_array_equal(got[:, :N], ref)
+            assert (got[:, N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("splits", [2, 3, 4, 5, 6, 7, 8, 9])
 @pytest.mark.parametrize("M,N", [(65, 136), (128, 1032)])
 def test_every_count_of_k_runs_exact(dev, tile128, M, N, splits):
