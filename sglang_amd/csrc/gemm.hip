@@ -197,9 +197,13 @@ static Plan plan_base(int64_t M, int64_t N, int64_t K, int cu) {
 // is 0.4 % behind the best of all plans on average, 14 % at worst.
 //  * tiles of 128 weight rows and TM = 128 or 64 activation rows: 0.43 (0.34) per K block - the serial chain of a trip more than its
 //    work - and a little more when the weights are new to the chip and the chip is full; 3 us of first loads and write-out per
-//    round of tiles, at most two rounds; a K cut adds the reduction launch and the float partials.  Below 12 us a cut gains nothing
-//    where the host makes the launches one by one: it takes 4 us for each (134 x 1280 x 2944 as a linear: 17 - 18 us with three
-//    K ranges, which are the quicker product by 0.4, and 15 without).
+//    round of tiles, at most two rounds; a K cut adds the reduction launch and the float partials.  A cut counts as 12 us at least:
+//    where the product without one takes that little, it is not cut, and among cuts below 12 us the fewest runs are taken.  Both
+//    sides, whole linears of 150 such shapes (N up to 2304, 4 % of all), us, replayed from a graph / launched one by one: without
+//    a cut 11.8 / 12.5, with the six runs the model would choose 12.4 / 13.7 (152 x 832 x 2304; 166 x 1216 x 2432 12.4 / 13.0 and
+//    12.8 / 14.4, but 218 x 640 x 2560 14.7 / 14.7 and 12.7 / 14.1); four runs 13.3 / 14.6, eight 12.2 / 13.7 (99 x 512 x 4736; 82 x
+//    2304 x 3328, four and seven: 13.2 / 14.2 and 13.7 / 14.6).  On average the model without that floor is 3 % ahead in a graph and 2 %
+//    outside of one.
 //  * 256x256 tiles: 1.5 per K block on a full chip (0.7 for a workgroup alone), 4.4 per tile, 15 us + partials for a cut last round.
 static double est_tile128(int64_t M, int64_t N, int kb, int cu, int* best_splits, int* best_tm) {
   double best = 1e30;
@@ -735,9 +739,11 @@ extern "C" int fp8k_token_linear(const void* x, const void* B, const float* sb, 
 
 // ---- batched per-tensor-scaled FP8 GEMM (the MLA absorbed products): every batch entry is a row-mode GEMM on the short-K
 // kernel or, for long K, on the 128x128 tile kernel (grid y = entry), whose per-row / per-column scale vectors are shared by all entries.
-// Up to eight K blocks the short-K kernel is ahead at every row count (1 .. 4096 rows, 16 and 128 entries: level to 3.6 times;
-// 128 entries of 64 x 512 x 128: 14.6 -> 5.7 us); at 16 and more blocks the tile kernel's ring and larger tile win from about
-// 1000 rows on and below it the two are within 15 % on a part-filled chip.
+// Up to eight K blocks the short-K kernel is ahead at every row count (1 .. 4096 rows, 16 and 128 entries: 1.03 - 3.7 times;
+// 128 entries of 64 x 512 x 128: 14.7 -> 6.2 us).  At 16 blocks the tile kernel's ring and larger tile are ahead with 4096 rows (16
+// entries 98 against 107 us, 128 entries 773 against 816) and at 32 blocks with 16 entries of up to 64 rows (17.1 against 19.1); in
+// between the short-K kernel still is, most with many entries of few rows (128 entries of 64 rows, K = 1536 / 2048 / 4096: 24.7 /
+// 31.6 / 54.1 against 47.7 / 56.1 / 93.1).  The line is where it is right for every count.
 constexpr int64_t kBmmShortK = 1024;
 static int bmm_impl(const void* A, const void* B, const float* sa, const float* sb, int64_t scale_stride, void* C, int64_t batch,
                     int64_t M, int64_t N, int64_t K, int64_t a_stride_b, int64_t lda, int64_t b_stride_b, int64_t ldb,

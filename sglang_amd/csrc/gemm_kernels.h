@@ -234,8 +234,9 @@ __device__ __forceinline__ void load_bias8(const void* bias, int64_t n, float (&
 // 256(n) x 256(m) x 128(k) workgroup tile, 8 wavefronts (2 along n x 4 along m), wave tile
 // 128(n) x 64(m) = 8 x 4 MFMA tiles of 16x16, K step 128 = one v_mfma_f32_16x16x128_f8f6f4.
 //
-// Bound: the matrix cores under the chip's power limit.  A bare loop of MFMAs on quantised normal data reaches 4.56 PFLOP/s in
-// the 16x16x128 form and 4.19 in the 32x32x64 form (4.94 both on zeros), with the same rounding error of a K block; the kernel
+// Bound: the matrix cores under the chip's power limit.  A bare loop of MFMAs on quantised normal data reaches 4.42 PFLOP/s in
+// the 16x16x128 form (fp8k_tune_mfma_peak) and 4.07 in the 32x32x64 form (form 0 of fp8k_tune_mfma_loop; 4.93 and 4.98 on zeros), with
+// the same rounding error of a K block; on one machine the kernel
 // with 32x32x64 tiles took 447 us at 4096 x 18432 x 7168 (block scales) where this one takes 426, 377 against 361 at 8192^3
 // (row scales), 200 against 193 at 2000 x 7168 x 18432 (UE8M0), 106 against 104 at 4096 x 32768 x 512.
 //

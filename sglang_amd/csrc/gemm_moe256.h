@@ -46,8 +46,8 @@ namespace fp8k {
 // weights that outgrow the last-level cache (moe256_once()).
 // The weights are then loaded non-temporally, and leave the L2 to the activation rows, which every n tile of the block reads
 // again; the result rows too are stored past it.  Whole layers, us, plain / ONCE: 256 experts, 7168 x 2048, top 8: 1024 tokens
-// 2105 / 1959, 4096 2622 / 2565; 7168 x 512: 1024 641 / 611, 3200 821 / 785; 64 experts, 7168 x 256, top 4, 1600 tokens
-// 187 / 184.  With several blocks per expert they share the tile in L2: 64 experts, 7168 x 2048, top 8, 2400 tokens 1248 / 1271.
+// 2040 / 1906, 4096 2518 / 2459; 7168 x 512: 1024 633 / 605, 3200 785 / 755; 64 experts, 7168 x 256, top 4, 1600 tokens
+// 177 / 171.  With several blocks per expert they share the tile in L2: 64 experts, 7168 x 2048, top 8, 2400 tokens 1248 / 1271.
 template <int OUT_DT, bool PAIRS, bool SORTED, bool FUSE = false, bool SCALED = false, bool ONCE = false>
 __global__ __launch_bounds__(512, 1) void moe_stream256_kernel(const GemmArgs p) {
   static_assert(!FUSE || (SORTED && !PAIRS), "the fused write-out is built for sorted activation scales");

@@ -563,8 +563,13 @@ static bool moe256_one_block(int64_t num_valid_tokens, int64_t num_experts) { re
 // Whether the 256-slot kernel loads its weights non-temporally (ONCE): one block per expert, so that no other workgroup reads the
 // tile, and weights that the 256 MB last-level cache cannot hold until the next call.  GEMM 1 counts the weights of GEMM 2 (half
 // as many) to its own: what GEMM 1 leaves alone, GEMM 2 finds again.  Whole layers, us, plain / this rule: 402 MB (64 experts,
-// 2048 x 1024, top 4, 512 tokens) 114 / 100, 352 MB (64 experts, 7168 x 256, 1600 tokens) 186 / 178; non-temporal all the same
+// 2048 x 1024, top 4, 512 tokens) 116 / 100, 352 MB (64 experts, 7168 x 256, 1600 tokens) 177 / 171; non-temporal all the same
 // at 201 MB (64 experts, 4096 x 256, 512 tokens) 73 / 93, at 100 MB (64 experts, 2048 x 256, 512 tokens) 50 / 56.
+// The number of blocks is that of even routing.  Where hot experts have several, their workgroups share a tile that was loaded to
+// pass by.  At some 32 slots per expert the rule is ahead whatever the skew (256 experts, 7168 x 2048, 1024 tokens: even 2036 / 1901,
+// Zipf's law 2462 / 2315, half the slots on 8 experts 2472 / 2304); at 94 - 140 it gains 3 - 6 % with even routing and 1 % on average
+// over skewed ones, between 3.5 % ahead and, with half the slots on a few experts, behind (3000 tokens: even 2309 / 2181, Zipf 3185 /
+// 3131, 32 hot experts 3255 / 3313; 256 experts, 2048 x 1024, 3000 tokens, 32 hot experts 580 / 616, the worst of 55 layers).
 static bool moe256_once(int64_t num_valid_tokens, int64_t num_experts, int64_t weight_bytes) {
   return moe256_one_block(num_valid_tokens, num_experts) && weight_bytes > (256LL << 20);
 }

@@ -180,7 +180,10 @@ __global__ __launch_bounds__(256) void group_quant_kernel(const void* __restrict
 // Segments per wave: four keep enough bytes in flight to stream a large input; up to a wave per wave slot of the chip (8192 segments,
 // 4 M elements) what counts is that the latency of one segment, not of four, stands in front of the product.  Whole linears,
 // quantisation and product, us, four / one: 32 x 4096 x 4096 10.7 / 9.5, 64 x 4096 x 4096 13.5 / 12.6, 200 x 7168 x 2304 15.0 / 14.1,
-// 128 x 7168 x 16384 43.2 / 42.4, 1000 x 24576 x 1536 50.6 / 49.8; level above (2048 x 7168 x 2304 41.2 / 41.2).
+// 128 x 7168 x 16384 41.3 / 40.5, 1000 x 24576 x 1536 50.6 / 49.8; level above (2048 x 7168 x 2304 41.2 / 41.2).
+// The kernel alone, row-major / column-major / packed UE8M0 scales: 32 x 4096 3.16 / 2.21, 3.23 / 2.33, 3.05 / 2.28; 512 x 8192 (8192
+// segments) 5.02 / 4.03, 4.94 / 4.06, 4.63 / 3.88; with silu_and_mul in front, which loads two streams, 32 x 4096 4.41 / 2.68, 4.38 /
+// 2.70, 4.23 / 2.69 and 512 x 8192 7.84 / 6.05, 7.70 / 6.07, 7.17 / 5.72; one segment in all is level in every form.
 constexpr int64_t kFewSegments = 8192;
 template <int DT, int GROUP, int KIND, int SEG, bool FUSE, bool MASKED>
 static int launch_group_quant_seg(const void* x, void* q, void* s, int64_t M, int64_t K, float eps, int64_t sm, int64_t sg,
