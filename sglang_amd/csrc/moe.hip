@@ -293,9 +293,10 @@ __global__ __launch_bounds__(256) void act_only_kernel(const void* __restrict__ 
 // 2.40 / 2.08, 512 x 8 x 2048 3.70 / 3.10, 1024 x 8 x 7168 20.0 / 20.3, 3000 x 6 x 7168 (258 MB) 47.7 / 45.6, 4096 x 8 x 7168
 // (470 MB) 100.5 / 103.1.
 // ELEM (moe_sum with 2..4 experts per token): the running sum is rounded to the element type after every addition.  16-bit rows, in
-// and out, go one by one from 256 MB on (on two machines: 20000 x 2 x 7168 158 / 169 and 151 / 155, 9000 x 2 x 7168 72 / 75 and 68.7 /
-// 69.4, 16384 x 4 x 4096 125 / 129 and 119 / 122; level for 16384 x 4 x 2048, 320 MB, 59 / 59); below, four are ahead or level (1 x 4 x 7168 2.86 / 2.60, 64 x 4 x 2048 2.92 / 2.66, 1024 x
-// 4 x 7168 12.9 / 12.8), and with 32-bit rows at every size (1024 x 4 x 7168 24.6 / 22.8, 16384 x 4 x 4096 257 / 253).
+// and out, go one by one from 256 MB on (one / four on two machines: 20000 x 2 x 7168 158 / 169 and 151 / 155, 9000 x 2 x 7168 72 / 75
+// and 68.7 / 69.4, 16384 x 4 x 4096 125 / 129 and 119 / 122; level for 16384 x 4 x 2048, 320 MB, 59 / 59); below, four are ahead or
+// level (1 x 4 x 7168 2.86 / 2.60, 64 x 4 x 2048 2.92 / 2.66, 1024 x 4 x 7168 12.9 / 12.8), and with 32-bit rows at every size
+// (1024 x 4 x 7168 24.6 / 22.8, 16384 x 4 x 4096 257 / 253).
 template <int DT, bool ELEM, int S>
 __device__ __forceinline__ void add_experts(const void* x, int64_t at, int64_t stride_k, int k0, float (&acc)[8]) {
   Raw8<DT> raw[S];
