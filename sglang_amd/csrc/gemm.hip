@@ -199,7 +199,7 @@ static Plan plan_base(int64_t M, int64_t N, int64_t K, int cu) {
 //    work - and a little more when the weights are new to the chip and the chip is full; 3 us of first loads and write-out per
 //    round of tiles, at most two rounds; a K cut adds the reduction launch and the float partials.  A cut counts as 12 us at least:
 //    where the product without one takes that little, it is not cut, and among cuts below 12 us the fewest runs are taken.  Both
-//    sides, whole linears of 150 such shapes (N up to 2304, 4 % of all), us, replayed from a graph / launched one by one: without
+//    sides, whole linears of 150 such shapes (N up to some 2500, 4 % of all), us, replayed from a graph / launched one by one: without
 //    a cut 11.8 / 12.5, with the six runs the model would choose 12.4 / 13.7 (152 x 832 x 2304; 166 x 1216 x 2432 12.4 / 13.0 and
 //    12.8 / 14.4, but 218 x 640 x 2560 14.7 / 14.7 and 12.7 / 14.1); four runs 13.3 / 14.6, eight 12.2 / 13.7 (99 x 512 x 4736; 82 x
 //    2304 x 3328, four and seven: 13.2 / 14.2 and 13.7 / 14.6).  On average the model without that floor is 3 % ahead in a graph and 2 %
