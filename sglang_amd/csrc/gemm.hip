@@ -9,6 +9,7 @@
 #include "gemm_direct_quant.h"
 #include "gemm_skinny.h"
 #include "gemm_tile128.h"
+#include "gemm_tile64.h"
 
 #include "../../include/fp8k_tune.h"
 
@@ -17,7 +18,7 @@ namespace fp8k {
 struct Plan {
   int kind;    // 0 = generic, 1 = tile256, 2 = weight-streaming through LDS (33..128 rows), 3 = direct (<= 32 rows),
                // 4 = tiles of 128 weight rows, 5 = direct with K cut across the waves of a workgroup (<= 16 rows, N below 16 K),
-               // 7 = skinny strips over all of K (<= 128 rows, N up to 16 K)
+               // 7 = skinny strips over all of K (<= 64 rows, N up to 16 K), 8 = tiles of 64 weight rows
   int splits;  // >1: split-K through the float workspace
   int kb_per_split;
   int tm;      // rows per block of the streaming kernels, activation rows of a tile (kind 4)
@@ -39,6 +40,12 @@ static Plan plan_tile128(int64_t M, int64_t N, int kb, int splits, int tm) {
   pl.kb_per_split = (kb + splits - 1) / splits;
   pl.splits = (kb + pl.kb_per_split - 1) / pl.kb_per_split;
   pl.ws_bytes = pl.splits > 1 ? (int64_t)pl.splits * M * N * 4 : 0;
+  return pl;
+}
+
+static Plan plan_tile64(int64_t M, int64_t N, int kb, int splits) {
+  Plan pl = plan_tile128(M, N, kb, splits, kT64);
+  pl.kind = 8;
   return pl;
 }
 
@@ -98,14 +105,13 @@ static Plan plan_wavek(int64_t M, int64_t N, int64_t K, int cu) {
   pl.kb_per_split = (kb + 8 / nw - 1) / (8 / nw);
   return pl;
 }
-// Up to 128 rows: the strips of weight rows that one workgroup each runs over all of K are as narrow as leaves every CU one.
+// Up to 64 rows: the strips of weight rows that one workgroup each runs over all of K are as narrow as leaves every CU one.
 constexpr int64_t kSkinnyMaxN = 16384;
 static Plan plan_skinny(int64_t M, int64_t N, int64_t K, int cu) {
   Plan pl{7, 1, 0, 0, 0, 0};
-  pl.tm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
+  pl.tm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
   pl.halves = N <= 16 * cu ? 1 : N <= 32 * cu ? 2 : 4;
   if (g_force_kind == 7 && (g_force_splits == 1 || g_force_splits == 2 || g_force_splits == 4)) pl.halves = g_force_splits;  // tuning aid
-  if (pl.tm == 128) pl.halves = 2;
   return pl;
 }
 // Where it is ahead (M = 4 .. 64 x 16 widths up to 20480 x 9 depths up to 18432, timed against the other decode kernels and the
@@ -122,7 +128,6 @@ static bool prefers_skinny(int64_t M, int64_t N, int64_t K, int cu) {
   if (M <= 8) return K <= 9216;  // above: the wave-cut kernel, whose waves keep all of their K range in flight
   if (M <= 16) return true;
   if (M <= 32) return !wide || fills || K <= 6144;
-  if (M > 64) return !wide && K >= 1536 && K <= (N >= 16 * cu ? 4608 : 3072);
   if (wide) return K > 1536 && K <= (fills ? 10240 : 4608);
   return K <= (N <= 16 * cu ? 7168 : 6144);
 }
@@ -225,6 +230,26 @@ static double est_tile128(int64_t M, int64_t N, int kb, int cu, int* best_splits
   return best;
 }
 
+// The same for tiles of 64 x 64, as many as the chip has CUs at most (one round), more than 64 rows and more than eight K blocks (up
+// to eight they are level with the larger tiles, 0.95 - 1.05): a wave runs 0.9 us per K block of its own, every fourth of the range, and
+// more where the weights come out of HBM for this tile alone and the chip is full.  Fitted to 137 pairs of shape and K cut (65 .. 1150
+// rows, N = 512 .. 9856, K = 896 .. 17664; rms error 6 %).  On 68 such shapes the choice between all tiles is 0.2 % behind the best
+// and 7 % ahead of the larger tiles alone (up to 23 %; whole linears, us, replayed from a graph, weights out of HBM / out of the
+// last-level cache: 238 x 3456 x 3072 18.1 -> 14.3 / 14.7 -> 12.8, 159 x 4288 x 4224 20.8 -> 16.2 / 17.4 -> 14.1, 73 x 576 x 2688
+// 14.6 -> 11.0 / 13.8 -> 10.4, 411 x 1024 x 3200 15.8 -> 13.6 / 15.7 -> 13.3).
+static double est_tile64(int64_t M, int64_t N, int kb, int cu, int* best_splits) {
+  double best = 1e30;
+  const int64_t tm = (M + kT64 - 1) / kT64, tiles = tm * ((N + kT64 - 1) / kT64);
+  if (M <= kT64 || kb <= 8) return best;
+  for (int s = 1; s <= 8 && tiles * s <= cu && (s == 1 || s <= kb / 8); ++s) {
+    const double cold = 1.0 / (double)tm, fill = (double)(tiles * s) / cu;
+    double t = 4.75 + (((kb + s - 1) / s + 3) / 4) * (0.91 + cold * (0.64 * fill - 0.26));
+    if (s > 1) t += 2.7 + (double)s * M * N * 8.0 / 6.9e6;
+    if (t < best) { best = t; *best_splits = s; }
+  }
+  return best;
+}
+
 static double est_tile256(const Plan& pl, int64_t M, int64_t N, int kb, int cu) {
   const int64_t tiles = ((M + kTileM - 1) / kTileM) * ((N + kTileN - 1) / kTileN), rest = tiles % cu;
   auto per_kb = [&](int64_t wgs) { return 0.68 + 0.87 * std::min(1.0, (double)wgs / cu); };
@@ -242,17 +267,17 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K) {
   const int kb = (int)(K / kTileK), cu = num_cu();  // once: asking the runtime for the device costs more than all of the arithmetic
   // tuning aid: the K cut in the low byte, 256 for tiles of 64 activation rows
   if (g_force_kind == 4 && N % 8 == 0) return plan_tile128(M, N, kb, g_force_splits & 255, g_force_splits & 256 ? 64 : 128);
+  if (g_force_kind == 8 && N % 8 == 0) return plan_tile64(M, N, kb, g_force_splits);
   pl = plan_base(M, N, K, cu);
   if (g_force_kind >= 0 || N % 8 != 0 || M <= 16) return pl;
-  int splits = 1, rows = 0;
-  if (pl.kind == 1) {
-    if (est_tile128(M, N, kb, cu, &splits, &rows) < est_tile256(pl, M, N, kb, cu)) return plan_tile128(M, N, kb, splits, rows);
-  } else if (pl.kind == 2) {
-    // The streaming kernel keeps 256-row tiles x 2 - 3 K ranges where 128-row tiles are a little more than half a chip and a K cut
-    // would be a second round: 97 x 18240 x 15104 70 us against 79, 97 x 17152 x 8192 41 against 45; 122 x 20288 x 6400 42 against 39,
-    // 106 x 23040 x 5760 41 against 35.  Everywhere else the tiles are ahead, up to twice (108 x 15616 x 1024 8.2 against 19.3).
-    if (!(N > 64 * cu && N <= 80 * cu && K >= 8192)) {
-      est_tile128(M, N, kb, cu, &splits, &rows);
+  int splits = 1, rows = 0, splits64 = 1;
+  // The streaming kernel keeps 256-row tiles x 2 - 3 K ranges where 128-row tiles are a little more than half a chip and a K cut
+  // would be a second round: 97 x 18240 x 15104 70 us against 79, 97 x 17152 x 8192 41 against 45; 122 x 20288 x 6400 42 against 39,
+  // 106 x 23040 x 5760 41 against 35.  Everywhere else the tiles are ahead, up to twice (108 x 15616 x 1024 8.2 against 19.3).
+  if (pl.kind == 1 || (pl.kind == 2 && !(N > 64 * cu && N <= 80 * cu && K >= 8192))) {
+    const double t128 = est_tile128(M, N, kb, cu, &splits, &rows), t64 = est_tile64(M, N, kb, cu, &splits64);
+    if (pl.kind == 2 || std::min(t128, t64) < est_tile256(pl, M, N, kb, cu)) {
+      if (t64 < t128) return plan_tile64(M, N, kb, splits64);
       if (rows) return plan_tile128(M, N, kb, splits, rows);
     }
   } else if (pl.kind == 3 && N > 32 * cu && N < 48 * cu && K > 6144) {
@@ -278,7 +303,7 @@ static int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 // The skinny kernel's waves fetch 16 scales per load instead of 32: there the copy (2 - 3 us) is level at 16 rows x 128 K blocks
 // and ahead above (without it 32 x 128 takes 34.8 us against 27.4 with column-major scales, 64 x 64 32.4 against 21.1).
 static bool wants_scale_copy(const Plan& pl, int64_t M, int64_t K) {
-  return pl.kind == 7 ? M * (K / kTileK) >= 2048 : M > 32 && (pl.kind == 1 || pl.kind == 2 || pl.kind == 4);
+  return pl.kind == 7 ? M * (K / kTileK) >= 2048 : M > 32 && (pl.kind == 1 || pl.kind == 2 || pl.kind == 4 || pl.kind == 8);
 }
 static int64_t block_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -293,7 +318,7 @@ __global__ __launch_bounds__(256) void scale_to_column_major_kernel(const float*
   dst[i] = src[(int64_t)m * stride_m + k];
 }
 
-// the two tile kernels (plan kinds 1 and 4); `a` carries the operands, the plan the tiling
+// the tile kernels (plan kinds 1, 4 and 8); `a` carries the operands, the plan the tiling
 template <int MODE, int OUT_DT, int BIAS_DT>
 static int launch_tiles(const GemmArgs& a0, const Plan& pl, hipStream_t st) {
   GemmArgs a = a0;
@@ -319,6 +344,18 @@ static int launch_tiles(const GemmArgs& a0, const Plan& pl, hipStream_t st) {
     const int64_t quads = (int64_t)a.M * (a.N / 4);
     hipLaunchKernelGGL((splitk_reduce_kernel<MODE, OUT_DT, BIAS_DT>), dim3((unsigned)((quads + 255) / 256)), dim3(256),
                        0, st, a);
+    return check_launch("splitk_reduce");
+  }
+  if (pl.kind == 8) {
+    a.tiles_m = (a.M + kT64 - 1) / kT64;
+    a.tiles_n = (a.N + kT64 - 1) / kT64;
+    const unsigned nwg = (unsigned)(((int64_t)a.tiles_m * a.tiles_n * pl.splits + 7) / 8 * 8);
+    if (pl.splits == 1) hipLaunchKernelGGL((gemm_tile64_kernel<MODE, OUT_DT, BIAS_DT, false>), dim3(nwg), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gemm_tile64_kernel<MODE, OUT_DT, BIAS_DT, true>), dim3(nwg), dim3(256), 0, st, a);
+    int rc = check_launch("gemm_tile64");
+    if (rc || pl.splits == 1) return rc;
+    const int64_t quads = (int64_t)a.M * (a.N / 4);
+    hipLaunchKernelGGL((splitk_reduce_kernel<MODE, OUT_DT, BIAS_DT>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, a);
     return check_launch("splitk_reduce");
   }
   const int ntiles = a.tiles_m * a.tiles_n;
@@ -397,8 +434,7 @@ static int launch(const GemmArgs& a0, const Plan& pl, hipStream_t st) {
   } while (0)
     if (pl.tm == 16) FP8K_SKINNY_NW(16);
     else if (pl.tm == 32) FP8K_SKINNY_NW(32);
-    else if (pl.tm == 64) FP8K_SKINNY_NW(64);
-    else FP8K_SKINNY(128, 2);
+    else FP8K_SKINNY_NW(64);
 #undef FP8K_SKINNY_NW
 #undef FP8K_SKINNY
     return check_launch("gemm_skinny");
@@ -580,7 +616,7 @@ extern "C" int fp8k_block_gemm_ue8m0(const void* A, const void* B, const int32_t
   // the matrix core applies the scales only in the tile kernels, and every plan for more than 128 rows and whole K blocks is one of
   // them; smaller problems take the float-scale entry point with the exponents expanded to floats
   const Plan pl = make_plan(M, N, K);
-  FP8K_REQUIRE(M > 128 && (pl.kind == 1 || pl.kind == 4), "%s: built for M > 128 with K a multiple of 128 (got M=%lld, K=%lld); expand the "
+  FP8K_REQUIRE(M > 128 && (pl.kind == 1 || pl.kind == 4 || pl.kind == 8), "%s: built for M > 128 with K a multiple of 128 (got M=%lld, K=%lld); expand the "
                "scales and call fp8k_block_gemm", op, (long long)M, (long long)K);
   const int64_t need = pl.ws_bytes;
   if (need > 0 && (!workspace || workspace_bytes_given < need))

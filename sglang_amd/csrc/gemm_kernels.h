@@ -111,7 +111,7 @@ __device__ __forceinline__ void spread_rows(uint32_t v, uint32_t (&out)[4]) {
 }
 
 template <int OUT_DT>
-__device__ __forceinline__ void store4(void* C, int64_t idx, float a, float b, float c, float d) {
+__device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
   uint2 o;
   if (OUT_DT == FP8K_BF16) {
     o.x = pack_bf16x2(a, b);
@@ -120,7 +120,11 @@ __device__ __forceinline__ void store4(void* C, int64_t idx, float a, float b, f
     o.x = f32_to_f16_bits(a) | (f32_to_f16_bits(b) << 16);
     o.y = f32_to_f16_bits(c) | (f32_to_f16_bits(d) << 16);
   }
-  *reinterpret_cast<uint2*>((u16*)C + idx) = o;
+  return o;
+}
+template <int OUT_DT>
+__device__ __forceinline__ void store4(void* C, int64_t idx, float a, float b, float c, float d) {
+  *reinterpret_cast<uint2*>((u16*)C + idx) = pack4<OUT_DT>(a, b, c, d);
 }
 
 template <int DT>

@@ -1,4 +1,4 @@
-// FP8 GEMM for decode batches (9 .. 128 activation rows), gfx950: no float partials, no reduction launch.
+// FP8 GEMM for decode batches (9 .. 64 activation rows), gfx950: no float partials, no reduction launch.
 //
 // The weights are a stream from HBM that has to be spread over all CUs.  With narrow strips of weight rows per workgroup (16 or
 // 32: one or two to a CU) every workgroup can run over the whole of K and write finished rows; the price is that each of them
@@ -7,8 +7,8 @@
 // empty the weight stream.  Loads of a wave return in order, so a wave that waits for an activation line also waits for every
 // weight line it asked for before.  Hence two kinds of waves:
 //
-//   * eight streaming waves, NW along n (16 weight rows each) x KS = 8 / NW along k.  A trip covers eight K blocks (four above 64
-//     rows), U consecutive ones per wave; a wave keeps its next D K blocks of weights in flight in registers (whole-line loads, re-laid
+//   * eight streaming waves, NW along n (16 weight rows each) x KS = 8 / NW along k.  A trip covers eight K blocks,
+//     U consecutive ones per wave; a wave keeps its next D K blocks of weights in flight in registers (whole-line loads, re-laid
 //     out through a private LDS slot as in gemm_direct_kernel) and takes its activations from LDS.  It never waits for a load
 //     of anybody else's.
 //   * NL loading waves, which bring the activations of a trip - [rows][1 KB], 1 KB per instruction straight into LDS - one
@@ -19,20 +19,20 @@
 //
 // GEMM alone, bf16, against what ran before (K cut across workgroups with partials, or across the waves of one whose lanes fetched
 // their own activations), weights rotated over 600 MB: 32 x 4096 x 4096 10.6 -> 7.6 us, 24 x 7168 x 16384 32.4 -> 26.7 (117 MB: 4.4
-// TB/s), 64 x 4096 x 4096 15.2 -> 10.3, 13 x 12224 x 3968 19.4 -> 11.8, 128 x 4096 x 4096 17.9 -> 15.6, 96 x 8192 x 4096 22.6 -> 16.1.
+// TB/s), 64 x 4096 x 4096 15.2 -> 10.3, 13 x 12224 x 3968 19.4 -> 11.8.
 #pragma once
 
 #include "gemm_direct.h"
 
 namespace fp8k {
 
-constexpr int kSkinnyMaxM = 128;
-constexpr int skinny_trip(int tm) { return tm <= 64 ? 8 : 4; }  // K blocks of a trip
+constexpr int kSkinnyMaxM = 64;
+constexpr int kSkinnyTrip = 8;  // K blocks of a trip
 
 template <int TM, int NW, int MODE, int OUT_DT, int BIAS_DT>
 __global__ __launch_bounds__(TM <= 32 ? 640 : 768) void gemm_skinny_kernel(const GemmArgs p) {
-  static_assert(TM == 16 || TM == 32 || TM == 64 || TM == 128, "16, 32, 64 or 128 rows");
-  constexpr int TRIP = skinny_trip(TM), ROW = TRIP * kTileK;  // K blocks of a trip, bytes of a staged row
+  static_assert(TM == 16 || TM == 32 || TM == 64, "16, 32 or 64 rows");
+  constexpr int TRIP = kSkinnyTrip, ROW = TRIP * kTileK;  // K blocks of a trip, bytes of a staged row
   static_assert((NW == 1 || NW == 2 || NW == 4) && TRIP * NW % 8 == 0, "waves along n");
   constexpr int MS = TM / 16, KS = 8 / NW, U = TRIP / KS;  // U: K blocks of a trip per wave
   // K blocks of weights in flight per wave (whole trips): more is slower, 24 x 7168 x 16384 25.2 us with 8 against 24.6
