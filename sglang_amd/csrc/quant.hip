@@ -389,23 +389,25 @@ __global__ __launch_bounds__(256) void tensor_quant_kernel(const void* __restric
 
 // ------------------------------------------------------------------------------------------------
 // per-tensor quant of a strided [H, S, D] tensor into a contiguous one (the MLA absorbed products): 8 elements (a chunk) a
-// lane, four chunks in flight, in grid-stride.  Bound by latency at decode sizes: with 2048 workgroups the maxima queued up
-// at the one atomic (8.0 us for 64 tokens x 128 heads x 128, 2 MB), so the maximum pass takes at most 512 workgroups and four
-// chunks per lane before it takes a second workgroup's atomic; IDX is 32-bit wherever the chunks can be counted so, because
+// lane, four chunks in flight, in grid-stride.  The maxima queue up at one atomic, so the maximum pass takes one workgroup of 1024
+// threads per CU at most, and four chunks per lane before it takes a second one's atomic (both passes, us, 512 of 256 threads / this:
+// 3.7 MB 7.9 / 7.1, 5.9 MB 10.0 / 8.4, 10 MB 13.0 / 10.3, 17 MB 15.5 / 13.2, 67 MB 33.9 / 31.6); IDX is 32-bit wherever the chunks can be counted so, because
 // the two divisions per chunk (row, then head) are the arithmetic of this kernel.
 // ------------------------------------------------------------------------------------------------
+constexpr int mla_threads(bool quant) { return quant ? 256 : 1024; }
 template <int DT, bool QUANT, typename IDX>
-__global__ __launch_bounds__(256) void rows_tensor_quant_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
+__global__ __launch_bounds__(mla_threads(QUANT)) void rows_tensor_quant_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
                                                                 float* __restrict__ s, int64_t rows, int S, int D,
                                                                 int64_t stride_h, int64_t stride_s, float eps) {
-  __shared__ float red[4];
+  constexpr int T = mla_threads(QUANT);
+  __shared__ float red[16];
   const IDX chunks = (IDX)(D / 8);          // per row; the host checks D % 8 == 0 and the alignment of every row
   const IDX total = (IDX)rows * chunks;
-  const IDX step = (IDX)gridDim.x * 256;
+  const IDX step = (IDX)gridDim.x * T;
   const float inv = QUANT ? 1.0f / s[0] : 0.f;
   float m = 0.f;
   constexpr int U = 4;
-  for (IDX i0 = (IDX)blockIdx.x * 256 + threadIdx.x; i0 < total; i0 += U * step) {
+  for (IDX i0 = (IDX)blockIdx.x * T + threadIdx.x; i0 < total; i0 += U * step) {
     Raw8<DT> t[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -436,7 +438,11 @@ __global__ __launch_bounds__(256) void rows_tensor_quant_kernel(const void* __re
     }
   }
   if (!QUANT) {
-    m = block_max_256(fmaxf(m, eps), red);
+    m = group_max<64>(fmaxf(m, eps));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < T / 64; ++i) m = fmaxf(m, red[i]);
     // non-negative floats order like their bit patterns
     if (threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned int*>(s), __float_as_uint(m / kFp8Max));
   }
@@ -786,13 +792,13 @@ static int tensor_quant_mla(const void* x, void* q, float* s, int64_t H, int64_t
   const int64_t rows = H * S, chunks = rows * (D / 8);
   const bool narrow = chunks < (1LL << 31);  // room for the four steps past the end
   const dim3 block(256);
-  const dim3 grid_max((unsigned)std::min<int64_t>(512, (chunks + 1023) / 1024)), grid_q((unsigned)std::min<int64_t>(2048, (chunks + 255) / 256));
+  const dim3 grid_max((unsigned)std::min<int64_t>(num_cu(), (chunks + 4095) / 4096)), grid_q((unsigned)std::min<int64_t>(2048, (chunks + 255) / 256));
   // one chunk per lane is enough to work on: the more workgroups share it, the shorter the loads
   const dim3 grid_once((unsigned)std::min<int64_t>(kMlaOnceGroups, (chunks + 1023) / 1024));
   FP8K_REQUIRE(!sync || fp8k_tensor_quant_mla_takes_sync(H * S * D), "%s: not a size of the one-launch form", op);
 #define FP8K_MLAQ2(DT, IDX)                                                                                                 \
   do {                                                                                                                      \
-    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, false, IDX>), grid_max, block, 0, st, x, (uint8_t*)q, s, rows, (int)S, \
+    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, false, IDX>), grid_max, dim3(mla_threads(false)), 0, st, x, (uint8_t*)q, s, rows, (int)S, \
                        (int)D, x_stride_h, x_stride_s, eps);                                                                \
     hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, true, IDX>), grid_q, block, 0, st, x, (uint8_t*)q, s, rows, (int)S,    \
                        (int)D, x_stride_h, x_stride_s, eps);                                                                \
