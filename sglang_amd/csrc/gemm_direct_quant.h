@@ -11,7 +11,9 @@
 // Whole linear, bf16, two launches -> this one, one weight: M = 1: 4608 x 7168 13.5 -> 8.7 us (33 MB: 5.3 us at the read ceiling),
 // 6144 x 4096 10.9 -> 7.4, 7168 x 18432 28.9 -> 22.1, 1024 x 1024 9.7 -> 5.2 (the host's time for one launch); M = 8, at the limit
 // of M * K: 6144 x 4096 11.7 -> 8.8, per-token 11.1 -> 9.1.  With the weights rotated over 600 MB, so that none comes out of the
-// memory-side cache: 9.4, 8.2, 22.4, 5.3; 9.6, 9.9.
+// memory-side cache: 9.4, 8.2, 22.4, 5.3; 9.6, 9.9.  Per token the row's scale is one more serial step; with the maxima of all rows
+// taken at once, 32 lanes to a row, rather than 64 lanes to two rows in turn, 13 x 3456 x 1152 6.2 -> 5.7 us (replayed from a graph),
+// 16 x 896 x 640 5.6 -> 5.2, 11 x 8640 x 2048 8.8 -> 8.4, 8 x 4096 x 2048 6.4 -> 6.2, 1 x 4608 x 7168 9.2 level.
 //
 // Split of the work, K order, LDS re-layout of the weights and summation are gemm_wavek_kernel's, and the quantisation is
 // that of group_quant_kernel (block mode) or token_quant_kernel (row mode), so results are those of the two launches bit for
@@ -98,11 +100,11 @@ __global__ __launch_bounds__(512, 4) void gemm_wavek_quant_kernel(const GemmArgs
       if (l8 == 0 && base + 4 * j < groups) sgrp[base + 4 * j] = m;
     }
     lds_barrier();
-    for (int m = w; m < p.M; m += 8) {
+    if (const int m = tid >> 5; m < p.M) {  // 32 lanes to a row, all 16 at once (64: two in turn)
       float mx = 0.f;
-      for (int g = lane; g < kb_all; g += 64) mx = fmaxf(mx, sgrp[m * kb_all + g]);
-      const float sc = group_max<64>(mx) / kFp8Max;
-      if (lane == 0) {
+      for (int g = lane & 31; g < kb_all; g += 32) mx = fmaxf(mx, sgrp[m * kb_all + g]);
+      const float sc = group_max<32>(mx) / kFp8Max;
+      if ((lane & 31) == 0) {
         srow[m] = sc;
         sinv[m] = sc == 0.f ? 0.f : 1.0f / sc;
       }
