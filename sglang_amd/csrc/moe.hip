@@ -672,6 +672,23 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
 #undef FP8K_SHORTK
     return check_launch(op);
   }
+  // Few blocks with 16 slots: at most four strips of 16 weight rows per CU, which tiles of 128 rows would put on half of the CUs.  Whole layers,
+  // time over that with the tiles, at 1 / 2 / 3 / 4 tokens: 64 experts, 7168 x 256, top 8 0.69 / 0.79 / 0.88 / 0.90 (39.8 -> 27.7 us at one
+  // token), 128 experts, 4096 x 512, top 4 0.75 / 0.81 / 0.88 / 0.88, 64 experts, 2048 x 256, top 6 0.90 - 0.97; 256 experts, 7168 x 2048, top 4, one
+  // token 0.82.  With six strips 64 experts, 2048 x 256 took 1.13 and 256 experts, 4096 x 512 1.05 times as long.  Waves along n: two
+  // from 1.5 strips per CU on (1.5: 0.80 - 0.81 against 0.85 - 0.87 with one; at one strip 0.78 - 0.82 against 0.73 - 0.78) or where eight
+  // would share less than four K blocks each, four from three on (three: 0.82 - 0.88 against 0.87 - 0.95 with two; 2.5: 0.95 against 0.85).
+  const int64_t strips = blocks_max * ((N + 15) / 16), cu = num_cu();
+  if (block_m == 16 && strips <= 4 * cu && K >= 8 * kTileK) {
+    const int kb = (int)(K / kTileK);
+    a.wk_nw = strips >= 3 * cu ? 4 : 2 * strips >= 3 * cu || kb < 32 ? 2 : 1;
+    a.tiles_n = (int)((N + 16 * a.wk_nw - 1) / (16 * a.wk_nw));
+    a.kb_per_split = (kb + 8 / a.wk_nw - 1) / (8 / a.wk_nw);
+    const dim3 grid((unsigned)(blocks_max * a.tiles_n)), block(512);
+    if (out_dtype == FP8K_BF16) hipLaunchKernelGGL((moe_wavek_kernel<FP8K_BF16>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((moe_wavek_kernel<FP8K_F16>), grid, block, 0, st, a);
+    return check_launch(op);
+  }
   if (direct) {
     if (out_dtype == FP8K_BF16) {
       if (block_m == 16) FP8K_MOE_DIRECT(16, FP8K_BF16);
