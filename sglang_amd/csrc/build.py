@@ -18,7 +18,7 @@ LIB = os.path.join(HERE, "libfp8k.so")
 HOST_SRC = "host.cpp"
 HOST = os.path.join(os.path.dirname(HERE), "_host.so")  # the extension module sglang_amd._host, linked against LIB
 SOURCES = ["api.hip", "quant.hip", "gemm.hip", "moe.hip", "tune.hip"]
-HEADERS = ["fp8k_common.h", "quant_math.h", "gemm_kernels.h", "gemm_direct.h", "gemm_direct_quant.h", "gemm_moe256.h", "gemm_moe_regx.h", "gemm_moe_shortk.h", "gemm_skinny.h", "gemm_tile128.h", "gemm_tile64.h", "gemm_bmm.h", os.path.join("..", "..", "include", "fp8k.h"),
+HEADERS = ["fp8k_common.h", "quant_math.h", "gemm_kernels.h", "gemm_direct.h", "gemm_direct_quant.h", "gemm_moe256.h", "gemm_moe_shortk.h", "gemm_skinny.h", "gemm_tile128.h", "gemm_tile64.h", "gemm_bmm.h", os.path.join("..", "..", "include", "fp8k.h"),
            os.path.join("..", "..", "include", "fp8k_tune.h")]
 
 # -packed-fp32-ops off: packed float32 VALU forms are not used on this hardware pool.

@@ -2,7 +2,6 @@
 // GEMM (host side; the device code is the grouped form of gemm_direct_kernel for 16/32-slot blocks, of
 // gemm_stream_kernel for 64/128 and moe_stream256_kernel or moe_regx_kernel for 256), silu_and_mul and the top-k sum.  No allocation, no synchronisation, no host reads of device data.
 #include "gemm_direct.h"
-#include "gemm_moe_regx.h"
 #include "gemm_moe_shortk.h"
 #include "gemm_moe256.h"
 
@@ -586,15 +585,6 @@ static int64_t moe_blocks_in_use(int64_t slots, int64_t num_experts, int64_t blo
   return std::min(capacity, std::min(slots, num_experts + 1 + slots / block_m));
 }
 
-// Whether a short K goes to moe_regx_kernel, which gains with the slots that its four waves can fill: time of whole layers over that with
-// the 256x256 tiles, at 90 / 130 / 200 / 300 / 500 slots per expert: 64 experts, 7168 rows, K = 256 0.95 / 0.99 / 0.89 / 0.87 / 0.88;
-// K = 512 1.00 / 1.00 / 0.92 / 0.90 / 0.90; 128 experts, 4096 rows, K = 512 1.02 / 0.97 / 0.94; 256 experts, 7168 rows, K = 512, 90
-// slots 1.03.  In between it also takes enough result to share out: 64 experts, 140 .. 175 slots, 2048 rows 1.02 - 1.04, 4096 rows 1.02 at
-// 140 and 0.97 - 0.98 at 150 and 160, 7168 rows 0.96 - 0.97.  Far beyond, 1800 slots, 0.89 - 0.91.
-static bool moe_regx_pays(int64_t slots, int64_t num_experts, int64_t N) {
-  return slots >= 192 * num_experts || (slots >= 144 * num_experts && slots * N >= (40LL << 20));
-}
-
 static int moe_block_gemm_impl(const void* A, const void* B, const float* As, const float* Bs, void* C,
                                const int32_t* sorted_token_ids, const int32_t* expert_ids,
                                const int32_t* num_tokens_post_padded, const float* topk_weights,
@@ -702,27 +692,6 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
 #undef FP8K_MOE_DIRECT
   FP8K_REQUIRE((as_sorted ? sorted_capacity : xrows) * as_stride_m + (K / kTileK) * as_stride_k < 0x38000000LL,
                "%s: activation scale tensor too large", op);
-  if (block_m == 256 && as_sorted && !pow2_scales && K >= 2 * kTileK && K <= kMoeRegxMaxKb * kTileK && N % 128 == 0 && ldc % 8 == 0 &&
-      aligned(C, 16) && num_valid_tokens * ldc * 2 <= 0xE0000000LL && N * ldb < (1LL << 31) &&
-      moe_regx_pays(num_valid_tokens, num_experts, N)) {
-    // runs per 128-slot part: about two rounds of two workgroups per CU (one round / two / three, us: 128 experts, 4096 x 256, 3200 tokens of
-    // top 8 320 / 304 / 306; 64 experts, 7168 x 256, 4000 of top 8 508 / 493 / 494), and no more weight scales than lanes
-    const int64_t tiles = N / 128, kb = K / kTileK, longest = kMoeRegxScales / kb;
-    const int64_t parts = std::min(2 * blocks_max, num_valid_tokens / 128 + num_experts / 2 + 1);
-    const int64_t runs = std::min(tiles, std::max(4 * num_cu() / parts + 1, (tiles + longest - 1) / longest));
-    a.tiles_n = (int)runs;
-    const dim3 grid((unsigned)((blocks_max + 7) / 8 * 8 * 2 * runs)), block(256);  // far below 2^31: so is the result
-#define FP8K_REGX(KB) \
-  do { \
-    if (out_dtype == FP8K_BF16) hipLaunchKernelGGL((moe_regx_kernel<KB, FP8K_BF16>), grid, block, 0, st, a); \
-    else hipLaunchKernelGGL((moe_regx_kernel<KB, FP8K_F16>), grid, block, 0, st, a); \
-  } while (0)
-    if (kb == 2) FP8K_REGX(2);
-    else if (kb == 3) FP8K_REGX(3);
-    else FP8K_REGX(4);
-#undef FP8K_REGX
-    return check_launch(op);
-  }
   if (block_m == 256) {
     // Up to about 200 slots per expert nearly every expert is one block and the items cost about the same: one walking
     // workgroup per CU (a multiple of 8: one share per XCD), which requests an item's first blocks in front of the
