@@ -388,9 +388,11 @@ __global__ __launch_bounds__(512, 2) void gemm_wavek_kernel(const GemmArgs p) {
 // The same for a grouped launch of few 16-slot blocks (the first GEMM of a decode step that hits few experts of a small or sharded
 // intermediate size): tiles of 128 weight rows, a wave per 16 of them over all of K, leave most CUs idle, and those at work stream
 // 128 x K bytes each.  Here a workgroup owns 16 * NW rows of a block's expert and its waves cut K.  The block's rows and the slots
-// they go to come from the slot table; workgroups of a block are dealt over all XCDs (every weight line is read once).  Bound by the
-// latency of the first lines and by launch: the first GEMM of one token, 8 experts of 512 x 7168 (29 MB, 5 us at the copy rate) 19.9 -> 8.0 us, 4
-// experts of 1024 x 4096 13.8 -> 6.7.  Eight K blocks in flight per wave are level to 10 % slower.
+// they go to come from the slot table; workgroups of a block are dealt over all XCDs, so a weight line is read once per block of its
+// expert.  Bound by the latency of the first lines and by launch: the first GEMM of one token, 8 experts of 512 x 7168 (29 MB, 5 us at
+// the copy rate) 19.9 -> 8.0 us, 4 experts of 1024 x 4096 13.8 -> 6.7.  Eight K blocks in flight per wave are level to 10 % slower.
+// The grid is sized for the blocks that a table aligned over the launch's own experts can have in use; a table may have more (blocks of
+// other ranks' experts, blocks without slots), so a workgroup goes on by that number of blocks.  The loop costs 2 % (0.1 - 0.2 us).
 // ------------------------------------------------------------------------------------------------
 template <int OUT_DT>
 __global__ __launch_bounds__(512, 4) void moe_wavek_kernel(const GemmArgs p) {
@@ -398,88 +400,94 @@ __global__ __launch_bounds__(512, 4) void moe_wavek_kernel(const GemmArgs p) {
   __shared__ __attribute__((aligned(16))) uint8_t wl[8][16 * kTileK];  // per wave: one K block of its 16 weight rows
   __shared__ __attribute__((aligned(16))) float red[8][64][4];
 
-  const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int r = lane & 15, kq = lane >> 4;
   const int NW = p.wk_nw, nw = w % NW, ks = w / NW;
-  const int mb = (int)blockIdx.x / p.tiles_n;
-  if (mb >= moe_blocks_used(p)) return;
-  const int expert = as_const_ints(p.expert_ids)[mb];
-  const int n0w = (((int)blockIdx.x - mb * p.tiles_n) * NW + nw) * 16;
-  const int slot = p.sorted_ids[mb * 16 + r];
-  const bool real = slot < p.num_valid;
-  const int row = real ? slot / p.top_k : 0;
-  const int kb_all = p.K / kTileK, kb0 = ks * p.kb_per_split;
-  // an expert of another rank: no K block, zeros are stored
-  const int nkb = n0w < p.N && expert >= 0 ? max(min(kb_all, kb0 + p.kb_per_split) - kb0, 0) : 0;
-  const uint32_t kbytes = (uint32_t)nkb * kTileK;
+  const int first = (int)blockIdx.x / p.tiles_n, tile_n = (int)blockIdx.x - first * p.tiles_n;
+  const int n0w = (tile_n * NW + nw) * 16;
+  const int used = min(as_const_ints(p.num_post_pad)[0] / 16, p.m_blocks);
+  for (int mb = first; mb < used; mb += p.walkers) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // what hangs on it is found again per block: kept across the loop the kernel took 2 - 4 % longer
+    const int r = lane & 15, kq = lane >> 4;
+    const int expert = as_const_ints(p.expert_ids)[mb];
+    const int slot = p.sorted_ids[mb * 16 + r];
+    const bool real = slot < p.num_valid;
+    const int row = real ? slot / p.top_k : 0;
+    const int kb_all = p.K / kTileK, kb0 = ks * p.kb_per_split;
+    // an expert of another rank: no K block, zeros are stored
+    const int nkb = n0w < p.N && expert >= 0 ? max(min(kb_all, kb0 + p.kb_per_split) - kb0, 0) : 0;
+    const uint32_t kbytes = (uint32_t)nkb * kTileK;
 
-  const uint8_t* const Wb = p.W + (int64_t)max(expert, 0) * p.w_expert_stride;
-  const int rowsW = min(16, p.N - n0w);
-  const rsrc_t rW = make_rsrc(Wb + (int64_t)n0w * p.ldw + (int64_t)kb0 * kTileK, nkb > 0 ? (uint32_t)((rowsW - 1) * p.ldw) + kbytes : 0u);
-  const int wrow = lane >> 3, wc = lane & 7;
-  const uint32_t voW0 = (uint32_t)(wrow * p.ldw + wc * 16), voW1 = (uint32_t)((wrow + 8) * p.ldw + wc * 16);
-  uint8_t* const wslot = wl[w];
-  const uint32_t wst0 = (uint32_t)(wrow * kTileK + ((wc ^ ((wrow >> 1) & 7)) << 4));
-  const uint32_t wst1 = (uint32_t)((wrow + 8) * kTileK + ((wc ^ (((wrow + 8) >> 1) & 7)) << 4));
-  const uint32_t wrd0 = (uint32_t)(r * kTileK + ((kq ^ ((r >> 1) & 7)) << 4));
-  const uint32_t wrd1 = (uint32_t)(r * kTileK + (((4 + kq) ^ ((r >> 1) & 7)) << 4));
-  const int64_t xrows = (p.num_valid + p.top_k - 1) / p.top_k;
-  const rsrc_t rX = make_rsrc(p.X + (int64_t)kb0 * kTileK, nkb > 0 ? (uint32_t)((xrows - 1) * p.ldx) + kbytes : 0u);
-  const uint32_t voX = (uint32_t)((int64_t)row * p.ldx) + kq * 16;
-  const float* const sxp = p.sx + (int64_t)row * p.sx_m + (int64_t)kb0 * p.sx_k;
-  const float* const swp = p.sw + (int64_t)max(expert, 0) * p.sw_expert_stride + (int64_t)(min(n0w, p.N - 1) >> 7) * p.sw_n + (int64_t)kb0 * p.sw_k;
+    const uint8_t* const Wb = p.W + (int64_t)max(expert, 0) * p.w_expert_stride;
+    const int rowsW = min(16, p.N - n0w);
+    const rsrc_t rW = make_rsrc(Wb + (int64_t)n0w * p.ldw + (int64_t)kb0 * kTileK, nkb > 0 ? (uint32_t)((rowsW - 1) * p.ldw) + kbytes : 0u);
+    const int wrow = lane >> 3, wc = lane & 7;
+    const uint32_t voW0 = (uint32_t)(wrow * p.ldw + wc * 16), voW1 = (uint32_t)((wrow + 8) * p.ldw + wc * 16);
+    uint8_t* const wslot = wl[w];
+    const uint32_t wst0 = (uint32_t)(wrow * kTileK + ((wc ^ ((wrow >> 1) & 7)) << 4));
+    const uint32_t wst1 = (uint32_t)((wrow + 8) * kTileK + ((wc ^ (((wrow + 8) >> 1) & 7)) << 4));
+    const uint32_t wrd0 = (uint32_t)(r * kTileK + ((kq ^ ((r >> 1) & 7)) << 4));
+    const uint32_t wrd1 = (uint32_t)(r * kTileK + (((4 + kq) ^ ((r >> 1) & 7)) << 4));
+    const int64_t xrows = (p.num_valid + p.top_k - 1) / p.top_k;
+    const rsrc_t rX = make_rsrc(p.X + (int64_t)kb0 * kTileK, nkb > 0 ? (uint32_t)((xrows - 1) * p.ldx) + kbytes : 0u);
+    const uint32_t voX = (uint32_t)((int64_t)row * p.ldx) + kq * 16;
+    const float* const sxp = p.sx + (int64_t)row * p.sx_m + (int64_t)kb0 * p.sx_k;
+    // constant like the tables: behind a store of the loop the compiler would take vector loads for these
+    const const_floats swp = (const_floats)(uintptr_t)(p.sw + (int64_t)max(expert, 0) * p.sw_expert_stride + (int64_t)(min(n0w, p.N - 1) >> 7) * p.sw_n + (int64_t)kb0 * p.sw_k);
 
-  v4i wreg[D][2], xreg[D][2];
-  float sxr[D], swr[D];
-  auto issue = [&](int d, int kb) {
-    const bool ok = kb < nkb, okx = ok && real;
-    const uint32_t ko = (uint32_t)kb * kTileK;
-    wreg[d][0] = buf_load16_stream(rW, ok ? voW0 + ko : kOutOfRange);
-    wreg[d][1] = buf_load16_stream(rW, ok ? voW1 + ko : kOutOfRange);
-    xreg[d][0] = buf_load16(rX, okx ? voX + ko : kOutOfRange);
-    xreg[d][1] = buf_load16(rX, okx ? voX + ko + 64 : kOutOfRange);
-    const int kc = min(kb, max(nkb - 1, 0));  // past the range the products are zero: any finite scale will do
-    sxr[d] = sxp[(int64_t)kc * p.sx_k];
-    swr[d] = swp[(int64_t)kc * p.sw_k];
-  };
-  v4f acc = {0.f, 0.f, 0.f, 0.f};
-  if (nkb > 0) {
+    v4i wreg[D][2], xreg[D][2];
+    float sxr[D], swr[D];
+    auto issue = [&](int d, int kb) {
+      const bool ok = kb < nkb, okx = ok && real;
+      const uint32_t ko = (uint32_t)kb * kTileK;
+      wreg[d][0] = buf_load16_stream(rW, ok ? voW0 + ko : kOutOfRange);
+      wreg[d][1] = buf_load16_stream(rW, ok ? voW1 + ko : kOutOfRange);
+      xreg[d][0] = buf_load16(rX, okx ? voX + ko : kOutOfRange);
+      xreg[d][1] = buf_load16(rX, okx ? voX + ko + 64 : kOutOfRange);
+      const int kc = min(kb, max(nkb - 1, 0));  // past the range the products are zero: any finite scale will do
+      sxr[d] = sxp[(int64_t)kc * p.sx_k];
+      swr[d] = swp[(int64_t)kc * p.sw_k];
+    };
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    if (nkb > 0) {
 #pragma unroll
-    for (int d = 0; d < D; ++d) issue(d, d);
-    for (int k0 = 0; k0 < nkb; k0 += D) {
+      for (int d = 0; d < D; ++d) issue(d, d);
+      for (int k0 = 0; k0 < nkb; k0 += D) {
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        *reinterpret_cast<v4i*>(wslot + wst0) = wreg[d][0];
-        *reinterpret_cast<v4i*>(wslot + wst1) = wreg[d][1];
-        const v8i wa = join(*reinterpret_cast<const v4i*>(wslot + wrd0), *reinterpret_cast<const v4i*>(wslot + wrd1));
-        const v8i xa = join(xreg[d][0], xreg[d][1]);
-        const float sc = sxr[d] * swr[d];
-        const bool live = k0 + d < nkb;
-        issue(d, k0 + d + D);
-        const v4f t = mfma_16x16x128(wa, xa, v4f{0.f, 0.f, 0.f, 0.f});
-        if (live) {
+        for (int d = 0; d < D; ++d) {
+          *reinterpret_cast<v4i*>(wslot + wst0) = wreg[d][0];
+          *reinterpret_cast<v4i*>(wslot + wst1) = wreg[d][1];
+          const v8i wa = join(*reinterpret_cast<const v4i*>(wslot + wrd0), *reinterpret_cast<const v4i*>(wslot + wrd1));
+          const v8i xa = join(xreg[d][0], xreg[d][1]);
+          const float sc = sxr[d] * swr[d];
+          const bool live = k0 + d < nkb;
+          issue(d, k0 + d + D);
+          const v4f t = mfma_16x16x128(wa, xa, v4f{0.f, 0.f, 0.f, 0.f});
+          if (live) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(t[i], sc, acc[i]);
+            for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(t[i], sc, acc[i]);
+          }
         }
       }
     }
-  }
-  *reinterpret_cast<v4f*>(red[w][lane]) = acc;
-  __syncthreads();
-  const int n = n0w + kq * 4;
-  if (ks != 0 || n >= p.N || !real) return;
-  for (int k = 1; k < 8 / NW; ++k) {
-    const v4f o = *reinterpret_cast<const v4f*>(red[k * NW + nw][lane]);
-    acc[0] += o[0]; acc[1] += o[1]; acc[2] += o[2]; acc[3] += o[3];
-  }
-  float v[4] = {acc[0], acc[1], acc[2], acc[3]};
-  if (p.topk_w) {
-    const float tw = p.topk_w[slot];
+    *reinterpret_cast<v4f*>(red[w][lane]) = acc;
+    __syncthreads();
+    const int n = n0w + kq * 4;
+    if (ks == 0 && n < p.N && real) {
+      for (int k = 1; k < 8 / NW; ++k) {
+        const v4f o = *reinterpret_cast<const v4f*>(red[k * NW + nw][lane]);
+        acc[0] += o[0]; acc[1] += o[1]; acc[2] += o[2]; acc[3] += o[3];
+      }
+      float v[4] = {acc[0], acc[1], acc[2], acc[3]};
+      if (p.topk_w) {
+        const float tw = p.topk_w[slot];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] *= tw;
+        for (int i = 0; i < 4; ++i) v[i] *= tw;
+      }
+      store4<OUT_DT>(p.C, (int64_t)slot * p.ldc + n, v[0], v[1], v[2], v[3]);
+    }
+    if (mb + p.walkers < used) __syncthreads();  // the sums are read before the next block's are written
   }
-  store4<OUT_DT>(p.C, (int64_t)slot * p.ldc + n, v[0], v[1], v[2], v[3]);
 }
 
 }  // namespace fp8k

@@ -30,7 +30,7 @@ struct GemmArgs {
   int kb_per_split;
   int tail_first;     // tile256 only: tiles [tail_first, tiles) are the ones cut along K or into halves
   int tail_halves;    // tile256 only: those tiles are computed as two 128-row halves, one workgroup each (no K cut)
-  int walkers;        // tile256 only: workgroups [0, walkers) walk the whole tiles (a multiple of 8)
+  int walkers;        // tile256: workgroups [0, walkers) walk the whole tiles (a multiple of 8); moe_wavek_kernel: blocks of the grid
   int tail_shared;    // tile256 only: unit u of the tail belongs to workgroup u (after its walk), else to workgroup walkers + u
   int wk_nw;          // gemm_wavek_kernel only: waves of a workgroup along n (1, 2, 4 or 8; the other 8 / wk_nw cut K)
   // grouped (MoE) form of the streaming kernel; all null / zero for a dense GEMM
@@ -800,6 +800,7 @@ struct MoeItem {
 // Tables of the launch that no kernel writes while it reads them, for scalar loads: in a kernel that also stores, the
 // compiler takes vector loads for them otherwise, and those return in order behind every weight load in flight.
 typedef const int32_t __attribute__((address_space(4)))* const_ints;
+typedef const float __attribute__((address_space(4)))* const_floats;
 __device__ __forceinline__ const_ints as_const_ints(const int32_t* p) { return (const_ints)(uintptr_t)p; }
 // blocks in use (a device-side count: the host sizes the grid for the worst case)
 __device__ __forceinline__ int moe_blocks_used(const GemmArgs& p) { return min(as_const_ints(p.num_post_pad)[0] / p.block_m, p.m_blocks); }

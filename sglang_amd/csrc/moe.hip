@@ -580,7 +580,10 @@ static bool moe256_walks(int64_t num_valid_tokens, int64_t num_experts, int64_t 
   return (balanced || moe256_one_block(num_valid_tokens, num_experts)) && K >= 2 * kTileK;
 }
 
-// blocks that can be in use: every one holds a slot, and only an expert's last (or that of the slots without one) is not full
+// Blocks in use, at most, of a table that was aligned over the launch's own experts: every one holds a slot, and only an expert's last
+// (or that of the slots without one) is not full.  A caller's table may have more - blocks of other ranks' experts one by one,
+// blocks without slots, several part-filled ones of an expert - so this chooses kernels and sizes grids, whose workgroups go on to
+// num_tokens_post_padded whatever it says.
 static int64_t moe_blocks_in_use(int64_t slots, int64_t num_experts, int64_t block_m, int64_t capacity) {
   return std::min(capacity, std::min(slots, num_experts + 1 + slots / block_m));
 }
@@ -674,6 +677,7 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
     a.wk_nw = strips >= 3 * cu ? 4 : 2 * strips >= 3 * cu || kb < 32 ? 2 : 1;
     a.tiles_n = (int)((N + 16 * a.wk_nw - 1) / (16 * a.wk_nw));
     a.kb_per_split = (kb + 8 / a.wk_nw - 1) / (8 / a.wk_nw);
+    a.walkers = (int)blocks_max;
     const dim3 grid((unsigned)(blocks_max * a.tiles_n)), block(512);
     if (out_dtype == FP8K_BF16) hipLaunchKernelGGL((moe_wavek_kernel<FP8K_BF16>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((moe_wavek_kernel<FP8K_F16>), grid, block, 0, st, a);

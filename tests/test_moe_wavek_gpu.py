@@ -37,3 +37,45 @@ def test_few_blocks_with_k_cut_between_waves_exact(dev, sizes, top_k, N, K, dtyp
             C = torch.full((slots, N), float("nan"), dtype=dtype, device=dev)
             moe_block_gemm(A, B, C, sc, wsd, twd, sorted_ids, expert_ids, npad, weigh, top_k, 16, slots)
             assert torch.equal(C.float().cpu(), (want * tw if weigh else want).to(dtype).float())
+
+
+def _table(blocks, pad, extra, dev):
+    """sorted_token_ids, expert_ids and num_tokens_post_padded of (expert, slots) blocks of 16, with `extra` unused blocks behind them."""
+    rows = [list(s) + [pad] * (16 - len(s)) for _, s in blocks] + [[pad] * 16] * extra
+    return (torch.tensor(rows, dtype=torch.int32, device=dev).flatten(), torch.tensor([e for e, _ in blocks] + [0] * extra, dtype=torch.int32, device=dev),
+            torch.tensor([16 * len(blocks)], dtype=torch.int32, device=dev))
+
+
+# What the caller's table may hold beyond what an aligner over B's experts would write: more blocks than slots, or than those experts fill.
+TABLES = {
+    # aligned over 64 experts of all ranks, of which this rank has every eighth: one slot each, foreign blocks at -1
+    "foreign_experts": (8, [(e // 8 if e % 8 == 3 else -1, [63 - e]) for e in range(64)]),
+    # one block per expert whatever the routing (the layout of a captured graph), three of 24 with slots
+    "fixed_blocks": (24, [(e, {3: [0, 1, 2], 17: [5], 23: [4, 3]}.get(e, [])) for e in range(24)]),
+    # two experts in turn, every block part-filled
+    "part_filled": (2, [(b % 2, [2 * b, 2 * b + 1]) for b in range(30)]),
+}
+
+
+@pytest.mark.parametrize("N,K", [(264, 4224), (1024, 1152), (776, 2048), (2056, 1280)])
+@pytest.mark.parametrize("table", sorted(TABLES))
+def test_tables_of_more_blocks_than_the_experts_fill(dev, table, N, K):
+    """Every block below num_tokens_post_padded is computed, whatever its number; the rows of foreign blocks are zeros; exact on integers."""
+    from sglang_amd.sgl_kernel import moe_block_gemm
+
+    E, blocks = TABLES[table]
+    slots = 1 + max(s for _, b in blocks for s in b)
+    g = torch.Generator().manual_seed(N + K + E)
+    powers = lambda *s: 2.0 ** torch.randint(-2, 2, s, generator=g).float()  # noqa: E731
+    x, w = torch.randint(-1, 2, (slots, K), generator=g).float(), torch.randint(-1, 2, (E, N, K), generator=g).float()
+    xs, ws = powers(slots, K // 128), powers(E, (N + 127) // 128, K // 128)
+    want = torch.zeros((slots, N))
+    for e, ids in blocks:
+        if e >= 0 and ids:
+            scaled = w[e] * ws[e].repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)
+            want[ids] = (x[ids] * xs[ids].repeat_interleave(128, 1)) @ scaled.t()
+    A, B = x.to(dev).to(torch.float8_e4m3fn), w.to(dev).to(torch.float8_e4m3fn)
+    for extra in (0, 5):
+        C = torch.full((slots, N), float("nan"), dtype=torch.bfloat16, device=dev)
+        moe_block_gemm(A, B, C, xs.to(dev), ws.to(dev), None, *_table(blocks, slots, extra, dev), False, 1, 16, slots)
+        assert torch.equal(C.float().cpu(), want.to(torch.bfloat16).float())
