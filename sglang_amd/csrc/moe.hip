@@ -672,7 +672,8 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
   // from 1.5 strips per CU on (1.5: 0.80 - 0.81 against 0.85 - 0.87 with one; at one strip 0.78 - 0.82 against 0.73 - 0.78) or where eight
   // would share less than four K blocks each, four from three on (three: 0.82 - 0.88 against 0.87 - 0.95 with two; 2.5: 0.95 against 0.85).
   const int64_t strips = blocks_max * ((N + 15) / 16), cu = num_cu();
-  if (block_m == 16 && strips <= 4 * cu && K >= 8 * kTileK) {
+  // Its K ranges are summed apart, so it is kept off every K whose sum fp8k_moe_act_block_gemm has to match bit for bit.
+  if (block_m == 16 && strips <= 4 * cu && K > kMoeShortKAct) {
     const int kb = (int)(K / kTileK);
     a.wk_nw = strips >= 3 * cu ? 4 : 2 * strips >= 3 * cu || kb < 32 ? 2 : 1;
     a.tiles_n = (int)((N + 16 * a.wk_nw - 1) / (16 * a.wk_nw));

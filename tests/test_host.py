@@ -253,6 +253,32 @@ def test_experts_are_the_dispatcher_path(dev, dispatcher, tokens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("inter", [256, 1024, 1152])
+@pytest.mark.parametrize("tokens", [1, 3])
+def test_experts_of_few_tokens_are_the_dispatcher_path(dev, dispatcher, tokens, inter):
+    """Few blocks, up to, at and above the longest second K that takes the activation inside.  The largest terms of the second product
+    cancel - its first K block against its last - so that another order of its sums shows in the 16-bit result."""
+    E, H, topk = 16, 2048, 4
+    x = _randn((tokens, H))
+    g = torch.Generator().manual_seed(inter + tokens)
+    fp8 = lambda t: t.to(dev).to(torch.float8_e4m3fn)  # noqa: E731
+    w13, w2 = torch.randn((E, 2, inter, H), generator=g), torch.randn((E, H, inter), generator=g)
+    w13[:, :, -128:] = w13[:, :, :128]
+    w2[:, :, -128:] = -w2[:, :, :128]
+    s13, s2 = torch.full((E, 2 * inter // 128, H // 128), 0.02), torch.rand((E, H // 128, inter // 128), generator=g) + 0.5
+    s2[:, :, -1] = s2[:, :, 0] = 1000.0
+    w13, w2, s13, s2 = fp8(w13.view(E, 2 * inter, H)), fp8(w2), s13.to(dev), s2.to(dev)
+    logits, bias = _randn((tokens, E), torch.float32, 7), _randn((E,), torch.float32, 8)
+
+    def layer():
+        tw, ids = fused_moe.biased_grouped_topk(x, logits, bias, topk, True, 4, 2)
+        return fused_moe.fused_experts_impl(x, w13, w2, tw, ids, use_fp8_w8a8=True, w1_scale=s13, w2_scale=s2, block_shape=BLOCK,
+                                            routed_scaling_factor=2.5)
+
+    assert _same(layer(), dispatcher(layer))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("b,m,n,k", [(1, 1, 8, 128), (9, 64, 128, 256), (8, 65, 136, 384), (17, 127, 120, 1024), (3, 70, 200, 1152)])
 def test_bmm_tile_edges(dev, b, m, n, k):
     """Row, column and batch remainders of the short-K kernel's 64 x 128 tiles, one to nine K blocks, strided operands and

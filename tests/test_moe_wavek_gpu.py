@@ -6,7 +6,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("sizes,top_k,N,K", [((1,), 1, 8, 1024), ((1, 0, 3, 16, 17), 1, 264, 1152), ((5, 1, 1, 1), 4, 512, 7168), ((2, 1, 1), 2, 1032, 4096),
-                                             ((40, 1, 16, 15), 1, 2048, 2048), ((1, 1), 1, 4096, 18432)])
+                                             ((40, 1, 16, 15), 1, 2048, 2048), ((1, 1), 1, 4096, 18432),
+                                             ((1,), 1, 8, 1152)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_blocks_with_k_cut_between_waves_exact(dev, sizes, top_k, N, K, dtype):
     """One, two and four waves along n, a K that the waves do not divide, a last strip of 8 weight rows, blocks of one slot and full
@@ -79,3 +80,36 @@ def test_tables_of_more_blocks_than_the_experts_fill(dev, table, N, K):
         C = torch.full((slots, N), float("nan"), dtype=torch.bfloat16, device=dev)
         moe_block_gemm(A, B, C, xs.to(dev), ws.to(dev), None, *_table(blocks, slots, extra, dev), False, 1, 16, slots)
         assert torch.equal(C.float().cpu(), want.to(torch.bfloat16).float())
+
+
+@pytest.mark.parametrize("T,E,topk,N,K", [(1, 16, 4, 2048, 1024), (3, 8, 2, 1032, 1024), (2, 16, 4, 2048, 896), (1, 4, 1, 512, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_few_blocks_have_the_bits_of_the_form_with_the_activation_inside(dev, T, E, topk, N, K, dtype):
+    """Whatever K fp8k_moe_act_block_gemm takes, the grouped GEMM adds its K blocks in the same order, also where few blocks are hit.  The
+    largest terms cancel - the first K block against the last - so that another order shows in the 16-bit result."""
+    from sglang_amd._lib import BF16, F16, check, lib, stream_ptr
+    from sglang_amd.fp8_kernel import sglang_per_token_group_quant_fp8
+    from sglang_amd.fused_moe import moe_align_block_size
+    from sglang_amd.sgl_kernel import moe_block_gemm
+
+    g = torch.Generator().manual_seed(K + T)
+    x = torch.randn((T * topk, 2, K), generator=g)
+    x[:, :, -128:] = x[:, :, :128]
+    x = x.to(dtype).to(dev).view(T * topk, 2 * K)
+    w = torch.randn((E, N, K), generator=g)
+    w[:, :, -128:] = -w[:, :, :128]
+    w = w.to(dev).to(torch.float8_e4m3fn)
+    ws = torch.rand((E, (N + 127) // 128, K // 128), generator=g) + 0.5
+    ws[:, :, -1] = ws[:, :, 0] = 1000.0
+    ws = ws.to(dev)
+    ids = torch.rand((T, E), generator=g).argsort(dim=1)[:, :topk].int().to(dev)
+    sorted_ids, expert_ids, npad = moe_align_block_size(ids, 16, E)
+    q, s = sglang_per_token_group_quant_fp8(x, 128, column_major_scales=True, fuse_silu_and_mul=True)
+    assert lib.fp8k_moe_act_block_gemm_takes(16, N, K, K) == 1
+    want, got = (torch.full((T * topk, N), 7.0, dtype=dtype, device=dev) for _ in range(2))
+    moe_block_gemm(q, w, want, s, ws, None, sorted_ids, expert_ids, npad, False, 1, 16, ids.numel())
+    check(lib.fp8k_moe_act_block_gemm(x.data_ptr(), w.data_ptr(), ws.data_ptr(), got.data_ptr(), sorted_ids.data_ptr(), expert_ids.data_ptr(),
+                                      npad.data_ptr(), None, sorted_ids.numel(), 16, ids.numel(), E, N, K, 2 * K, N * K, K, *ws.stride(), N, 1e-10,
+                                      BF16 if dtype == torch.bfloat16 else F16, stream_ptr(dev)))
+    torch.cuda.synchronize()
+    assert torch.equal(want, got)
