@@ -650,7 +650,7 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
   // At K = 2048 with 32 slots, where one workgroup fits a CU, whole layers took 1 - 26 % longer as runs: 256 experts, H = 7168,
   // 256 / 512 / 700 tokens 1807 / 1900 / 2020 us against 1738 / 1852 / 2010, 64 experts, H = 2048, 150 tokens 186 against 149.
   const int64_t blocks_max = moe_blocks_in_use(num_valid_tokens, num_experts, block_m, a.m_blocks);
-  const int64_t most = 2 * (int64_t)num_cu() / 8 * 8;
+  const int64_t cu = num_cu(), most = 2 * cu / 8 * 8;
   if (direct && K <= (block_m == 16 ? kMoeShortKFew : kMoeShortKMax) && blocks_max * a.tiles_n > most && N * ldb < (1LL << 31)) {
     const dim3 grid((unsigned)most), block(512);
     const unsigned lds = (unsigned)(block_m * moe_shortk_row((int)K));
@@ -665,15 +665,24 @@ static int moe_block_gemm_impl(const void* A, const void* B, const float* As, co
 #undef FP8K_SHORTK
     return check_launch(op);
   }
-  // Few blocks with 16 slots: at most four strips of 16 weight rows per CU, which tiles of 128 rows would put on half of the CUs.  Whole layers,
-  // time over that with the tiles, at 1 / 2 / 3 / 4 tokens: 64 experts, 7168 x 256, top 8 0.69 / 0.79 / 0.88 / 0.90 (39.8 -> 27.7 us at one
-  // token), 128 experts, 4096 x 512, top 4 0.75 / 0.81 / 0.88 / 0.88, 64 experts, 2048 x 256, top 6 0.90 - 0.97; 256 experts, 7168 x 2048, top 4, one
-  // token 0.82.  With six strips 64 experts, 2048 x 256 took 1.13 and 256 experts, 4096 x 512 1.05 times as long.  Waves along n: two
-  // from 1.5 strips per CU on (1.5: 0.80 - 0.81 against 0.85 - 0.87 with one; at one strip 0.78 - 0.82 against 0.73 - 0.78) or where eight
-  // would share less than four K blocks each, four from three on (three: 0.82 - 0.88 against 0.87 - 0.95 with two; 2.5: 0.95 against 0.85).
-  const int64_t strips = blocks_max * ((N + 15) / 16), cu = num_cu();
+  // Few blocks with 16 slots: strips of 16 weight rows, at most four per CU, which tiles of 128 rows would put on half of the CUs.  A wave
+  // pays for its share of K with activations: it fetches its rows' bytes for itself, from as many lines as its block has rows, where
+  // the waves of a tile share them.  So the line lies by the strips per CU, the depth and the rows that a block can have: one per token
+  // where a token's experts differ.  GEMM alone, time over the tiles', median (range), weights out of HBM / out of the cache, 405 shapes with
+  // even and skewed routing:
+  //   up to one strip, K >= 4096, any rows    0.47 (0.35 - 0.78) / 0.51 (0.33 - 0.81)
+  //   up to one, K below, up to 8 rows        0.75 (0.61 - 0.93) / 0.80 (0.59 - 0.96)
+  //   up to two, up to 8 rows                 0.72 (0.44 - 0.83) / 0.75 (0.42 - 0.97)
+  //   up to four, K >= 4096, up to 6 rows     0.81 (0.58 - 0.96) / 0.80 (0.56 - 0.98)
+  // and outside: above one strip, K >= 4096, full blocks up to 1.09 / 1.13, above two 1.67; up to one, K below, full blocks 0.95 / 1.11; above
+  // two, K below, up to 8 rows up to 1.15 / 1.30.  (Six strips, even routing, whole layers: 1.05 - 1.13.)
   // Its K ranges are summed apart, so it is kept off every K whose sum fp8k_moe_act_block_gemm has to match bit for bit.
-  if (block_m == 16 && strips <= 4 * cu && K > kMoeShortKAct) {
+  // Waves along n: two from 1.5 strips per CU on (1.5: 0.80 - 0.81 against 0.85 - 0.87 with one; at one strip 0.78 - 0.82 against 0.73 -
+  // 0.78) or where eight would share less than four K blocks each, four from three on (three: 0.82 - 0.88 against 0.87 - 0.95 with two;
+  // 2.5: 0.95 against 0.85); whole layers of one to six tokens.
+  const int64_t strips = blocks_max * ((N + 15) / 16);
+  if (block_m == 16 && K > kMoeShortKAct &&
+      (strips <= cu ? xrows <= 8 || K >= 4096 : strips <= 2 * cu ? xrows <= 8 : strips <= 4 * cu && xrows <= 6 && K >= 4096)) {
     const int kb = (int)(K / kTileK);
     a.wk_nw = strips >= 3 * cu ? 4 : 2 * strips >= 3 * cu || kb < 32 ? 2 : 1;
     a.tiles_n = (int)((N + 16 * a.wk_nw - 1) / (16 * a.wk_nw));

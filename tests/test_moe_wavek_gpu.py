@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("sizes,top_k,N,K", [((1,), 1, 8, 1024), ((1, 0, 3, 16, 17), 1, 264, 1152), ((5, 1, 1, 1), 4, 512, 7168), ((2, 1, 1), 2, 1032, 4096),
                                              ((40, 1, 16, 15), 1, 2048, 2048), ((1, 1), 1, 4096, 18432),
-                                             ((1,), 1, 8, 1152)])
+                                             ((1,), 1, 8, 1152), ((1, 0, 3, 16, 17), 8, 264, 1152), ((40, 1, 16, 15), 16, 776, 4096), ((40, 1, 16, 15), 16, 1400, 4224)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_blocks_with_k_cut_between_waves_exact(dev, sizes, top_k, N, K, dtype):
     """One, two and four waves along n, a K that the waves do not divide, a last strip of 8 weight rows, blocks of one slot and full
@@ -58,7 +58,7 @@ TABLES = {
 }
 
 
-@pytest.mark.parametrize("N,K", [(264, 4224), (1024, 1152), (776, 2048), (2056, 1280)])
+@pytest.mark.parametrize("N,K", [(264, 4224), (1024, 1152), (776, 4096), (1032, 4224), (2056, 4224)])
 @pytest.mark.parametrize("table", sorted(TABLES))
 def test_tables_of_more_blocks_than_the_experts_fill(dev, table, N, K):
     """Every block below num_tokens_post_padded is computed, whatever its number; the rows of foreign blocks are zeros; exact on integers."""
@@ -66,19 +66,22 @@ def test_tables_of_more_blocks_than_the_experts_fill(dev, table, N, K):
 
     E, blocks = TABLES[table]
     slots = 1 + max(s for _, b in blocks for s in b)
+    top_k = (slots + 3) // 4  # few tokens
+    rows = (slots + top_k - 1) // top_k
     g = torch.Generator().manual_seed(N + K + E)
     powers = lambda *s: 2.0 ** torch.randint(-2, 2, s, generator=g).float()  # noqa: E731
-    x, w = torch.randint(-1, 2, (slots, K), generator=g).float(), torch.randint(-1, 2, (E, N, K), generator=g).float()
-    xs, ws = powers(slots, K // 128), powers(E, (N + 127) // 128, K // 128)
+    x, w = torch.randint(-1, 2, (rows, K), generator=g).float(), torch.randint(-1, 2, (E, N, K), generator=g).float()
+    xs, ws = powers(rows, K // 128), powers(E, (N + 127) // 128, K // 128)
     want = torch.zeros((slots, N))
     for e, ids in blocks:
         if e >= 0 and ids:
             scaled = w[e] * ws[e].repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)
-            want[ids] = (x[ids] * xs[ids].repeat_interleave(128, 1)) @ scaled.t()
+            at = torch.tensor(ids) // top_k
+            want[ids] = (x[at] * xs[at].repeat_interleave(128, 1)) @ scaled.t()
     A, B = x.to(dev).to(torch.float8_e4m3fn), w.to(dev).to(torch.float8_e4m3fn)
     for extra in (0, 5):
         C = torch.full((slots, N), float("nan"), dtype=torch.bfloat16, device=dev)
-        moe_block_gemm(A, B, C, xs.to(dev), ws.to(dev), None, *_table(blocks, slots, extra, dev), False, 1, 16, slots)
+        moe_block_gemm(A, B, C, xs.to(dev), ws.to(dev), None, *_table(blocks, slots, extra, dev), False, top_k, 16, slots)
         assert torch.equal(C.float().cpu(), want.to(torch.bfloat16).float())
 
 
