@@ -389,17 +389,18 @@ __global__ __launch_bounds__(256) void tensor_quant_kernel(const void* __restric
 
 // ------------------------------------------------------------------------------------------------
 // per-tensor quant of a strided [H, S, D] tensor into a contiguous one (the MLA absorbed products): 8 elements (a chunk) a
-// lane, four chunks in flight, in grid-stride.  The maxima queue up at one atomic, so the maximum pass takes one workgroup of 1024
-// threads per CU at most, and four chunks per lane before it takes a second one's atomic (both passes, us, 512 of 256 threads / this:
-// 3.7 MB 7.9 / 7.1, 5.9 MB 10.0 / 8.4, 10 MB 13.0 / 10.3, 17 MB 15.5 / 13.2, 67 MB 33.9 / 31.6); IDX is 32-bit wherever the chunks can be counted so, because
-// the two divisions per chunk (row, then head) are the arithmetic of this kernel.
+// lane, four chunks in flight, in grid-stride.  The maxima queue up at one atomic, so a workgroup of the maximum pass takes four chunks
+// per lane before a second one's atomic is taken, and above kMlaMaxWide chunks (2 MB of 16-bit input) it has 1024 threads, one per CU at
+// most: both passes, us, up to 512 workgroups of 256 threads / 1024 threads: 3.1 MB 7.0 / 6.6, 5.9 MB 9.7 / 7.7, 10.9 MB 12.8 / 9.7,
+// 20 MB 15.6 / 13.2, 36 MB 20.3 / 18.7; 2.1 MB 6.16 / 6.14, and below, where the chip is idle, the many small ones are ahead: 1.4 MB 5.6 /
+// 6.0, 0.5 MB 4.9 / 5.8, 0.1 MB 4.5 / 5.5.  IDX is 32-bit wherever the chunks can be counted so, because the two divisions per
+// chunk (row, then head) are the arithmetic of this kernel.
 // ------------------------------------------------------------------------------------------------
-constexpr int mla_threads(bool quant) { return quant ? 256 : 1024; }
-template <int DT, bool QUANT, typename IDX>
-__global__ __launch_bounds__(mla_threads(QUANT)) void rows_tensor_quant_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
+constexpr int64_t kMlaMaxWide = 131072;
+template <int DT, int T, bool QUANT, typename IDX>
+__global__ __launch_bounds__(T) void rows_tensor_quant_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
                                                                 float* __restrict__ s, int64_t rows, int S, int D,
                                                                 int64_t stride_h, int64_t stride_s, float eps) {
-  constexpr int T = mla_threads(QUANT);
   __shared__ float red[16];
   const IDX chunks = (IDX)(D / 8);          // per row; the host checks D % 8 == 0 and the alignment of every row
   const IDX total = (IDX)rows * chunks;
@@ -792,15 +793,21 @@ static int tensor_quant_mla(const void* x, void* q, float* s, int64_t H, int64_t
   const int64_t rows = H * S, chunks = rows * (D / 8);
   const bool narrow = chunks < (1LL << 31);  // room for the four steps past the end
   const dim3 block(256);
-  const dim3 grid_max((unsigned)std::min<int64_t>(num_cu(), (chunks + 4095) / 4096)), grid_q((unsigned)std::min<int64_t>(2048, (chunks + 255) / 256));
+  const bool wide = chunks > kMlaMaxWide;
+  const dim3 grid_max((unsigned)(wide ? std::min<int64_t>(num_cu(), (chunks + 4095) / 4096) : (chunks + 1023) / 1024));
+  const dim3 grid_q((unsigned)std::min<int64_t>(2048, (chunks + 255) / 256));
   // one chunk per lane is enough to work on: the more workgroups share it, the shorter the loads
   const dim3 grid_once((unsigned)std::min<int64_t>(kMlaOnceGroups, (chunks + 1023) / 1024));
   FP8K_REQUIRE(!sync || fp8k_tensor_quant_mla_takes_sync(H * S * D), "%s: not a size of the one-launch form", op);
 #define FP8K_MLAQ2(DT, IDX)                                                                                                 \
   do {                                                                                                                      \
-    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, false, IDX>), grid_max, dim3(mla_threads(false)), 0, st, x, (uint8_t*)q, s, rows, (int)S, \
-                       (int)D, x_stride_h, x_stride_s, eps);                                                                \
-    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, true, IDX>), grid_q, block, 0, st, x, (uint8_t*)q, s, rows, (int)S,    \
+    if (wide)                                                                                                               \
+      hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, 1024, false, IDX>), grid_max, dim3(1024), 0, st, x, (uint8_t*)q, s,  \
+                         rows, (int)S, (int)D, x_stride_h, x_stride_s, eps);                                                \
+    else                                                                                                                    \
+      hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, 256, false, uint32_t>), grid_max, block, 0, st, x, (uint8_t*)q, s,   \
+                         rows, (int)S, (int)D, x_stride_h, x_stride_s, eps);                                                \
+    hipLaunchKernelGGL((rows_tensor_quant_kernel<DT, 256, true, IDX>), grid_q, block, 0, st, x, (uint8_t*)q, s, rows, (int)S, \
                        (int)D, x_stride_h, x_stride_s, eps);                                                                \
   } while (0)
 #define FP8K_MLAQ(DT)                                                                                                          \

@@ -44,6 +44,29 @@ def test_per_tensor_quant_mla(dev, H, S, D, transposed, dtype):
     assert np.array_equal(q.view(torch.uint8).cpu().numpy(), oq)
 
 
+@pytest.mark.parametrize("H,S", [(128, 16), (5, 3001), (64, 256), (1, 16385), (3, 5462), (16, 4096), (257, 1024)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_per_tensor_quant_mla_in_two_launches(dev, H, S, dtype):
+    """Both forms of the maximum pass - workgroups of 256 threads up to 131072 chunks of eight elements, of 1024 above - below, at, a row
+    above and far above that line, with more chunks than one round takes; the largest value first, in the middle and last, and a
+    scale on entry that is larger than the tensor's."""
+    from sglang_amd._lib import BF16, F32, check, lib, stream_ptr
+
+    D = 64
+    base = torch.randn((S, H, D), generator=torch.Generator().manual_seed(H)).to(dtype)
+    for (s_at, h_at), start in (((0, 0), 0.0), ((S // 2, H // 2), 0.0), ((S - 1, H - 1), 0.0), ((0, 0), 1.0)):
+        x_cpu = base.clone()
+        x_cpu[s_at, h_at, -1 if s_at else 0] = -41.0
+        x = x_cpu.to(dev).transpose(0, 1)
+        q, s = torch.empty((H, S, D), dtype=torch.float8_e4m3fn, device=dev), torch.full((1,), start, device=dev)
+        check(lib.fp8k_tensor_quant_mla(x.data_ptr(), q.data_ptr(), s.data_ptr(), H, S, D, x.stride(0), x.stride(1), 1e-12,
+                                        BF16 if dtype == torch.bfloat16 else F32, stream_ptr(dev)))
+        scale = torch.tensor(max(np.float32(41.0) / np.float32(448.0), np.float32(start)))
+        assert s.cpu()[0] == scale
+        want = (x_cpu.transpose(0, 1).float() * (1.0 / scale)).clamp(-448, 448).to(torch.float8_e4m3fn)
+        assert torch.equal(q.cpu().view(torch.uint8), want.contiguous().view(torch.uint8))
+
+
 def test_per_tensor_quant_mla_zero_tensor_and_errors(dev):
     from sglang_amd.fp8_kernel import per_tensor_quant_mla_fp8
 
