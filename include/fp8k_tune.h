@@ -16,12 +16,13 @@ extern "C" {
 /*
  * Tuning and test aid (no counterpart in the reference): pins the kernel family that the dense GEMM entry points
  * pick for later calls made by the calling thread (the setting is thread-local; other threads keep the automatic
- * choice).  kind -1: automatic (the default).  kind 4: the 128x128 tile kernel with K
- * cut into `splits` runs (0 or 1: none; | 256: the form with 64 activation rows).  kind 0: the choice by the number of rows alone, without the 128x128
- * kernel.  kind 1: 256x256 tiles; kind 2: the streaming kernel (up to 128 rows); kind 3: the direct kernel (up to 32
- * rows, `splits` > 0 pins its K cut too); kind 5: the direct kernel that cuts K across the waves of a workgroup (up to
- * 32 rows); kind 8: the 64x64 tile kernel with K cut into `splits` runs; where a pinned family cannot take the shape, the choice by rows stands.
- * `splits` is ignored for kinds 0..2.
+ * choice).  kind -1: automatic (the default).  kind 4: the tile kernel of 128 weight rows with K cut into `splits` runs (0 or 1:
+ * none; | 256: the form with 64 activation rows); kind 8: the 64x64 tile kernel with K cut into `splits` runs; both for N a
+ * multiple of 8.  kind 0: the choice by the number of rows alone, without these two.  kind 1: 256x256 tiles; kind 2: the streaming
+ * kernel (up to 128 rows); kind 3: the direct kernel (up to 32 rows, `splits` > 0 pins its K cut too); kind 5: the kernel that cuts
+ * K across the waves of a workgroup (up to 16 rows, `splits` 1, 2, 4 or 8 pins its waves along n); kind 7: the strips over all of K
+ * (up to 64 rows, `splits` 1, 2 or 4 pins their waves along n).  Where a pinned family cannot take the shape, the choice by rows
+ * stands.  `splits` is ignored for kinds 0..2.
  * kind -2: automatic, but the last round of 256x256 tiles is kept whole instead of being computed in 128-row halves.
  * fp8k_*_workspace_bytes, called from the same thread, follows the pinned choice.
  */

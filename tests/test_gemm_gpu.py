@@ -245,8 +245,9 @@ def test_block_gemm_random_shapes_every_plan(dev):
 @pytest.mark.parametrize("nw", [0, 1, 2, 4])
 def test_skinny_gemm_is_exact_on_integers(dev, nw):
     """The decode-batch kernel with loading and streaming waves, pinned with every wave layout (0 = the plan's own): one to 33 K blocks
-    (one trip, remainders of a trip, more trips than stages), 1 .. 128 rows around the row counts it is built for, strips that end
-    inside their 16, 32 or 64 rows, both scale layouts, both outputs; exact whatever the order of the sums; then row mode."""
+    (one trip, remainders of a trip, more trips than stages), 1 .. 64 rows around the row counts it is built for, strips that end
+    inside their 16, 32 or 64 rows, both scale layouts, both outputs; exact whatever the order of the sums; then row mode.  65 and
+    128 rows are more than it takes: there the pin leaves the choice by rows."""
     from sglang_amd._lib import lib
     from sglang_amd.sgl_kernel import fp8_scaled_mm
 
@@ -275,7 +276,7 @@ def test_skinny_gemm_is_exact_on_integers(dev, nw):
 def test_decode_gemm_with_k_cut_across_waves_is_exact_on_integers(dev, nw):
     """The decode kernel that cuts K across the waves of a workgroup (partial sums meet in LDS), pinned with every
     wave layout (0 = the plan's own): K block counts that do not divide by the number of K ranges (waves with short or
-    empty ranges), N not a multiple of the 16 rows of a wave, 1 .. 32 rows, both scale layouts, bf16 and fp16 output -
+    empty ranges), N not a multiple of the 16 rows of a wave, 1 .. 16 rows (above, the choice by rows stands), both scale layouts, bf16 and fp16 output -
     integer data with power-of-two scales, so the sums are exact whatever their order - and the same through
     fp8_scaled_mm with a bias."""
     from sglang_amd._lib import lib

@@ -1,5 +1,6 @@
 """GPU parity of the 64x64 tile kernel (gemm_tile64_kernel), pinned through fp8k_tune_force_gemm_plan: fewer K blocks than waves, remainders
-of a round of four waves, rows and columns around the edges of a tile, K cuts, every mode, both scale layouts, strided output rows.
+of a round of four waves, rows and columns around the edges of a tile, K cuts, every mode, both scale layouts, biases, strided operand and
+output rows in both store forms.
 Integer data with power-of-two scales: the sums are exact whatever their order.
 """
 import numpy as np
@@ -77,3 +78,57 @@ def test_hardware_scales_match_float_scales(dev, tile64, M, N, K, splits):
             q = (x.float().view(M, -1, 128) / s[..., None]).clamp(-448, 448).view(M, K).to(torch.float8_e4m3fn)
         outs.append(fp8_kernel.w8a8_block_fp8_matmul(q, w, s, ws, [128, 128], torch.bfloat16))
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("splits", [1, 2])
+@pytest.mark.parametrize("mode", ["block", "row"])
+@pytest.mark.parametrize("dtype,code,name", [(torch.bfloat16, 2, "bf16"), (torch.float16, 1, "f16")])
+def test_strided_rows_and_both_store_forms(dev, tile64, splits, mode, dtype, code, name):
+    """Operand rows longer than K, output rows longer than N: rows of a multiple of eight elements from a 16-byte aligned start take
+    16-byte stores, any other ldc or start the 8-byte ones; what lies between the rows stays as it was.  Exact on integers."""
+    from sglang_amd._lib import check, lib, stream_ptr
+
+    M, N, K = 131, 200, 128 * 9
+    rng, xq, wq, xs, ws = _integers(M, N, K)
+    sa, sb = ((2.0 ** rng.integers(-3, 3, (n,))).astype(np.float32) for n in (M, N))
+    A, B = torch.zeros((M, K + 48), dtype=torch.uint8, device=dev), torch.zeros((N, K + 16), dtype=torch.uint8, device=dev)
+    A[:, :K], B[:, :K] = torch.from_numpy(xq).to(dev).view(torch.uint8), torch.from_numpy(wq).to(dev).view(torch.uint8)
+    if mode == "block":
+        want = O.w8a8_block_fp8_matmul(xq, wq, xs, ws, out_dtype=name, acc=np.float64)
+    else:
+        want = O.fp8_scaled_mm(xq, wq, sa, sb, out_dtype=name)
+    xs, ws, sa, sb = (torch.from_numpy(t).to(dev) for t in (xs, ws, sa, sb))
+    tile64(splits)
+    need = max(lib.fp8k_block_gemm_workspace_bytes(M, N, K), lib.fp8k_scaled_mm_workspace_bytes(M, N, K))
+    work = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+    for ldc, start in ((N, 0), (N + 8, 0), (N + 4, 0), (N, 4), (N + 8, 4)):
+        buf = torch.full((M * ldc + 8,), 7.0, dtype=dtype, device=dev)
+        C = buf[start:start + M * ldc].view(M, ldc)
+        if mode == "block":
+            check(lib.fp8k_block_gemm(A.data_ptr(), B.data_ptr(), xs.data_ptr(), ws.data_ptr(), C.data_ptr(), M, N, K, K + 48, K + 16, xs.stride(0),
+                                      xs.stride(1), ws.stride(0), ws.stride(1), ldc, code, work.data_ptr(), need, stream_ptr(dev)))
+        else:
+            check(lib.fp8k_scaled_mm(A.data_ptr(), B.data_ptr(), sa.data_ptr(), sb.data_ptr(), None, C.data_ptr(), M, N, K, K + 48, K + 16, ldc, code, 0,
+                                     work.data_ptr(), need, stream_ptr(dev)))
+        assert np.array_equal(C[:, :N].float().cpu().numpy(), want), (ldc, start)
+        assert (C[:, N:] == 7.0).all() and (buf[:start] == 7.0).all() and (buf[start + M * ldc:] == 7.0).all(), (ldc, start)
+
+
+@pytest.mark.parametrize("splits", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_block_linear_adds_its_bias_to_the_rounded_product(dev, tile64, splits, dtype):
+    """Block mode's bias.  Every group's largest value is 448 times a power of two, so the quantisation is exact, and so are the sums."""
+    from sglang_amd.fp8_utils import w8a8_block_fp8_linear
+
+    M, N, K = 133, 136, 128 * 9
+    rng, _, wq, _, ws = _integers(M, N, K)
+    x = rng.integers(-4, 5, (M, K // 128, 128)).astype(np.float32)
+    x[:, :, 5] = 448.0 * rng.choice([-1, 1], (M, K // 128))
+    scale = (2.0 ** rng.integers(-3, 3, (M, K // 128))).astype(np.float32)
+    bias = torch.from_numpy(rng.standard_normal(N).astype(np.float32) * 100).to(dtype)
+    product = O.w8a8_block_fp8_matmul(O.f32_to_e4m3fn(x.reshape(M, K)), wq, scale, ws, out_dtype="f32", acc=np.float64)
+    want = (torch.from_numpy(product).to(dtype).float() + bias.float()).to(dtype)
+    tile64(splits)
+    got = w8a8_block_fp8_linear(torch.from_numpy((x * scale[:, :, None]).reshape(M, K)).to(dtype).to(dev), fp8_tensor(wq, dev), [128, 128],
+                                torch.from_numpy(ws).to(dev), bias=bias.to(dev))
+    assert torch.equal(got.cpu(), want)

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 def test_few_blocks_with_k_cut_between_waves_exact(dev, sizes, top_k, N, K, dtype):
     """One, two and four waves along n, a K that the waves do not divide, a last strip of 8 weight rows, blocks of one slot and full
     ones, an expert with several blocks and one without slots, slots of another rank's expert (stored as zeros), routed weights on and off, activation
-    scales by row and by column.  Integers below 2^11 times powers of two, exact in float32 in any order of the sums."""
+    scales by row and by column.  Integers below 2^11 times powers of two, exact in float32 in any order of the sums.  K = 1024, 2048 weight
+    rows and the first sizes with top_k = 1 and K = 1152 are past the lines of the rule: the kernel with tiles, the same results."""
     from sglang_amd.fused_moe import moe_align_block_size
     from sglang_amd.sgl_kernel import moe_block_gemm
 
