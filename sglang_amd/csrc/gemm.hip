@@ -233,10 +233,11 @@ static double est_tile128(int64_t M, int64_t N, int kb, int cu, int* best_splits
 // The same for tiles of 64 x 64, as many as the chip has CUs at most (one round), more than 64 rows and more than eight K blocks (up
 // to eight they are level with the larger tiles, 0.95 - 1.05): a wave runs 0.9 us per K block of its own, every fourth of the range, and
 // more where the weights come out of HBM for this tile alone and the chip is full.  Fitted to 137 pairs of shape and K cut (65 .. 1150
-// rows, N = 512 .. 9856, K = 896 .. 17664; rms error 6 %).  On 68 such shapes the choice between all tiles is 0.2 % behind the best
-// and 7 % ahead of the larger tiles alone (up to 23 %; whole linears, us, replayed from a graph, weights out of HBM / out of the
-// last-level cache: 238 x 3456 x 3072 18.1 -> 14.3 / 14.7 -> 12.8, 159 x 4288 x 4224 20.8 -> 16.2 / 17.4 -> 14.1, 73 x 576 x 2688
-// 14.6 -> 11.0 / 13.8 -> 10.4, 411 x 1024 x 3200 15.8 -> 13.6 / 15.7 -> 13.3).
+// rows, N = 512 .. 9856, K = 896 .. 17664; rms error 6 %).  On 105 other such shapes, even over the logarithm of 65 .. 1300 rows, N up
+// to 12000 and K up to 18000, the GEMM takes 0.92 (0.73 - 1.00) of the time that the larger tiles and the strips took there with
+// weights out of HBM, 0.88 (0.73 - 1.04) out of the last-level cache; whole linears, us, replayed from a graph, HBM / cache: 238 x 3456 x
+// 3072 18.2 -> 14.5 / 13.1 -> 10.8, 159 x 4288 x 4224 20.8 -> 16.4 / 15.8 -> 12.4, 73 x 576 x 2688 13.9 -> 11.6 / 13.3 -> 10.2, 411 x 1024 x
+// 3200 15.6 -> 13.3 / 14.7 -> 12.5, 128 x 4096 x 4096 18.1 -> 16.4 / 15.7 -> 11.2.
 static double est_tile64(int64_t M, int64_t N, int kb, int cu, int* best_splits) {
   double best = 1e30;
   const int64_t tm = (M + kT64 - 1) / kT64, tiles = tm * ((N + kT64 - 1) / kT64);

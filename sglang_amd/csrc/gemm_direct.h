@@ -390,7 +390,8 @@ __global__ __launch_bounds__(512, 2) void gemm_wavek_kernel(const GemmArgs p) {
 // 128 x K bytes each.  Here a workgroup owns 16 * NW rows of a block's expert and its waves cut K.  The block's rows and the slots
 // they go to come from the slot table; workgroups of a block are dealt over all XCDs, so a weight line is read once per block of its
 // expert.  Bound by the latency of the first lines and by launch: the first GEMM of one token, 8 experts of 512 x 7168 (29 MB, 5 us at
-// the copy rate) 19.9 -> 8.0 us, 4 experts of 1024 x 4096 13.8 -> 6.7.  Eight K blocks in flight per wave are level to 10 % slower.
+// the copy rate) 21.0 -> 8.8 us, 4 experts of 1024 x 4096 13.4 -> 7.3, weights out of HBM.  Eight K blocks in flight per wave are level to
+// 10 % slower.
 // The grid is sized for the blocks that a table aligned over the launch's own experts can have in use; a table may have more (blocks of
 // other ranks' experts, blocks without slots), so a workgroup goes on by that number of blocks.  The loop costs 2 % (0.1 - 0.2 us).
 // ------------------------------------------------------------------------------------------------

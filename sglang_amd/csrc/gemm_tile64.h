@@ -5,8 +5,9 @@
 // 16x16x128 per block, eight operand fragments for them out of LDS), its loads go to LDS that nobody else touches, and no barrier
 // stands in the K loop.  The four sums meet in LDS at the end, in ascending order.
 //
-// Bound: the CU's load path.  A block is 16 KB for 128 clocks of matrix-core time per SIMD and wave; with one tile per CU it takes 0.19
-// us (86 bytes a ns; 0.10 without the loads; plain loads of the same rows out of L2 reach 120 - 150).  Measured, and no faster: loads
+// Bound: the CU's load path.  A block is 16 KB for 512 clocks of its wave's matrix core, so 128 clocks per block with the four waves at
+// work; with one tile per CU it takes 0.24 us (69 bytes a ns: 1024 x 1024 x 4096 / 8192 / 16384 12.1 / 19.8 / 35.0 us), for a tile alone on
+// the chip 0.13 (64 x 64: 8.5 / 12.8 / 21.0), where plain loads of such rows out of L2 reach 120 - 150.  Measured, and no faster: loads
 // straight into operand registers (half lines: 2.4 times the time), eight waves with one block each in LDS, weights two blocks ahead
 // instead of one, the operands landing in registers and shared by eight waves through LDS (a barrier per four blocks).
 //
